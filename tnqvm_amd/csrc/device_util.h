@@ -29,22 +29,50 @@ __device__ __forceinline__ double2 cfmac(double2 a, double2 b, double2 c) {
 }
 __device__ __forceinline__ double cabs2(double2 a) { return a.x * a.x + a.y * a.y; }
 
+// Loads and stores through a pointer that came out of a task descriptor.  The compiler cannot tell
+// which memory such a pointer names and emits flat accesses, which count as LDS accesses too and
+// complete in no known order, so that every wait on an LDS read also waits for every load in flight.
+// These go through the global address space.
+typedef double gvec_d2 __attribute__((ext_vector_type(2)));
+typedef float gvec_f2 __attribute__((ext_vector_type(2)));
+#define HIPMPS_GLOBAL __attribute__((address_space(1)))
+__device__ __forceinline__ double2 gld(const double2* p) {
+  const gvec_d2 v = *(const HIPMPS_GLOBAL gvec_d2*)p;
+  return make_double2(v.x, v.y);
+}
+__device__ __forceinline__ float2 gld(const float2* p) {
+  const gvec_f2 v = *(const HIPMPS_GLOBAL gvec_f2*)p;
+  return make_float2(v.x, v.y);
+}
+__device__ __forceinline__ void gst(double2* p, double2 v) {
+  gvec_d2 x;
+  x.x = v.x;
+  x.y = v.y;
+  *(HIPMPS_GLOBAL gvec_d2*)p = x;
+}
+__device__ __forceinline__ void gst(float2* p, float2 v) {
+  gvec_f2 x;
+  x.x = v.x;
+  x.y = v.y;
+  *(HIPMPS_GLOBAL gvec_f2*)p = x;
+}
+
 template <typename T>
 __device__ __forceinline__ double2 ld(const T* p, size_t i);
 template <>
-__device__ __forceinline__ double2 ld<double2>(const double2* p, size_t i) { return p[i]; }
+__device__ __forceinline__ double2 ld<double2>(const double2* p, size_t i) { return gld(p + i); }
 template <>
 __device__ __forceinline__ double2 ld<float2>(const float2* p, size_t i) {
-  float2 v = p[i];
+  const float2 v = gld(p + i);
   return make_double2((double)v.x, (double)v.y);
 }
 template <typename T>
 __device__ __forceinline__ void st(T* p, size_t i, double2 v);
 template <>
-__device__ __forceinline__ void st<double2>(double2* p, size_t i, double2 v) { p[i] = v; }
+__device__ __forceinline__ void st<double2>(double2* p, size_t i, double2 v) { gst(p + i, v); }
 template <>
 __device__ __forceinline__ void st<float2>(float2* p, size_t i, double2 v) {
-  p[i] = make_float2((float)v.x, (float)v.y);
+  gst(p + i, make_float2((float)v.x, (float)v.y));
 }
 
 // Largest t with begin(t) <= b, for task arrays sorted by their first block.

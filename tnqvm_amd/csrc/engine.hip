@@ -190,7 +190,6 @@ struct hipmps_engine_s {
   int max_sweeps = 40;
   double tol = 1e-13;       // FP64 path: relative orthogonality of converged rows
   double tol_mixed = 1e-8;  // mixed path: factors are stored in complex64
-  int inner_sweeps = 1;
   int debug_sweeps = 0;  // HIPMPS_DEBUG_SWEEPS: per-sweep rotated / visited block pairs on stderr
   int lq_min_rank = 64;  // Jacobi on the double-LQ factor when min(m, n) >= this (0: never)
   // LQ with look-ahead (next panel factored in LDS on one stream while the trailing rows update
@@ -989,8 +988,8 @@ int run_wave(hipmps_engine E, std::vector<WaveItem>& items) {
     for (int round = 0; round < max_rounds; ++round)
       for (int l = 0; l < lanes; ++l)
         if (lane_n[l] > 0 && round < lane_rounds[l])
-          HIP_TRY(launch_jacobi_round(djt + lane_begin[l], lane_n[l], lane_pairs[l], round, E->inner_sweeps,
-                                      E->lane_stream[l], true));
+          HIP_TRY(launch_jacobi_round(djt + lane_begin[l], lane_n[l], lane_pairs[l], round, E->lane_stream[l],
+                                      true));
     for (int l = 1; l < lanes; ++l) {
       HIP_TRY(hipEventRecord(E->lane_ev[l], E->lane_stream[l]));
       HIP_TRY(hipStreamWaitEvent(st, E->lane_ev[l], 0));
@@ -1389,7 +1388,7 @@ int run_kraus_waves(hipmps_engine E, const std::vector<hipmps_state_s*>& states)
     HIP_TRY(hipMemcpyAsync(djt, hja, active.size() * sizeof(JacTask), hipMemcpyHostToDevice, st));
     HIP_TRY(hipMemsetAsync(d_counts, 0, 2 * (size_t)C * sizeof(int), st));
     for (int round = 0; round < rounds; ++round)
-      HIP_TRY(launch_jacobi_round(djt, (int)active.size(), pairs, round, E->inner_sweeps, st));
+      HIP_TRY(launch_jacobi_round(djt, (int)active.size(), pairs, round, st));
     HIP_TRY(hipMemcpyAsync(hcount, d_counts, 2 * (size_t)C * sizeof(int), hipMemcpyDeviceToHost, st));
     HIP_TRY(hipStreamSynchronize(st));
     std::vector<int> next;

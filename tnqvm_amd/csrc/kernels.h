@@ -163,8 +163,8 @@ hipError_t launch_jacobi_prep(const SplitTask* d_split, const JacTask* d_jac, in
 constexpr double JAC_FLOOR2 = 1e-30;
 // *jt[t].fro2 = ||theta'_t||_F^2 (= ||X||_F^2 = ||R2||_F^2), one workgroup per task, fixed order
 hipError_t launch_fro2(const SplitTask* d_split, const JacTask* d_jac, int ntasks, hipStream_t s);
-hipError_t launch_jacobi_round(const JacTask* d_tasks, int ntasks, int total_pairs, int round,
-                               int inner_sweeps, hipStream_t s, bool tiled = false);
+hipError_t launch_jacobi_round(const JacTask* d_tasks, int ntasks, int total_pairs, int round, hipStream_t s,
+                               bool tiled = false);
 // Y (row-major, ldy) <-> Yt (tiled, ntc) for every task: rows [0, r_pad), columns [0, c_tot);
 // to_tiles writes zeros into the tile columns past c_tot.  max_blocks = largest r_pad / 16.
 hipError_t launch_to_tiles(const JacTask* d_tasks, int ntasks, int max_blocks, int max_ntc, hipStream_t s);

@@ -250,47 +250,249 @@ __device__ __forceinline__ double nr_rcp(double d) {
 // Rotation that annihilates gamma in the Hermitian 2x2 [[alpha, gamma], [conj(gamma), beta]]
 // (Golub & Van Loan Alg. 8.4.1 with a phase): h = beta - alpha,
 // tau = 2 sign(h) gamma / (|h| + sqrt(h^2 + 4|gamma|^2))  (|tau| = t, the smaller root),
-// c = 1/sqrt(1 + |tau|^2), se = c tau;  J = [[c, se], [-conj(se), c]].
-// Returns the identity when |gamma| <= tol sqrt(alpha beta) or a diagonal entry is 0.
-__device__ __forceinline__ void jacobi_rotation(double alpha, double beta, double2 gamma, double tol, double floor2,
-                                                double& c, double2& se) {
+// c = 1/sqrt(1 + |tau|^2);  J = c [[1, tau], [-conj(tau), 1]].
+// The rotated diagonal is alpha - f |gamma|^2, beta + f |gamma|^2 with tau = f gamma; it replaces
+// alpha and beta.  The identity when |gamma| <= tol sqrt(alpha beta) or a diagonal entry is 0.
+__device__ __forceinline__ void jacobi_rotation(double& alpha, double& beta, double2 gamma, double tol, double floor2,
+                                                double& c, double2& tau) {
   const double g2 = cabs2(gamma);
   if (!(alpha > floor2) || !(beta > floor2) || !(g2 > tol * tol * alpha * beta)) {
     c = 1.0;
-    se = make_double2(0.0, 0.0);
+    tau = make_double2(0.0, 0.0);
     return;
   }
   const double h = beta - alpha;
   const double a = fma(h, h, 4.0 * g2);
   const double d = fabs(h) + a * nr_rsq(a);
   const double f = (h >= 0.0 ? 2.0 : -2.0) * nr_rcp(d);
-  const double2 tau = make_double2(f * gamma.x, f * gamma.y);
+  tau = make_double2(f * gamma.x, f * gamma.y);
   c = nr_rsq(1.0 + cabs2(tau));
-  se = make_double2(c * tau.x, c * tau.y);
+  alpha = fma(-f, g2, alpha);
+  beta = fma(f, g2, beta);
 }
 
-// Thread -> 2x2 block of rotation pairs (bk, bl) of the inner sweep, packed bk << 4 | bl.  The 16
-// blocks that form the next step's rotations -- (0, 1), (j + 1, j - 1) for 1 <= j <= 14, (15, 14)
-// -- go to threads 0..15 (wave 0), so that the other three waves skip that code; the remaining
-// 240 blocks follow in row order.
-struct InnerBlockMap {
-  unsigned char v[256];
-};
-constexpr bool inner_owner(int bk, int bl) {
-  return (bk == 0 && bl == 1) || (bk >= 2 && bl == bk - 2) || (bk == 15 && bl == 14);
+// A value moved one lane along its row of 16 lanes: from the next lane (lane 15 keeps `edge`) or from
+// the previous one (lane 0 keeps `edge`).
+template <int CTRL>
+__device__ __forceinline__ double dpp_move(double edge, double v) {
+  const long long e = __double_as_longlong(edge), x = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_update_dpp((int)e, (int)x, CTRL, 0xf, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp((int)(e >> 32), (int)(x >> 32), CTRL, 0xf, 0xf, false);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
 }
+__device__ __forceinline__ double2 flip_im(double2 v, int sign) {  // sign: 0, or the sign bit
+  const long long y = __double_as_longlong(v.y) ^ ((long long)sign << 32);
+  return make_double2(v.x, __longlong_as_double(y));
+}
+__device__ __forceinline__ double2 from_next(double2 edge, double2 v) {
+  return make_double2(dpp_move<0x101>(edge.x, v.x), dpp_move<0x101>(edge.y, v.y));  // row_shl:1
+}
+__device__ __forceinline__ double2 from_next_cyclic(double2 v) {  // lane 15 takes lane 0's
+  return make_double2(dpp_move<0x12f>(v.x, v.x), dpp_move<0x12f>(v.y, v.y));  // row_ror:15
+}
+__device__ __forceinline__ double2 from_prev(double2 edge, double2 v) {
+  return make_double2(dpp_move<0x111>(edge.x, v.x), dpp_move<0x111>(edge.y, v.y));  // row_shr:1
+}
+
+// The two orderings of the inner sweep.  G is held by slot: at every step, pair k is slots k and
+// JP-1-k.
+//   full (CROSS = false): the circle ordering, 31 steps, every pair of the 32 rows once.  From one
+//     step to the next a row moves from slot x to x-1, slot 1 to JP-1, slot 0 stays.
+//   cross (CROSS = true): 16 steps, every row of the first block with every row of the second.  The
+//     first block's rows keep their slots k, the second's move from pair k to pair k-1 (mod 16).
+// A sweep over all block pairs that uses the full ordering everywhere rotates the pairs within a
+// block nb-1 times; the cross ordering in most rounds leaves those out (jacobi_full_round).
+template <bool CROSS>
+constexpr int inner_next_slot(int x) {
+  return CROSS ? (x < JB ? x : (x == JP - 1 ? JB : x + 1)) : (x == 0 ? 0 : (x == 1 ? JP - 1 : x - 1));
+}
+
+// The 120 blocks (k, l), k < l, of rotation pairs that the threads 0..119 update, packed k << 4 | l.
+// The next step's pair j is formed from one entry of one block -- full: (0, 1) for pair 0, (j - 1,
+// j + 1), (14, 15) for pair 15; cross: (j, j + 1), (0, 15) for pair 15 -- and these 16 blocks come
+// first (wave 0, so that wave 1 skips the rotation), the others in row order.
+struct InnerBlockMap {
+  unsigned char v[128];
+};
+template <bool CROSS>
+constexpr int inner_owner_block(int j) {
+  const int k = CROSS ? (j < 15 ? j : 0) : (j == 0 ? 0 : j - 1);
+  const int l = CROSS ? (j < 15 ? j + 1 : 15) : (j == 0 ? 1 : (j == 15 ? 15 : j + 1));
+  return k << 4 | l;
+}
+template <bool CROSS>
 constexpr InnerBlockMap make_inner_block_map() {
   InnerBlockMap m{};
-  m.v[0] = (unsigned char)(0 << 4 | 1);
-  for (int j = 1; j <= 14; ++j) m.v[j] = (unsigned char)((j + 1) << 4 | (j - 1));
-  m.v[15] = (unsigned char)(15 << 4 | 14);
-  int n = 16;
-  for (int bk = 0; bk < 16; ++bk)
-    for (int bl = 0; bl < 16; ++bl)
-      if (!inner_owner(bk, bl)) m.v[n++] = (unsigned char)(bk << 4 | bl);
+  int n = 0;
+  for (; n < 16; ++n) m.v[n] = (unsigned char)inner_owner_block<CROSS>(n);
+  for (int k = 0; k < 16; ++k)
+    for (int l = k + 1; l < 16; ++l) {
+      bool owner = false;
+      for (int j = 0; j < 16; ++j) owner = owner || inner_owner_block<CROSS>(j) == (k << 4 | l);
+      if (!owner) m.v[n++] = (unsigned char)(k << 4 | l);
+    }
+  for (; n < 128; ++n) m.v[n] = 1;  // threads 120..127 (see inner_sweep)
   return m;
 }
-__constant__ InnerBlockMap c_inner_blocks = make_inner_block_map();
+__constant__ InnerBlockMap c_inner_full = make_inner_block_map<false>();
+__constant__ InnerBlockMap c_inner_cross = make_inner_block_map<true>();
+
+// Rounds of a sweep whose inner sweep is the full ordering: every 2nd for SVDs of up to 4 blocks,
+// every 4th up to 14, every 8th above.  In an emulation on preconditioned 64 x 64 to 256 x 256
+// matrices (random, and theta' of decaying spectra; tolerances 1e-13 and 1e-8) these periods keep
+// the sweep count within one of the full ordering's with 16 to 41% fewer inner steps; once a sweep
+// takes one more sweep, and twice as often gains nothing.
+__device__ __forceinline__ bool jacobi_full_round(int round, int nb) {
+  return round % (nb <= 4 ? 2 : (nb < 16 ? 4 : 8)) == 0;
+}
+
+struct InnerShared {
+  double2 G[2][JP][JP + 1];
+  double2 tau[2][JB];  // rotations of the current / next step
+  double c[2][JB];
+  double d[2][JP];     // diagonal by slot, rotated
+  int rot[4];          // per wave: an entry of the Gram is above the tolerance
+};
+
+// One cyclic two-sided Jacobi sweep on the Hermitian S.G[0]; leaves W (its rotations) in S.G[0].
+// Waves 0 and 1 hold one 2x2 block each of rotation pairs k < l (the other half is its conjugate,
+// a rotated diagonal block is diag(d) with a zero off-diagonal entry), waves 2 and 3 hold W.
+template <bool CROSS>
+__device__ __forceinline__ void inner_sweep(InnerShared& S, double itol, double floor2) {
+  const int tid = threadIdx.x, wave = tid >> 6, l16 = tid & 15;
+  if (tid < JB) {
+    double alpha = S.G[0][tid][tid].x, beta = S.G[0][JP - 1 - tid][JP - 1 - tid].x, c;
+    double2 tau;
+    jacobi_rotation(alpha, beta, S.G[0][tid][JP - 1 - tid], itol, floor2, c, tau);
+    S.c[0][tid] = c;
+    S.tau[0][tid] = tau;
+    S.d[0][tid] = alpha;
+    S.d[0][JP - 1 - tid] = beta;
+  }
+  __syncthreads();
+  constexpr int STEPS = CROSS ? JB : JP - 1;
+  constexpr int LDG = JP + 1;
+  if (wave < 2) {
+    const int blk = CROSS ? c_inner_cross.v[tid] : c_inner_full.v[tid];
+    const int bk = blk >> 4, bl = blk & 15;
+    // where this thread's four entries go: the next step's slots, in the half with the smaller pair
+    // first, conjugated (sign bit) where that swaps row and column.  The entry that becomes a
+    // pair's own off-diagonal goes to the unused column JP.  Threads 120..127 write the zeros that
+    // the rotated off-diagonal entries of two pairs each become.
+    const bool zeros = tid >= 120;
+    int dst[4], flip[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      int x = (e & 2) ? JP - 1 - bk : bk, y = (e & 1) ? JP - 1 - bl : bl;
+      if (zeros) {
+        x = 2 * (tid - 120) + (e & 1);
+        y = JP - 1 - x;
+      }
+      const int dx = inner_next_slot<CROSS>(x), dy = inner_next_slot<CROSS>(y);
+      const int px = dx < JB ? dx : JP - 1 - dx, py = dy < JB ? dy : JP - 1 - dy;
+      dst[e] = px == py ? dx * LDG + JP : (px < py ? dx * LDG + dy : dy * LDG + dx);
+      flip[e] = px > py ? (int)0x80000000 : 0;
+    }
+    // owners (threads 0..15): slots of the next pair's members, which entry of the block couples
+    // them and whether it is stored conjugated
+    const bool owner = tid < JB;
+    int xa, xb;
+    bool conj_g, e10 = false, e11 = false;
+    if (CROSS) {
+      xa = tid & 15;
+      xb = JP - 1 - ((tid + 1) & 15);
+      e10 = conj_g = tid == 15;
+    } else {
+      xa = tid == 0 ? 0 : (tid == 15 ? JB : (tid + 1) & 15);
+      xb = tid == 0 ? 1 : JP - 1 - ((tid - 1) & 15);
+      conj_g = tid != 0;
+      e11 = tid == 15;
+      e10 = conj_g && !e11;
+    }
+    double2* gA = &S.G[0][0][0];
+    double2* gB = &S.G[1][0][0];
+    const int pk = bk * LDG, qk = (JP - 1 - bk) * LDG, pl = bl, ql = JP - 1 - bl;
+#pragma unroll 1
+    for (int st = 0; st < STEPS; ++st) {
+      const int buf = st & 1;
+      const double2 tl = S.tau[buf][bl];
+      const double2 b00 = gA[pk + pl], b01 = gA[pk + ql], b10 = gA[qk + pl], b11 = gA[qk + ql];
+      const double2 tk = S.tau[buf][bk];
+      const double ck = S.c[buf][bk], cl = S.c[buf][bl];
+      double alpha = 0.0, beta = 0.0;
+      if (wave == 0) {
+        alpha = S.d[buf][xa];
+        beta = S.d[buf][xb];
+      }
+      const double rho = zeros ? 0.0 : ck * cl;
+      // block B' = Jk^H B Jl
+      const double2 ntl = make_double2(-tl.x, tl.y);
+      const double2 m00 = cfma(b01, ntl, b00), m01 = cfma(b00, tl, b01);
+      const double2 m10 = cfma(b11, ntl, b10), m11 = cfma(b10, tl, b11);
+      const double2 ntk = make_double2(-tk.x, -tk.y), ctk = cconj(tk);
+      const double2 n00 = cscale(cfma(ntk, m10, m00), rho), n01 = cscale(cfma(ntk, m11, m01), rho);
+      const double2 n10 = cscale(cfma(ctk, m00, m10), rho), n11 = cscale(cfma(ctk, m01, m11), rho);
+      gB[dst[0]] = flip_im(n00, flip[0]);
+      gB[dst[1]] = flip_im(n01, flip[1]);
+      gB[dst[2]] = flip_im(n10, flip[2]);
+      gB[dst[3]] = flip_im(n11, flip[3]);
+      if (wave == 0) {  // the next step's rotations
+        double cn;
+        double2 tau;
+        double2 gam = CROSS ? (e10 ? n10 : n01) : (e10 ? n10 : (e11 ? n11 : n00));
+        gam = flip_im(gam, conj_g ? (int)0x80000000 : 0);
+        jacobi_rotation(alpha, beta, gam, itol, floor2, cn, tau);
+        if (owner) {
+          S.tau[buf ^ 1][tid] = tau;
+          S.c[buf ^ 1][tid] = cn;
+          S.d[buf ^ 1][tid] = alpha;
+          S.d[buf ^ 1][JP - 1 - tid] = beta;
+        }
+      }
+      __syncthreads();
+      double2* tmp = gA;
+      gA = gB;
+      gB = tmp;
+    }
+    __syncthreads();  // W is in place
+  } else {
+    // W rows wr .. wr + 3 at slots l16 (t) and JP-1-l16 (b)
+    const int wr = 4 * ((tid - 128) >> 4);
+    double2 t[4], b[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      t[i] = make_double2(wr + i == l16 ? 1.0 : 0.0, 0.0);
+      b[i] = make_double2(wr + i == JP - 1 - l16 ? 1.0 : 0.0, 0.0);
+    }
+#pragma unroll 1
+    for (int st = 0; st < STEPS; ++st) {
+      const double c = S.c[st & 1][l16];
+      const double2 tau = S.tau[st & 1][l16], ntau = make_double2(-tau.x, tau.y);
+      // W' = W J, then to the next step's slots; full: the top slot of pair k takes pair k + 1's top
+      // (pair 15: its own bottom, pair 0 keeps its top), the bottom slot pair k - 1's bottom (pair
+      // 0: pair 1's top)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const double2 u = cscale(cfma(b[i], ntau, t[i]), c), d = cscale(cfma(t[i], tau, b[i]), c);
+        if (CROSS) {
+          t[i] = u;
+          b[i] = from_next_cyclic(d);
+        } else {
+          const double2 x = from_next(d, u);
+          b[i] = from_prev(x, d);
+          t[i] = l16 == 0 ? u : x;
+        }
+      }
+      __syncthreads();
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      S.G[0][wr + i][l16] = t[i];
+      S.G[0][wr + i][JP - 1 - l16] = b[i];
+    }
+    __syncthreads();
+  }
+}
 
 // Design notes (gfx950):
 //  * Gram and apply stream their MFMA operands straight from memory into registers; no
@@ -299,26 +501,29 @@ __constant__ InnerBlockMap c_inner_blocks = make_inner_block_map();
 //    four partial Grams are summed once in LDS.
 //  * In the apply each wave owns whole 32-row x 16-column tiles, so the in-place update
 //    never overwrites a column another wave still reads.
-//  * Inner sweep: thread (k, l) owns the 2x2 block of rotation pairs k and l, updates it
-//    two-sided in one pass (B' = Jk^H B Jl, G double-buffered in LDS), updates two W
-//    entries pairs, and -- when the next step's pair (p', q') has p' in pair k and q' in
-//    pair l -- also forms that pair's rotation from values it already holds.  One barrier
-//    per step; every LDS read of a step is issued before any arithmetic.
-//    In the circle ordering the pair owner is static: next pair 0 <- (0,1), next pair j
-//    <- (j+1, j-1) for 1 <= j <= 14, next pair 15 <- (15,14); and each row index moves
-//    to x+1 (31 -> 1) from one step to the next, except row 0.
+//  * Inner sweep: a thread owns the 2x2 block of rotation pairs k < l and updates it two-sided
+//    in one pass (B' = Jk^H B Jl, G double-buffered in LDS); when an entry of it couples the
+//    members of a next step's pair, it also forms that pair's rotation from values it already
+//    holds and the rotated diagonal entries, which travel with the rotations.  One barrier per
+//    step; every LDS read of a step is issued before any arithmetic.  Each step writes its
+//    rotated blocks where the next step reads them, so every G address is fixed per thread; after
+//    the last step the slots are back in row order.
+//  * W stays in registers of two waves of its own, each thread four rows at the two slots of one
+//    pair: the slots' move to the next step is a shift by one lane within a row of 16 lanes.
+//  A step is bound by its serial chain (LDS read, block update, rotation, LDS write, barrier) and
+//  by LDS bandwidth: the whole G and W in LDS (20 16-byte accesses a thread and step, all four
+//  waves) took 1590 clocks a step, a half of G on two waves and W in registers 1200.
+//  Measured, 768 workgroups on 32 rows x 512 columns (three per CU): 156 us a launch before
+//  (inner sweep 93k clocks), 142 us with the full ordering, 126 us with the cross one, which is
+//  4.8 TB/s over its three passes; one workgroup alone on 32 x 32: 32 us before, 26 and 18 us.
 // BLK is the block size JB (a template parameter: the kernel's register allocation on
-// gfx950 comes out at 150 VGPRs, three waves per SIMD, in this form).
+// gfx950 comes out at 168 VGPRs, three waves per SIMD, in the tiled form).
 template <int BLK, bool TILED>
-__global__ __launch_bounds__(256, 2) void k_jacobi_round(const JacTask* tasks, int ntasks, int round,
-                                                         int inner_sweeps) {
+__global__ __launch_bounds__(256, 2) void k_jacobi_round(const JacTask* tasks, int ntasks, int round) {
   static_assert(BLK == 16 && JB == BLK && JP == 2 * BLK, "256 threads map onto 16 x 16 rotation-pair blocks");
-  __shared__ double2 sG[JP][JP + 1];
-  __shared__ double2 sG2[JP][JP + 1];
-  __shared__ double2 sW[JP][JP + 1];
-  __shared__ double s_c[2][JP / 2 + 1];  // rotations of the current / next step;
-  __shared__ double2 s_se[2][JP / 2 + 1];  // entry JP/2 takes the writes of non-owners
-  __shared__ double s_red[4];  // per-wave maxima of the convergence test
+  __shared__ InnerShared S;
+  double2 (*sG)[JP + 1] = S.G[0];
+  double2 (*sG2)[JP + 1] = S.G[1];
 
   const int t = find_task(tasks, ntasks, (int)blockIdx.x, [](const JacTask& x) { return x.pair_begin; });
   const JacTask& T = tasks[t];
@@ -335,23 +540,26 @@ __global__ __launch_bounds__(256, 2) void k_jacobi_round(const JacTask* tasks, i
   const int tid = threadIdx.x;
   const int wave = tid >> 6, lane = tid & 63;
   const int l16 = lane & 15, k4 = lane >> 4;
-  // element (row, col) of the pair's rows; row-major: row * ld + col
-  auto at = [&](int row, int col) -> size_t {
-    return TILED ? jac_tile_offset(row, col, ntc) : (size_t)row * ld + col;
-  };
+  // element (row, col) of the row-major layout
+  auto at = [&](int row, int col) -> size_t { return (size_t)row * ld + col; };
   const int rowa = ba * JB + l16, rowb = bb * JB + l16;  // pair rows l16 and 16 + l16
 
   // ---- Gram tiles (0,0), (0,1), (1,1) over this wave's 4-column units u = wave, wave + 4, ... ----
   // FP64 MFMA, or in the early sweeps of large SVDs FP32 MFMA at twice the rate: the rotations
   // they give are still applied in FP64 and are unitary, so the rows only lose the accuracy of
-  // the rotation angles, which the FP64 sweeps that end every SVD make up for
-  const int nu = (C + 3) >> 2;
+  // the rotation angles, which the FP64 sweeps that end every SVD make up for.
+  // Tiled rows (c = c_tot, the last tile's missing columns zero): unit wave + 4 d is the wave's
+  // quarter of tile d, so both operands advance by one tile a step; row-major rows are bounded by
+  // their columns.
+  const int nd = TILED ? ntc : (((C + 3) >> 2) + 3) >> 2;
+  const double2* ga = TILED ? Y + (size_t)ba * ntc * 256 + (l16 >> 2) * 64 + wave * 16 + (l16 & 3) * 4 + k4 : Y;
+  const double2* gb = TILED ? Y + (size_t)bb * ntc * 256 + (l16 >> 2) * 64 + wave * 16 + (l16 & 3) * 4 + k4 : Y;
   constexpr int PD = 2;
-  auto ld_unit = [&](int u, double2& v0, double2& v1) {
-    const int col = 4 * u + k4;
-    if (u < nu && col < C) {
-      v0 = Y[at(rowa, col)];
-      v1 = Y[at(rowb, col)];
+  auto ld_unit = [&](int d, double2& v0, double2& v1) {
+    const int col = 4 * (wave + 4 * d) + k4;
+    if (TILED ? d < nd : col < C) {
+      v0 = gld(TILED ? ga + (size_t)d * 256 : Y + at(rowa, col));
+      v1 = gld(TILED ? gb + (size_t)d * 256 : Y + at(rowb, col));
     } else {
       v0 = make_double2(0, 0);
       v1 = make_double2(0, 0);
@@ -368,12 +576,13 @@ __global__ __launch_bounds__(256, 2) void k_jacobi_round(const JacTask* tasks, i
     mfma_d4 k1 = {0, 0, 0, 0}, k2 = {0, 0, 0, 0}, k3 = {0, 0, 0, 0};
     double2 x0[PD], x1[PD];
 #pragma unroll
-    for (int d = 0; d < PD; ++d) ld_unit(wave + 4 * d, x0[d], x1[d]);
-    for (int u0 = wave; u0 < nu; u0 += 4 * PD) {
+    for (int d = 0; d < PD; ++d) ld_unit(d, x0[d], x1[d]);
+#pragma unroll 1
+    for (int e0 = 0; e0 < nd; e0 += PD) {
 #pragma unroll
       for (int d = 0; d < PD; ++d) {
         const double2 v0 = x0[d], v1 = x1[d];
-        ld_unit(u0 + 4 * (d + PD), x0[d], x1[d]);
+        ld_unit(e0 + d + PD, x0[d], x1[d]);
         a00r = mfma64(v0.x, v0.x, a00r);
         a11r = mfma64(v1.x, v1.x, a11r);
         a00x = mfma64(v0.x, v0.y, a00x);
@@ -386,8 +595,9 @@ __global__ __launch_bounds__(256, 2) void k_jacobi_round(const JacTask* tasks, i
       }
     }
     // f64 D[i][j]: lane j + 16 (i % 4), register i / 4
-    for (int w = 0; w < 4; ++w) {
-      if (wave == w) {
+    for (int w = 0; w < 4; w += 2) {  // waves 0, 1 store, then 2, 3 add: two partial sums
+      if ((wave & 2) == w) {
+        double2 (*P)[JP + 1] = S.G[wave & 1];
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
           const int i = 4 * v + k4, j = l16;
@@ -395,13 +605,13 @@ __global__ __launch_bounds__(256, 2) void k_jacobi_round(const JacTask* tasks, i
           double2 g01 = make_double2(k1[v] - k3[v], k1[v] + k2[v]);
           double2 g11 = make_double2(a11r[v], a11x[v]);
           if (w) {
-            g00 = cadd(g00, sG[i][j]);
-            g01 = cadd(g01, sG[i][JB + j]);
-            g11 = cadd(g11, sG[JB + i][JB + j]);
+            g00 = cadd(g00, P[i][j]);
+            g01 = cadd(g01, P[i][JB + j]);
+            g11 = cadd(g11, P[JB + i][JB + j]);
           }
-          sG[i][j] = g00;
-          sG[i][JB + j] = g01;
-          sG[JB + i][JB + j] = g11;
+          P[i][j] = g00;
+          P[i][JB + j] = g01;
+          P[JB + i][JB + j] = g11;
         }
       }
       __syncthreads();
@@ -412,12 +622,13 @@ __global__ __launch_bounds__(256, 2) void k_jacobi_round(const JacTask* tasks, i
     mfma_f4 h1 = {0, 0, 0, 0}, h2 = {0, 0, 0, 0}, h3 = {0, 0, 0, 0};
     double2 x0[PD], x1[PD];
 #pragma unroll
-    for (int d = 0; d < PD; ++d) ld_unit(wave + 4 * d, x0[d], x1[d]);
-    for (int u0 = wave; u0 < nu; u0 += 4 * PD) {
+    for (int d = 0; d < PD; ++d) ld_unit(d, x0[d], x1[d]);
+#pragma unroll 1
+    for (int e0 = 0; e0 < nd; e0 += PD) {
 #pragma unroll
       for (int d = 0; d < PD; ++d) {
         const float p0 = (float)x0[d].x, q0 = (float)x0[d].y, p1 = (float)x1[d].x, q1 = (float)x1[d].y;
-        ld_unit(u0 + 4 * (d + PD), x0[d], x1[d]);
+        ld_unit(e0 + d + PD, x0[d], x1[d]);
         b00r = __builtin_amdgcn_mfma_f32_16x16x4f32(p0, p0, b00r, 0, 0, 0);
         b11r = __builtin_amdgcn_mfma_f32_16x16x4f32(p1, p1, b11r, 0, 0, 0);
         b00x = __builtin_amdgcn_mfma_f32_16x16x4f32(p0, q0, b00x, 0, 0, 0);
@@ -431,8 +642,9 @@ __global__ __launch_bounds__(256, 2) void k_jacobi_round(const JacTask* tasks, i
     }
     // f32 D[i][j]: lane j + 16 (i / 4), register i % 4; the four waves' partial tiles are
     // summed in FP64
-    for (int w = 0; w < 4; ++w) {
-      if (wave == w) {
+    for (int w = 0; w < 4; w += 2) {  // waves 0, 1 store, then 2, 3 add: two partial sums
+      if ((wave & 2) == w) {
+        double2 (*P)[JP + 1] = S.G[wave & 1];
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
           const int i = 4 * k4 + v, j = l16;
@@ -440,168 +652,78 @@ __global__ __launch_bounds__(256, 2) void k_jacobi_round(const JacTask* tasks, i
           double2 g01 = make_double2((double)h1[v] - (double)h3[v], (double)h1[v] + (double)h2[v]);
           double2 g11 = make_double2((double)b11r[v], (double)b11x[v]);
           if (w) {
-            g00 = cadd(g00, sG[i][j]);
-            g01 = cadd(g01, sG[i][JB + j]);
-            g11 = cadd(g11, sG[JB + i][JB + j]);
+            g00 = cadd(g00, P[i][j]);
+            g01 = cadd(g01, P[i][JB + j]);
+            g11 = cadd(g11, P[JB + i][JB + j]);
           }
-          sG[i][j] = g00;
-          sG[i][JB + j] = g01;
-          sG[JB + i][JB + j] = g11;
+          P[i][j] = g00;
+          P[i][JB + j] = g01;
+          P[JB + i][JB + j] = g11;
         }
       }
       __syncthreads();
     }
   }
   {
-    // Im of the diagonal tiles from X (X[i][j] - X[j][i]), and the lower off-diagonal tile
+    // the two partial sums; Im of the diagonal tiles from X (X[i][j] - X[j][i]), and the lower
+    // off-diagonal tile
     const int i = tid >> 4, j = tid & 15;
-    const double x00 = sG[i][j].y - sG[j][i].y, x11 = sG[JB + i][JB + j].y - sG[JB + j][JB + i].y;
-    const double2 g10 = cconj(sG[j][JB + i]);
+    const double2 g00 = cadd(sG[i][j], sG2[i][j]), g11 = cadd(sG[JB + i][JB + j], sG2[JB + i][JB + j]);
+    const double y00 = sG[j][i].y + sG2[j][i].y, y11 = sG[JB + j][JB + i].y + sG2[JB + j][JB + i].y;
+    const double2 g01 = cadd(sG[i][JB + j], sG2[i][JB + j]), g10 = cadd(sG[j][JB + i], sG2[j][JB + i]);
     __syncthreads();
-    sG[i][j].y = x00;
-    sG[JB + i][JB + j].y = x11;
-    sG[JB + i][j] = g10;
+    sG[i][j] = make_double2(g00.x, g00.y - y00);
+    sG[JB + i][JB + j] = make_double2(g11.x, g11.y - y11);
+    sG[i][JB + j] = g01;
+    sG[JB + i][j] = cconj(g10);
   }
   __syncthreads();
-  // ---- convergence test of this block pair: max |G_ij|^2 / (G_ii G_jj) over i != j ----
+  // ---- convergence test of this block pair: |G_ij|^2 > tol^2 G_ii G_jj for some i < j ----
   {
-    double m = 0.0;
+    int above = 0;
+    const double tol2 = tol * tol;
     for (int e = tid; e < JP * JP; e += 256) {
-      int i = e / JP, j = e % JP;
-      if (i == j) continue;
-      double aii = sG[i][i].x, ajj = sG[j][j].x;
-      if (aii > floor2 && ajj > floor2) m = fmax(m, cabs2(sG[i][j]) / (aii * ajj));
+      const int i = e / JP, j = e % JP;
+      const double aii = sG[i][i].x, ajj = sG[j][j].x;
+      if (i < j && aii > floor2 && ajj > floor2 && cabs2(sG[i][j]) > tol2 * (aii * ajj)) above = 1;
     }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) m = fmax(m, __shfl_xor(m, o, 64));
-    if (lane == 0) s_red[wave] = m;
+    above = __any(above);
+    if (lane == 0) S.rot[wave] = above;
     __syncthreads();
   }
   if (tid == 0) atomicAdd(T.visited, 1);
-  if (fmax(fmax(s_red[0], s_red[1]), fmax(s_red[2], s_red[3])) <= tol * tol) return;
+  if (!(S.rot[0] | S.rot[1] | S.rot[2] | S.rot[3])) return;
 
   // ---- apply prefetch: this wave's first column tile, all 32 rows ----
-  const int nt = (CT + 15) >> 4;
+  // element (4 kk + k4, column l16 of the tile) of the pair's rows, kk = 0..7
+  const int nt = TILED ? ntc : (CT + 15) >> 4;
+  double2* ya = TILED ? Y + (size_t)ba * ntc * 256 + (l16 >> 2) * 16 + k4 * 4 + (l16 & 3) : Y + at(ba * JB + k4, l16);
+  double2* yb = TILED ? Y + (size_t)bb * ntc * 256 + (l16 >> 2) * 16 + k4 * 4 + (l16 & 3) : Y + at(bb * JB + k4, l16);
+  const size_t step_row = TILED ? 64 : 4 * ld, step_tile = TILED ? 256 : 16;
+  auto ok_tile = [&](int ctile) { return TILED ? ctile < nt : ctile < nt && ctile * 16 + l16 < CT; };
+  auto elem = [&](int kk, int ctile) { return (kk < 4 ? ya + kk * step_row : yb + (kk - 4) * step_row) + ctile * step_tile; };
   double2 bq[8];
-  auto ld_tile = [&](int ctile, double2* b) {
-    const int col = ctile * 16 + l16;
-    const bool ok = ctile < nt && col < CT;
 #pragma unroll
-    for (int kk = 0; kk < 8; ++kk) {
-      const int row = kk * 4 + k4;
-      b[kk] = ok ? Y[at(row < JB ? ba * JB + row : bb * JB + row - JB, col)] : make_double2(0, 0);
-    }
-  };
-  ld_tile(wave, bq);
+  for (int kk = 0; kk < 8; ++kk) bq[kk] = ok_tile(wave) ? gld(elem(kk, wave)) : make_double2(0, 0);
 
-  for (int e = tid; e < JP * JP; e += 256) sW[e / JP][e % JP] = make_double2((e / JP) == (e % JP) ? 1.0 : 0.0, 0.0);
-  const double itol = tol * 0.25;
-  if (tid < JP / 2) {
-    const int p = circle_slot(tid, 0, JP), q = circle_slot(JP - 1 - tid, 0, JP);
-    double c;
-    double2 se;
-    jacobi_rotation(sG[p][p].x, sG[q][q].x, sG[p][q], itol, floor2, c, se);
-    s_c[0][tid] = c;
-    s_se[0][tid] = se;
-  }
-  __syncthreads();
-  // ---- inner sweep (one barrier per step) ----
-  // G is held by slot: at every step, pair k is rows k and JP-1-k of the buffer.  Each step
-  // writes its rotated 2x2 blocks where the next step reads them (a row moves from slot x to
-  // x-1, slot 1 to JP-1, slot 0 stays), so every G address is fixed per thread; after JP-1
-  // steps the slots are back in row order.  W stays in row order (single buffer).
-  const int blk = c_inner_blocks.v[tid];
-  const int bk = blk >> 4, bl = blk & 15;  // G block of rotation pairs bk, bl
-  const int wi = tid >> 3, wl = tid & 7;   // W row wi, rotation pairs wl and wl + 8
-  auto nxt = [](int x) { return x == JP - 1 ? 1 : x + 1; };  // row index one step later
-  auto prv = [](int x) { return x == 0 ? 0 : (x == 1 ? JP - 1 : x - 1); };  // slot one step later
-  const int pk = bk, qk = JP - 1 - bk, pl = bl, ql = JP - 1 - bl;
-  const int dpk = prv(pk), dqk = prv(qk), dpl = prv(pl), dql = prv(ql);
-  int pw0 = wl, qw0 = JP - 1 - wl, pw1 = wl + 8, qw1 = JP - 1 - (wl + 8);
-  // next-step pair owned by this thread (jn), and which row of pair bk (rra) and of pair
-  // bl (rrb) its members are
-  int jn = -1, rra = 0, rrb = 0;
-  if (bk == 0 && bl == 1) { jn = 0; rra = 0; rrb = 0; }
-  else if (bk >= 2 && bl == bk - 2) { jn = bk - 1; rra = 0; rrb = 1; }
-  else if (bk == 15 && bl == 14) { jn = 15; rra = 1; rrb = 1; }
-  const int nsteps = inner_sweeps * (JP - 1);
-  double2 (*gA)[JP + 1] = sG;
-  double2 (*gB)[JP + 1] = sG2;
-  const int slot = jn >= 0 ? jn : JP / 2;  // non-owners write a dummy slot
-  for (int st = 0; st < nsteps; ++st) {
-    const int buf = st & 1;
-    // ---- all LDS reads of the step ----
-    const double ck = s_c[buf][bk], cl = s_c[buf][bl];
-    const double2 sek = s_se[buf][bk], sel = s_se[buf][bl];
-    const double2 b00 = gA[pk][pl], b01 = gA[pk][ql], b10 = gA[qk][pl], b11 = gA[qk][ql];
-    const double c2 = s_c[buf][wl], c3 = s_c[buf][wl + 8];
-    const double2 se2 = s_se[buf][wl], se3 = s_se[buf][wl + 8];
-    const double2 w0p = sW[wi][pw0], w0q = sW[wi][qw0], w1p = sW[wi][pw1], w1q = sW[wi][qw1];
-    // ---- block B' = Jk^H B Jl,  J = [[c, se], [-conj(se), c]] ----
-    const double2 nsel = make_double2(-sel.x, sel.y);
-    const double2 m00 = cfma(b01, nsel, cscale(b00, cl)), m01 = cfma(b00, sel, cscale(b01, cl));
-    const double2 m10 = cfma(b11, nsel, cscale(b10, cl)), m11 = cfma(b10, sel, cscale(b11, cl));
-    const double2 nsek = make_double2(-sek.x, -sek.y), csek = cconj(sek);
-    const double2 n00 = cfma(nsek, m10, cscale(m00, ck)), n01 = cfma(nsek, m11, cscale(m01, ck));
-    const double2 n10 = cfma(csek, m00, cscale(m10, ck)), n11 = cfma(csek, m01, cscale(m11, ck));
-    // ---- W' = W J on this thread's two pairs (identity rotations leave W unchanged) ----
-    const double2 v0p = cfma(w0q, make_double2(-se2.x, se2.y), cscale(w0p, c2));
-    const double2 v0q = cfma(w0p, se2, cscale(w0q, c2));
-    const double2 v1p = cfma(w1q, make_double2(-se3.x, se3.y), cscale(w1p, c3));
-    const double2 v1q = cfma(w1p, se3, cscale(w1q, c3));
-    // ---- the next step's rotation: wave 0 (threads 0..15 own one each) ----
-    double cn = 1.0;
-    double2 sen = make_double2(0.0, 0.0);
-    if (wave == 0) {
-      const double ak = gA[pk][pk].x, bk2 = gA[qk][qk].x, al2 = gA[pl][pl].x, bl2 = gA[ql][ql].x;
-      const double2 gk = gA[pk][qk], gl = gA[pl][ql];
-      const double rk = 2.0 * ck * (gk.x * sek.x + gk.y * sek.y);
-      const double ek = cabs2(sek), c2k = ck * ck;
-      const double alpha = rra ? (ek * ak + c2k * bk2 + rk) : (c2k * ak + ek * bk2 - rk);
-      const double rl = 2.0 * cl * (gl.x * sel.x + gl.y * sel.y);
-      const double el = cabs2(sel), c2l = cl * cl;
-      const double beta = rrb ? (el * al2 + c2l * bl2 + rl) : (c2l * al2 + el * bl2 - rl);
-      const double2 gam = rra ? (rrb ? n11 : n10) : (rrb ? n01 : n00);
-      jacobi_rotation(alpha, beta, gam, itol, floor2, cn, sen);
-    }
-    // ---- all LDS writes of the step ----
-    gB[dpk][dpl] = n00;
-    gB[dpk][dql] = n01;
-    gB[dqk][dpl] = n10;
-    gB[dqk][dql] = n11;
-    sW[wi][pw0] = v0p;
-    sW[wi][qw0] = v0q;
-    sW[wi][pw1] = v1p;
-    sW[wi][qw1] = v1q;
-    if (wave == 0) {
-      s_c[buf ^ 1][slot] = cn;
-      s_se[buf ^ 1][slot] = sen;
-    }
-    __syncthreads();
-    double2 (*tmp)[JP + 1] = gA;
-    gA = gB;
-    gB = tmp;
-    if (wl) pw0 = nxt(pw0);
-    qw0 = nxt(qw0);
-    pw1 = nxt(pw1);
-    qw1 = nxt(qw1);
-  }
+  if (jacobi_full_round(round, nb)) inner_sweep<false>(S, tol * 0.25, floor2);
+  else inner_sweep<true>(S, tol * 0.25, floor2);
+  double2 (*sW)[JP + 1] = S.G[0];
 
   // ---- apply Y' = W^T Y; wave owns column tiles wave, wave + 4, ... (all 32 rows) ----
+#pragma unroll 1
   for (int ctile = wave; ctile < nt; ctile += 4) {
     // (A + iB)(C + iD) with three real products (Gauss): K1 = (A + B) C, K2 = A (D - C),
     // K3 = B (C + D); Re = K1 - K3, Im = K1 + K2
     mfma_d4 e0 = {0, 0, 0, 0}, f0 = {0, 0, 0, 0}, g0 = {0, 0, 0, 0};
     mfma_d4 e1 = {0, 0, 0, 0}, f1 = {0, 0, 0, 0}, g1 = {0, 0, 0, 0};
-    const int ncol = (ctile + 4) * 16 + l16;
-    const bool nok = ctile + 4 < nt && ncol < CT;
+    const bool nok = ok_tile(ctile + 4);
 #pragma unroll
     for (int kk = 0; kk < 8; ++kk) {
       const double2 b = bq[kk];
       const double2 w0 = sW[kk * 4 + k4][l16];       // A[i][k] = W[k][i], rows 0..15
       const double2 w1 = sW[kk * 4 + k4][16 + l16];  // rows 16..31
-      const int row = kk * 4 + k4;
-      bq[kk] = nok ? Y[at(row < JB ? ba * JB + row : bb * JB + row - JB, ncol)] : make_double2(0, 0);
+      bq[kk] = nok ? gld(elem(kk, ctile + 4)) : make_double2(0, 0);
       const double dmc = b.y - b.x, cpd = b.x + b.y;
       e0 = mfma64(w0.x + w0.y, b.x, e0);
       e1 = mfma64(w1.x + w1.y, b.x, e1);
@@ -610,12 +732,11 @@ __global__ __launch_bounds__(256, 2) void k_jacobi_round(const JacTask* tasks, i
       g0 = mfma64(w0.y, cpd, g0);
       g1 = mfma64(w1.y, cpd, g1);
     }
-    const int col = ctile * 16 + l16;
-    if (col < CT) {
+    if (ok_tile(ctile)) {
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
-        Y[at(ba * JB + 4 * v + k4, col)] = make_double2(e0[v] - g0[v], e0[v] + f0[v]);
-        Y[at(bb * JB + 4 * v + k4, col)] = make_double2(e1[v] - g1[v], e1[v] + f1[v]);
+        gst(elem(v, ctile), make_double2(e0[v] - g0[v], e0[v] + f0[v]));
+        gst(elem(4 + v, ctile), make_double2(e1[v] - g1[v], e1[v] + f1[v]));
       }
     }
   }
@@ -643,15 +764,13 @@ hipError_t launch_fro2(const SplitTask* d_split, const JacTask* d_jac, int ntask
   return hipGetLastError();
 }
 
-hipError_t launch_jacobi_round(const JacTask* d_tasks, int ntasks, int total_pairs, int round,
-                               int inner_sweeps, hipStream_t s, bool tiled) {
+hipError_t launch_jacobi_round(const JacTask* d_tasks, int ntasks, int total_pairs, int round, hipStream_t s,
+                               bool tiled) {
   if (total_pairs <= 0) return hipSuccess;
   if (tiled)
-    hipLaunchKernelGGL((k_jacobi_round<JB, true>), dim3(total_pairs), dim3(256), 0, s, d_tasks, ntasks, round,
-                       inner_sweeps);
+    hipLaunchKernelGGL((k_jacobi_round<JB, true>), dim3(total_pairs), dim3(256), 0, s, d_tasks, ntasks, round);
   else
-    hipLaunchKernelGGL((k_jacobi_round<JB, false>), dim3(total_pairs), dim3(256), 0, s, d_tasks, ntasks, round,
-                       inner_sweeps);
+    hipLaunchKernelGGL((k_jacobi_round<JB, false>), dim3(total_pairs), dim3(256), 0, s, d_tasks, ntasks, round);
   return hipGetLastError();
 }
 
