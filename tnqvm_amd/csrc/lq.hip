@@ -21,24 +21,42 @@ namespace hipmps {
 
 constexpr int LQB = 16;  // rows per panel (reflectors per block reflector)
 constexpr int LQR = 16;  // rows per MFMA tile in the block-reflector application
+constexpr long long LQ_ONE_STREAM_ROWS = 4096;  // launch_lq_lookahead: rows of all tasks on one stream up to this
 
+// Sum over the wave, the same value in every lane: four DPP steps within the rows of 16 lanes, then
+// the four row sums through scalar registers.  A shuffle-based tree goes through the LDS crossbar at
+// every level (about 7 times the latency, and these sums are most of a reflector's serial chain).
+template <int CTRL>
+__device__ __forceinline__ double dpp_add(double v) {
+  const long long x = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)x, CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(x >> 32), CTRL, 0xf, 0xf, true);
+  return v + __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+__device__ __forceinline__ double lane_value(double v, int lane) {  // lane: wave-uniform
+  const long long x = __double_as_longlong(v);
+  const unsigned int lo = (unsigned int)__builtin_amdgcn_readlane((int)x, lane);
+  const unsigned int hi = (unsigned int)__builtin_amdgcn_readlane((int)(x >> 32), lane);
+  return __longlong_as_double(((long long)hi << 32) | lo);
+}
 __device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
+  v = dpp_add<0xb1>(v);   // quad_perm [1, 0, 3, 2]
+  v = dpp_add<0x4e>(v);   // quad_perm [2, 3, 0, 1]
+  v = dpp_add<0x124>(v);  // row_ror:4
+  v = dpp_add<0x128>(v);  // row_ror:8
+  return (lane_value(v, 0) + lane_value(v, 16)) + (lane_value(v, 32) + lane_value(v, 48));
 }
 __device__ __forceinline__ double2 wave_sum2(double2 v) { return make_double2(wave_sum(v.x), wave_sum(v.y)); }
 
 // Element w_k[col] of reflector k of M (support col >= k; head in W0, tail in M's row k).
 __device__ __forceinline__ double2 refl(const double2* M, size_t ld, const double2* W0, int k, int col) {
   if (col < k) return make_double2(0, 0);
-  if (col == k) return W0[k];
-  return M[(size_t)k * ld + col];
+  return gld(col == k ? W0 + k : M + (size_t)k * ld + col);
 }
 
 // Factor rows [k0, k0 + 16) of T.M over columns [k0, cols) and form the panel's T factor.
 // Whole workgroup (256 threads); rows stay in memory (L2), each wave updates every fourth row.
-__device__ void lq_factor_panel(const LqTask& T, int k0, double2 (*sG)[LQB + 1], double2 (*sT)[LQB + 1]) {
+__device__ __forceinline__ void lq_factor_panel(const LqTask& T, int k0, double2 (*sG)[LQB + 1], double2 (*sT)[LQB + 1]) {
   double2* M = T.M;
   const size_t ld = T.ld;
   const int C = T.cols;
@@ -47,9 +65,9 @@ __device__ void lq_factor_panel(const LqTask& T, int k0, double2 (*sG)[LQB + 1],
   for (int k = k0; k < k1; ++k) {
     const double2* rk = M + (size_t)k * ld;
     double s = 0.0;
-    for (int l = k + 1 + lane; l < C; l += 64) s += cabs2(rk[l]);
+    for (int l = k + 1 + lane; l < C; l += 64) s += cabs2(gld(rk + l));
     s = wave_sum(s);
-    const double2 a = rk[k];
+    const double2 a = gld(rk + k);
     const double nrm = sqrt(cabs2(a) + s);
     double2 beta = make_double2(0, 0), w0 = make_double2(0, 0);
     double scale = 0.0;
@@ -65,18 +83,18 @@ __device__ void lq_factor_panel(const LqTask& T, int k0, double2 (*sG)[LQB + 1],
     for (int i = k + 1; i < k1; ++i) {
       if (((i - k0) & 3) != wave) continue;
       double2* yi = M + (size_t)i * ld;
-      double2 d = lane == 0 ? cfmac(w0, yi[k], make_double2(0, 0)) : make_double2(0, 0);
-      for (int l = k + 1 + lane; l < C; l += 64) d = cfmac(cscale(rk[l], scale), yi[l], d);
+      double2 d = lane == 0 ? cfmac(w0, gld(yi + k), make_double2(0, 0)) : make_double2(0, 0);
+      for (int l = k + 1 + lane; l < C; l += 64) d = cfmac(cscale(gld(rk + l), scale), gld(yi + l), d);
       d = wave_sum2(d);  // <y, w> = sum y_l conj(w_l)  (cfmac(a, b) adds conj(a) b)
       const double2 m2d = cscale(d, -2.0);
-      if (lane == 0) yi[k] = cfma(m2d, w0, yi[k]);
-      for (int l = k + 1 + lane; l < C; l += 64) yi[l] = cfma(m2d, cscale(rk[l], scale), yi[l]);
+      if (lane == 0) gst(yi + k, cfma(m2d, w0, gld(yi + k)));
+      for (int l = k + 1 + lane; l < C; l += 64) gst(yi + l, cfma(m2d, cscale(gld(rk + l), scale), gld(yi + l)));
     }
     __syncthreads();  // every read of row k done
-    for (int l = k + 1 + tid; l < C; l += 256) M[(size_t)k * ld + l] = cscale(rk[l], scale);
+    for (int l = k + 1 + tid; l < C; l += 256) gst(M + (size_t)k * ld + l, cscale(gld(rk + l), scale));
     if (tid == 0) {
-      M[(size_t)k * ld + k] = beta;
-      T.W0[k] = w0;
+      gst(M + (size_t)k * ld + k, beta);
+      gst(T.W0 + k, w0);
     }
     __syncthreads();
   }
@@ -109,7 +127,7 @@ __device__ void lq_factor_panel(const LqTask& T, int k0, double2 (*sG)[LQB + 1],
     __syncthreads();
   }
   double2* Tp = T.T + (size_t)(k0 / LQB) * LQB * LQB;
-  for (int e = tid; e < LQB * LQB; e += 256) Tp[e] = sT[e / LQB][e % LQB];
+  for (int e = tid; e < LQB * LQB; e += 256) gst(Tp + e, sT[e / LQB][e % LQB]);
   __syncthreads();
 }
 
@@ -117,13 +135,14 @@ __device__ void lq_factor_panel(const LqTask& T, int k0, double2 (*sG)[LQB + 1],
 // T' = T (conjT = 0) or T^H (conjT = 1), W the LQB reflector rows of the panel at k0.
 // P = Y W^H (16 x LQB) by MFMA with the column range split over the 4 waves and the next
 // 4-column unit prefetched, Q = P T' with T' staged in LDS, then Y -= Q W by MFMA, each wave
-// owning whole 16-column tiles.
-__device__ void lq_apply_panel(const LqTask& T, int k0, double2* Y, size_t ly, int r0, int r1, int conjT,
+// owning whole 16-column tiles.  Run by teams of four waves (a workgroup of 256 threads is one
+// team, one of 512 threads two, each with rows and LDS of its own).
+__device__ __forceinline__ void lq_apply_panel(const LqTask& T, int k0, double2* Y, size_t ly, int r0, int r1, int conjT,
                                double2 (*sP)[LQB + 1], double2 (*sQ)[LQB + 1], double2 (*sT)[LQB + 1]) {
   const double2* M = T.M;
   const size_t ld = T.ld;
   const int C = T.cols;
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int tid = threadIdx.x & 255, wave = tid >> 6, lane = tid & 63;
   const int l16 = lane & 15, k4 = lane >> 4;
   const int k1 = min(k0 + LQB, T.rows);
   const bool rowok = r0 + l16 < r1;
@@ -142,7 +161,7 @@ __device__ void lq_apply_panel(const LqTask& T, int k0, double2* Y, size_t ly, i
   const int nu = (C - k0 + 3) >> 2;
   int u = wave;
   int col = k0 + 4 * u + k4;
-  double2 a = (u < nu && rowok && col < C) ? yrow[col] : make_double2(0, 0);
+  double2 a = (u < nu && rowok && col < C) ? gld(yrow + col) : make_double2(0, 0);
   double2 wv[NG];
 #pragma unroll
   for (int g = 0; g < NG; ++g) wv[g] = u < nu ? wload(k0 + LQR * g + l16, col) : make_double2(0, 0);
@@ -153,7 +172,7 @@ __device__ void lq_apply_panel(const LqTask& T, int k0, double2* Y, size_t ly, i
     for (int g = 0; g < NG; ++g) y[g] = wv[g];
     const int ncol = col + 16;
     const bool nok = u + 4 < nu;
-    a = (nok && rowok && ncol < C) ? yrow[ncol] : make_double2(0, 0);
+    a = (nok && rowok && ncol < C) ? gld(yrow + ncol) : make_double2(0, 0);
 #pragma unroll
     for (int g = 0; g < NG; ++g) wv[g] = nok ? wload(k0 + LQR * g + l16, ncol) : make_double2(0, 0);
     col = ncol;
@@ -188,7 +207,7 @@ __device__ void lq_apply_panel(const LqTask& T, int k0, double2* Y, size_t ly, i
     for (int h = 0; h < NG; ++h) {  // rows 16h .. 16h + 15 of T'
       for (int e = tid; e < LQR * LQB; e += 256) {
         const int m = e / LQB, j = e % LQB, mm = LQR * h + m;
-        sT[m][j] = conjT ? cconj(Tp[j * LQB + mm]) : Tp[mm * LQB + j];
+        sT[m][j] = conjT ? cconj(gld(Tp + j * LQB + mm)) : gld(Tp + mm * LQB + j);
       }
       __syncthreads();
 #pragma unroll
@@ -230,8 +249,9 @@ __device__ void lq_apply_panel(const LqTask& T, int k0, double2* Y, size_t ly, i
       for (int v = 0; v < 4; ++v) {
         const int row = r0 + 4 * v + k4;
         if (row < r1) {
-          double2* y = Y + (size_t)row * ly + c0;
-          *y = make_double2(y->x - dr[v], y->y - di[v]);
+          double2* yp = Y + (size_t)row * ly + c0;
+          const double2 y = gld(yp);
+          gst(yp, make_double2(y.x - dr[v], y.y - di[v]));
         }
       }
     }
@@ -270,17 +290,18 @@ __global__ __launch_bounds__(256) void k_lq_update(const LqTask* tasks, int p) {
   lq_apply_panel(T, k0, T.M, T.ld, r0, min(r0 + LQR, T.rows), 0, sP, sQ, sT);
 }
 
-// Tgt <- Tgt (I - W_p^H T_p^H W_p) on rows [16x, 16x + 16) of Tgt.
-__global__ __launch_bounds__(256) void k_lq_apply_q(const LqTask* tasks, int p) {
+// Tgt <- Tgt (I - W_p^H T_p^H W_p) for every panel p from the last to the first, on rows [16x, 16x +
+// 16) of Tgt: the rows are independent of each other, so one launch applies all panels, each
+// workgroup to its rows (one launch a panel left gaps of several us between launches of 7 to 20 us).
+__global__ __launch_bounds__(256) void k_lq_apply_q(const LqTask* tasks) {
   __shared__ double2 sP[LQB][LQB + 1];
   __shared__ double2 sQ[LQB][LQB + 1];
   __shared__ double2 sT[LQR][LQB + 1];
-  const LqTask& T = tasks[blockIdx.y];
-  const int k0 = p * LQB;
-  if (k0 >= T.rows) return;
-  const int r0 = LQR * (int)blockIdx.x;
+  const LqTask& T = tasks[blockIdx.x];
+  const int r0 = LQR * (int)blockIdx.y;
   if (r0 >= T.rows_t) return;
-  lq_apply_panel(T, k0, T.Tgt, T.ld_t, r0, min(r0 + LQR, T.rows_t), 1, sP, sQ, sT);
+  for (int p = (T.rows - 1) / LQB; p >= 0; --p)
+    lq_apply_panel(T, p * LQB, T.Tgt, T.ld_t, r0, min(r0 + LQR, T.rows_t), 1, sP, sQ, sT);
 }
 
 // dst[i][j] = conj(src[j][i]) for j >= i and i < n, 0 otherwise (the conjugate transpose of
@@ -312,133 +333,171 @@ __global__ __launch_bounds__(256) void k_widen(const TriTask* tasks) {
   T.dst[e] = j < T.n ? T.src[(size_t)i * T.ld_src + j] : make_double2(0, 0);
 }
 
-// ---- factorisation with the panel in registers, look-ahead on two streams ----------------------
-// Factor rows [k0, k1) of T.M (panel p) over columns [k0, cols) with the panel in LDS (16 rows of
-// at most LQ_REG_MAX_COLS columns, 128 KiB): the same reflectors as lq_factor_panel, with every
-// dependent access of the 16 serial steps in LDS instead of memory.  Eight waves; wave w updates
-// the rows i = w (mod 8), its inner products reduced within the wave.
-__global__ __launch_bounds__(512) void k_lq_factor_lds(const LqTask* tasks, int p) {
-  constexpr int NT = 512, NW = NT / 64;
-  __shared__ double2 sy[LQB][LQ_REG_MAX_COLS];
-  __shared__ double2 sG[LQB][LQB + 1];
-  __shared__ double2 sT[LQB][LQB + 1];
-  __shared__ double2 s_w0[LQB];
-  __shared__ double s_scale[LQB];
-  const LqTask& T = tasks[blockIdx.x];
+// ---- factorisation with the panel in registers ------------------------------------------------
+struct LqStepShared {
+  double2 P[2][LQB][LQB + 1], Q[2][LQB][LQB + 1], T[2][LQR][LQB + 1];  // lq_apply_panel, per team
+  double2 w0[LQB];
+};
+
+// Factor rows [k0, k1) of T.M (panel p) over columns [k0, cols), at most 64 NC of them, with the
+// panel in registers: wave w of eight holds the rows w and w + 8, lane l the columns l + 64 j.  The
+// reflectors are those of lq_factor_panel.  Per reflector, its row w_r goes to LDS (zero before column
+// r), every wave forms the inner products of its rows with it -- <y_i, w_r> updates a row i > r, and
+// is G_ir of the T factor for a row i < r -- and the wave with row r + 1 goes on to the next reflector
+// as soon as that row is updated; T's column r - 1 is formed by another wave meanwhile.  One barrier
+// per reflector.  Bound by that serial chain; with the rows in LDS and shuffle reductions a panel of
+// 128 .. 512 columns took 48 .. 59 us, this form @US@.
+template <int NC>
+__device__ __forceinline__ void lq_factor_regs(const LqTask& T, int p, LqStepShared& S, double2* srow) {
   const int k0 = p * LQB;
-  if (k0 >= T.rows) return;
   const int k1 = min(k0 + LQB, T.rows), nr = k1 - k0;
-  const int W = T.cols - k0;  // columns k0 .. cols - 1 (local index c = column - k0)
-  double2* M = T.M;
+  const int W = T.cols - k0;  // local column c = column - k0
+  double2* M = T.M + (size_t)k0 * T.ld + k0;
   const size_t ld = T.ld;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  for (int e = tid; e < LQB * W; e += NT) {
-    const int i = e / W, c = e % W;
-    sy[i][c] = i < nr ? M[(size_t)(k0 + i) * ld + k0 + c] : make_double2(0, 0);
-  }
-  __syncthreads();
-  // Reflector of row k (wave 0 only): w = (w0 at column k, scale * row k beyond), beta onto the
-  // diagonal.  Row k's tail stays unscaled in LDS: every use multiplies by s_scale[k], the same
-  // single rounding as storing it scaled.
-  auto reflector = [&](int k) {
+  double2 (*sG)[LQB + 1] = S.P[0];
+  double2 (*sT)[LQB + 1] = S.T[0];
+  double2 y[2][NC];
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int j = 0; j < NC; ++j) {
+      const int i = wave + 8 * h, c = lane + 64 * j;
+      y[h][j] = (i < nr && c < W) ? gld(M + (size_t)i * ld + c) : make_double2(0, 0);
+    }
+  if (tid < LQB * LQB) sG[tid / LQB][tid % LQB] = sT[tid / LQB][tid % LQB] = make_double2(0, 0);
+  // reflector of row r, held by this wave in y[h]: w into srow[r & 1], beta and the scaled tail in place
+  auto reflector = [&](double2 (&v)[NC], int r) __attribute__((always_inline)) {
     double s = 0.0;
-    for (int c = k + 1 + lane; c < W; c += 64) s += cabs2(sy[k][c]);
+#pragma unroll
+    for (int j = 0; j < NC; ++j)
+      if (j > 0 || lane > r) s += cabs2(v[j]);
     s = wave_sum(s);
-    if (lane == 0) {
-      const double2 a = sy[k][k];
-      const double nrm = sqrt(cabs2(a) + s);
-      double2 beta = make_double2(0, 0), w0 = make_double2(0, 0);
-      double scale = 0.0;
-      if (nrm > 0.0) {
-        const double aa = sqrt(cabs2(a));
-        const double2 ph = aa > 0.0 ? cscale(a, 1.0 / aa) : make_double2(1.0, 0.0);
-        beta = cscale(ph, -nrm);  // -e^{i arg a} |x|: no cancellation in a - beta
-        const double2 v0 = make_double2(a.x - beta.x, a.y - beta.y);
-        scale = 1.0 / sqrt(cabs2(v0) + s);
-        w0 = cscale(v0, scale);
-      }
-      sy[k][k] = beta;
-      s_w0[k] = w0;
-      s_scale[k] = scale;
+    const double2 a = make_double2(lane_value(v[0].x, r), lane_value(v[0].y, r));
+    const double nrm = sqrt(cabs2(a) + s);
+    double2 beta = make_double2(0, 0), w0 = make_double2(0, 0);
+    double scale = 0.0;
+    if (nrm > 0.0) {
+      const double aa = sqrt(cabs2(a));
+      const double2 ph = aa > 0.0 ? cscale(a, 1.0 / aa) : make_double2(1.0, 0.0);
+      beta = cscale(ph, -nrm);  // -e^{i arg a} |x|: no cancellation in a - beta
+      const double2 v0 = make_double2(a.x - beta.x, a.y - beta.y);
+      scale = 1.0 / sqrt(cabs2(v0) + s);
+      w0 = cscale(v0, scale);
     }
+    double2* row = srow + (r & 1) * NC * 64;
+#pragma unroll
+    for (int j = 0; j < NC; ++j) {
+      const double2 t = cscale(v[j], scale);
+      if (j > 0) {
+        v[j] = t;
+        row[lane + 64 * j] = t;
+      } else {
+        row[lane] = make_double2(lane > r ? t.x : (lane == r ? w0.x : 0.0), lane > r ? t.y : (lane == r ? w0.y : 0.0));
+        v[0] = make_double2(lane > r ? t.x : (lane == r ? beta.x : v[0].x),
+                            lane > r ? t.y : (lane == r ? beta.y : v[0].y));
+      }
+    }
+    if (lane == 0) S.w0[r] = w0;
   };
-  if (wave == 0 && nr > 0) reflector(0);
-  __syncthreads();
-  // One barrier per reflector: wave w updates rows i = r + 1 + w (mod 8); wave 0 owns row r + 1,
-  // the next pivot, and forms its reflector as soon as that row is updated.
-  for (int r = 0; r < nr; ++r) {
-    const double2 w0 = s_w0[r];
-    const double scale = s_scale[r];
-    for (int i = r + 1 + wave; i < nr; i += NW) {
-      double2 d = lane == 0 ? cfmac(w0, sy[i][r], make_double2(0, 0)) : make_double2(0, 0);
-      for (int c = r + 1 + lane; c < W; c += 64) d = cfmac(cscale(sy[r][c], scale), sy[i][c], d);
-      d = wave_sum2(d);  // <y, w> = sum y_l conj(w_l)
-      const double2 m2d = cscale(d, -2.0);
-      if (lane == 0) sy[i][r] = cfma(m2d, w0, sy[i][r]);
-      for (int c = r + 1 + lane; c < W; c += 64) sy[i][c] = cfma(m2d, cscale(sy[r][c], scale), sy[i][c]);
-      if (i == r + 1) {
-        // the row's new values were written by other lanes of this wave: order them before the
-        // reflector's reads
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        reflector(i);
-      }
+  // column j of T (T_jj = 2, T_ij = -2 sum_{i <= m < j} T_im G_mj): four lanes a row
+  auto t_column = [&](int j) __attribute__((always_inline)) {
+    const int i = lane >> 2, q = lane & 3;
+    double2 t = make_double2(0, 0);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int m = q + 4 * e;
+      if (m >= i && m < j) t = cfma(sT[i][m], sG[m][j], t);
     }
+    t.x = dpp_add<0x4e>(dpp_add<0xb1>(t.x));
+    t.y = dpp_add<0x4e>(dpp_add<0xb1>(t.y));
+    if (q == 0 && i <= j) sT[i][j] = i == j ? make_double2(2.0, 0.0) : cscale(t, -2.0);
+  };
+  double2 w[NC];
+  auto inner = [&](const double2 (&v)[NC]) __attribute__((always_inline)) {  // <v, w> = sum v conj(w)
+    double2 d = make_double2(0, 0);
+#pragma unroll
+    for (int j = 0; j < NC; ++j) d = cfmac(w[j], v[j], d);
+    return wave_sum2(d);
+  };
+  auto update = [&](double2 (&v)[NC]) __attribute__((always_inline)) {
+    const double2 m2d = cscale(inner(v), -2.0);
+#pragma unroll
+    for (int j = 0; j < NC; ++j) v[j] = cfma(m2d, w[j], v[j]);
+  };
+  auto gram = [&](const double2 (&v)[NC], int i, int r) __attribute__((always_inline)) {
+    const double2 d = inner(v);
+    if (lane == 0) sG[i][r] = d;
+  };
+  auto load_w = [&](int r) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < NC; ++j) w[j] = srow[(r & 1) * NC * 64 + lane + 64 * j];
+  };
+  if (wave == 0 && nr > 0) reflector(y[0], 0);
+  __syncthreads();
+  // pivots 0 .. 6: the next pivot is among the rows 0 .. 7, the rows 8 .. 15 all update
+#pragma unroll 1
+  for (int r = 0; r < min(nr, 7); ++r) {
+    load_w(r);
+    if (wave > r) {
+      update(y[0]);
+      if (wave == r + 1 && wave < nr) reflector(y[0], r + 1);
+    } else if (wave < r) {
+      gram(y[0], wave, r);
+    }
+    update(y[1]);
+    if (r > 0 && wave == ((r + 4) & 7)) t_column(r - 1);
     __syncthreads();
   }
-  // G_ij = <w_i, w_j> = sum_l conj(w_j[l]) w_i[l] for i < j, support from local column j on
-  for (int pr = wave; pr < LQB * LQB; pr += NW) {
-    const int i = pr / LQB, j = pr % LQB;
-    if (j <= i) continue;
-    double2 d = make_double2(0, 0);
-    if (j < nr) {
-      const double si = s_scale[i], sj = s_scale[j];
-      if (lane == 0) d = cfmac(s_w0[j], cscale(sy[i][j], si), d);
-      for (int c = j + 1 + lane; c < W; c += 64) d = cfmac(cscale(sy[j][c], sj), cscale(sy[i][c], si), d);
+  // pivots 7 .. 15: the next pivot is among the rows 8 .. 15, the rows 0 .. 7 are done
+#pragma unroll 1
+  for (int r = 7; r < nr; ++r) {
+    load_w(r);
+    if (wave + 8 > r) {
+      update(y[1]);
+      if (wave + 8 == r + 1 && r + 1 < nr) reflector(y[1], r + 1);
+    } else if (wave + 8 < r) {
+      gram(y[1], wave + 8, r);
     }
-    d = wave_sum2(d);
-    if (lane == 0) sG[i][j] = d;
+    if (wave < r) gram(y[0], wave, r);
+    if (wave == ((r + 4) & 7)) t_column(r - 1);
+    __syncthreads();
   }
-  __syncthreads();
-  // T column by column in wave 0 (lanes 0..15), ordered within the wave
-  if (wave == 0) {
-    for (int j = 0; j < LQB; ++j) {
-      if (lane < LQB) {
-        double2 t = make_double2(0, 0);
-        if (lane < j) {
-          for (int m = lane; m < j; ++m) t = cfma(sT[lane][m], sG[m][j], t);
-          t = cscale(t, -2.0);
-        } else if (lane == j) {
-          t = make_double2(k0 + j < k1 ? 2.0 : 0.0, 0.0);
-        }
-        sT[lane][j] = t;
-      }
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    }
-  }
+  if (nr > 0 && wave == 0) t_column(nr - 1);
   __syncthreads();
   double2* Tp = T.T + (size_t)p * LQB * LQB;
-  for (int e = tid; e < LQB * LQB; e += NT) Tp[e] = sT[e / LQB][e % LQB];
-  if (tid < nr) T.W0[k0 + tid] = s_w0[tid];
-  for (int e = tid; e < nr * W; e += NT) {
-    const int i = e / W, c = e % W;
-    M[(size_t)(k0 + i) * ld + k0 + c] = c > i ? cscale(sy[i][c], s_scale[i]) : sy[i][c];
-  }
+  if (tid < LQB * LQB) gst(Tp + tid, sT[tid / LQB][tid % LQB]);
+  if (tid < nr) gst(T.W0 + k0 + tid, S.w0[tid]);
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int j = 0; j < NC; ++j) {
+      const int i = wave + 8 * h, c = lane + 64 * j;
+      if (i < nr && c < W) gst(M + (size_t)i * ld + c, y[h][j]);
+    }
 }
 
-// Rows of panel p + 1 (16 rows from k1) with the block reflector of panel p
-__global__ __launch_bounds__(256) void k_lq_next(const LqTask* tasks, int p) {
-  __shared__ double2 sP[LQB][LQB + 1];
-  __shared__ double2 sQ[LQB][LQB + 1];
-  __shared__ double2 sT[LQR][LQB + 1];
+// One panel's step, p = -1 .. panels - 2: workgroup (task, 0) applies the block reflector of panel p
+// to the rows of panel p + 1 and factors them; workgroup (task, x > 0) applies it to the 32 rows
+// from k0 + 2 LQB + 32 (x - 1) (two teams of four waves).  The factoring workgroups come first.
+template <int NC>
+__global__ __launch_bounds__(512) void k_lq_step(const LqTask* tasks, int p) {
+  __shared__ LqStepShared S;
+  __shared__ double2 srow[2 * NC * 64];
   const LqTask& T = tasks[blockIdx.x];
-  const int k0 = p * LQB;
-  const int k1 = min(k0 + LQB, T.rows);
+  const int team = threadIdx.x >> 8;
+  const int k0 = p * LQB, k1 = k0 + LQB;
   if (k1 >= T.rows) return;
-  lq_apply_panel(T, k0, T.M, T.ld, k1, min(k1 + LQB, T.rows), 0, sP, sQ, sT);
+  if (blockIdx.y == 0) {
+    const int e1 = min(k1 + LQB, T.rows);
+    if (p >= 0) lq_apply_panel(T, k0, T.M, T.ld, k1, team ? k1 : e1, 0, S.P[team], S.Q[team], S.T[team]);
+    lq_factor_regs<NC>(T, p + 1, S, srow);
+    return;
+  }
+  const int r0 = k1 + LQB + 2 * LQR * ((int)blockIdx.y - 1);
+  if (r0 >= T.rows) return;
+  const int rt = min(r0 + LQR * team, T.rows);
+  lq_apply_panel(T, k0, T.M, T.ld, rt, min(rt + LQR, T.rows), 0, S.P[team], S.Q[team], S.T[team]);
 }
 
 // Rows beyond panel p + 1 with the block reflector of panel p, 16 rows per workgroup
@@ -446,9 +505,9 @@ __global__ __launch_bounds__(256) void k_lq_rest(const LqTask* tasks, int p) {
   __shared__ double2 sP[LQB][LQB + 1];
   __shared__ double2 sQ[LQB][LQB + 1];
   __shared__ double2 sT[LQR][LQB + 1];
-  const LqTask& T = tasks[blockIdx.y];
+  const LqTask& T = tasks[blockIdx.x];
   const int k0 = p * LQB;
-  const int r0 = k0 + 2 * LQB + LQR * (int)blockIdx.x;
+  const int r0 = k0 + 2 * LQB + LQR * (int)blockIdx.y;
   if (r0 >= T.rows) return;
   lq_apply_panel(T, k0, T.M, T.ld, r0, min(r0 + LQR, T.rows), 0, sP, sQ, sT);
 }
@@ -457,26 +516,42 @@ hipError_t launch_lq_lookahead(const LqTask* d_tasks, int ntasks, int max_rows, 
                                hipStream_t sb, hipEvent_t ea, hipEvent_t eb) {
   if (ntasks <= 0 || max_rows <= 0) return hipSuccess;
   if (max_cols > LQ_REG_MAX_COLS) return hipErrorNotSupported;
-  auto factor = [&](int p) { hipLaunchKernelGGL(k_lq_factor_lds, dim3(ntasks), dim3(512), 0, sa, d_tasks, p); };
+  const int panels = (max_rows + LQB - 1) / LQB;
+  // columns per lane of the panel's registers; the results are the same for every NC that holds them
+  auto step = [&](int p, int blocks) {
+    const int w = max_cols - (p + 1) * LQB;
+    const dim3 g(ntasks, blocks), b(512);
+    if (w <= 128) hipLaunchKernelGGL(k_lq_step<2>, g, b, 0, sa, d_tasks, p);
+    else if (w <= 256) hipLaunchKernelGGL(k_lq_step<4>, g, b, 0, sa, d_tasks, p);
+    else if (w <= 512) hipLaunchKernelGGL(k_lq_step<8>, g, b, 0, sa, d_tasks, p);
+    else hipLaunchKernelGGL(k_lq_step<16>, g, b, 0, sa, d_tasks, p);
+  };
+  // Few trailing rows: one launch per panel for both, on one stream.  Many: the trailing update in
+  // workgroups of its own (a third of the registers) on the second stream, beside the next panel.
+  if ((long long)ntasks * max_rows <= LQ_ONE_STREAM_ROWS || sb == nullptr) {
+    for (int p = -1; p + 1 < panels; ++p) {
+      const int trailing = p < 0 ? 0 : max_rows - (p + 2) * LQB;
+      step(p, 1 + (trailing > 0 ? (trailing + 2 * LQR - 1) / (2 * LQR) : 0));
+    }
+    return hipGetLastError();
+  }
   hipError_t e = hipSuccess;
   // sb starts after what sa has queued so far (the matrices are ready there)
   if ((e = hipEventRecord(ea, sa)) != hipSuccess) return e;
   if ((e = hipStreamWaitEvent(sb, ea, 0)) != hipSuccess) return e;
-  factor(0);
+  step(-1, 1);
   if ((e = hipEventRecord(ea, sa)) != hipSuccess) return e;
-  const int panels = (max_rows + LQB - 1) / LQB;
   for (int p = 0; p + 1 < panels; ++p) {
     // sa: rows of panel p + 1 need the rest-update of panel p - 1 (recorded in eb), sb: the rest
     // update of panel p needs panel p's reflectors (recorded in ea); both waits are enqueued before
     // the events are recorded again below
     if (p > 0 && (e = hipStreamWaitEvent(sa, eb, 0)) != hipSuccess) return e;
     if ((e = hipStreamWaitEvent(sb, ea, 0)) != hipSuccess) return e;
-    hipLaunchKernelGGL(k_lq_next, dim3(ntasks), dim3(256), 0, sa, d_tasks, p);
-    factor(p + 1);
+    step(p, 1);
     if ((e = hipEventRecord(ea, sa)) != hipSuccess) return e;
     const int trailing = max_rows - (p + 2) * LQB;
     if (trailing > 0)
-      hipLaunchKernelGGL(k_lq_rest, dim3((trailing + LQR - 1) / LQR, ntasks), dim3(256), 0, sb, d_tasks, p);
+      hipLaunchKernelGGL(k_lq_rest, dim3(ntasks, (trailing + LQR - 1) / LQR), dim3(256), 0, sb, d_tasks, p);
     if ((e = hipEventRecord(eb, sb)) != hipSuccess) return e;
   }
   // everything after this on sa sees both streams' work
@@ -506,9 +581,7 @@ hipError_t launch_lq(const LqTask* d_tasks, int ntasks, int max_rows, hipStream_
 
 hipError_t launch_lq_apply_q(const LqTask* d_tasks, int ntasks, int max_rows, int max_rows_t, hipStream_t s) {
   if (ntasks <= 0 || max_rows <= 0) return hipSuccess;
-  const int panels = (max_rows + LQB - 1) / LQB;
-  for (int p = panels - 1; p >= 0; --p)
-    hipLaunchKernelGGL(k_lq_apply_q, dim3((max_rows_t + LQR - 1) / LQR, ntasks), dim3(256), 0, s, d_tasks, p);
+  hipLaunchKernelGGL(k_lq_apply_q, dim3(ntasks, (max_rows_t + LQR - 1) / LQR), dim3(256), 0, s, d_tasks);
   return hipGetLastError();
 }
 
