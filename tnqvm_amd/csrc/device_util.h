@@ -57,6 +57,19 @@ __device__ __forceinline__ void gst(float2* p, float2 v) {
   *(HIPMPS_GLOBAL gvec_f2*)p = x;
 }
 
+// base uniform over the wave, idx < 2^28: one scalar base and a 32-bit offset instead of a 64-bit
+// address per load
+__device__ __forceinline__ double2 gld_at(const double2* base, unsigned idx) {
+  const gvec_d2 v = *(const HIPMPS_GLOBAL gvec_d2*)((const HIPMPS_GLOBAL char*)base + (size_t)(idx * 16u));
+  return make_double2(v.x, v.y);
+}
+__device__ __forceinline__ void gst_at(double2* base, unsigned idx, double2 v) {
+  gvec_d2 x;
+  x.x = v.x;
+  x.y = v.y;
+  *(HIPMPS_GLOBAL gvec_d2*)((HIPMPS_GLOBAL char*)base + (size_t)(idx * 16u)) = x;
+}
+
 template <typename T>
 __device__ __forceinline__ double2 ld(const T* p, size_t i);
 template <>

@@ -132,96 +132,105 @@ __device__ __forceinline__ void lq_factor_panel(const LqTask& T, int k0, double2
 }
 
 // Rows [r0, r0 + 16) (clipped to r1) of Y (ld ly): Y <- Y (I - W^H T' W) over columns [k0, C),
-// T' = T (conjT = 0) or T^H (conjT = 1), W the LQB reflector rows of the panel at k0.
-// P = Y W^H (16 x LQB) by MFMA with the column range split over the 4 waves and the next
-// 4-column unit prefetched, Q = P T' with T' staged in LDS, then Y -= Q W by MFMA, each wave
-// owning whole 16-column tiles.  Run by teams of four waves (a workgroup of 256 threads is one
-// team, one of 512 threads two, each with rows and LDS of its own).
-__device__ __forceinline__ void lq_apply_panel(const LqTask& T, int k0, double2* Y, size_t ly, int r0, int r1, int conjT,
-                               double2 (*sP)[LQB + 1], double2 (*sQ)[LQB + 1], double2 (*sT)[LQB + 1]) {
+// T' = T (conjT = 0) or T^H (conjT = 1), W the reflector rows [k0, k1) of the panel at k0 (at most
+// LQB).  P = Y W^H (16 x LQB) by MFMA with the column range split over the 4 waves, Q = P T' with T'
+// staged in LDS, then Y -= Q W by MFMA, each wave owning whole 16-column tiles.  PD units of P and a
+// whole tile of the update are in flight; the loads of whole 16-column groups past the panel's own
+// columns, nearly all, are plain (no reflector starts there, no column is past the end).  With one
+// unit ahead and a branch around every load, a workgroup alone on its CU waited for one load latency
+// per 16 columns.  Run by teams of four waves (a workgroup of 256 threads is one team, one of 512
+// threads two, each with rows and LDS of its own).
+template <int PD>
+__device__ __forceinline__ void lq_apply_panel(const LqTask& T, int k0, int k1, double2* Y, size_t ly, int r0, int r1,
+                                               int conjT, double2 (*sP)[LQB + 1], double2 (*sQ)[LQB + 1],
+                                               double2 (*sT)[LQB + 1]) {
   const double2* M = T.M;
+  const double2* W0 = T.W0;
   const size_t ld = T.ld;
   const int C = T.cols;
   const int tid = threadIdx.x & 255, wave = tid >> 6, lane = tid & 63;
   const int l16 = lane & 15, k4 = lane >> 4;
-  const int k1 = min(k0 + LQB, T.rows);
-  const bool rowok = r0 + l16 < r1;
-  const double2* yrow = Y + (size_t)(r0 + l16) * ly;
-  constexpr int NG = LQB / LQR;  // 16-column groups of P
-  auto wload = [&](int j, int col) -> double2 {
-    return (j < k1 && col < C) ? refl(M, ld, T.W0, j, col) : make_double2(0, 0);
+  // element w_j[col] of reflector j (support col >= j; head in W0, tail in M's row j).  A reflector
+  // past k1 repeats the last one: its rows and columns of T are zero.
+  auto wload = [&](int j, int g, int off) __attribute__((always_inline)) {  // 16-column group at k0 + 16 g
+    const int c0 = k0 + 16 * g, col = c0 + off;
+    const unsigned row = (unsigned)min(j, k1 - 1) * (unsigned)ld;
+    if (g > 0 && c0 + 16 <= C) return gld_at(M, row + col);
+    const int jc = min(j, k1 - 1), cc = min(col, C - 1);
+    const double2 v = gld_at(M, row + cc), h = gld_at(W0, jc);
+    const bool head = col == jc, zero = col < jc || col >= C;
+    return make_double2(zero ? 0.0 : (head ? h.x : v.x), zero ? 0.0 : (head ? h.y : v.y));
   };
-  // ---- P[i][j] = sum_c Y[r0+i][c] conj(w_j[c]); B operand of group g: reflector k0 + 16g + l16 ----
-  mfma_d4 pr[NG], pim[NG];
+  // ---- P[i][j] = sum_c Y[r0+i][c] conj(w_j[c]); B operand: reflector k0 + l16 ----
+  const unsigned yrow = (unsigned)min(r0 + l16, r1 - 1) * (unsigned)ly;  // a row past the end: a repeat, not stored
+  auto yload = [&](int g, int off) __attribute__((always_inline)) {
+    const int c0 = k0 + 16 * g, col = c0 + off;
+    if (c0 + 16 <= C) return gld_at(Y, yrow + col);
+    const double2 v = gld_at(Y, yrow + min(col, C - 1));
+    return make_double2(col < C ? v.x : 0.0, col < C ? v.y : 0.0);
+  };
+  mfma_d4 pr = {0, 0, 0, 0}, pim = {0, 0, 0, 0};
+  const int nt = (C - k0 + 15) >> 4;  // 16-column groups; this wave's unit of a group: 4 columns
+  const int uo = 4 * wave + k4;
+  double2 a[PD], w[PD];
 #pragma unroll
-  for (int g = 0; g < NG; ++g) {
-    pr[g] = mfma_d4{0, 0, 0, 0};
-    pim[g] = mfma_d4{0, 0, 0, 0};
-  }
-  const int nu = (C - k0 + 3) >> 2;
-  int u = wave;
-  int col = k0 + 4 * u + k4;
-  double2 a = (u < nu && rowok && col < C) ? gld(yrow + col) : make_double2(0, 0);
-  double2 wv[NG];
+  for (int d = 0; d < PD; ++d)
+    if (d < nt) {
+      a[d] = yload(d, uo);
+      w[d] = wload(k0 + l16, d, uo);
+    }
+#pragma unroll 1
+  for (int d0 = 0; d0 < nt; d0 += PD) {
 #pragma unroll
-  for (int g = 0; g < NG; ++g) wv[g] = u < nu ? wload(k0 + LQR * g + l16, col) : make_double2(0, 0);
-  for (; u < nu; u += 4) {
-    const double2 x = a;
-    double2 y[NG];
-#pragma unroll
-    for (int g = 0; g < NG; ++g) y[g] = wv[g];
-    const int ncol = col + 16;
-    const bool nok = u + 4 < nu;
-    a = (nok && rowok && ncol < C) ? gld(yrow + ncol) : make_double2(0, 0);
-#pragma unroll
-    for (int g = 0; g < NG; ++g) wv[g] = nok ? wload(k0 + LQR * g + l16, ncol) : make_double2(0, 0);
-    col = ncol;
-    // x conj(y): re = x.x y.x + x.y y.y, im = x.y y.x - x.x y.y
-#pragma unroll
-    for (int g = 0; g < NG; ++g) {
-      pr[g] = mfma64(x.x, y[g].x, pr[g]);
-      pr[g] = mfma64(x.y, y[g].y, pr[g]);
-      pim[g] = mfma64(x.y, y[g].x, pim[g]);
-      pim[g] = mfma64(-x.x, y[g].y, pim[g]);
+    for (int d = 0; d < PD; ++d) {
+      if (d0 + d < nt) {
+        const double2 x = a[d], y = w[d];
+        if (d0 + d + PD < nt) {
+          a[d] = yload(d0 + d + PD, uo);
+          w[d] = wload(k0 + l16, d0 + d + PD, uo);
+        }
+        // x conj(y): re = x.x y.x + x.y y.y, im = x.y y.x - x.x y.y
+        pr = mfma64(x.x, y.x, pr);
+        pim = mfma64(x.y, y.x, pim);
+        pr = mfma64(x.y, y.y, pr);
+        pim = mfma64(-x.x, y.y, pim);
+      }
     }
   }
-  for (int w = 0; w < 4; ++w) {
-    if (wave == w) {
+  // first tile of the update, while P is summed
+  double2 tw[LQB / 4], ty[4];
+  unsigned ry[4];
 #pragma unroll
-      for (int g = 0; g < NG; ++g)
+  for (int v = 0; v < 4; ++v) ry[v] = (unsigned)min(r0 + 4 * v + k4, r1 - 1) * (unsigned)ly;
+  auto tile = [&](int t) __attribute__((always_inline)) {
+    const int c = min(k0 + 16 * t + l16, C - 1);
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          double2 e = make_double2(pr[g][v], pim[g][v]);
-          if (w) e = cadd(e, sP[4 * v + k4][LQR * g + l16]);
-          sP[4 * v + k4][LQR * g + l16] = e;
-        }
+    for (int kk = 0; kk < LQB / 4; ++kk) tw[kk] = wload(k0 + kk * 4 + k4, t, l16);  // B[k][c] = w_j[c]
+#pragma unroll
+    for (int v = 0; v < 4; ++v) ty[v] = gld_at(Y, ry[v] + c);
+  };
+  if (wave < nt) tile(wave);
+  for (int q = 0; q < 4; ++q) {
+    if (wave == q) {
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        double2 e = make_double2(pr[v], pim[v]);
+        if (q) e = cadd(e, sP[4 * v + k4][l16]);
+        sP[4 * v + k4][l16] = e;
+      }
     }
     __syncthreads();
   }
-  // ---- Q = P T' (16 x LQB), T' staged 16 rows at a time in sT ----
+  // ---- Q = P T' (16 x LQB) ----
   {
     const double2* Tp = T.T + (size_t)(k0 / LQB) * LQB * LQB;
-    double2 q[NG];
-    const int i = tid >> 4, j0 = tid & 15;
-#pragma unroll
-    for (int h = 0; h < NG; ++h) {  // rows 16h .. 16h + 15 of T'
-      for (int e = tid; e < LQR * LQB; e += 256) {
-        const int m = e / LQB, j = e % LQB, mm = LQR * h + m;
-        sT[m][j] = conjT ? cconj(gld(Tp + j * LQB + mm)) : gld(Tp + mm * LQB + j);
-      }
-      __syncthreads();
-#pragma unroll
-      for (int x = 0; x < NG; ++x) {
-        const int j = j0 + LQR * x;
-        double2 acc = h ? q[x] : make_double2(0, 0);
+    const int i = tid >> 4, j = tid & 15;
+    sT[i][j] = conjT ? cconj(gld(Tp + j * LQB + i)) : gld(Tp + i * LQB + j);
+    __syncthreads();
+    double2 acc = make_double2(0, 0);
 #pragma unroll 4
-        for (int m = 0; m < LQR; ++m) acc = cfma(sP[i][LQR * h + m], sT[m][j], acc);
-        q[x] = acc;
-      }
-      __syncthreads();
-    }
-#pragma unroll
-    for (int x = 0; x < NG; ++x) sQ[i][LQR * x + j0] = q[x];
+    for (int m = 0; m < LQB; ++m) acc = cfma(sP[i][m], sT[m][j], acc);
+    sQ[i][j] = acc;
   }
   __syncthreads();
   // ---- Y -= Q W over 16-column tiles ----
@@ -232,27 +241,28 @@ __device__ __forceinline__ void lq_apply_panel(const LqTask& T, int k0, double2*
     qr[kk] = q.x;
     qi[kk] = q.y;
   }
-  const int nt = (C - k0 + 15) >> 4;
+#pragma unroll 1
   for (int t = wave; t < nt; t += 4) {
-    const int c0 = k0 + 16 * t + l16;
+    const int c = k0 + 16 * t + l16;
+    double2 cwv[LQB / 4], cy[4];
+#pragma unroll
+    for (int kk = 0; kk < LQB / 4; ++kk) cwv[kk] = tw[kk];
+#pragma unroll
+    for (int v = 0; v < 4; ++v) cy[v] = ty[v];
+    if (t + 4 < nt) tile(t + 4);
     mfma_d4 dr = {0, 0, 0, 0}, di = {0, 0, 0, 0};
 #pragma unroll
     for (int kk = 0; kk < LQB / 4; ++kk) {
-      const double2 w = wload(k0 + kk * 4 + k4, c0);  // B[k][c] = w_j[c]
-      dr = mfma64(qr[kk], w.x, dr);
-      dr = mfma64(-qi[kk], w.y, dr);
-      di = mfma64(qr[kk], w.y, di);
-      di = mfma64(qi[kk], w.x, di);
+      dr = mfma64(qr[kk], cwv[kk].x, dr);
+      di = mfma64(qr[kk], cwv[kk].y, di);
+      dr = mfma64(-qi[kk], cwv[kk].y, dr);
+      di = mfma64(qi[kk], cwv[kk].x, di);
     }
-    if (c0 < C) {
+    if (c < C) {
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
         const int row = r0 + 4 * v + k4;
-        if (row < r1) {
-          double2* yp = Y + (size_t)row * ly + c0;
-          const double2 y = gld(yp);
-          gst(yp, make_double2(y.x - dr[v], y.y - di[v]));
-        }
+        if (row < r1) gst_at(Y, ry[v] + c, make_double2(cy[v].x - dr[v], cy[v].y - di[v]));
       }
     }
   }
@@ -281,13 +291,13 @@ __global__ __launch_bounds__(256) void k_lq_update(const LqTask* tasks, int p) {
   if (blockIdx.x == 0) {
     if (k1 >= T.rows) return;
     const int e1 = min(k1 + LQB, T.rows);
-    for (int r0 = k1; r0 < e1; r0 += LQR) lq_apply_panel(T, k0, T.M, T.ld, r0, e1, 0, sP, sQ, sT);
+    lq_apply_panel<4>(T, k0, k1, T.M, T.ld, k1, e1, 0, sP, sQ, sT);
     lq_factor_panel(T, k1, sP, sQ);
     return;
   }
   const int r0 = k1 + LQB + LQR * ((int)blockIdx.x - 1);
   if (r0 >= T.rows) return;
-  lq_apply_panel(T, k0, T.M, T.ld, r0, min(r0 + LQR, T.rows), 0, sP, sQ, sT);
+  lq_apply_panel<4>(T, k0, k1, T.M, T.ld, r0, min(r0 + LQR, T.rows), 0, sP, sQ, sT);
 }
 
 // Tgt <- Tgt (I - W_p^H T_p^H W_p) for every panel p from the last to the first, on rows [16x, 16x +
@@ -301,7 +311,7 @@ __global__ __launch_bounds__(256) void k_lq_apply_q(const LqTask* tasks) {
   const int r0 = LQR * (int)blockIdx.y;
   if (r0 >= T.rows_t) return;
   for (int p = (T.rows - 1) / LQB; p >= 0; --p)
-    lq_apply_panel(T, p * LQB, T.Tgt, T.ld_t, r0, min(r0 + LQR, T.rows_t), 1, sP, sQ, sT);
+    lq_apply_panel<2>(T, p * LQB, min(p * LQB + LQB, T.rows), T.Tgt, T.ld_t, r0, min(r0 + LQR, T.rows_t), 1, sP, sQ, sT);
 }
 
 // dst[i][j] = conj(src[j][i]) for j >= i and i < n, 0 otherwise (the conjugate transpose of
@@ -336,18 +346,22 @@ __global__ __launch_bounds__(256) void k_widen(const TriTask* tasks) {
 // ---- factorisation with the panel in registers ------------------------------------------------
 struct LqStepShared {
   double2 P[2][LQB][LQB + 1], Q[2][LQB][LQB + 1], T[2][LQR][LQB + 1];  // lq_apply_panel, per team
+  double2 G[LQB][LQB + 1], Tf[LQB][LQB + 1];                           // lq_factor_regs
   double2 w0[LQB];
 };
 
 // Factor rows [k0, k1) of T.M (panel p) over columns [k0, cols), at most 64 NC of them, with the
-// panel in registers: wave w of eight holds the rows w and w + 8, lane l the columns l + 64 j.  The
-// reflectors are those of lq_factor_panel.  Per reflector, its row w_r goes to LDS (zero before column
-// r), every wave forms the inner products of its rows with it -- <y_i, w_r> updates a row i > r, and
-// is G_ir of the T factor for a row i < r -- and the wave with row r + 1 goes on to the next reflector
-// as soon as that row is updated; T's column r - 1 is formed by another wave meanwhile.  One barrier
-// per reflector.  Bound by that serial chain; with the rows in LDS and shuffle reductions a panel of
-// 128 .. 512 columns took 48 .. 59 us, this form @US@.
-template <int NC>
+// panel in registers: lane l holds the columns l + 64 j, wave w of eight the rows w and w + 8 (RW = 2),
+// or, where two rows of a lane do not fit its registers, first row w and then, after the first eight
+// reflectors, row w + 8 (RW = 1).  The reflectors are those of lq_factor_panel.  Per reflector, its
+// row w_r goes to LDS (zero before column r), every wave forms the inner products of its rows with it
+// -- <y_i, w_r> updates a row i > r, and is G_ir of the T factor for a row i < r -- and the wave with
+// row r + 1 goes on to the next reflector as soon as that row is updated; T's column r - 1 is formed by
+// another wave meanwhile.  One barrier per reflector.  Bound by that serial chain.  Measured, with the
+// update of the panel's rows by the panel before: 26, 34 and 48 us at up to 128, 256 and 512 columns
+// (rows in LDS, shuffle reductions: 55, 73 and 100 us), 80 us at 1024 and 218 us at 1536 (rows in L2:
+// 350 to 700 us).
+template <int NC, int RW>
 __device__ __forceinline__ void lq_factor_regs(const LqTask& T, int p, LqStepShared& S, double2* srow) {
   const int k0 = p * LQB;
   const int k1 = min(k0 + LQB, T.rows), nr = k1 - k0;
@@ -355,18 +369,25 @@ __device__ __forceinline__ void lq_factor_regs(const LqTask& T, int p, LqStepSha
   double2* M = T.M + (size_t)k0 * T.ld + k0;
   const size_t ld = T.ld;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  double2 (*sG)[LQB + 1] = S.P[0];
-  double2 (*sT)[LQB + 1] = S.T[0];
-  double2 y[2][NC];
-#pragma unroll
-  for (int h = 0; h < 2; ++h)
+  double2 (*sG)[LQB + 1] = S.G;
+  double2 (*sT)[LQB + 1] = S.Tf;
+  constexpr bool WREG = NC <= 16;  // the pivot row in registers too
+  double2 y[RW][NC], w[WREG ? NC : 1];
+  auto load = [&](double2 (&v)[NC], int i) __attribute__((always_inline)) {
 #pragma unroll
     for (int j = 0; j < NC; ++j) {
-      const int i = wave + 8 * h, c = lane + 64 * j;
-      y[h][j] = (i < nr && c < W) ? gld(M + (size_t)i * ld + c) : make_double2(0, 0);
+      const int c = lane + 64 * j;
+      v[j] = (i < nr && c < W) ? gld(M + (size_t)i * ld + c) : make_double2(0, 0);
     }
-  if (tid < LQB * LQB) sG[tid / LQB][tid % LQB] = sT[tid / LQB][tid % LQB] = make_double2(0, 0);
-  // reflector of row r, held by this wave in y[h]: w into srow[r & 1], beta and the scaled tail in place
+  };
+  auto store = [&](const double2 (&v)[NC], int i) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < NC; ++j) {
+      const int c = lane + 64 * j;
+      if (i < nr && c < W) gst(M + (size_t)i * ld + c, v[j]);
+    }
+  };
+  // reflector of row r, held by this wave in v: w into srow[r & 1], beta and the scaled tail in place
   auto reflector = [&](double2 (&v)[NC], int r) __attribute__((always_inline)) {
     double s = 0.0;
 #pragma unroll
@@ -413,68 +434,124 @@ __device__ __forceinline__ void lq_factor_regs(const LqTask& T, int p, LqStepSha
     t.y = dpp_add<0x4e>(dpp_add<0xb1>(t.y));
     if (q == 0 && i <= j) sT[i][j] = i == j ? make_double2(2.0, 0.0) : cscale(t, -2.0);
   };
-  double2 w[NC];
-  auto inner = [&](const double2 (&v)[NC]) __attribute__((always_inline)) {  // <v, w> = sum v conj(w)
-    double2 d = make_double2(0, 0);
-#pragma unroll
-    for (int j = 0; j < NC; ++j) d = cfmac(w[j], v[j], d);
-    return wave_sum2(d);
-  };
-  auto update = [&](double2 (&v)[NC]) __attribute__((always_inline)) {
-    const double2 m2d = cscale(inner(v), -2.0);
-#pragma unroll
-    for (int j = 0; j < NC; ++j) v[j] = cfma(m2d, w[j], v[j]);
-  };
-  auto gram = [&](const double2 (&v)[NC], int i, int r) __attribute__((always_inline)) {
-    const double2 d = inner(v);
-    if (lane == 0) sG[i][r] = d;
+  auto pivot = [&](int j, int r) __attribute__((always_inline)) {  // w_r at this lane's column j
+    return WREG ? w[WREG ? j : 0] : srow[(r & 1) * NC * 64 + lane + 64 * j];
   };
   auto load_w = [&](int r) __attribute__((always_inline)) {
+    if (WREG) {
 #pragma unroll
-    for (int j = 0; j < NC; ++j) w[j] = srow[(r & 1) * NC * 64 + lane + 64 * j];
+      for (int j = 0; j < NC; ++j) w[WREG ? j : 0] = srow[(r & 1) * NC * 64 + lane + 64 * j];
+    }
   };
-  if (wave == 0 && nr > 0) reflector(y[0], 0);
-  __syncthreads();
-  // pivots 0 .. 6: the next pivot is among the rows 0 .. 7, the rows 8 .. 15 all update
-#pragma unroll 1
-  for (int r = 0; r < min(nr, 7); ++r) {
-    load_w(r);
-    if (wave > r) {
-      update(y[0]);
-      if (wave == r + 1 && wave < nr) reflector(y[0], r + 1);
-    } else if (wave < r) {
-      gram(y[0], wave, r);
-    }
-    update(y[1]);
-    if (r > 0 && wave == ((r + 4) & 7)) t_column(r - 1);
-    __syncthreads();
-  }
-  // pivots 7 .. 15: the next pivot is among the rows 8 .. 15, the rows 0 .. 7 are done
-#pragma unroll 1
-  for (int r = 7; r < nr; ++r) {
-    load_w(r);
-    if (wave + 8 > r) {
-      update(y[1]);
-      if (wave + 8 == r + 1 && r + 1 < nr) reflector(y[1], r + 1);
-    } else if (wave + 8 < r) {
-      gram(y[1], wave + 8, r);
-    }
-    if (wave < r) gram(y[0], wave, r);
-    if (wave == ((r + 4) & 7)) t_column(r - 1);
-    __syncthreads();
-  }
-  if (nr > 0 && wave == 0) t_column(nr - 1);
-  __syncthreads();
-  double2* Tp = T.T + (size_t)p * LQB * LQB;
-  if (tid < LQB * LQB) gst(Tp + tid, sT[tid / LQB][tid % LQB]);
-  if (tid < nr) gst(T.W0 + k0 + tid, S.w0[tid]);
-#pragma unroll
-  for (int h = 0; h < 2; ++h)
+  auto inner = [&](const double2 (&v)[NC], int r) __attribute__((always_inline)) {  // <v, w> = sum v conj(w)
+    double2 d = make_double2(0, 0);
 #pragma unroll
     for (int j = 0; j < NC; ++j) {
-      const int i = wave + 8 * h, c = lane + 64 * j;
-      if (i < nr && c < W) gst(M + (size_t)i * ld + c, y[h][j]);
+      d = cfmac(pivot(j, r), v[j], d);
+      if (!WREG && j % 8 == 7) __builtin_amdgcn_sched_barrier(0);  // 8 LDS reads ahead, not all of them
     }
+    return wave_sum2(d);
+  };
+  auto update = [&](double2 (&v)[NC], int r) __attribute__((always_inline)) {
+    const double2 m2d = cscale(inner(v, r), -2.0);
+#pragma unroll
+    for (int j = 0; j < NC; ++j) {
+      v[j] = cfma(m2d, pivot(j, r), v[j]);
+      if (!WREG && j % 8 == 7) __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  auto gram = [&](const double2 (&v)[NC], int i, int r) __attribute__((always_inline)) {
+    const double2 d = inner(v, r);
+    if (lane == 0) sG[i][r] = d;
+  };
+  auto store_t = [&]() __attribute__((always_inline)) {
+    double2* Tp = T.T + (size_t)p * LQB * LQB;
+    if (tid < LQB * LQB) gst(Tp + tid, sT[tid / LQB][tid % LQB]);
+    if (tid < nr) gst(T.W0 + k0 + tid, S.w0[tid]);
+  };
+
+  if (tid < LQB) S.w0[tid] = make_double2(0, 0);
+  if (tid < LQB * LQB) sG[tid / LQB][tid % LQB] = sT[tid / LQB][tid % LQB] = make_double2(0, 0);
+  if constexpr (RW == 2) {
+    load(y[0], wave);
+    load(y[1], wave + 8);
+    __syncthreads();
+    if (wave == 0 && nr > 0) reflector(y[0], 0);
+    __syncthreads();
+    // pivots 0 .. 6: the next pivot is among the rows 0 .. 7, the rows 8 .. 15 all update
+#pragma unroll 1
+    for (int r = 0; r < min(nr, 7); ++r) {
+      load_w(r);
+      if (wave > r) {
+        update(y[0], r);
+        if (wave == r + 1 && wave < nr) reflector(y[0], r + 1);
+      } else if (wave < r) {
+        gram(y[0], wave, r);
+      }
+      update(y[1], r);
+      if (r > 0 && wave == ((r + 4) & 7)) t_column(r - 1);
+      __syncthreads();
+    }
+    // pivots 7 .. 15: the next pivot is among the rows 8 .. 15, the rows 0 .. 7 are done
+#pragma unroll 1
+    for (int r = 7; r < nr; ++r) {
+      load_w(r);
+      if (wave + 8 > r) {
+        update(y[1], r);
+        if (wave + 8 == r + 1 && r + 1 < nr) reflector(y[1], r + 1);
+      } else if (wave + 8 < r) {
+        gram(y[1], wave + 8, r);
+      }
+      if (wave < r) gram(y[0], wave, r);
+      if (wave == ((r + 4) & 7)) t_column(r - 1);
+      __syncthreads();
+    }
+    if (nr > 0 && wave == 0) t_column(nr - 1);
+    __syncthreads();
+    store_t();
+    store(y[0], wave);
+    store(y[1], wave + 8);
+  } else {
+#pragma unroll 1
+    for (int base = 0; base < nr; base += 8) {
+      if (base > 0) {  // rows 8 .. 15 through the first eight reflectors
+        const int r0 = k0 + 8;
+        const int team = tid >> 8;
+        lq_apply_panel<4>(T, k0, r0, T.M, ld, r0, team ? r0 : k1, 0, S.P[team], S.Q[team], S.T[team]);
+      }
+      load(y[0], wave + base);
+      __syncthreads();
+      if (wave == 0) reflector(y[0], base);
+      __syncthreads();
+      const int end = min(nr, base + 8);
+#pragma unroll 1
+      for (int r = base; r < end; ++r) {
+        if (wave + base > r) {
+          update(y[0], r);
+          if (wave + base == r + 1 && r + 1 < end) reflector(y[0], r + 1);
+        } else if (wave + base < r) {
+          gram(y[0], wave + base, r);
+        }
+        if (base > 0) {  // G with the finished row `wave`, from memory
+          double2 d = make_double2(0, 0);
+#pragma unroll 8
+          for (int j = 0; j < NC; ++j) {
+            const int c = lane + 64 * j;
+            d = cfmac(srow[(r & 1) * NC * 64 + c], gld(M + (size_t)wave * ld + min(c, W - 1)), d);  // w_r is 0 past W
+          }
+          d = wave_sum2(d);
+          if (lane == 0) sG[wave][r] = d;
+        }
+        if (r > 0 && wave == ((r + 4) & 7)) t_column(r - 1);
+        __syncthreads();
+      }
+      if (wave == 0) t_column(end - 1);
+      __syncthreads();
+      store_t();
+      store(y[0], wave + base);
+      __syncthreads();
+    }
+  }
 }
 
 // One panel's step, p = -1 .. panels - 2: workgroup (task, 0) applies the block reflector of panel p
@@ -490,14 +567,14 @@ __global__ __launch_bounds__(512) void k_lq_step(const LqTask* tasks, int p) {
   if (k1 >= T.rows) return;
   if (blockIdx.y == 0) {
     const int e1 = min(k1 + LQB, T.rows);
-    if (p >= 0) lq_apply_panel(T, k0, T.M, T.ld, k1, team ? k1 : e1, 0, S.P[team], S.Q[team], S.T[team]);
-    lq_factor_regs<NC>(T, p + 1, S, srow);
+    if (p >= 0) lq_apply_panel<4>(T, k0, k1, T.M, T.ld, k1, team ? k1 : e1, 0, S.P[team], S.Q[team], S.T[team]);
+    lq_factor_regs<NC, (NC <= 16 ? 2 : 1)>(T, p + 1, S, srow);
     return;
   }
   const int r0 = k1 + LQB + 2 * LQR * ((int)blockIdx.y - 1);
   if (r0 >= T.rows) return;
   const int rt = min(r0 + LQR * team, T.rows);
-  lq_apply_panel(T, k0, T.M, T.ld, rt, min(rt + LQR, T.rows), 0, S.P[team], S.Q[team], S.T[team]);
+  lq_apply_panel<4>(T, k0, k1, T.M, T.ld, rt, min(rt + LQR, T.rows), 0, S.P[team], S.Q[team], S.T[team]);
 }
 
 // Rows beyond panel p + 1 with the block reflector of panel p, 16 rows per workgroup
@@ -509,7 +586,7 @@ __global__ __launch_bounds__(256) void k_lq_rest(const LqTask* tasks, int p) {
   const int k0 = p * LQB;
   const int r0 = k0 + 2 * LQB + LQR * (int)blockIdx.y;
   if (r0 >= T.rows) return;
-  lq_apply_panel(T, k0, T.M, T.ld, r0, min(r0 + LQR, T.rows), 0, sP, sQ, sT);
+  lq_apply_panel<2>(T, k0, k0 + LQB, T.M, T.ld, r0, min(r0 + LQR, T.rows), 0, sP, sQ, sT);
 }
 
 hipError_t launch_lq_lookahead(const LqTask* d_tasks, int ntasks, int max_rows, int max_cols, hipStream_t sa,
@@ -524,7 +601,9 @@ hipError_t launch_lq_lookahead(const LqTask* d_tasks, int ntasks, int max_rows, 
     if (w <= 128) hipLaunchKernelGGL(k_lq_step<2>, g, b, 0, sa, d_tasks, p);
     else if (w <= 256) hipLaunchKernelGGL(k_lq_step<4>, g, b, 0, sa, d_tasks, p);
     else if (w <= 512) hipLaunchKernelGGL(k_lq_step<8>, g, b, 0, sa, d_tasks, p);
-    else hipLaunchKernelGGL(k_lq_step<16>, g, b, 0, sa, d_tasks, p);
+    else if (w <= 1024) hipLaunchKernelGGL(k_lq_step<16>, g, b, 0, sa, d_tasks, p);
+    else if (w <= 1536) hipLaunchKernelGGL(k_lq_step<24>, g, b, 0, sa, d_tasks, p);
+    else hipLaunchKernelGGL(k_lq_step<32>, g, b, 0, sa, d_tasks, p);
   };
   // Few trailing rows: one launch per panel for both, on one stream.  Many: the trailing update in
   // workgroups of its own (a third of the registers) on the second stream, beside the next panel.
