@@ -525,6 +525,14 @@ int state_init_product(hipmps_state_s* s) {
 // ------------------------------------------------------------------------------------
 // wave execution (many states, many bonds)
 // ------------------------------------------------------------------------------------
+// output tiles of a GEMM task, whose first is `begin`; returns the one after its last
+int gemm_tiles(GemmTask& g, int begin) {
+  g.tiles_m = (g.M + GEMM_TM - 1) / GEMM_TM;
+  g.tiles_n = (g.N + GEMM_TN - 1) / GEMM_TN;
+  g.tile_begin = begin;
+  return begin + g.tiles_m * g.tiles_n;
+}
+
 struct WaveItem {
   hipmps_state_s* s;
   int i;          // left site
@@ -801,10 +809,7 @@ int run_wave(hipmps_engine E, std::vector<WaveItem>& items) {
         G.Mdyn = S.K;
         G.rowscale = S.inv_sig;
       }
-      G.tiles_m = (G.M + 31) / 32;
-      G.tiles_n = (G.N + 31) / 32;
-      G.tile_begin = tiles;
-      tiles += G.tiles_m * G.tiles_n;
+      tiles = gemm_tiles(G, tiles);
     }
     granges.push_back({q, e, tiles});
     q = e;
@@ -1493,7 +1498,6 @@ struct EnvJob {
   int z;              // 1: apply diag(d0, d1) on the physical index of this site
   double d0 = 1.0, d1 = -1.0;
   int kap = 1;        // Kraus leg of the site, traced with the physical index
-  const void* Abra = nullptr;  // bra-side site when it differs from A (projected copies)
 };
 
 // left step: E'(cr x cr) = A^H D (E A), D = diag(+-1) on the physical index when z; the two
@@ -1505,16 +1509,16 @@ void env_tasks_left(const EnvJob& j, GemmTask& a, GemmTask& b) {
   a.B = j.A; a.ldb = d * j.cr;
   a.C = j.X; a.ldc = d * j.cr;
   a.M = j.cl; a.N = d * j.cr; a.K = j.cl;
-  a.tiles_m = (a.M + 31) / 32; a.tiles_n = (a.N + 31) / 32;
+  (void)gemm_tiles(a, 0);
   memset(&b, 0, sizeof(b));
-  b.A = j.Abra ? j.Abra : j.A; b.lda = j.cr;
+  b.A = j.A; b.lda = j.cr;
   b.B = j.X; b.ldb = j.cr;
   b.C = j.Eout; b.ldc = j.cr;
   b.M = j.cr; b.N = j.cr; b.K = d * j.cl;
   b.sign_div = j.z ? j.kap : 0;
   b.kd0 = j.d0;
   b.kd1 = j.d1;
-  b.tiles_m = (b.M + 31) / 32; b.tiles_n = (b.N + 31) / 32;
+  (void)gemm_tiles(b, 0);
 }
 
 // right step: E'(cl x cl) = conj(A) (A R^T)^T with the physical sign when z
@@ -1525,7 +1529,7 @@ void env_tasks_right(const EnvJob& j, GemmTask& a, GemmTask& b) {
   a.B = j.Ein; a.ldb = j.cr;               // R^T
   a.C = j.X; a.ldc = j.cr;
   a.M = d * j.cl; a.N = j.cr; a.K = j.cr;
-  a.tiles_m = (a.M + 31) / 32; a.tiles_n = (a.N + 31) / 32;
+  (void)gemm_tiles(a, 0);
   memset(&b, 0, sizeof(b));
   b.A = j.A; b.lda = d * j.cr;             // conj, cl x (d cr)
   b.B = j.X; b.ldb = d * j.cr;             // X viewed cl x (d cr), transposed
@@ -1534,11 +1538,11 @@ void env_tasks_right(const EnvJob& j, GemmTask& a, GemmTask& b) {
   b.sign_div = j.z ? j.kap * j.cr : 0;
   b.kd0 = j.d0;
   b.kd1 = j.d1;
-  b.tiles_m = (b.M + 31) / 32; b.tiles_n = (b.N + 31) / 32;
+  (void)gemm_tiles(b, 0);
 }
 
-// independent steps, one launch per GEMM for all of them
-int env_steps(hipmps_engine E, std::vector<EnvJob>& jobs, bool left, int fp32) {
+// independent left steps, one launch per GEMM for all of them
+int env_steps(hipmps_engine E, std::vector<EnvJob>& jobs, int fp32) {
   if (jobs.empty()) return 0;
   const int N = (int)jobs.size();
   RC_TRY(E->hdesc.ensure(2 * N * sizeof(GemmTask)));
@@ -1546,130 +1550,180 @@ int env_steps(hipmps_engine E, std::vector<EnvJob>& jobs, bool left, int fp32) {
   GemmTask* h = (GemmTask*)E->hdesc.p;
   int t1 = 0, t2 = 0;
   for (int q = 0; q < N; ++q) {
-    GemmTask& a = h[q];
-    GemmTask& b = h[N + q];
-    if (left) env_tasks_left(jobs[q], a, b);
-    else env_tasks_right(jobs[q], a, b);
-    a.tile_begin = t1; t1 += a.tiles_m * a.tiles_n;
-    b.tile_begin = t2; t2 += b.tiles_m * b.tiles_n;
+    env_tasks_left(jobs[q], h[q], h[N + q]);
+    t1 = gemm_tiles(h[q], t1);
+    t2 = gemm_tiles(h[N + q], t2);
   }
   GemmTask* d = (GemmTask*)E->desc.p;
   HIP_TRY(hipMemcpyAsync(d, h, 2 * N * sizeof(GemmTask), hipMemcpyHostToDevice, E->stream));
-  if (left) {
-    HIP_TRY(launch_gemm(d, N, t1, 0, 0, 0, fp32, 0, E->stream));
-    HIP_TRY(launch_gemm(d + N, N, t2, 2, 0, fp32, 0, 0, E->stream));
-  } else {
-    HIP_TRY(launch_gemm(d, N, t1, 0, 3, fp32, 0, 0, E->stream));
-    HIP_TRY(launch_gemm(d + N, N, t2, 1, 3, fp32, 0, 0, E->stream));
-  }
+  HIP_TRY(launch_gemm(d, N, t1, 0, 0, 0, fp32, 0, E->stream));
+  HIP_TRY(launch_gemm(d + N, N, t2, 2, 0, fp32, 0, 0, E->stream));
   HIP_TRY(hipStreamSynchronize(E->stream));  // staging reuse
   return 0;
 }
 
-int env_left(hipmps_engine E, std::vector<EnvJob>& jobs, int fp32) { return env_steps(E, jobs, true, fp32); }
-int env_right(hipmps_engine E, std::vector<EnvJob>& jobs, int fp32) { return env_steps(E, jobs, false, fp32); }
-
-// a chain of steps, each reading the environment the one before wrote (a sweep over the
-// sites): every descriptor is staged at once and the steps launch back to back in stream
-// order (the X scratch they share is rewritten only after the step before has read it), with
-// one synchronisation at the end instead of one per site
-int env_chain(hipmps_engine E, const std::vector<EnvJob>& jobs, bool left, int fp32) {
-  if (jobs.empty()) return 0;
-  const int N = (int)jobs.size();
-  RC_TRY(E->hdesc.ensure(2 * N * sizeof(GemmTask)));
-  RC_TRY(E->desc.ensure(2 * N * sizeof(GemmTask)));
-  GemmTask* h = (GemmTask*)E->hdesc.p;
-  for (int q = 0; q < N; ++q) {
-    if (left) env_tasks_left(jobs[q], h[2 * q], h[2 * q + 1]);
-    else env_tasks_right(jobs[q], h[2 * q], h[2 * q + 1]);
-  }
-  GemmTask* d = (GemmTask*)E->desc.p;
-  HIP_TRY(hipMemcpyAsync(d, h, 2 * N * sizeof(GemmTask), hipMemcpyHostToDevice, E->stream));
-  for (int q = 0; q < N; ++q) {
-    const GemmTask& a = h[2 * q];
-    const GemmTask& b = h[2 * q + 1];
-    if (left) {
-      HIP_TRY(launch_gemm(d + 2 * q, 1, a.tiles_m * a.tiles_n, 0, 0, 0, fp32, 0, E->stream));
-      HIP_TRY(launch_gemm(d + 2 * q + 1, 1, b.tiles_m * b.tiles_n, 2, 0, fp32, 0, 0, E->stream));
-    } else {
-      HIP_TRY(launch_gemm(d + 2 * q, 1, a.tiles_m * a.tiles_n, 0, 3, fp32, 0, 0, E->stream));
-      HIP_TRY(launch_gemm(d + 2 * q + 1, 1, b.tiles_m * b.tiles_n, 1, 3, fp32, 0, 0, E->stream));
-    }
-  }
-  HIP_TRY(hipStreamSynchronize(E->stream));  // staging reuse
-  return 0;
-}
-
-// environment storage: all left (L_0..L_n) and right (R_0..R_n) environments + scratch
+// Environments of a measurement.  Every site's X_k = L_k A_k (chi_k x d_k x chi_(k+1)) and, with
+// `right`, P_k = A_k R_(k+1)^T of the same shape are kept: with them <Z_k> and the end of a <ZZ> pair
+// are one dot product each, sum_e z_e X_e conj(P_e) (R is Hermitian), instead of two more products
+// and a trace.  Environments themselves only live from one step to the next (two buffers a chain),
+// so a sweep without `keep` holds one X.
 struct EnvLayout {
-  std::vector<size_t> offL, offR;
-  size_t offX = 0, offT = 0, total = 0;
+  size_t mat = 0;                 // bytes of one environment
+  size_t L = 0, R = 0;            // two environments each
+  std::vector<size_t> X, P;       // per site
+  size_t total = 0;
 };
 
-EnvLayout env_layout(const hipmps_state_s* s, size_t extra_mats, size_t extra_elems) {
-  EnvLayout L;
-  size_t off = 0;
-  L.offL.resize(s->n + 1);
-  L.offR.resize(s->n + 1);
+EnvLayout env_layout(const hipmps_state_s* s, bool keep, bool right) {
+  EnvLayout E;
   int cmax = 1;
+  size_t xmax = 1;
   for (int k = 0; k <= s->n; ++k) cmax = std::max(cmax, s->chi[k]);
-  for (int k = 0; k <= s->n; ++k) {
-    L.offL[k] = off;
-    off = align_up(off + (size_t)s->chi[k] * s->chi[k] * 16);
+  for (int k = 0; k < s->n; ++k) xmax = std::max(xmax, site_elems(s, k));
+  E.mat = align_up((size_t)cmax * cmax * 16);
+  size_t off = 2 * E.mat;
+  if (right) {
+    E.R = off;
+    off += 2 * E.mat;
   }
-  for (int k = 0; k <= s->n; ++k) {
-    L.offR[k] = off;
-    off = align_up(off + (size_t)s->chi[k] * s->chi[k] * 16);
+  for (int side = 0; side < (right ? 2 : 1); ++side) {
+    std::vector<size_t>& v = side ? E.P : E.X;
+    v.resize(s->n);
+    for (int k = 0; k < s->n; ++k) {
+      v[k] = off;
+      if (keep) off += align_up(site_elems(s, k) * 16);
+    }
+    if (!keep) off += align_up(xmax * 16);
   }
-  L.offX = off;
-  off = align_up(off + align_up((size_t)cmax * 2 * max_kap(s) * cmax * 16) * std::max<size_t>(1, extra_mats));
-  L.offT = off;
-  off = align_up(off + std::max<size_t>(extra_elems, 1) * 16);
-  L.total = off;
-  return L;
+  E.total = off;
+  return E;
 }
 
-// diag: empty (identity everywhere) or 2n values diag(d_k0, d_k1) per site
-int compute_left_envs_diag(hipmps_state_s* s, const EnvLayout& L, const std::vector<double>& diag) {
-  hipmps_engine E = s->e;
-  char* base = (char*)E->env.p;
-  HIP_TRY(launch_fill_identity1((double2*)(base + L.offL[0]), E->stream));
+// jobs of the left sweep (ends in environment buffer n % 2) and of the right one, in their order
+std::vector<EnvJob> left_jobs(hipmps_state_s* s, const EnvLayout& L, char* base, const std::vector<double>& diag) {
   std::vector<EnvJob> jobs(s->n);
   for (int k = 0; k < s->n; ++k) {
-    jobs[k] = {s->sites[k].p, s->chi[k], s->chi[k + 1], (const double2*)(base + L.offL[k]),
-               (double2*)(base + L.offX), (double2*)(base + L.offL[k + 1]), 0};
-    jobs[k].kap = s->kap[k];
+    EnvJob& j = jobs[k];
+    j = {s->sites[k].p, s->chi[k], s->chi[k + 1], (const double2*)(base + L.L + (k & 1) * L.mat),
+         (double2*)(base + L.X[k]), (double2*)(base + L.L + ((k + 1) & 1) * L.mat), 0};
+    j.kap = s->kap[k];
     if (!diag.empty() && !(diag[2 * k] == 1.0 && diag[2 * k + 1] == 1.0)) {
-      jobs[k].z = 1;
-      jobs[k].d0 = diag[2 * k];
-      jobs[k].d1 = diag[2 * k + 1];
+      j.z = 1;
+      j.d0 = diag[2 * k];
+      j.d1 = diag[2 * k + 1];
     }
   }
-  return env_chain(E, jobs, true, s->fp32);
+  return jobs;
 }
 
-int compute_left_envs(hipmps_state_s* s, const EnvLayout& L, const std::vector<int>& zmask) {
-  std::vector<double> diag;
-  if (!zmask.empty()) {
-    diag.assign(2 * s->n, 1.0);
-    for (int k = 0; k < s->n; ++k)
-      if (zmask[k]) diag[2 * k + 1] = -1.0;
-  }
-  return compute_left_envs_diag(s, L, diag);
-}
-
-int compute_right_envs(hipmps_state_s* s, const EnvLayout& L) {
-  hipmps_engine E = s->e;
-  char* base = (char*)E->env.p;
-  HIP_TRY(launch_fill_identity1((double2*)(base + L.offR[s->n]), E->stream));
+std::vector<EnvJob> right_jobs(hipmps_state_s* s, const EnvLayout& L, char* base) {
   std::vector<EnvJob> jobs;
   for (int k = s->n - 1; k >= 0; --k) {
-    EnvJob j{s->sites[k].p, s->chi[k], s->chi[k + 1], (const double2*)(base + L.offR[k + 1]),
-             (double2*)(base + L.offX), (double2*)(base + L.offR[k]), 0};
+    EnvJob j{s->sites[k].p, s->chi[k], s->chi[k + 1], (const double2*)(base + L.R + ((k + 1) & 1) * L.mat),
+             (double2*)(base + L.P[k]), (double2*)(base + L.R + (k & 1) * L.mat), 0};
     j.kap = s->kap[k];
     jobs.push_back(j);
   }
-  return env_chain(E, jobs, false, s->fp32);
+  return jobs;
+}
+
+// Measurement plan of one state: GEMM tasks and dot tasks staged in one buffer, one upload, then every
+// launch back to back.  The left sweep runs on the engine's stream, the right one beside it on the
+// first lane's: each is a chain of small products, bound by their latency.
+struct EnvPlan {
+  std::vector<GemmTask> g;
+  std::vector<DotTask> dots;
+  struct Launch {
+    size_t off;
+    int n, tiles, kind;  // kind 0: E A, 1: A^H X, 2: A R^T, 3: conj(A) X^T
+    bool second;         // on the right sweep's stream
+  };
+  std::vector<Launch> sweeps, steps;  // steps: after both sweeps
+  void add(std::vector<Launch>& to, const std::vector<GemmTask>& tasks, int kind, bool second) {
+    Launch l{g.size(), (int)tasks.size(), 0, kind, second};
+    for (GemmTask t : tasks) {
+      l.tiles = gemm_tiles(t, l.tiles);
+      g.push_back(t);
+    }
+    if (l.n > 0) to.push_back(l);
+  }
+};
+
+// runs the plan; with dots, their values go to `out`; *last: the final left environment (1 x 1)
+int env_run(hipmps_state_s* s, const EnvLayout& L, EnvPlan& P, std::vector<double>* out, double* last) {
+  hipmps_engine E = s->e;
+  char* base = (char*)E->env.p;
+  const hipStream_t st = E->stream;
+  const size_t gb = align_up(P.g.size() * sizeof(GemmTask)), db = align_up(P.dots.size() * sizeof(DotTask));
+  const size_t rb = P.dots.size() * DOT_BLOCKS * sizeof(double);
+  RC_TRY(E->desc.ensure(gb + db + rb));
+  RC_TRY(E->hdesc.ensure(gb + db + rb + sizeof(double2)));
+  char* h = (char*)E->hdesc.p;
+  char* d = (char*)E->desc.p;
+  if (!P.g.empty()) memcpy(h, P.g.data(), P.g.size() * sizeof(GemmTask));
+  if (!P.dots.empty()) memcpy(h + gb, P.dots.data(), P.dots.size() * sizeof(DotTask));
+  HIP_TRY(hipMemcpyAsync(d, h, gb + db, hipMemcpyHostToDevice, st));
+  bool two = false;
+  for (const auto& l : P.sweeps) two = two || l.second;
+  HIP_TRY(launch_fill_identity1((double2*)(base + L.L), st));
+  if (two) HIP_TRY(launch_fill_identity1((double2*)(base + L.R + (s->n & 1) * L.mat), st));
+  const hipStream_t s2 = two && E->lane_stream[1] && E->lane_ev[0] && E->lane_ev[1] ? E->lane_stream[1] : st;
+  auto run = [&](const std::vector<EnvPlan::Launch>& v) -> int {
+    static const int opa[4] = {0, 2, 0, 1}, opb[4] = {0, 0, 3, 3};
+    for (const auto& l : v) {
+      const int ta = l.kind == 0 ? 0 : s->fp32, tb = l.kind == 0 ? s->fp32 : 0;
+      HIP_TRY(launch_gemm((const GemmTask*)d + l.off, l.n, l.tiles, opa[l.kind], opb[l.kind], ta, tb, 0,
+                          l.second ? s2 : st));
+    }
+    return 0;
+  };
+  if (s2 != st) {
+    HIP_TRY(hipEventRecord(E->lane_ev[0], st));
+    HIP_TRY(hipStreamWaitEvent(s2, E->lane_ev[0], 0));
+  }
+  RC_TRY(run(P.sweeps));
+  if (s2 != st) {
+    HIP_TRY(hipEventRecord(E->lane_ev[1], s2));
+    HIP_TRY(hipStreamWaitEvent(st, E->lane_ev[1], 0));
+  }
+  RC_TRY(run(P.steps));
+  double* hr = (double*)(h + gb + db);
+  double2* hl = (double2*)(h + gb + db + rb);
+  if (!P.dots.empty()) {
+    HIP_TRY(launch_dot((const DotTask*)(d + gb), (double*)(d + gb + db), (int)P.dots.size(), st));
+    HIP_TRY(hipMemcpyAsync(hr, d + gb + db, rb, hipMemcpyDeviceToHost, st));
+  }
+  if (last)
+    HIP_TRY(hipMemcpyAsync(hl, base + L.L + (s->n & 1) * L.mat, sizeof(double2), hipMemcpyDeviceToHost, st));
+  HIP_TRY(hipStreamSynchronize(st));  // staging reuse
+  if (last) *last = hl->x;
+  if (out) {
+    out->assign(P.dots.size(), 0.0);
+    for (size_t t = 0; t < P.dots.size(); ++t)
+      for (int b = 0; b < DOT_BLOCKS; ++b) (*out)[t] += hr[t * DOT_BLOCKS + b];
+  }
+  return 0;
+}
+
+// the sweeps' launches; the two sweeps' steps alternate, so that both streams are fed
+void env_sweeps(EnvPlan& P, const std::vector<EnvJob>& left, const std::vector<EnvJob>& right) {
+  GemmTask a, b;
+  for (size_t k = 0; k < std::max(left.size(), right.size()); ++k) {
+    if (k < left.size()) {
+      env_tasks_left(left[k], a, b);
+      P.add(P.sweeps, {a}, 0, false);
+      P.add(P.sweeps, {b}, 1, false);
+    }
+    if (k < right.size()) {
+      env_tasks_right(right[k], a, b);
+      P.add(P.sweeps, {a}, 2, true);
+      P.add(P.sweeps, {b}, 3, true);
+    }
+  }
+}
+
+DotTask site_dot(const hipmps_state_s* s, int k, const void* x, const void* p, double z1) {
+  return {(const double2*)x, (const double2*)p, s->chi[k], 2 * s->kap[k], s->chi[k + 1], 1.0, z1};
 }
 
 int read_scalar(hipmps_engine E, const void* dptr, double2* out) {
@@ -1705,143 +1759,247 @@ int trace_products(hipmps_engine E, const std::vector<const double2*>& A, const 
   return 0;
 }
 
-// <Z_i> for every site; with norm, also <psi|psi> (the closed left environment L_n against the
-// identity R_n, one more pair of the same trace products)
+// <Z_i> for every site; with norm, also <psi|psi> (the closed left environment)
 int measure_z_all(hipmps_state_s* s, double* out, double* norm = nullptr) {
   hipmps_engine E = s->e;
-  const int n = s->n;
-  int cmax = 1;
-  for (int k = 0; k <= n; ++k) cmax = std::max(cmax, s->chi[k]);
-  // M_i buffers (n of them) + pointer tables
-  size_t mbytes = 0;
-  std::vector<size_t> offM(n);
-  for (int i = 0; i < n; ++i) {
-    offM[i] = mbytes;
-    mbytes = align_up(mbytes + (size_t)s->chi[i + 1] * s->chi[i + 1] * 16);
-  }
-  EnvLayout L = env_layout(s, (size_t)n, mbytes / 16 + 4096);
+  const EnvLayout L = env_layout(s, true, true);
   RC_TRY(E->env.ensure(L.total));
   char* base = (char*)E->env.p;
-  RC_TRY(compute_left_envs(s, L, {}));
-  RC_TRY(compute_right_envs(s, L));
-  // M_i = env update of L_i with Z at i (batched); X scratch per job
-  std::vector<EnvJob> jobs;
-  size_t xstride = align_up((size_t)cmax * 2 * max_kap(s) * cmax * 16);
-  for (int i = 0; i < n; ++i) {
-    jobs.push_back({s->sites[i].p, s->chi[i], s->chi[i + 1], (const double2*)(base + L.offL[i]),
-                    (double2*)(base + L.offX + i * xstride), (double2*)(base + L.offT + offM[i]), 1});
-    jobs.back().kap = s->kap[i];
-  }
-  RC_TRY(env_left(E, jobs, s->fp32));
-  std::vector<const double2*> A, B;
-  std::vector<int> dims;
-  for (int i = 0; i < n; ++i) {
-    A.push_back((const double2*)(base + L.offT + offM[i]));
-    B.push_back((const double2*)(base + L.offR[i + 1]));
-    dims.push_back(s->chi[i + 1]);
-  }
-  if (norm) {
-    A.push_back((const double2*)(base + L.offL[n]));
-    B.push_back((const double2*)(base + L.offR[n]));
-    dims.push_back(s->chi[n]);
-  }
-  std::vector<double2> res;
-  // pointer tables go right after the M buffers
-  RC_TRY(trace_products(E, A, B, dims, base + L.offT + align_up(mbytes), res));
-  for (int i = 0; i < n; ++i) out[i] = res[i].x;
-  if (norm) *norm = res[n].x;
+  EnvPlan P;
+  env_sweeps(P, left_jobs(s, L, base, {}), right_jobs(s, L, base));
+  for (int i = 0; i < s->n; ++i) P.dots.push_back(site_dot(s, i, base + L.X[i], base + L.P[i], -1.0));
+  std::vector<double> v;
+  RC_TRY(env_run(s, L, P, &v, norm));
+  std::copy(v.begin(), v.end(), out);
   return 0;
 }
 
+// <Z_i Z_j> of pairs i < j: one chain per distinct i, from M_i = A_i^H Z X_i on, advanced together;
+// at every site j that ends a pair, X = M A_j against P_j
 int measure_zz(hipmps_state_s* s, const int* pairs, int k, double* out) {
   hipmps_engine E = s->e;
   const int n = s->n;
-  int cmax = 1;
-  for (int b = 0; b <= n; ++b) cmax = std::max(cmax, s->chi[b]);
-  size_t mat = align_up((size_t)cmax * cmax * 16);
-  size_t xmat = align_up((size_t)cmax * 2 * max_kap(s) * cmax * 16);
-  EnvLayout L = env_layout(s, 1, 0);
-  size_t per_pair = 2 * mat + xmat;
-  size_t total = L.total + per_pair * (size_t)k + 4096 + (size_t)k * 64;
-  RC_TRY(E->env.ensure(total));
-  char* base = (char*)E->env.p;
-  RC_TRY(compute_left_envs(s, L, {}));
-  RC_TRY(compute_right_envs(s, L));
-  char* pb = base + L.total;
-  struct P { int i, j, cur; int pp; };
-  std::vector<P> ps(k);
-  std::vector<double> norm_val(1, 0.0);
-  double2 nrm;
-  RC_TRY(read_scalar(E, base + L.offL[n], &nrm));
+  std::vector<std::vector<int>> ends(n);  // per first site: the sites at which its pairs end
   for (int t = 0; t < k; ++t) {
-    int a = pairs[2 * t], b = pairs[2 * t + 1];
+    const int a = pairs[2 * t], b = pairs[2 * t + 1];
     if (a < 0 || a >= n || b < 0 || b >= n) return fail(HIPMPS_E_ARG, "zz pair out of range");
-    if (a > b) std::swap(a, b);
-    ps[t] = {a, b, a, 0};
+    if (a != b) ends[std::min(a, b)].push_back(std::max(a, b));
   }
-  // advance all pairs in lock-step
-  bool any = true;
-  while (any) {
-    any = false;
-    std::vector<EnvJob> jobs;
-    std::vector<int> who;
-    for (int t = 0; t < k; ++t) {
-      P& p = ps[t];
-      if (p.i == p.j || p.cur > p.j) continue;
-      any = true;
-      char* buf = pb + per_pair * t;
-      const double2* ein = (p.cur == p.i) ? (const double2*)(base + L.offL[p.i]) : (const double2*)(buf + mat * p.pp);
-      double2* eout = (double2*)(buf + mat * (1 - p.pp));
-      int z = (p.cur == p.i || p.cur == p.j) ? 1 : 0;
-      jobs.push_back({s->sites[p.cur].p, s->chi[p.cur], s->chi[p.cur + 1], ein, (double2*)(buf + 2 * mat), eout, z});
-      jobs.back().kap = s->kap[p.cur];
-      who.push_back(t);
-    }
-    if (!any) break;
-    RC_TRY(env_left(E, jobs, s->fp32));
-    for (int t : who) {
-      ps[t].cur++;
-      ps[t].pp = 1 - ps[t].pp;
-    }
+  EnvLayout L = env_layout(s, true, true);
+  size_t xmax = 1;
+  for (int q = 0; q < n; ++q) xmax = std::max(xmax, site_elems(s, q));
+  // a chain holds two environments, the X of every site at which a pair ends (the dot products run
+  // after all steps) and one X for the sites between
+  struct Chain {
+    int i, last;
+    size_t E, X;                 // offsets; X: scratch of the sites where no pair ends
+    std::vector<size_t> Xend;    // per site i + 1 .. last: offset, or 0
+  };
+  std::vector<Chain> chains;
+  size_t off = L.total;
+  for (int i = 0; i < n; ++i) {
+    if (ends[i].empty()) continue;
+    Chain c;
+    c.i = i;
+    c.last = *std::max_element(ends[i].begin(), ends[i].end());
+    c.E = off;
+    off += 2 * L.mat;
+    c.X = off;
+    off += align_up(xmax * 16);
+    c.Xend.assign(c.last - i + 1, 0);
+    for (int j : ends[i])
+      if (!c.Xend[j - i]) {
+        c.Xend[j - i] = off;
+        off += align_up(site_elems(s, j) * 16);
+      }
+    chains.push_back(std::move(c));
   }
-  std::vector<const double2*> A, B;
-  std::vector<int> dims, idx;
+  RC_TRY(E->env.ensure(off));
+  char* base = (char*)E->env.p;
+  EnvPlan P;
+  env_sweeps(P, left_jobs(s, L, base, {}), right_jobs(s, L, base));
+  std::map<std::pair<int, int>, size_t> where;
+  for (int step = 0;; ++step) {
+    std::vector<GemmTask> ket, bra;
+    for (const Chain& c : chains) {
+      const int site = c.i + step;
+      if (site > c.last) continue;
+      const size_t xo = step == 0 ? L.X[site] : (c.Xend[step] ? c.Xend[step] : c.X);
+      EnvJob j{s->sites[site].p, s->chi[site], s->chi[site + 1],
+               (const double2*)(base + c.E + (step & 1) * L.mat), (double2*)(base + xo),
+               (double2*)(base + c.E + ((step + 1) & 1) * L.mat), step == 0 ? 1 : 0};
+      j.kap = s->kap[site];
+      GemmTask a, b;
+      env_tasks_left(j, a, b);
+      if (step > 0) ket.push_back(a);
+      if (site < c.last) bra.push_back(b);
+      if (step > 0 && c.Xend[step]) {
+        where[{c.i, site}] = P.dots.size();
+        P.dots.push_back(site_dot(s, site, base + xo, base + L.P[site], -1.0));
+      }
+    }
+    if (ket.empty() && bra.empty()) break;
+    P.add(P.steps, ket, 0, false);
+    P.add(P.steps, bra, 1, false);
+  }
+  std::vector<double> v;
+  double norm = 0.0;
+  RC_TRY(env_run(s, L, P, &v, &norm));
   for (int t = 0; t < k; ++t) {
-    P& p = ps[t];
-    if (p.i == p.j) {
-      out[t] = nrm.x;  // Z_i Z_i = I
-      continue;
-    }
-    A.push_back((const double2*)(pb + per_pair * t + mat * p.pp));
-    B.push_back((const double2*)(base + L.offR[p.j + 1]));
-    dims.push_back(s->chi[p.j + 1]);
-    idx.push_back(t);
+    const int a = pairs[2 * t], b = pairs[2 * t + 1];
+    out[t] = a == b ? norm : v[where[{std::min(a, b), std::max(a, b)}]];  // Z_i Z_i = I
   }
-  std::vector<double2> res;
-  RC_TRY(trace_products(E, A, B, dims, pb + per_pair * k, res));
-  for (size_t q = 0; q < idx.size(); ++q) out[idx[q]] = res[q].x;
   return 0;
+}
+
+// <psi| (x)_k diag(d[2k], d[2k+1]) |psi>, diag empty: <psi|psi>
+int measure_diag(hipmps_state_s* s, const std::vector<double>& diag, double* out) {
+  hipmps_engine E = s->e;
+  const EnvLayout L = env_layout(s, false, false);
+  RC_TRY(E->env.ensure(L.total));
+  EnvPlan P;
+  env_sweeps(P, left_jobs(s, L, (char*)E->env.p, diag), {});
+  return env_run(s, L, P, nullptr, out);
 }
 
 int measure_parity(hipmps_state_s* s, const std::vector<int>& zmask, double* out) {
+  std::vector<double> diag;
+  if (!zmask.empty()) {
+    diag.assign(2 * s->n, 1.0);
+    for (int k = 0; k < s->n; ++k)
+      if (zmask[k]) diag[2 * k + 1] = -1.0;
+  }
+  return measure_diag(s, diag, out);
+}
+
+// all right environments R_0 .. R_n, kept (sampling), with one X for the sweep
+struct RightEnvs {
+  std::vector<size_t> R;
+  size_t X = 0, total = 0;
+};
+
+RightEnvs right_env_layout(const hipmps_state_s* s) {
+  RightEnvs L;
+  size_t xmax = 1;
+  for (int k = 0; k < s->n; ++k) xmax = std::max(xmax, site_elems(s, k));
+  for (int k = 0; k <= s->n; ++k) {
+    L.R.push_back(L.total);
+    L.total += align_up((size_t)s->chi[k] * s->chi[k] * 16);
+  }
+  L.X = L.total;
+  L.total += align_up(xmax * 16);
+  return L;
+}
+
+int compute_right_envs(hipmps_state_s* s, const RightEnvs& L) {
   hipmps_engine E = s->e;
-  EnvLayout L = env_layout(s, 1, 0);
-  RC_TRY(E->env.ensure(L.total));
-  RC_TRY(compute_left_envs(s, L, zmask));
-  double2 v;
-  RC_TRY(read_scalar(E, (char*)E->env.p + L.offL[s->n], &v));
-  *out = v.x;
+  char* base = (char*)E->env.p;
+  const size_t bytes = 2 * (size_t)s->n * sizeof(GemmTask);
+  RC_TRY(E->hdesc.ensure(bytes));
+  RC_TRY(E->desc.ensure(bytes));
+  GemmTask* h = (GemmTask*)E->hdesc.p;
+  const GemmTask* d = (const GemmTask*)E->desc.p;
+  for (int k = s->n - 1; k >= 0; --k) {
+    EnvJob j{s->sites[k].p, s->chi[k], s->chi[k + 1], (const double2*)(base + L.R[k + 1]), (double2*)(base + L.X),
+             (double2*)(base + L.R[k]), 0};
+    j.kap = s->kap[k];
+    env_tasks_right(j, h[2 * k], h[2 * k + 1]);
+  }
+  HIP_TRY(hipMemcpyAsync(E->desc.p, h, bytes, hipMemcpyHostToDevice, E->stream));
+  HIP_TRY(launch_fill_identity1((double2*)(base + L.R[s->n]), E->stream));
+  for (int k = s->n - 1; k >= 0; --k)
+    for (int g = 0; g < 2; ++g) {
+      const GemmTask& t = h[2 * k + g];
+      HIP_TRY(launch_gemm(d + 2 * k + g, 1, t.tiles_m * t.tiles_n, g, 3, s->fp32, 0, 0, E->stream));
+    }
+  HIP_TRY(hipStreamSynchronize(E->stream));  // staging reuse
   return 0;
 }
 
-int measure_diag(hipmps_state_s* s, const std::vector<double>& diag, double* out) {
+// sample_measure with factored environments: per site one product for all shots, and at a measured one
+// a second against the right environment and the choice, all on the device
+int sample_factored(hipmps_state_s* s, const int* qubits, int k, int shots, const double* draws, char* out,
+                    const RightEnvs& L, size_t row_elems) {
   hipmps_engine E = s->e;
-  EnvLayout L = env_layout(s, 1, 0);
-  RC_TRY(E->env.ensure(L.total));
-  RC_TRY(compute_left_envs_diag(s, L, diag));
-  double2 v;
-  RC_TRY(read_scalar(E, (char*)E->env.p + L.offL[s->n], &v));
-  *out = v.x;
+  const hipStream_t st = E->stream;
+  const int n = s->n;
+  // per shot: V, X and U of at most row_elems elements, its draws, characters and f
+  const size_t per_shot = 3 * row_elems * 16 + (size_t)k * 9 + 8;
+  const size_t budget = std::max<size_t>((size_t)256 << 20, 8 * per_shot);
+  const size_t limit = std::min<size_t>(budget / per_shot, ((size_t)1 << 30) / row_elems);
+  const int B = (int)std::max<size_t>(1, std::min<size_t>((size_t)shots, limit));
+  const size_t vb = align_up(B * row_elems * 16), drb = align_up((size_t)B * k * 8), fb = align_up((size_t)B * 8);
+  RC_TRY(E->env.ensure(L.total + 3 * vb + drb + fb + align_up((size_t)B * k)));
+  char* base = (char*)E->env.p;
+  RC_TRY(compute_right_envs(s, L));
+  double2* V = (double2*)(base + L.total);
+  double2* X = (double2*)(base + L.total + vb);
+  double2* U = (double2*)(base + L.total + 2 * vb);
+  double* d_draws = (double*)(base + L.total + 3 * vb);
+  double* d_f = (double*)(base + L.total + 3 * vb + drb);
+  char* d_out = base + L.total + 3 * vb + drb + fb;
+  for (int s0 = 0; s0 < shots; s0 += B) {
+    const int nb = std::min(B, shots - s0);
+    // the products of every site up to the last measured one; the buffers V, X, U change roles
+    std::vector<GemmTask> g;
+    struct Step {
+      bool meas;
+      int rho, site;
+      double2 *v, *x, *u;
+    };
+    std::vector<Step> steps;
+    int rho = 1;
+    double2 *v = V, *x = X, *u = U;
+    for (int site = 0, mi = 0; site < n && mi < k; ++site) {
+      const bool meas = qubits[mi] == site;
+      const int cl = s->chi[site], cr = s->chi[site + 1], d = 2 * s->kap[site];
+      steps.push_back({meas, rho, site, v, x, u});
+      GemmTask a;
+      memset(&a, 0, sizeof(a));
+      a.A = v; a.lda = cl;                    // X = V A: (nb rho) x cl times cl x (d cr)
+      a.B = s->sites[site].p; a.ldb = d * cr;
+      a.C = x; a.ldc = d * cr;
+      a.M = nb * rho; a.N = d * cr; a.K = cl;
+      (void)gemm_tiles(a, 0);
+      g.push_back(a);
+      if (meas) {
+        memset(&a, 0, sizeof(a));
+        a.A = x; a.lda = cr;                  // U = X R^T: (nb rho d) x cr
+        a.B = base + L.R[site + 1]; a.ldb = cr;
+        a.C = u; a.ldc = cr;
+        a.M = nb * rho * d; a.N = cr; a.K = cr;
+        (void)gemm_tiles(a, 0);
+        g.push_back(a);
+        rho *= d / 2;                         // V' is written over V
+        ++mi;
+      } else {
+        rho *= d;                             // V' is X
+        std::swap(v, x);
+      }
+    }
+    RC_TRY(E->hdesc.ensure(g.size() * sizeof(GemmTask)));
+    RC_TRY(E->desc.ensure(g.size() * sizeof(GemmTask)));
+    memcpy(E->hdesc.p, g.data(), g.size() * sizeof(GemmTask));
+    HIP_TRY(hipMemcpyAsync(E->desc.p, E->hdesc.p, g.size() * sizeof(GemmTask), hipMemcpyHostToDevice, st));
+    HIP_TRY(hipMemcpyAsync(d_draws, draws + (size_t)s0 * k, (size_t)nb * k * 8, hipMemcpyHostToDevice, st));
+    HIP_TRY(launch_fill_c(V, (size_t)nb, make_double2(1.0, 0.0), st));  // E_t = [1]
+    HIP_TRY(launch_fill_c((double2*)d_f, (size_t)(nb + 1) / 2, make_double2(1.0, 1.0), st));
+    const GemmTask* dg = (const GemmTask*)E->desc.p;
+    int mi = 0;
+    size_t q = 0;
+    for (const Step& S : steps) {
+      HIP_TRY(launch_gemm(dg + q, 1, g[q].tiles_m * g[q].tiles_n, 0, 0, 0, s->fp32, 0, st));
+      ++q;
+      if (!S.meas) continue;
+      HIP_TRY(launch_gemm(dg + q, 1, g[q].tiles_m * g[q].tiles_n, 0, 3, 0, 0, 0, st));
+      ++q;
+      const SampleTask t{S.x, S.u, S.v, d_draws + mi, d_f, d_out + mi, k, nb, S.rho, s->kap[S.site], s->chi[S.site + 1]};
+      HIP_TRY(launch_sample_pick(t, st));
+      ++mi;
+    }
+    HIP_TRY(hipMemcpyAsync(out + (size_t)s0 * k, d_out, (size_t)nb * k, hipMemcpyDeviceToHost, st));
+    HIP_TRY(hipStreamSynchronize(st));  // staging reuse
+  }
   return 0;
 }
 
@@ -1857,11 +2015,26 @@ int measure_diag(hipmps_state_s* s, const std::vector<double>& diag, double* out
 int sample_measure(hipmps_state_s* s, const int* qubits, int k, int shots, const double* draws, char* out) {
   hipmps_engine E = s->e;
   const int n = s->n;
-  int cmax = 1;
+  int cmax = 1, kmax = max_kap(s);
   for (int b = 0; b <= n; ++b) cmax = std::max(cmax, s->chi[b]);
-  const EnvLayout L = env_layout(s, 1, 0);
+  RightEnvs L = right_env_layout(s);
+  // Factored environments, E_t = V^H V: a measured site keeps kap rows of V per row, a traced one 2 kap.
+  // With every site measured V is one row, and a site costs chi^2 per shot instead of chi^3.  Taken when
+  // its products are fewer: few traced sites, short Kraus legs.
+  double dense = 0.0, factored = 0.0, rho = 1.0, rows_max = 1.0;
+  for (int site = 0, mi = 0; site < n && mi < k; ++site) {
+    const double cl = s->chi[site], cr = s->chi[site + 1], d = 2.0 * s->kap[site];
+    const bool meas = qubits[mi] == site;
+    dense += (meas ? 2.0 : 1.0) * d * cl * cr * (cl + cr);
+    factored += rho * d * cr * (meas ? cl + cr : cl);
+    rho *= meas ? d / 2 : d;
+    rows_max = std::max(rows_max, std::max(rho * cr, meas ? 2.0 * rho * cr : 0.0));
+    mi += meas;
+  }
+  if (factored < dense && rows_max < (double)(1 << 24))
+    return sample_factored(s, qubits, k, shots, draws, out, L, (size_t)rows_max);
   const size_t mat = align_up((size_t)cmax * cmax * 16);
-  const size_t xs = align_up((size_t)cmax * 2 * max_kap(s) * cmax * 16);
+  const size_t xs = align_up((size_t)cmax * 2 * kmax * cmax * 16);
   const size_t per_shot = 3 * mat + 2 * xs;  // E and two candidates, two X scratches
   const size_t budget = std::max<size_t>((size_t)256 << 20, 8 * per_shot);
   const int B = (int)std::max<size_t>(1, std::min<size_t>((size_t)shots, budget / per_shot));
@@ -1901,7 +2074,7 @@ int sample_measure(hipmps_state_s* s, const int* qubits, int k, int shots, const
           jobs.push_back(j);
         }
       }
-      RC_TRY(env_steps(E, jobs, true, s->fp32));
+      RC_TRY(env_steps(E, jobs, s->fp32));
       if (!meas) {
         for (int t = 0; t < nb; ++t) cur[t] = (cur[t] + 1) % 3;
         continue;
@@ -1911,7 +2084,7 @@ int sample_measure(hipmps_state_s* s, const int* qubits, int k, int shots, const
       for (int t = 0; t < nb; ++t)
         for (int b = 0; b < 2; ++b) {
           A.push_back(mat_at(t, (cur[t] + 1 + b) % 3));
-          R.push_back((const double2*)(base + L.offR[site + 1]));
+          R.push_back((const double2*)(base + L.R[site + 1]));
           dims.push_back(s->chi[site + 1]);
         }
       std::vector<double2> pr;
@@ -1968,8 +2141,9 @@ struct RdmPlan {
 };
 
 constexpr size_t RDM_INT_MAX = ((size_t)1 << 31) - 1;
-// k_gemm runs one 256-thread block per tile and a dispatch holds at most 2^32 work-items
-constexpr size_t RDM_TILES_MAX = ((size_t)1 << 24) - 1;
+// tiles of a launch are counted in int (k_gemm: one block per tile)
+constexpr size_t RDM_TILES_MAX = (size_t)1 << 30;
+inline size_t rdm_tiles(size_t m, size_t n) { return ((m + GEMM_TM - 1) / GEMM_TM) * ((n + GEMM_TN - 1) / GEMM_TN); }
 
 // block of s that X holds for a site with `per` = cl |A| cr elements and `tiles` ket-side GEMM
 // tiles per s
@@ -1989,7 +2163,7 @@ int rdm_half(hipmps_engine E, const std::vector<RdmSite>& v, int fp32, size_t es
     const int cl = S.cl, d = S.d, cr = S.cr;
     char* out = (t + 1 == v.size()) ? dst : eb;
     const size_t per = (size_t)cl * nA * cr;
-    const int w = rdm_block(d, per, xcap, ((cl * nA + 31) / 32) * (((size_t)cr + 31) / 32));
+    const int w = rdm_block(d, per, xcap, rdm_tiles(cl * nA, (size_t)cr));
     const int nket = S.meas ? 2 : 1, nbra = nket;
     const int nch = (d + w - 1) / w;
     const size_t ndesc = (size_t)nket * (d + (size_t)nch * nbra);
@@ -2018,10 +2192,7 @@ int rdm_half(hipmps_engine E, const std::vector<RdmSite>& v, int fp32, size_t es
           g.N = cr;
           g.C = (double2*)xs + (size_t)sl * per;
           g.ldc = cr;
-          g.tiles_m = (g.M + 31) / 32;
-          g.tiles_n = (g.N + 31) / 32;
-          g.tile_begin = t1;
-          t1 += g.tiles_m * g.tiles_n;
+          t1 = gemm_tiles(g, t1);
         }
         launches.push_back({o, ws, t1, 0});
         o += ws;
@@ -2039,10 +2210,7 @@ int rdm_half(hipmps_engine E, const std::vector<RdmSite>& v, int fp32, size_t es
           g.C = (double2*)out + (size_t)slot * nA * cr;
           g.ldc = (int)((S.meas ? 4 : 1) * nA * cr);
           g.accumulate = s0 > 0;
-          g.tiles_m = (g.M + 31) / 32;
-          g.tiles_n = (g.N + 31) / 32;
-          g.tile_begin = t2;
-          t2 += g.tiles_m * g.tiles_n;
+          t2 = gemm_tiles(g, t2);
         }
         launches.push_back({o, nbra, t2, 1});
         o += nbra;
@@ -2095,18 +2263,18 @@ int measure_rdm(hipmps_state_s* s, const std::vector<int>& qubits, double* out) 
     max_e = std::max(max_e, std::max(P.el, P.er));
     P.es = max_e;
     P.xcap = std::max(max_e, (size_t)E->rdm_block_elems);
-    bool ok = cm * cm <= RDM_INT_MAX && ((P.nl + 31) / 32) * ((P.nr + 31) / 32) <= RDM_TILES_MAX;
+    bool ok = cm * cm <= RDM_INT_MAX && rdm_tiles(P.nl, P.nr) <= RDM_TILES_MAX;
     auto pass_x = [&](int q0, int q1, int step) {
       size_t nA = 1;
       for (int q = q0; q != q1; q += step) {
         const size_t cl = step > 0 ? s->chi[q] : s->chi[q + 1], cr = step > 0 ? s->chi[q + 1] : s->chi[q];
         const int d = 2 * s->kap[q];
         const size_t per = cl * nA * cr;
-        const size_t tiles = ((cl * nA + 31) / 32) * ((cr + 31) / 32);
+        const size_t tiles = rdm_tiles(cl * nA, cr);
         const int w = rdm_block(d, per, P.xcap, tiles);
         P.xs = std::max(P.xs, (size_t)w * per);
         ok = ok && cl * nA <= RDM_INT_MAX && tiles * w <= RDM_TILES_MAX && 4 * nA * cr <= RDM_INT_MAX &&
-             ((cr + 31) / 32) * ((nA * cr + 31) / 32) * 2 <= RDM_TILES_MAX && (size_t)w * cl <= RDM_INT_MAX;
+             rdm_tiles(cr, nA * cr) * 2 <= RDM_TILES_MAX && (size_t)w * cl <= RDM_INT_MAX;
         nA *= pos[q] >= 0 ? 4 : 1;
       }
     };
@@ -2217,8 +2385,7 @@ int measure_rdm(hipmps_state_s* s, const std::vector<int>& qubits, double* out) 
   g->N = (int)best.nr;
   g->C = cbuf;
   g->ldc = (int)best.nr;
-  g->tiles_m = (g->M + 31) / 32;
-  g->tiles_n = (g->N + 31) / 32;
+  (void)gemm_tiles(*g, 0);
   HIP_TRY(hipMemcpyAsync(E->desc.p, g, sizeof(GemmTask), hipMemcpyHostToDevice, st));
   HIP_TRY(launch_gemm((GemmTask*)E->desc.p, 1, g->tiles_m * g->tiles_n, 0, 3, 0, 0, 0, st));
   // joined label A_L |A_R| + A_R: the right half's measured sites (in its sweep order, from

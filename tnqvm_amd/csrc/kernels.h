@@ -93,6 +93,9 @@ struct SplitTask {
                          // 1: keep i (Kraus leg, ExaTnPmpsVisitor.cpp:1060-1072)
 };
 
+// Output tile of one k_gemm workgroup
+constexpr int GEMM_TM = 32, GEMM_TN = 16;
+
 // Generic batched complex GEMM: C (M x N) = rowscale . op(A) op(B) . colscale
 // op codes: 0 N, 1 C (conjugate), 2 H (conjugate transpose), 3 T (transpose).
 struct GemmTask {
@@ -200,6 +203,31 @@ hipError_t launch_chain(const ChainTask* d_tasks, int ntasks, int total_blocks, 
                         hipStream_t s);
 hipError_t launch_trace_prod(const double2* const* d_a, const double2* const* d_b,
                              const int* d_dims, double2* d_out, int ntasks, hipStream_t s);
+// sum_e z_e a[e] conj(b[e]) over the rows x d x cr elements e = ((l d) + s) cr + r, z_e = z[s >= d / 2]: the
+// expectation value of diag(z) on a site from X = L A and P = A R^T
+struct DotTask {
+  const double2* a;
+  const double2* b;
+  int rows, d, cr;
+  double z0, z1;
+};
+// One measured site of getMeasureSample for `shots` shots whose left environments are held as V^H V, V
+// (rho x chi) per shot: X = V A (rho d rows of chi_r per shot, d = 2 kap) and U = X R^T are given.  Per
+// shot: p_b = sum over the rows of outcome b of Re U conj(X), scaled by f (1e-12 cut to 0), bit = draw >
+// p_0, f /= p_bit, V' = the rows of the outcome (rho kap x chi_r).
+struct SampleTask {
+  const double2* X;
+  const double2* U;
+  double2* V;
+  const double* draws;  // draw of shot t: draws[t * stride]
+  double* f;
+  char* out;            // '0' / '1' of shot t: out[t * stride]
+  int stride, shots, rho, kap, cr;
+};
+hipError_t launch_sample_pick(const SampleTask& task, hipStream_t s);
+// DOT_BLOCKS partial sums per task, to be added in order
+constexpr int DOT_BLOCKS = 16;
+hipError_t launch_dot(const DotTask* d_tasks, double* d_out, int ntasks, hipStream_t s);
 hipError_t launch_check_finite(const void* p, size_t n_complex, int fp32, int* d_flag,
                                hipStream_t s);
 hipError_t launch_fill_identity1(double2* p, hipStream_t s);

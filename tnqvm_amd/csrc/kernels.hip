@@ -1074,110 +1074,112 @@ hipError_t launch_normalize(const SplitTask* d_split, int ntasks, int max_k, int
 //   b(k,j): N  B[k*ldb + j]       T B[gB(j)*ldb + k]   H conj(B[gB(j)*ldb + k])
 // optional diagonal operator diag(kd0, kd1) on a(i,k), selected by the physical index
 // (k / sign_div) & 1 (Z, projectors, ... inserted on the contracted physical leg).
-constexpr int GM = 32, GN = 32, GK = 16;
+//
+// FP64 MFMA, complex64 operands converted on the way in.  A workgroup owns a 32 x 16 tile of C and its
+// four waves split K (unit u of 4 to wave u mod 4, so that the four waves read whole lines of a row of
+// A), each streaming its operands from memory into MFMA registers, GEMM_PD units in flight; the four
+// partial tiles are summed in LDS in a fixed order.  No LDS staging and no barrier in the loop: the
+// operands of these products (environments, sites) are L2-resident, and a chain of them is bound by
+// each product's latency.  Split K and the small tile put a 256 x 512 x 256 product, one step of an
+// environment sweep at bond 256, on all 256 CUs (32 x 32 tiles through LDS on vector FMA took 38 to 60
+// us a step and half of the CUs).
+constexpr int GEMM_PD = 4;
 
 template <typename TA, typename TB, typename TC, int OPA, int OPB>
-__global__ __launch_bounds__(256) void k_gemm(const GemmTask* tasks, int ntasks) {
-  __shared__ double2 sA[GM][GK + 1];
-  __shared__ double2 sB[GK][GN + 1];
-  const int t = find_task(tasks, ntasks, (int)blockIdx.x, [](const GemmTask& x) { return x.tile_begin; });
+__global__ __launch_bounds__(256) void k_gemm(const GemmTask* tasks, int ntasks, int tile_base) {
+  __shared__ double2 sC[4][GEMM_TM][GEMM_TN + 1];
+  const int block = tile_base + (int)blockIdx.x;
+  const int t = find_task(tasks, ntasks, block, [](const GemmTask& x) { return x.tile_begin; });
   const GemmTask& T = tasks[t];
-  const int tile = blockIdx.x - T.tile_begin;
+  const int tile = block - T.tile_begin;
   if (tile >= T.tiles_m * T.tiles_n) return;
   int M = T.M, N = T.N;
   if (T.Mdyn) M = min(M, *T.Mdyn);
   if (T.Ndyn) N = min(N, *T.Ndyn);
-  const int i0 = (tile / T.tiles_n) * GM, j0 = (tile % T.tiles_n) * GN;
+  const int i0 = (tile / T.tiles_n) * GEMM_TM, j0 = (tile % T.tiles_n) * GEMM_TN;
   if (i0 >= M || j0 >= N) return;
-  const int Kd = T.K;
+  const int K = T.K;
   const int ldc = T.ldc > 0 ? T.ldc : N;
+  const size_t lda = T.lda, ldb = T.ldb;
   const TA* A = (const TA*)T.A;
   const TB* B = (const TB*)T.B;
-  const int tid = threadIdx.x;
-  const int ty = tid / 16, tx = tid % 16;
-  double2 acc[2][2];
+  const int sign_div = T.sign_div;
+  const double kd0 = T.kd0, kd1 = T.kd1;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int l16 = lane & 15, k4 = lane >> 4;
+  // rows of A and columns of B of this lane; past the end: a repeat, not stored
+  const int ia = min(i0 + l16, M - 1), ib = min(i0 + 16 + l16, M - 1), jb = min(j0 + l16, N - 1);
+  const bool a_rows = OPA == 0 || OPA == 1;
+  const TA* pa = A + (a_rows ? (size_t)(T.gatherA ? T.gatherA[ia] : ia) * lda : (size_t)ia);
+  const TA* pb = A + (a_rows ? (size_t)(T.gatherA ? T.gatherA[ib] : ib) * lda : (size_t)ib);
+  const TB* pj = B + (OPB == 0 ? (size_t)jb : (size_t)(T.gatherB ? T.gatherB[jb] : jb) * ldb);
+  const size_t sa = a_rows ? 1 : lda, sb = OPB == 0 ? ldb : 1;
+  const int nu = (K + 3) >> 2, nd = (nu - wave + 3) >> 2;  // this wave's units wave, wave + 4, ...
+  auto load = [&](int d, double2& x0, double2& x1, double2& y) __attribute__((always_inline)) {
+    const int k = 4 * (wave + 4 * d) + k4, kc = min(k, K - 1);
+    x0 = ld(pa, (size_t)kc * sa);
+    x1 = ld(pb, (size_t)kc * sa);
+    y = ld(pj, (size_t)kc * sb);
+    double f = k < K ? 1.0 : 0.0;
+    if (sign_div > 0) f *= ((kc / sign_div) & 1) ? kd1 : kd0;
+    if (k >= K || sign_div > 0) {
+      x0 = cscale(x0, f);
+      x1 = cscale(x1, f);
+    }
+  };
+  mfma_d4 re0 = {0, 0, 0, 0}, im0 = {0, 0, 0, 0}, re1 = {0, 0, 0, 0}, im1 = {0, 0, 0, 0};
+  double2 x0[GEMM_PD], x1[GEMM_PD], y[GEMM_PD];
 #pragma unroll
-  for (int x = 0; x < 2; ++x)
+  for (int d = 0; d < GEMM_PD; ++d)
+    if (d < nd) load(d, x0[d], x1[d], y[d]);
+#pragma unroll 1
+  for (int d0 = 0; d0 < nd; d0 += GEMM_PD) {
 #pragma unroll
-    for (int y = 0; y < 2; ++y) acc[x][y] = make_double2(0, 0);
-
-  for (int k0 = 0; k0 < Kd; k0 += GK) {
-#pragma unroll
-    for (int q = 0; q < 2; ++q) {
-      int e = tid + 256 * q;  // 512 = 32 x 16
-      int i, k;
-      if (OPA == 0 || OPA == 1) { i = e / GK; k = e % GK; }
-      else { k = e / GM; i = e % GM; }
-      double2 v = make_double2(0, 0);
-      int gi = i0 + i, gk = k0 + k;
-      if (gi < M && gk < Kd) {
-        if (OPA == 0 || OPA == 1) {
-          int sr = T.gatherA ? T.gatherA[gi] : gi;
-          v = ld(A, (size_t)sr * T.lda + gk);
-        } else {
-          v = ld(A, (size_t)gk * T.lda + gi);
-        }
-        if (OPA == 1 || OPA == 2) v = cconj(v);
-        if (T.sign_div > 0) v = cscale(v, ((gk / T.sign_div) & 1) ? T.kd1 : T.kd0);
+    for (int d = 0; d < GEMM_PD; ++d) {
+      if (d0 + d < nd) {
+        const double2 a0 = x0[d], a1 = x1[d], b = y[d];
+        if (d0 + d + GEMM_PD < nd) load(d0 + d + GEMM_PD, x0[d], x1[d], y[d]);
+        // conj(A) (OPA 1, 2): -a.y for a.y; conj(B) (OPB 2): -b.y for b.y
+        const double a0y = OPA == 1 || OPA == 2 ? -a0.y : a0.y, a1y = OPA == 1 || OPA == 2 ? -a1.y : a1.y;
+        const double by = OPB == 2 ? -b.y : b.y;
+        re0 = mfma64(a0.x, b.x, re0);
+        im0 = mfma64(a0.x, by, im0);
+        re1 = mfma64(a1.x, b.x, re1);
+        im1 = mfma64(a1.x, by, im1);
+        re0 = mfma64(-a0y, by, re0);
+        im0 = mfma64(a0y, b.x, im0);
+        re1 = mfma64(-a1y, by, re1);
+        im1 = mfma64(a1y, b.x, im1);
       }
-      sA[i][k] = v;
     }
-#pragma unroll
-    for (int q = 0; q < 2; ++q) {
-      int e = tid + 256 * q;  // 512 = 16 x 32
-      int k, j;
-      if (OPB == 0) { k = e / GN; j = e % GN; }
-      else { j = e / GK; k = e % GK; }
-      double2 v = make_double2(0, 0);
-      int gj = j0 + j, gk = k0 + k;
-      if (gj < N && gk < Kd) {
-        if (OPB == 0) {
-          v = ld(B, (size_t)gk * T.ldb + gj);
-        } else {
-          int sr = T.gatherB ? T.gatherB[gj] : gj;
-          v = ld(B, (size_t)sr * T.ldb + gk);
-          if (OPB == 2) v = cconj(v);
-        }
-      }
-      sB[k][j] = v;
-    }
-    __syncthreads();
-#pragma unroll 4
-    for (int k = 0; k < GK; ++k) {
-      double2 a0 = sA[ty * 2][k], a1 = sA[ty * 2 + 1][k];
-      double2 b0 = sB[k][tx * 2], b1 = sB[k][tx * 2 + 1];
-      acc[0][0] = cfma(a0, b0, acc[0][0]);
-      acc[0][1] = cfma(a0, b1, acc[0][1]);
-      acc[1][0] = cfma(a1, b0, acc[1][0]);
-      acc[1][1] = cfma(a1, b1, acc[1][1]);
-    }
-    __syncthreads();
   }
+#pragma unroll
+  for (int v = 0; v < 4; ++v) {
+    sC[wave][4 * v + k4][l16] = make_double2(re0[v], im0[v]);
+    sC[wave][16 + 4 * v + k4][l16] = make_double2(re1[v], im1[v]);
+  }
+  __syncthreads();
   TC* Cp = (TC*)T.C;
 #pragma unroll
-  for (int x = 0; x < 2; ++x) {
-    int i = i0 + ty * 2 + x;
-    if (i >= M) continue;
-    double rs = T.rowscale ? T.rowscale[i] : 1.0;
-#pragma unroll
-    for (int y = 0; y < 2; ++y) {
-      int j = j0 + tx * 2 + y;
-      if (j >= N) continue;
-      double s = rs * (T.colscale ? T.colscale[j] : 1.0);
-      double2 v = cscale(acc[x][y], s);
-      size_t o = (size_t)i * ldc + j;
-      if (T.accumulate) v = cadd(v, ld(Cp, o));
-      st(Cp, o, v);
-    }
+  for (int q = 0; q < 2; ++q) {
+    const int li = (tid >> 4) + 16 * q, i = i0 + li, j = j0 + l16;
+    if (i >= M || j >= N) continue;
+    double2 v = cadd(cadd(sC[0][li][l16], sC[1][li][l16]), cadd(sC[2][li][l16], sC[3][li][l16]));
+    const double s = (T.rowscale ? T.rowscale[i] : 1.0) * (T.colscale ? T.colscale[j] : 1.0);
+    v = cscale(v, s);
+    const size_t o = (size_t)i * ldc + j;
+    if (T.accumulate) v = cadd(v, ld(Cp, o));
+    st(Cp, o, v);
   }
 }
 
 template <int OPA, int OPB>
 static hipError_t gemm_types(const GemmTask* d, int nt, int tiles, int ta, int tb, int tc, hipStream_t s) {
-  dim3 g(tiles), b(256);
+  constexpr int CHUNK = 1 << 23;  // a dispatch holds at most 2^32 work-items
 #define HIPMPS_GEMM_CASE(A_, B_, C_, a, b_, c)                                                   \
   if (ta == a && tb == b_ && tc == c) {                                                          \
-    hipLaunchKernelGGL((k_gemm<A_, B_, C_, OPA, OPB>), g, b, 0, s, d, nt);                       \
+    for (int t0 = 0; t0 < tiles; t0 += CHUNK)                                                    \
+      hipLaunchKernelGGL((k_gemm<A_, B_, C_, OPA, OPB>), dim3(std::min(CHUNK, tiles - t0)), dim3(256), 0, s, d, nt, t0); \
     return hipGetLastError();                                                                    \
   }
   HIPMPS_GEMM_CASE(double2, double2, double2, 0, 0, 0)
@@ -1260,6 +1262,69 @@ hipError_t launch_trace_prod(const double2* const* d_a, const double2* const* d_
                              double2* d_out, int ntasks, hipStream_t s) {
   if (ntasks <= 0) return hipSuccess;
   hipLaunchKernelGGL(k_trace_prod, dim3(ntasks), dim3(256), 0, s, d_a, d_b, d_dims, d_out);
+  return hipGetLastError();
+}
+
+// ------------------------------------------------------------------ one measured site of the sampling
+// One wave per shot: the rows' products, the choice and the copy of the chosen rows (bound by the read
+// of X and U, 2 rho d chi_r complex128 per shot; the choice stays on the device, so that a site costs
+// no round trip to the host).
+__global__ __launch_bounds__(256) void k_sample_pick(SampleTask T) {
+  const int t = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (t >= T.shots) return;
+  const int half = T.kap * T.cr, per = T.rho * half;  // elements of one outcome: of a row group, of a shot
+  const size_t base = (size_t)t * 2 * per;
+  double p[2];
+#pragma unroll
+  for (int b = 0; b < 2; ++b) {
+    double acc = 0.0;
+    for (int e = lane; e < per; e += 64) {
+      const size_t o = base + (size_t)(e / half) * 2 * half + (size_t)b * half + e % half;
+      const double2 x = T.X[o], u = T.U[o];
+      acc += fma(u.x, x.x, u.y * x.y);
+    }
+    for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o, 64);
+    p[b] = acc * T.f[t];
+    if (fabs(p[b]) < 1e-12) p[b] = 0.0;
+  }
+  const int bit = T.draws[(size_t)t * T.stride] <= p[0] ? 0 : 1;
+  const double pb = bit ? p[1] : p[0];
+  if (lane == 0) {
+    T.out[(size_t)t * T.stride] = bit ? '1' : '0';
+    if (pb > 0.0) T.f[t] /= pb;
+  }
+  for (int e = lane; e < per; e += 64)
+    T.V[(size_t)t * per + e] = T.X[base + (size_t)(e / half) * 2 * half + (size_t)bit * half + e % half];
+}
+
+hipError_t launch_sample_pick(const SampleTask& task, hipStream_t s) {
+  if (task.shots <= 0) return hipSuccess;
+  hipLaunchKernelGGL(k_sample_pick, dim3((task.shots + 3) / 4), dim3(256), 0, s, task);
+  return hipGetLastError();
+}
+
+// ------------------------------------------------------------------ sum_e z_e a_e conj(b_e), real part
+__global__ __launch_bounds__(256) void k_dot(const DotTask* tasks, double* out) {
+  __shared__ double red[4];
+  const DotTask& T = tasks[blockIdx.x];
+  const size_t per = (size_t)T.d * T.cr, n = (size_t)T.rows * per, half = per / 2;
+  double acc0 = 0.0, acc1 = 0.0;
+  for (size_t e = (size_t)blockIdx.y * 256 + threadIdx.x; e < n; e += (size_t)DOT_BLOCKS * 256) {
+    const double2 a = gld(T.a + e), b = gld(T.b + e);
+    const double v = fma(a.x, b.x, a.y * b.y);
+    if (e % per < half) acc0 += v;
+    else acc1 += v;
+  }
+  double acc = T.z0 * acc0 + T.z1 * acc1;
+  for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o, 64);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
+  __syncthreads();
+  if (threadIdx.x == 0) out[(size_t)blockIdx.x * DOT_BLOCKS + blockIdx.y] = (red[0] + red[1]) + (red[2] + red[3]);
+}
+
+hipError_t launch_dot(const DotTask* d_tasks, double* d_out, int ntasks, hipStream_t s) {
+  if (ntasks <= 0) return hipSuccess;
+  hipLaunchKernelGGL(k_dot, dim3(ntasks, DOT_BLOCKS), dim3(256), 0, s, d_tasks, d_out);
   return hipGetLastError();
 }
 
