@@ -109,4 +109,72 @@ __device__ __forceinline__ mfma_d4 mfma64(double a, double b, mfma_d4 c) {
   return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
 }
 
+// Sum over the wave, the same value in every lane: four DPP steps within the rows of 16 lanes, then
+// the four row sums through scalar registers.  A shuffle-based tree goes through the LDS crossbar at
+// every level (about 7 times the latency, and these sums are most of a reflector's serial chain).
+template <int CTRL>
+__device__ __forceinline__ double dpp_add(double v) {
+  const long long x = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)x, CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(x >> 32), CTRL, 0xf, 0xf, true);
+  return v + __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+__device__ __forceinline__ double lane_value(double v, int lane) {  // lane: wave-uniform
+  const long long x = __double_as_longlong(v);
+  const unsigned int lo = (unsigned int)__builtin_amdgcn_readlane((int)x, lane);
+  const unsigned int hi = (unsigned int)__builtin_amdgcn_readlane((int)(x >> 32), lane);
+  return __longlong_as_double(((long long)hi << 32) | lo);
+}
+__device__ __forceinline__ double wave_sum(double v) {
+  v = dpp_add<0xb1>(v);   // quad_perm [1, 0, 3, 2]
+  v = dpp_add<0x4e>(v);   // quad_perm [2, 3, 0, 1]
+  v = dpp_add<0x124>(v);  // row_ror:4
+  v = dpp_add<0x128>(v);  // row_ror:8
+  return (lane_value(v, 0) + lane_value(v, 16)) + (lane_value(v, 32) + lane_value(v, 48));
+}
+__device__ __forceinline__ double2 wave_sum2(double2 v) { return make_double2(wave_sum(v.x), wave_sum(v.y)); }
+
+// Round-robin ("circle") ordering of nb slots: slot 0 holds 0, slot s > 0 holds 1 + (s - 1 + round) mod
+// (nb - 1); slots i and nb - 1 - i meet.
+__device__ __forceinline__ int circle_slot(int s, int round, int nb) {
+  return s == 0 ? 0 : 1 + (s - 1 + round) % (nb - 1);
+}
+
+// 1/sqrt(a) and 1/d: the hardware approximations refined by one Newton step, which
+// brings them to the last bit or two of FP64 (all that a rotation needs: only
+// c^2 + |s|^2 = 1 has to hold to working precision, not the angle itself).
+__device__ __forceinline__ double nr_rsq(double a) {
+  const double y = __builtin_amdgcn_rsq(a);
+  const double hy = 0.5 * a * y;
+  return fma(y, fma(-hy, y, 0.5), y);
+}
+__device__ __forceinline__ double nr_rcp(double d) {
+  const double x = __builtin_amdgcn_rcp(d);
+  return fma(x, fma(-d, x, 1.0), x);
+}
+
+// Rotation that annihilates gamma in the Hermitian 2x2 [[alpha, gamma], [conj(gamma), beta]]
+// (Golub & Van Loan Alg. 8.4.1 with a phase): h = beta - alpha,
+// tau = 2 sign(h) gamma / (|h| + sqrt(h^2 + 4|gamma|^2))  (|tau| = t, the smaller root),
+// c = 1/sqrt(1 + |tau|^2);  J = c [[1, tau], [-conj(tau), 1]].
+// The rotated diagonal is alpha - f |gamma|^2, beta + f |gamma|^2 with tau = f gamma; it replaces
+// alpha and beta.  The identity when |gamma| <= tol sqrt(alpha beta) or a diagonal entry is 0.
+__device__ __forceinline__ void jacobi_rotation(double& alpha, double& beta, double2 gamma, double tol, double floor2,
+                                                double& c, double2& tau) {
+  const double g2 = cabs2(gamma);
+  if (!(alpha > floor2) || !(beta > floor2) || !(g2 > tol * tol * alpha * beta)) {
+    c = 1.0;
+    tau = make_double2(0.0, 0.0);
+    return;
+  }
+  const double h = beta - alpha;
+  const double a = fma(h, h, 4.0 * g2);
+  const double d = fabs(h) + a * nr_rsq(a);
+  const double f = (h >= 0.0 ? 2.0 : -2.0) * nr_rcp(d);
+  tau = make_double2(f * gamma.x, f * gamma.y);
+  c = nr_rsq(1.0 + cabs2(tau));
+  alpha = fma(-f, g2, alpha);
+  beta = fma(f, g2, beta);
+}
+
 }  // namespace hipmps

@@ -32,6 +32,7 @@
 #include <cstdio>
 #include <cstring>
 #include <deque>
+#include <functional>
 #include <map>
 #include <mutex>
 #include <stdexcept>
@@ -206,6 +207,7 @@ struct hipmps_engine_s {
   DevBuf env;    // environments for measurements
   HostBuf hdesc;
   HostBuf hsmall;
+  HostBuf hgate;  // descriptors and results of k_gate_small, read and written by the device in place
   std::mutex mu;
   bool timing = false;
   hipmps_profile_t prof{};
@@ -543,17 +545,45 @@ struct WaveItem {
   void* old_j;
   size_t off_theta, off_y, off_vec;
   int lq;                            // Jacobi on the double-LQ factor R2 of X
+  int small;                         // runs in k_gate_small
   size_t off_z, off_j, off_yt, off_lq;
   int ki, kj;                        // Kraus legs of the two sites (fused into cl and cr)
   size_t off_pin, off_pout;          // left site with its Kraus leg moved next to the left bond
   size_t off_jt;                     // the Jacobi matrix in tiles during the sweeps
 };
 
-int run_wave(hipmps_engine E, std::vector<WaveItem>& items) {
-  if (items.empty()) return 0;
+// bookkeeping of a state after one of its gates: new bond, weights (SplitTask::wstats), sweeps
+void finish_gate(const WaveItem& it, int K, const double* w, int sweeps, bool converged) {
+  hipmps_state_s* s = it.s;
+  s->chi[it.i + 1] = K;
+  s->maxb = std::max(s->maxb, K);
+  const double disc = w[0], kept = w[1];
+  if (w[5] != 0.0 || !std::isfinite(kept + disc)) s->status = HIPMPS_E_NUMERIC;
+  s->discarded += disc;
+  if (kept + disc > 0) s->fid *= kept / (kept + disc);
+  // post-SVD norm validation (ExaTnMpsVisitor.cpp:1634-1661): Frobenius norms of the two
+  // factors before truncation, sqrt(sum sigma) each for the sqrt(S) split; the reference
+  // prints an error when either is below 1e-3 and carries on (its assert is debug-only)
+  const double nf_i = s->t.absorb == HIPMPS_ABSORB_RIGHT ? std::sqrt((double)it.r) : std::sqrt(w[4]);
+  const double nf_j = s->t.absorb == HIPMPS_ABSORB_RIGHT ? std::sqrt(w[2]) : std::sqrt(w[4]);
+  if (std::fabs(nf_i) < 1e-3 || std::fabs(nf_j) < 1e-3) s->norm_warnings++;
+  s->n2q++;
+  s->sweeps_max = std::max(s->sweeps_max, sweeps);
+  s->sweeps_total += sweeps;
+  if (!converged) {
+    if (s->status == 0) s->status = HIPMPS_E_CONVERGENCE;  // NaN / Inf is the graver report
+    s->nonconverged++;
+  }
+}
+
+int run_wave_general(hipmps_engine E, std::vector<WaveItem>& items, const std::function<int()>& grow,
+                     const std::function<int()>& join);
+
+int run_wave(hipmps_engine E, std::vector<WaveItem>& all) {
+  if (all.empty()) return 0;
   const hipStream_t st = E->stream;
   // order: fp64 before fp32, non-transposed before transposed (contiguous launch groups)
-  for (auto& it : items) {
+  for (auto& it : all) {
     hipmps_state_s* s = it.s;
     it.ki = s->kap[it.i];
     it.kj = s->kap[it.i + 1];
@@ -570,14 +600,124 @@ int run_wave(hipmps_engine E, std::vector<WaveItem>& items) {
     it.kub = std::min(it.r, maxb);
     it.fp32 = s->fp32;
     it.lq = E->lq_min_rank > 0 && it.r >= E->lq_min_rank;
+    it.small = gate_small(it.r, it.c);
   }
-  std::stable_sort(items.begin(), items.end(), [](const WaveItem& a, const WaveItem& b) {
+  std::stable_sort(all.begin(), all.end(), [](const WaveItem& a, const WaveItem& b) {
     if (a.fp32 != b.fp32) return a.fp32 < b.fp32;
     return a.transposed < b.transposed;
   });
-  const int N = (int)items.size();
-  for (auto& it : items)
+  for (auto& it : all)
     if (it.r > 4096) return fail(HIPMPS_E_UNSUPPORTED, "bond dimension above 2048 is not supported");
+  // small gates, by launch variant (precision, LDS size): one workgroup each, in one launch per variant
+  std::vector<WaveItem> small[4], items;
+  int ns = 0;
+  for (auto& it : all) {
+    if (it.small) {
+      small[2 * it.fp32 + (small_rows(it.r) * small_stride(it.c) > SMALL_CAP_LO)].push_back(it);
+      ++ns;
+    } else {
+      items.push_back(it);
+    }
+  }
+  RC_TRY(E->hgate.ensure((size_t)ns * (sizeof(GateTask) + sizeof(GateResult))));
+  GateTask* ht = (GateTask*)E->hgate.p;
+  GateResult* hr = (GateResult*)(ht + ns);
+  // site capacity, after every engine buffer exists (new sites are written after theta has
+  // read the old ones); all-or-nothing across the wave.  Then the small gates' launches, beside the
+  // general path's when there is one.
+  hipStream_t ss = st;
+  auto start = [&]() -> int {
+    std::vector<SiteGrowth> growth;
+    auto need_of = [&](WaveItem& it) {
+      const size_t need[2] = {(size_t)it.cl * 2 * it.kub, (size_t)it.kub * 2 * it.cr};
+      for (int h = 0; h < 2; ++h) {
+        Site& S = it.s->sites[it.i + h];
+        (h ? it.old_j : it.old_i) = S.p;
+        if (need[h] > S.cap)
+          growth.push_back({it.s, it.i + h, grown_capacity(it.s, it.i + h, need[h], S.cap), nullptr});
+      }
+    };
+    for (auto& it : items) need_of(it);
+    for (auto& v : small)
+      for (auto& it : v) need_of(it);
+    if (!growth.empty()) RC_TRY(grow_sites(E, growth));
+    if (ns == 0) return 0;
+    void* dev = nullptr;
+    HIP_TRY(hipHostGetDevicePointer(&dev, E->hgate.p, 0));
+    int q = 0;
+    for (auto& v : small)
+      for (auto& it : v) {
+        GateTask& T = ht[q];
+        const hipmps_trunc_opts& to = it.s->t;
+        T.Ai = it.old_i;
+        T.Aj = it.old_j;
+        T.Oi = it.s->sites[it.i].p;
+        T.Oj = it.s->sites[it.i + 1].p;
+        T.res = (GateResult*)((GateTask*)dev + ns) + q;
+        T.chi_l = it.s->chi[it.i];
+        T.ki = it.ki;
+        T.cm = it.cm;
+        T.cr = it.cr;
+        T.m = it.m;
+        T.n = it.n;
+        T.r = it.r;
+        T.c = it.c;
+        T.transposed = it.transposed;
+        T.max_bond = to.max_bond_dim > 0 ? to.max_bond_dim : INT_MAX - 1;
+        T.pn_l2 = to.partial_norm == HIPMPS_PN_L2;
+        T.absorb = to.absorb == HIPMPS_ABSORB_RIGHT ? 1 : 0;
+        T.renorm = to.renormalize ? 1 : 0;
+        T.max_sweeps = E->max_sweeps;
+        T.cutoff = to.svd_cutoff;
+        T.tol = it.fp32 ? E->tol_mixed : E->tol;
+        for (int k = 0; k < 16; ++k) T.G[k] = make_double2(it.G[k].real(), it.G[k].imag());
+        ++q;
+      }
+    constexpr int LANE = hipmps_engine_s::MAX_LANES - 1;
+    if (!items.empty() && E->lane_stream[LANE] && E->lane_ev[0]) {
+      ss = E->lane_stream[LANE];
+      HIP_TRY(hipEventRecord(E->lane_ev[0], st));
+      HIP_TRY(hipStreamWaitEvent(ss, E->lane_ev[0], 0));
+    }
+    const GateTask* dt = (const GateTask*)dev;
+    for (int v = 0; v < 4; ++v) {
+      HIP_TRY(launch_gate_small(dt, (int)small[v].size(), v >> 1, (v & 1) == 0, ss));
+      dt += small[v].size();
+    }
+    return 0;
+  };
+  auto join = [&]() -> int {
+    if (ss != st) HIP_TRY(hipStreamSynchronize(ss));
+    return 0;
+  };
+  if (items.empty()) {
+    RC_TRY(start());
+    HIP_TRY(hipStreamSynchronize(st));
+    E->prof.waves += 1;
+  } else {
+    RC_TRY(run_wave_general(E, items, start, join));
+  }
+  int q = 0;
+  for (auto& v : small)
+    for (auto& it : v) {
+      const GateResult& R = hr[q++];
+      finish_gate(it, R.K, R.w, R.sweeps, R.converged != 0);
+      int lg = 0;
+      while (lg < 13 && (2 << lg) <= it.r) ++lg;
+      E->prof.applies_by_rank[lg] += 1;
+      E->prof.wave_tasks += 1;
+      E->prof.jacobi_sweeps += R.sweeps;
+    }
+  for (auto& it : all) release_deferred(it.s);
+  return 0;
+}
+
+// the gates that do not fit k_gate_small, as batched launches; `grow` reserves the sites of the whole wave
+// and launches its small gates, `join` waits for those
+int run_wave_general(hipmps_engine E, std::vector<WaveItem>& items, const std::function<int()>& grow,
+                     const std::function<int()>& join) {
+  const hipStream_t st = E->stream;
+  const int N = (int)items.size();
   // arena
   size_t off = 0;
   for (auto& it : items) {
@@ -626,20 +766,7 @@ int run_wave(hipmps_engine E, std::vector<WaveItem>& items) {
   // host staging: descriptors | counts (2N ints) | active Jacobi list / results
   const size_t stage_bytes = desc_bytes + align_up(2 * N * sizeof(int)) + N * sizeof(JacTask) + WS_N * N * sizeof(double) + 4096;
   RC_TRY(E->hdesc.ensure(stage_bytes));
-  // site capacity, after every engine buffer exists (new sites are written after theta has
-  // read the old ones); all-or-nothing across the wave
-  {
-    std::vector<SiteGrowth> grow;
-    for (auto& it : items) {
-      const size_t need[2] = {(size_t)it.cl * 2 * it.kub, (size_t)it.kub * 2 * it.cr};
-      for (int h = 0; h < 2; ++h) {
-        Site& S = it.s->sites[it.i + h];
-        (h ? it.old_j : it.old_i) = S.p;
-        if (need[h] > S.cap) grow.push_back({it.s, it.i + h, grown_capacity(it.s, it.i + h, need[h], S.cap), nullptr});
-      }
-    }
-    if (!grow.empty()) RC_TRY(grow_sites(E, grow));
-  }
+  RC_TRY(grow());
   char* hd = (char*)E->hdesc.p;
   ThetaTask* hth = (ThetaTask*)hd;
   SplitTask* hsp = (SplitTask*)(hd + align_up(N * sizeof(ThetaTask)));
@@ -1088,6 +1215,7 @@ int run_wave(hipmps_engine E, std::vector<WaveItem>& items) {
   HIP_TRY(hipMemcpyAsync(hw, d_w, WS_N * N * sizeof(double), hipMemcpyDeviceToHost, st));
   if (E->timing) HIP_TRY(hipEventRecord(E->ev[3], st));
   HIP_TRY(hipStreamSynchronize(st));
+  RC_TRY(join());
   if (E->timing) {
     float a = 0, b = 0, c = 0, d = 0;
     (void)hipEventElapsedTime(&a, E->ev[0], E->ev[6]);
@@ -1113,32 +1241,7 @@ int run_wave(hipmps_engine E, std::vector<WaveItem>& items) {
       E->prof.sweeps_large += sweeps_used[q];
     }
   }
-  for (int q = 0; q < N; ++q) {
-    auto& it = items[q];
-    hipmps_state_s* s = it.s;
-    int K = hK[q];
-    s->chi[it.i + 1] = K;
-    s->maxb = std::max(s->maxb, K);
-    const double* w = hw + WS_N * q;
-    double disc = w[0], kept = w[1];
-    if (w[5] != 0.0 || !std::isfinite(kept + disc)) s->status = HIPMPS_E_NUMERIC;
-    s->discarded += disc;
-    if (kept + disc > 0) s->fid *= kept / (kept + disc);
-    // post-SVD norm validation (ExaTnMpsVisitor.cpp:1634-1661): Frobenius norms of the two
-    // factors before truncation, sqrt(sum sigma) each for the sqrt(S) split; the reference
-    // prints an error when either is below 1e-3 and carries on (its assert is debug-only)
-    const double nf_i = s->t.absorb == HIPMPS_ABSORB_RIGHT ? std::sqrt((double)it.r) : std::sqrt(w[4]);
-    const double nf_j = s->t.absorb == HIPMPS_ABSORB_RIGHT ? std::sqrt(w[2]) : std::sqrt(w[4]);
-    if (std::fabs(nf_i) < 1e-3 || std::fabs(nf_j) < 1e-3) s->norm_warnings++;
-    s->n2q++;
-    s->sweeps_max = std::max(s->sweeps_max, sweeps_used[q]);
-    s->sweeps_total += sweeps_used[q];
-    if (!converged[q]) {
-      if (s->status == 0) s->status = HIPMPS_E_CONVERGENCE;  // NaN / Inf is the graver report
-      s->nonconverged++;
-    }
-  }
-  for (auto& it : items) release_deferred(it.s);
+  for (int q = 0; q < N; ++q) finish_gate(items[q], hK[q], hw + WS_N * q, sweeps_used[q], converged[q] != 0);
   return 0;
 }
 
@@ -2571,6 +2674,7 @@ int hipmps_engine_destroy(hipmps_engine e) {
   e->env.release();
   e->hdesc.release();
   e->hsmall.release();
+  e->hgate.release();
   for (auto& ev : e->ev)
     if (ev) (void)hipEventDestroy(ev);
   for (auto& ev : e->lane_ev)

@@ -96,6 +96,37 @@ struct SplitTask {
 // Output tile of one k_gemm workgroup
 constexpr int GEMM_TM = 32, GEMM_TN = 16;
 
+// A whole 2-qubit gate of small bonds in one workgroup (k_gate_small, small.hip).  Descriptor and result
+// live in mapped host memory: a wave of such gates is one launch and one synchronisation.
+struct GateResult {
+  int K, sweeps, converged, pad;
+  double w[WS_N];        // as SplitTask::wstats
+};
+struct GateTask {
+  const void* Ai;        // left site [l][a][kap][m], l < chi_l, kap < ki
+  const void* Aj;        // right site cm x 2 x cr
+  void* Oi;              // the new sites (may be the old buffers: both are read first)
+  void* Oj;
+  GateResult* res;
+  int chi_l, ki, cm, cr;
+  int m, n, r, c, transposed;  // theta' m x n, r = min, c = max, X = theta'^H when transposed (m > n)
+  int max_bond, pn_l2, absorb, renorm, max_sweeps;
+  double cutoff, tol;
+  double2 G[16];
+};
+// Jacobi rows of a small SVD: an even number of rows, whole groups of 16 columns
+__host__ __device__ inline int small_rows(int r) { return r + (r & 1); }
+__host__ __device__ inline int small_stride(int c) { return (c <= 16 ? 16 : c <= 32 ? 32 : c <= 64 ? 64 : 128) + 1; }
+// complex128 elements of X (and of Y) that fit a workgroup's LDS, and the largest row count
+constexpr int SMALL_MAX_ROWS = 64;
+constexpr int SMALL_CAP = 64 * 65;
+constexpr int SMALL_CAP_LO = 32 * 33;  // variant of 256 threads, several workgroups per CU
+inline bool gate_small(int r, int c) {
+  return r <= SMALL_MAX_ROWS && c <= 128 && small_rows(r) * small_stride(c) <= SMALL_CAP;
+}
+// lo: every task fits SMALL_CAP_LO
+hipError_t launch_gate_small(const GateTask* d_tasks, int ntasks, int fp32, bool lo, hipStream_t s);
+
 // Generic batched complex GEMM: C (M x N) = rowscale . op(A) op(B) . colscale
 // op codes: 0 N, 1 C (conjugate), 2 H (conjugate transpose), 3 T (transpose).
 struct GemmTask {

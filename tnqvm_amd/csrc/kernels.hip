@@ -230,47 +230,6 @@ hipError_t launch_jacobi_prep(const SplitTask* d_split, const JacTask* d_jac, in
 // For the 2*JB rows:  Gram  Gam[i][j] = sum_c conj(Y[i][c]) Y[j][c]
 //                     Gam ~ W Lambda W^H  by one cyclic two-sided Jacobi sweep (FP64)
 //                     Y' = W^T Y          (rows become mutually orthogonal)
-__device__ __forceinline__ int circle_slot(int s, int round, int nb) {
-  return s == 0 ? 0 : 1 + (s - 1 + round) % (nb - 1);
-}
-
-// 1/sqrt(a) and 1/d: the hardware approximations refined by one Newton step, which
-// brings them to the last bit or two of FP64 (all that a rotation needs: only
-// c^2 + |s|^2 = 1 has to hold to working precision, not the angle itself).
-__device__ __forceinline__ double nr_rsq(double a) {
-  const double y = __builtin_amdgcn_rsq(a);
-  const double hy = 0.5 * a * y;
-  return fma(y, fma(-hy, y, 0.5), y);
-}
-__device__ __forceinline__ double nr_rcp(double d) {
-  const double x = __builtin_amdgcn_rcp(d);
-  return fma(x, fma(-d, x, 1.0), x);
-}
-
-// Rotation that annihilates gamma in the Hermitian 2x2 [[alpha, gamma], [conj(gamma), beta]]
-// (Golub & Van Loan Alg. 8.4.1 with a phase): h = beta - alpha,
-// tau = 2 sign(h) gamma / (|h| + sqrt(h^2 + 4|gamma|^2))  (|tau| = t, the smaller root),
-// c = 1/sqrt(1 + |tau|^2);  J = c [[1, tau], [-conj(tau), 1]].
-// The rotated diagonal is alpha - f |gamma|^2, beta + f |gamma|^2 with tau = f gamma; it replaces
-// alpha and beta.  The identity when |gamma| <= tol sqrt(alpha beta) or a diagonal entry is 0.
-__device__ __forceinline__ void jacobi_rotation(double& alpha, double& beta, double2 gamma, double tol, double floor2,
-                                                double& c, double2& tau) {
-  const double g2 = cabs2(gamma);
-  if (!(alpha > floor2) || !(beta > floor2) || !(g2 > tol * tol * alpha * beta)) {
-    c = 1.0;
-    tau = make_double2(0.0, 0.0);
-    return;
-  }
-  const double h = beta - alpha;
-  const double a = fma(h, h, 4.0 * g2);
-  const double d = fabs(h) + a * nr_rsq(a);
-  const double f = (h >= 0.0 ? 2.0 : -2.0) * nr_rcp(d);
-  tau = make_double2(f * gamma.x, f * gamma.y);
-  c = nr_rsq(1.0 + cabs2(tau));
-  alpha = fma(-f, g2, alpha);
-  beta = fma(f, g2, beta);
-}
-
 // A value moved one lane along its row of 16 lanes: from the next lane (lane 15 keeps `edge`) or from
 // the previous one (lane 0 keeps `edge`).
 template <int CTRL>

@@ -23,31 +23,6 @@ constexpr int LQB = 16;  // rows per panel (reflectors per block reflector)
 constexpr int LQR = 16;  // rows per MFMA tile in the block-reflector application
 constexpr long long LQ_ONE_STREAM_ROWS = 4096;  // launch_lq_lookahead: rows of all tasks on one stream up to this
 
-// Sum over the wave, the same value in every lane: four DPP steps within the rows of 16 lanes, then
-// the four row sums through scalar registers.  A shuffle-based tree goes through the LDS crossbar at
-// every level (about 7 times the latency, and these sums are most of a reflector's serial chain).
-template <int CTRL>
-__device__ __forceinline__ double dpp_add(double v) {
-  const long long x = __double_as_longlong(v);
-  const int lo = __builtin_amdgcn_update_dpp(0, (int)x, CTRL, 0xf, 0xf, true);
-  const int hi = __builtin_amdgcn_update_dpp(0, (int)(x >> 32), CTRL, 0xf, 0xf, true);
-  return v + __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
-}
-__device__ __forceinline__ double lane_value(double v, int lane) {  // lane: wave-uniform
-  const long long x = __double_as_longlong(v);
-  const unsigned int lo = (unsigned int)__builtin_amdgcn_readlane((int)x, lane);
-  const unsigned int hi = (unsigned int)__builtin_amdgcn_readlane((int)(x >> 32), lane);
-  return __longlong_as_double(((long long)hi << 32) | lo);
-}
-__device__ __forceinline__ double wave_sum(double v) {
-  v = dpp_add<0xb1>(v);   // quad_perm [1, 0, 3, 2]
-  v = dpp_add<0x4e>(v);   // quad_perm [2, 3, 0, 1]
-  v = dpp_add<0x124>(v);  // row_ror:4
-  v = dpp_add<0x128>(v);  // row_ror:8
-  return (lane_value(v, 0) + lane_value(v, 16)) + (lane_value(v, 32) + lane_value(v, 48));
-}
-__device__ __forceinline__ double2 wave_sum2(double2 v) { return make_double2(wave_sum(v.x), wave_sum(v.y)); }
-
 // Element w_k[col] of reflector k of M (support col >= k; head in W0, tail in M's row k).
 __device__ __forceinline__ double2 refl(const double2* M, size_t ld, const double2* W0, int k, int col) {
   if (col < k) return make_double2(0, 0);

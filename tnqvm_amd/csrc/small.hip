@@ -1,0 +1,287 @@
+// small.hip -- a whole 2-qubit gate of small bonds in one workgroup.
+//
+// theta' = G (Ai Aj), its SVD, the truncation and the two new sites (ExaTnMpsVisitor.cpp:1387-1730,
+// :2366-2536) for theta' of at most 64 rows or columns whose other side fits the LDS beside it.  The
+// general path takes about 15 launches and, per Jacobi sweep, two copies, a memset, a launch per round
+// and a synchronisation; at these sizes each launch works for a few us on a few kilobytes, and a wave
+// took 0.3 to 0.9 ms.  Here theta', its rows and every intermediate stay in LDS, convergence is tested
+// on the device, and a wave is one launch.
+//
+// The SVD is the one-sided Jacobi of the general path on single rows: the rows of X = theta' (or
+// theta'^H) in circle order, r / 2 disjoint pairs a step.  A pair belongs to 16 lanes (one DPP row): they
+// form both squared norms and the inner product from the rows, rotate and write them back, so every angle
+// comes from the rows themselves and no Gram matrix is carried.  A step is bound by its chain (LDS read,
+// products, four DPP sums, the rotation, LDS write, barrier), and at 64 rows by FP64 issue of the one CU.
+// Measured, a wave: 13 us at bonds up to 4, 60 to 80 us up to 16, 320 to 465 us up to 32.
+#include <cfloat>
+
+#include "kernels.h"
+#include "device_util.h"
+
+namespace hipmps {
+
+// Sum over the 16 lanes of a DPP row, bit for bit the same in each of them: every step adds two lanes'
+// values in both (rotations by 4 and 8 would add the four quads in two different orders, and lanes that
+// disagree on an angle of nearly equal rows rotate their columns differently).
+__device__ __forceinline__ double row16_sum(double v) {
+  v = dpp_add<0xb1>(v);          // quad_perm [1, 0, 3, 2]
+  v = dpp_add<0x4e>(v);          // quad_perm [2, 3, 0, 1]
+  v = dpp_add<0x141>(v);         // row_half_mirror
+  return dpp_add<0x140>(v);      // row_mirror
+}
+
+// One-sided Jacobi on the rows of Y (nr even, stride elements apart, 16 NJ columns): sweeps until no pair's
+// relative inner product exceeds tol.  Returns the sweeps used; *flag (LDS) is 0 when converged.
+template <int NT, int NJ>
+__device__ __forceinline__ int jacobi_rows(double2* Y, int stride, int nr, double tol, double floor2, int max_sweeps,
+                                           int* flag) {
+  const int tid = threadIdx.x, group = tid >> 4, l16 = tid & 15;
+  const double itol = 0.25 * tol, tol2 = tol * tol;
+  int sweep = 0;
+  for (; sweep < max_sweeps; ++sweep) {
+    if (tid == 0) *flag = 0;
+    __syncthreads();
+    for (int step = 0; step < nr - 1; ++step) {
+      for (int p = group; p < nr / 2; p += NT / 16) {
+        double2* yp = Y + circle_slot(p, step, nr) * stride + l16;
+        double2* yq = Y + circle_slot(nr - 1 - p, step, nr) * stride + l16;
+        double2 a[NJ], b[NJ];
+        double alpha = 0.0, beta = 0.0;
+        double2 g = make_double2(0, 0);
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+          a[j] = yp[16 * j];
+          b[j] = yq[16 * j];
+        }
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+          alpha = fma(a[j].x, a[j].x, fma(a[j].y, a[j].y, alpha));
+          beta = fma(b[j].x, b[j].x, fma(b[j].y, b[j].y, beta));
+          g = cfmac(a[j], b[j], g);
+        }
+        alpha = row16_sum(alpha);
+        beta = row16_sum(beta);
+        g = make_double2(row16_sum(g.x), row16_sum(g.y));
+        if (alpha > floor2 && beta > floor2 && cabs2(g) > tol2 * (alpha * beta) && l16 == 0) *flag = 1;
+        double c;
+        double2 tau;
+        jacobi_rotation(alpha, beta, g, itol, floor2, c, tau);
+        if (tau.x != 0.0 || tau.y != 0.0) {  // rows' = W^T rows, W = c [[1, tau], [-conj(tau), 1]]
+          const double2 nt = make_double2(-tau.x, tau.y);
+#pragma unroll
+          for (int j = 0; j < NJ; ++j) {
+            yp[16 * j] = cscale(cfma(nt, b[j], a[j]), c);
+            yq[16 * j] = cscale(cfma(tau, a[j], b[j]), c);
+          }
+        }
+      }
+      __syncthreads();
+    }
+    const int again = *flag;
+    __syncthreads();
+    if (!again) return sweep + 1;
+  }
+  return sweep;
+}
+
+template <int NT>
+__device__ __forceinline__ int jacobi_rows_n(double2* Y, int stride, int nr, double tol, double floor2, int max_sweeps,
+                                             int* flag) {
+  switch (stride >> 4) {
+    case 1: return jacobi_rows<NT, 1>(Y, stride, nr, tol, floor2, max_sweeps, flag);
+    case 2: return jacobi_rows<NT, 2>(Y, stride, nr, tol, floor2, max_sweeps, flag);
+    case 4: return jacobi_rows<NT, 4>(Y, stride, nr, tol, floor2, max_sweeps, flag);
+    default: return jacobi_rows<NT, 8>(Y, stride, nr, tol, floor2, max_sweeps, flag);
+  }
+}
+
+template <typename S, int NT, int CAP>
+__global__ __launch_bounds__(NT) void k_gate_small(const GateTask* tasks) {
+  __shared__ GateTask T;
+  __shared__ double2 sX[CAP], sY[CAP];
+  __shared__ double s_sig[SMALL_MAX_ROWS], s_scy[SMALL_MAX_ROWS], s_scw[SMALL_MAX_ROWS], s_inv[SMALL_MAX_ROWS];
+  __shared__ int s_perm[SMALL_MAX_ROWS];
+  __shared__ double s_red[NT / 64];
+  __shared__ int s_flag, s_K, s_bad;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, group = tid >> 4, l16 = tid & 15;
+  for (int e = tid; e < (int)(sizeof(GateTask) / 4); e += NT) ((int*)&T)[e] = ((const int*)(tasks + blockIdx.x))[e];
+  if (tid == 0) {
+    s_flag = 0;
+    s_bad = 0;
+  }
+  __syncthreads();
+  const int m = T.m, n = T.n, r = T.r, cr = T.cr, cm = T.cm, ki = T.ki, tr = T.transposed;
+  const int nr = small_rows(r);
+  const int stride = small_stride(T.c);
+  for (int e = tid; e < nr * stride; e += NT) sX[e] = sY[e] = make_double2(0, 0);
+  __syncthreads();
+  // ---- theta' (rows (l, kap, a), columns (b, r)), one thread per (l, kap, r) ----
+  double f2 = 0.0;
+  {
+    const S* Ai = (const S*)T.Ai;
+    const S* Aj = (const S*)T.Aj;
+    const int cl = T.chi_l * ki;
+    for (int e = tid; e < cl * cr; e += NT) {
+      const int lk = e / cr, rr = e - lk * cr, l = lk / ki, k = lk - l * ki;
+      const size_t a0 = ((size_t)(2 * l) * ki + k) * cm, a1 = ((size_t)(2 * l + 1) * ki + k) * cm;
+      double2 x[4] = {make_double2(0, 0), make_double2(0, 0), make_double2(0, 0), make_double2(0, 0)};
+#pragma unroll 4
+      for (int q = 0; q < cm; ++q) {
+        const double2 u0 = ld(Ai, a0 + q), u1 = ld(Ai, a1 + q);
+        const double2 v0 = ld(Aj, (size_t)(2 * q) * cr + rr), v1 = ld(Aj, (size_t)(2 * q + 1) * cr + rr);
+        x[0] = cfma(u0, v0, x[0]);
+        x[1] = cfma(u0, v1, x[1]);
+        x[2] = cfma(u1, v0, x[2]);
+        x[3] = cfma(u1, v1, x[3]);
+      }
+#pragma unroll
+      for (int ab = 0; ab < 4; ++ab) {
+        double2 o = make_double2(0, 0);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) o = cfma(T.G[ab * 4 + q], x[q], o);
+        // stabilizeTensorBody: |x| < 1e-100 -> 0 (ExaTnMpsVisitor.cpp:141-161)
+        if (cabs2(o) < 1e-200) o = make_double2(0, 0);
+        f2 += cabs2(o);
+        const int i = 2 * lk + (ab >> 1), j = (ab & 1) * cr + rr;
+        const int at = tr ? j * stride + i : i * stride + j;
+        if (tr) o = cconj(o);
+        sX[at] = o;
+        sY[at] = o;
+      }
+    }
+  }
+  f2 = wave_sum(f2);
+  if (lane == 0) s_red[wave] = f2;
+  __syncthreads();
+  f2 = 0.0;
+  for (int w = 0; w < NT / 64; ++w) f2 += s_red[w];
+  __syncthreads();
+  const int sweeps = jacobi_rows_n<NT>(sY, stride, nr, T.tol, JAC_FLOOR2 * f2, T.max_sweeps, &s_flag);
+  __syncthreads();
+  // ---- singular values (row norms), sorted descending, ties by row; NaN / Inf sorted as 0 and flagged ----
+  for (int i = group; i < r; i += NT / 16) {
+    double a = 0.0;
+    for (int j = l16; j < T.c; j += 16) a += cabs2(sY[i * stride + j]);
+    a = sqrt(row16_sum(a));
+    if (l16 == 0) {
+      if (!(a >= 0.0 && a <= DBL_MAX)) {
+        a = 0.0;
+        s_bad = 1;
+      }
+      s_inv[i] = a;
+    }
+  }
+  __syncthreads();
+  if (tid < r) {
+    const double a = s_inv[tid];
+    int rank = 0;
+    for (int j = 0; j < r; ++j) {
+      const double b = s_inv[j];
+      rank += b > a || (b == a && j < tid);
+    }
+    s_sig[rank] = a;
+    s_perm[rank] = tid;
+  }
+  __syncthreads();
+  // ---- truncation rule and factor scales, as k_select ----
+  if (wave == 0) {
+    const double sg = lane < r ? s_sig[lane] : 0.0;
+    const double pn = T.pn_l2 ? sqrt(sg) : sg;
+    const unsigned long long below = __ballot(lane < r && pn < T.cutoff);
+    int K = below ? (int)__ffsll(below) : r;  // first sub-threshold index i: keep i + 1
+    K = max(1, min(K, T.max_bond));
+    const double kept = wave_sum(lane < K ? sg * sg : 0.0), disc = wave_sum(lane >= K ? sg * sg : 0.0);
+    const double ssum = wave_sum(sg);
+    const double f = T.renorm && kept > 0.0 ? sqrt((kept + disc) / kept) : 1.0;
+    if (lane < r) {
+      double gy = 0.0, gw = 0.0, is = 0.0;
+      if (lane < K && sg > 1e-150) {
+        // exponents of f sigma: left aL, right 1 - aL; Y's side is the right one unless transposed
+        const double sf = sg * f, h = sqrt(sf);
+        const double left = T.absorb == 0 ? h : 1.0, right = T.absorb == 0 ? h : sf;
+        gy = (tr ? left : right) / sg;
+        gw = tr ? right : left;
+        is = 1.0 / sg;
+      }
+      s_scy[lane] = gy;
+      s_scw[lane] = gw;
+      s_inv[lane] = is;
+    }
+    if (lane == 0) {
+      s_K = K;
+      GateResult R;
+      R.K = K;
+      R.sweeps = sweeps;
+      R.converged = s_flag == 0;
+      R.pad = 0;
+      R.w[0] = disc;
+      R.w[1] = kept;
+      R.w[2] = kept + disc;
+      R.w[3] = f;
+      R.w[4] = ssum;
+      R.w[5] = s_bad ? 1.0 : 0.0;
+      *T.res = R;
+    }
+  }
+  __syncthreads();
+  const int K = s_K;
+  S* Oi = (S*)T.Oi;
+  S* Oj = (S*)T.Oj;
+  // left site element of theta' row i = (l, kap, a) and bond index k
+  auto left = [&](int i, int k) {
+    const int lk = i >> 1, l = lk / ki;
+    return ((size_t)(2 * l + (i & 1)) * ki + (lk - l * ki)) * K + k;
+  };
+  // ---- factor on Y's side ----
+  for (int e = tid; e < K * T.c; e += NT) {
+    if (!tr) {
+      const int k = e / n, j = e - k * n;
+      st(Oj, (size_t)e, cscale(sY[s_perm[k] * stride + j], s_scy[k]));
+    } else {
+      const int i = e / K, k = e - i * K;
+      st(Oi, left(i, k), cscale(cconj(sY[s_perm[k] * stride + i]), s_scy[k]));
+    }
+  }
+  // ---- the other factor: X's rows on the kept rows of Y, each vector scaled to its length ----
+  for (int k = group; k < K; k += NT / 16) {
+    const double2* y = sY + s_perm[k] * stride;
+    const double is = s_inv[k];
+    double2 u[SMALL_MAX_ROWS / 16];
+    double t = 0.0;
+#pragma unroll
+    for (int q = 0; q < SMALL_MAX_ROWS / 16; ++q) {
+      u[q] = make_double2(0, 0);
+      const int i = l16 + 16 * q;
+      if (i < r) {
+        const double2* x = sX + i * stride;
+        double2 d = make_double2(0, 0);
+        for (int c = 0; c < T.c; ++c) d = cfmac(y[c], x[c], d);
+        u[q] = cscale(d, is);
+        t += cabs2(u[q]);
+      }
+    }
+    t = row16_sum(t);
+    const double f = t > 0.0 ? s_scw[k] / sqrt(t) : 0.0;
+#pragma unroll
+    for (int q = 0; q < SMALL_MAX_ROWS / 16; ++q) {
+      const int i = l16 + 16 * q;
+      if (i >= r) continue;
+      if (!tr) st(Oi, left(i, k), cscale(u[q], f));
+      else st(Oj, (size_t)k * n + i, cscale(cconj(u[q]), f));
+    }
+  }
+}
+
+hipError_t launch_gate_small(const GateTask* d_tasks, int ntasks, int fp32, bool lo, hipStream_t s) {
+  if (ntasks <= 0) return hipSuccess;
+  if (fp32) {
+    if (lo) hipLaunchKernelGGL((k_gate_small<float2, 256, SMALL_CAP_LO>), dim3(ntasks), dim3(256), 0, s, d_tasks);
+    else hipLaunchKernelGGL((k_gate_small<float2, 512, SMALL_CAP>), dim3(ntasks), dim3(512), 0, s, d_tasks);
+  } else {
+    if (lo) hipLaunchKernelGGL((k_gate_small<double2, 256, SMALL_CAP_LO>), dim3(ntasks), dim3(256), 0, s, d_tasks);
+    else hipLaunchKernelGGL((k_gate_small<double2, 512, SMALL_CAP>), dim3(ntasks), dim3(512), 0, s, d_tasks);
+  }
+  return hipGetLastError();
+}
+
+}  // namespace hipmps
