@@ -197,9 +197,7 @@ struct hipmps_engine_s {
   // on another) for rows of at most LQ_REG_MAX_COLS columns; HIPMPS_LQ_LOOKAHEAD=0 turns it off
   int lq_lookahead = 1;
   hipEvent_t lq_ev[2 * MAX_LANES] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
-  // completion of a wave's descriptor upload: the host edits the staged Jacobi descriptors
-  // after enqueuing that copy, and the copy may still wait behind earlier work on the stream
-  hipEvent_t stage_ev = nullptr;
+  hipEvent_t sweep_ev[2] = {nullptr, nullptr};  // counts of the last two sweeps queued have arrived
   long long stage_delay_ticks = 0;  // test hook: the upload held back this long (wall-clock ticks)
   DevBuf ws;     // per-wave arena
   DevBuf desc;   // task descriptors
@@ -750,21 +748,24 @@ int run_wave_general(hipmps_engine E, std::vector<WaveItem>& items, const std::f
   }
   RC_TRY(E->ws.ensure(off));
   char* ws = (char*)E->ws.p;
-  // small: counts (2N ints), K (N ints), wstats (WS_N doubles per item), ||X||_F^2 (N doubles)
-  size_t small_bytes = align_up(3 * N * sizeof(int)) + align_up(WS_N * N * sizeof(double)) + N * sizeof(double);
-  RC_TRY(E->small.ensure(small_bytes));
-  int* d_counts = (int*)E->small.p;
-  int* d_K = d_counts + 2 * N;
-  double* d_w = (double*)((char*)E->small.p + align_up(3 * N * sizeof(int)));
-  double* d_fro2 = (double*)((char*)d_w + align_up(WS_N * N * sizeof(double)));
+  // small: K (N ints) and wstats (WS_N doubles per item), read back together; ||X||_F^2 and its partial
+  // sums; per sweep the counts (2N ints), and N ints, all zeroed at the start
+  const size_t res_bytes = align_up(N * sizeof(int)) + align_up(WS_N * N * sizeof(double));
+  const size_t fro_bytes = align_up((size_t)(1 + FRO_BLOCKS) * N * sizeof(double));
+  const size_t cnt_bytes = align_up(((size_t)2 * E->max_sweeps + 1) * N * sizeof(int));
+  RC_TRY(E->small.ensure(res_bytes + fro_bytes + cnt_bytes));
+  int* d_K = (int*)E->small.p;
+  double* d_w = (double*)((char*)E->small.p + align_up(N * sizeof(int)));
+  double* d_fro2 = (double*)((char*)E->small.p + res_bytes);
+  int* d_counts = (int*)((char*)E->small.p + res_bytes + fro_bytes);
   // descriptors
   size_t desc_bytes = align_up(N * sizeof(ThetaTask)) + align_up(N * sizeof(SplitTask)) +
                       align_up(N * sizeof(JacTask)) + align_up(N * sizeof(GemmTask)) +
                       align_up(2 * N * sizeof(LqTask)) + align_up(3 * N * sizeof(TriTask)) +
-                      align_up(N * sizeof(double));
+                      align_up(N * sizeof(double)) + 2 * align_up(N * sizeof(JacTask));
   RC_TRY(E->desc.ensure(desc_bytes));
-  // host staging: descriptors | counts (2N ints) | active Jacobi list / results
-  const size_t stage_bytes = desc_bytes + align_up(2 * N * sizeof(int)) + N * sizeof(JacTask) + WS_N * N * sizeof(double) + 4096;
+  // host staging: descriptors | active Jacobi lists of the last two sweeps queued | counts | results
+  const size_t stage_bytes = desc_bytes + 2 * align_up(N * sizeof(JacTask)) + cnt_bytes + res_bytes;
   RC_TRY(E->hdesc.ensure(stage_bytes));
   RC_TRY(grow());
   char* hd = (char*)E->hdesc.p;
@@ -775,6 +776,9 @@ int run_wave_general(hipmps_engine E, std::vector<WaveItem>& items, const std::f
   LqTask* hlq = (LqTask*)((char*)hgm + align_up(N * sizeof(GemmTask)));
   TriTask* htr = (TriTask*)((char*)hlq + align_up(2 * N * sizeof(LqTask)));
   double* hcut = (double*)((char*)htr + align_up(3 * N * sizeof(TriTask)));  // rank cut, per LQ item
+  // Jacobi tasks of X (hjt: k_jacobi_prep), of the sweeps (hjs: R2 of LQ items, tiled), and a region for
+  // the sweeps' active lists
+  JacTask* hjs = (JacTask*)((char*)hcut + align_up(N * sizeof(double)));
   char* dd = (char*)E->desc.p;
   ThetaTask* dth = (ThetaTask*)dd;
   SplitTask* dsp = (SplitTask*)(dd + align_up(N * sizeof(ThetaTask)));
@@ -783,11 +787,13 @@ int run_wave_general(hipmps_engine E, std::vector<WaveItem>& items, const std::f
   LqTask* dlq = (LqTask*)((char*)dgm + align_up(N * sizeof(GemmTask)));
   TriTask* dtr = (TriTask*)((char*)dlq + align_up(2 * N * sizeof(LqTask)));
   const double* dcut = (const double*)((char*)dtr + align_up(3 * N * sizeof(TriTask)));
+  JacTask* djs = (JacTask*)((char*)dcut + align_up(N * sizeof(double)));
+  JacTask* dja = (JacTask*)((char*)djs + align_up(N * sizeof(JacTask)));
 
   // group boundaries
   int n64 = 0;
   while (n64 < N && !items[n64].fp32) ++n64;
-  int max_r = 0, max_c = 0, max_rpad = 0, max_k = 0;
+  int max_r = 0, max_c = 0, max_rpad = 0, max_k = 0, jt_blocks = 0, jt_ntc = 0;
   int tile_acc[2] = {0, 0};
   for (int q = 0; q < N; ++q) {
     auto& it = items[q];
@@ -838,19 +844,31 @@ int run_wave_general(hipmps_engine E, std::vector<WaveItem>& items, const std::f
     S.site_fp32 = it.fp32;
 
     JacTask& J = hjt[q];
-    J.Y = (double2*)(ws + it.off_y);  // X; for LQ items replaced by R2 after the factorizations
+    J.Y = (double2*)(ws + it.off_y);
     J.ldy = S.ldy;
     J.r = it.r;
     J.r_pad = it.r_pad;
     J.c = it.c;
     J.c_tot = it.c;
     J.nb = it.r_pad / JB;
-    J.counter = d_counts + 2 * q;
-    J.visited = d_counts + 2 * q + 1;
+    J.counts = d_counts + 2 * q;
+    J.cstride = 2 * N;
     J.fro2 = d_fro2 + q;
     J.tol = it.fp32 ? E->tol_mixed : E->tol;
-    J.gram32 = 0;
-    J.pad = 0;
+    J.gram32 = it.fp32 && it.r >= 256 ? E->gram32_sweeps : 0;
+    J.Yt = nullptr;
+    J.ntc = 0;
+    J.pad2 = 0;
+    JacTask& Js = hjs[q];  // the sweeps run on R2 (LQ items) or X, in tiles
+    Js = J;
+    if (it.lq) {
+      Js.Y = (double2*)(ws + it.off_j);
+      Js.ldy = Js.c = Js.c_tot = it.r;
+    }
+    Js.Yt = (double2*)(ws + it.off_jt);
+    Js.ntc = (Js.c_tot + 15) / 16;
+    jt_blocks = std::max(jt_blocks, Js.r_pad / 16);
+    jt_ntc = std::max(jt_ntc, Js.ntc);
 
     max_r = std::max(max_r, it.r);
     max_rpad = std::max(max_rpad, it.r_pad);
@@ -946,15 +964,7 @@ int run_wave_general(hipmps_engine E, std::vector<WaveItem>& items, const std::f
     HIP_TRY(hipGetLastError());
   }
   HIP_TRY(hipMemcpyAsync(dd, hd, desc_bytes, hipMemcpyHostToDevice, st));
-  HIP_TRY(hipEventRecord(E->stage_ev, st));
-  // the copy reads the staging buffer when the stream reaches it; the host edits the Jacobi
-  // descriptors there (LQ items switch to R2) only once it has been read
-  bool staged = false;
-  auto wait_staged = [&]() -> int {
-    if (!staged) HIP_TRY(hipEventSynchronize(E->stage_ev));
-    staged = true;
-    return 0;
-  };
+  HIP_TRY(hipMemsetAsync(d_counts, 0, cnt_bytes, st));
 
   if (E->timing) HIP_TRY(hipEventRecord(E->ev[0], st));
   // purified left sites: Kraus leg next to the left bond, [l][p][k][m] -> [l][k][p][m]
@@ -965,7 +975,7 @@ int run_wave_general(hipmps_engine E, std::vector<WaveItem>& items, const std::f
   if (n64 > 0) HIP_TRY(launch_theta(dth, n64, tile_acc[0], 0, st));
   if (N - n64 > 0) HIP_TRY(launch_theta(dth + n64, N - n64, tile_acc[1], 1, st));
   HIP_TRY(launch_jacobi_prep(dsp, djt, N, max_rpad, max_c, st));
-  HIP_TRY(launch_fro2(dsp, djt, N, st));
+  HIP_TRY(launch_fro2(dsp, djt, d_fro2 + N, d_counts + (size_t)2 * E->max_sweeps * N, N, st));
   if (E->timing) HIP_TRY(hipEventRecord(E->ev[6], st));
   // LQ lanes: with many items, contiguous slices of the LQ task arrays run their panel
   // sequences on separate streams, so that one slice's launch tails overlap another's work
@@ -1030,145 +1040,126 @@ int run_wave_general(hipmps_engine E, std::vector<WaveItem>& items, const std::f
     }
     RC_TRY(join_lanes(lq_lanes));
     if (any_cut) HIP_TRY(launch_rank_cut(dtr + N, dcut, nlq, st));
-    RC_TRY(wait_staged());
-    for (int q = 0; q < N; ++q) {
-      auto& it = items[q];
-      if (!it.lq) continue;
-      JacTask& J = hjt[q];
-      J.Y = (double2*)(ws + it.off_j);
-      J.ldy = it.r;
-      J.c = it.r;
-      J.c_tot = it.r;
-    }
   }
   if (E->timing) HIP_TRY(hipEventRecord(E->ev[1], st));
 
   // ---- Jacobi sweeps, on a tiled copy of every Jacobi matrix ----
-  int jt_blocks = 0, jt_ntc = 0;
-  RC_TRY(wait_staged());
-  for (int q = 0; q < N; ++q) {
-    JacTask& J = hjt[q];
-    J.Yt = (double2*)(ws + items[q].off_jt);
-    J.ntc = (J.c_tot + 15) / 16;
-    jt_blocks = std::max(jt_blocks, J.r_pad / 16);
-    jt_ntc = std::max(jt_ntc, J.ntc);
-  }
-  HIP_TRY(hipMemcpyAsync(djt, hjt, N * sizeof(JacTask), hipMemcpyHostToDevice, st));
-  HIP_TRY(launch_to_tiles(djt, N, jt_blocks, jt_ntc, st));
-  std::vector<int> active(N);
+  HIP_TRY(launch_to_tiles(djs, N, jt_blocks, jt_ntc, st));
+  std::vector<int> active(N), listed;
   for (int q = 0; q < N; ++q) active[q] = q;
   std::vector<int> sweeps_used(N, E->max_sweeps);
   std::vector<char> converged(N, 0);
-  // pairs each item rotated in the previous sweep: within a lane, the busiest items' block pairs
+  // pairs each item rotated in the last sweep seen: within a lane, the busiest items' block pairs
   // come first in the launch, so that the workgroups starting last (in the launch's tail) are
   // mostly the short ones of nearly converged items, which only form their Gram
   std::vector<long long> prev_rot(N, LLONG_MAX);
-  int* hcounts = (int*)((char*)E->hdesc.p + desc_bytes);
-  for (int sweep = 0; sweep < E->max_sweeps && !active.empty(); ++sweep) {
+  JacTask* hja[2] = {(JacTask*)(hd + desc_bytes), (JacTask*)(hd + desc_bytes + align_up(N * sizeof(JacTask)))};
+  int* hcounts = (int*)(hd + desc_bytes + 2 * align_up(N * sizeof(JacTask)));
+  constexpr int ML = hipmps_engine_s::MAX_LANES;
+  int lanes = 1, lane_begin[ML] = {0, 0, 0, 0}, lane_n[ML] = {0, 0, 0, 0}, lane_pairs[ML] = {0, 0, 0, 0},
+      lane_rounds[ML] = {0, 0, 0, 0};
+  // queue sweep `sweep` of the items in `active`, and the copy of its counts
+  auto enqueue = [&](int sweep) -> int {
     // active task list with pair prefix; with several lanes, the items are dealt to lists
     // of about equal work (largest first), each a prefix-indexed launch on its own stream
-    constexpr int ML = hipmps_engine_s::MAX_LANES;
-    int nact = (int)active.size();
-    JacTask* hja = (JacTask*)((char*)E->hdesc.p + desc_bytes + align_up(2 * N * sizeof(int)));
-    // lanes only pay when one launch would already fill the chip twice over (768 resident
-    // workgroups: 256 CUs x 3 at the kernel's register count); below that they add launches
-    int total_pairs = 0;
-    for (int q : active) total_pairs += hjt[q].nb / 2;
-    const int lanes = total_pairs >= E->lane_min_pairs ? std::max(1, std::min(E->jacobi_lanes, nact)) : 1;
-    std::vector<int> order(active);
-    if (lanes > 1)
-      std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return hjt[a].nb > hjt[b].nb; });
-    std::vector<int> lane_items[ML];
-    long long lane_load[ML] = {0, 0, 0, 0};
-    for (int q : order) {
-      int l = 0;
-      for (int k = 1; k < lanes; ++k)
-        if (lane_load[k] < lane_load[l]) l = k;
-      lane_items[l].push_back(q);
-      lane_load[l] += (long long)(hjt[q].nb / 2) * hjt[q].c * (hjt[q].nb - 1);
-    }
-    for (int l = 0; l < lanes; ++l)
-      std::stable_sort(lane_items[l].begin(), lane_items[l].end(),
-                       [&](int a, int b) { return prev_rot[a] > prev_rot[b]; });
-    int lane_begin[ML] = {0, 0, 0, 0}, lane_n[ML] = {0, 0, 0, 0}, lane_pairs[ML] = {0, 0, 0, 0},
-        lane_rounds[ML] = {0, 0, 0, 0};
-    {
+    if (active != listed) {
+      const int nact = (int)active.size();
+      JacTask* ha = hja[sweep & 1];  // its last reader, an upload two sweeps back, has run
+      // lanes only pay when one launch would already fill the chip twice over (768 resident
+      // workgroups: 256 CUs x 3 at the kernel's register count); below that they add launches
+      int total_pairs = 0;
+      for (int q : active) total_pairs += hjs[q].nb / 2;
+      lanes = total_pairs >= E->lane_min_pairs ? std::max(1, std::min(E->jacobi_lanes, nact)) : 1;
+      std::vector<int> order(active);
+      if (lanes > 1)
+        std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return hjs[a].nb > hjs[b].nb; });
+      std::vector<int> lane_items[ML];
+      long long lane_load[ML] = {0, 0, 0, 0};
+      for (int q : order) {
+        int l = 0;
+        for (int k = 1; k < lanes; ++k)
+          if (lane_load[k] < lane_load[l]) l = k;
+        lane_items[l].push_back(q);
+        lane_load[l] += (long long)(hjs[q].nb / 2) * hjs[q].c * (hjs[q].nb - 1);
+      }
       int a = 0;
       for (int l = 0; l < lanes; ++l) {
+        std::stable_sort(lane_items[l].begin(), lane_items[l].end(),
+                         [&](int x, int y) { return prev_rot[x] > prev_rot[y]; });
         lane_begin[l] = a;
+        lane_pairs[l] = lane_rounds[l] = 0;
         for (int q : lane_items[l]) {
-          hja[a] = hjt[q];
-          hja[a].gram32 = (sweep < E->gram32_sweeps && items[q].fp32 && hjt[q].r >= 256) ? 1 : 0;
-          hja[a].pair_begin = lane_pairs[l];
-          lane_pairs[l] += hja[a].nb / 2;
-          lane_rounds[l] = std::max(lane_rounds[l], hja[a].nb - 1);
+          ha[a] = hjs[q];
+          ha[a].pair_begin = lane_pairs[l];
+          lane_pairs[l] += ha[a].nb / 2;
+          lane_rounds[l] = std::max(lane_rounds[l], ha[a].nb - 1);
           ++a;
         }
         lane_n[l] = a - lane_begin[l];
       }
+      HIP_TRY(hipMemcpyAsync(dja, ha, nact * sizeof(JacTask), hipMemcpyHostToDevice, st));
+      listed = active;
     }
-    // reuse the JacTask region of the device descriptor block for the active list
-    HIP_TRY(hipMemcpyAsync(djt, hja, nact * sizeof(JacTask), hipMemcpyHostToDevice, st));
-    HIP_TRY(hipMemsetAsync(d_counts, 0, 2 * N * sizeof(int), st));
-    if (E->timing) HIP_TRY(hipEventRecord(E->ev[4], st));
+    if (E->timing && sweep == 0) HIP_TRY(hipEventRecord(E->ev[4], st));
     int max_rounds = 0;
     for (int l = 0; l < lanes; ++l) max_rounds = std::max(max_rounds, lane_rounds[l]);
-    if (lanes > 1) {
-      HIP_TRY(hipEventRecord(E->lane_ev[0], st));
-      for (int l = 1; l < lanes; ++l) HIP_TRY(hipStreamWaitEvent(E->lane_stream[l], E->lane_ev[0], 0));
-    }
+    RC_TRY(fork_lanes(lanes));
     for (int round = 0; round < max_rounds; ++round)
       for (int l = 0; l < lanes; ++l)
         if (lane_n[l] > 0 && round < lane_rounds[l])
-          HIP_TRY(launch_jacobi_round(djt + lane_begin[l], lane_n[l], lane_pairs[l], round, E->lane_stream[l],
+          HIP_TRY(launch_jacobi_round(dja + lane_begin[l], lane_n[l], lane_pairs[l], sweep, round, E->lane_stream[l],
                                       true));
-    for (int l = 1; l < lanes; ++l) {
-      HIP_TRY(hipEventRecord(E->lane_ev[l], E->lane_stream[l]));
-      HIP_TRY(hipStreamWaitEvent(st, E->lane_ev[l], 0));
-    }
-    if (E->timing) HIP_TRY(hipEventRecord(E->ev[5], st));
+    RC_TRY(join_lanes(lanes));
     for (int l = 0; l < lanes; ++l) E->prof.jacobi_launches += lane_rounds[l];
-    HIP_TRY(hipMemcpyAsync(hcounts, d_counts, 2 * N * sizeof(int), hipMemcpyDeviceToHost, st));
-    HIP_TRY(hipStreamSynchronize(st));
-    if (E->timing) {
-      float ms = 0;
-      (void)hipEventElapsedTime(&ms, E->ev[4], E->ev[5]);
-      E->prof.ms_jacobi_rounds += ms;
-    }
-    if (E->debug_sweeps) {
-      long long R = 0, V = 0;
-      for (int a = 0; a < nact; ++a) R += hcounts[2 * active[a]], V += hcounts[2 * active[a] + 1];
-      fprintf(stderr, "[hipmps sweep] wave %lld sweep %d active %d rotated %lld visited %lld\n", E->prof.waves, sweep,
-              nact, R, V);
-      if (sweep >= 25)
-        for (int a = 0; a < nact; ++a) {
-          const int q = active[a];
-          fprintf(stderr, "[hipmps sweep]   item %d: m %d n %d r %d lq %d fp32 %d rotated %d visited %d\n", q,
-                  items[q].m, items[q].n, items[q].r, items[q].lq, items[q].fp32, hcounts[2 * q], hcounts[2 * q + 1]);
-        }
-    }
+    const size_t at = (size_t)2 * N * sweep;
+    HIP_TRY(hipMemcpyAsync(hcounts + at, d_counts + at, 2 * N * sizeof(int), hipMemcpyDeviceToHost, st));
+    HIP_TRY(hipEventRecord(E->sweep_ev[sweep & 1], st));
+    return 0;
+  };
+  // wait for a sweep's counts; returns whether few pairs rotated (few or none will in the next sweep)
+  bool nearly = false;
+  auto finish = [&](int sweep) -> int {
+    HIP_TRY(hipEventSynchronize(E->sweep_ev[sweep & 1]));
+    const int* cnt = hcounts + (size_t)2 * N * sweep;
+    long long R = 0, V = 0;
     std::vector<int> next;
-    for (int a = 0; a < nact; ++a) {
-      int q = active[a];
-      long long rot = hcounts[2 * q], vis = hcounts[2 * q + 1];
+    for (int q : active) {
+      const long long rot = cnt[2 * q], vis = cnt[2 * q + 1];
+      R += rot;
+      V += vis;
       prev_rot[q] = rot;
-      E->prof.jacobi_pairs_rotated += rot;
-      E->prof.jacobi_pairs_visited += vis;
-      const double c = items[q].lq ? items[q].r : items[q].c;  // columns the Jacobi works on
-      E->prof.jacobi_flops += 8.0 * JP * JP * c * (double)(vis + rot);
-      const bool g32 = sweep < E->gram32_sweeps && items[q].fp32 && hjt[q].r >= 256;
-      if (rot == 0 && !g32) {
+      E->prof.jacobi_flops += 8.0 * JP * JP * hjs[q].c * (double)(vis + rot);
+      if (rot == 0 && sweep >= hjs[q].gram32) {
         sweeps_used[q] = sweep + 1;
         converged[q] = 1;
       } else {
         next.push_back(q);
       }
     }
+    E->prof.jacobi_pairs_rotated += R;
+    E->prof.jacobi_pairs_visited += V;
+    nearly = R * 20 <= V;
+    if (E->debug_sweeps) {
+      fprintf(stderr, "[hipmps sweep] wave %lld sweep %d active %d rotated %lld visited %lld\n", E->prof.waves, sweep,
+              (int)active.size(), R, V);
+      if (sweep >= 25)
+        for (int q : active)
+          fprintf(stderr, "[hipmps sweep]   item %d: m %d n %d r %d lq %d fp32 %d rotated %d visited %d\n", q,
+                  items[q].m, items[q].n, items[q].r, items[q].lq, items[q].fp32, cnt[2 * q], cnt[2 * q + 1]);
+    }
     active.swap(next);
+    return 0;
+  };
+  // One sweep is queued ahead of the one whose counts the host waits for, so that the device does not
+  // idle between sweeps (it did for 40 us, a fifth of a sweep at rank 128); converged items return at
+  // once.  Not when the last sweep seen rotated few pairs: then the one in flight is the last or nearly
+  // so, and an empty sweep of nb - 1 launches would follow it.
+  for (int sweep = 0, seen = 0; sweep < E->max_sweeps && !active.empty(); ++sweep) {
+    RC_TRY(enqueue(sweep));
+    while (seen < sweep || (seen == sweep && (nearly || sweep + 1 == E->max_sweeps))) RC_TRY(finish(seen++));
   }
-  // rows back from the tiles (the full task list: the device copy held the last active list)
-  HIP_TRY(hipMemcpyAsync(djt, hjt, N * sizeof(JacTask), hipMemcpyHostToDevice, st));
-  HIP_TRY(launch_from_tiles(djt, N, jt_blocks, jt_ntc, st));
+  if (E->timing) HIP_TRY(hipEventRecord(E->ev[5], st));
+  HIP_TRY(launch_from_tiles(djs, N, jt_blocks, jt_ntc, st));
   if (nlq > 0) {  // rows of the Jacobi result back to the column space of X
     RC_TRY(fork_lanes(lq_lanes));
     for (int l = 0; l < lq_lanes; ++l) {
@@ -1209,10 +1200,9 @@ int run_wave_general(hipmps_engine E, std::vector<WaveItem>& items, const std::f
                               it.fp32, st));
   }
   // results
-  int* hK = hcounts;  // reuse staging
-  double* hw = (double*)((char*)E->hdesc.p + desc_bytes + align_up(2 * N * sizeof(int)));
-  HIP_TRY(hipMemcpyAsync(hK, d_K, N * sizeof(int), hipMemcpyDeviceToHost, st));
-  HIP_TRY(hipMemcpyAsync(hw, d_w, WS_N * N * sizeof(double), hipMemcpyDeviceToHost, st));
+  const int* hK = (const int*)((char*)hcounts + cnt_bytes);
+  const double* hw = (const double*)((const char*)hK + align_up(N * sizeof(int)));
+  HIP_TRY(hipMemcpyAsync((char*)hcounts + cnt_bytes, d_K, res_bytes, hipMemcpyDeviceToHost, st));
   if (E->timing) HIP_TRY(hipEventRecord(E->ev[3], st));
   HIP_TRY(hipStreamSynchronize(st));
   RC_TRY(join());
@@ -1222,6 +1212,9 @@ int run_wave_general(hipmps_engine E, std::vector<WaveItem>& items, const std::f
     (void)hipEventElapsedTime(&d, E->ev[6], E->ev[1]);
     (void)hipEventElapsedTime(&b, E->ev[1], E->ev[2]);
     (void)hipEventElapsedTime(&c, E->ev[2], E->ev[3]);
+    float rounds = 0;
+    (void)hipEventElapsedTime(&rounds, E->ev[4], E->ev[5]);
+    E->prof.ms_jacobi_rounds += rounds;
     E->prof.ms_theta += a;
     E->prof.ms_lq += d;
     E->prof.ms_jacobi += b;
@@ -1454,12 +1447,11 @@ int run_kraus_waves(hipmps_engine E, const std::vector<hipmps_state_s*>& states)
     J.c = h.jc;
     J.c_tot = h.ld;
     J.nb = h.r_pad / JB;
-    J.counter = d_counts + 2 * i;
-    J.visited = d_counts + 2 * i + 1;
+    J.counts = d_counts + 2 * i;
+    J.cstride = 0;
     J.fro2 = nullptr;
     J.tol = s->fp32 ? E->tol_mixed : E->tol;
     J.gram32 = 0;
-    J.pad = 0;
     J.Yt = nullptr;  // row-major sweeps
     J.ntc = 0;
     J.pad2 = 0;
@@ -1496,7 +1488,7 @@ int run_kraus_waves(hipmps_engine E, const std::vector<hipmps_state_s*>& states)
     HIP_TRY(hipMemcpyAsync(djt, hja, active.size() * sizeof(JacTask), hipMemcpyHostToDevice, st));
     HIP_TRY(hipMemsetAsync(d_counts, 0, 2 * (size_t)C * sizeof(int), st));
     for (int round = 0; round < rounds; ++round)
-      HIP_TRY(launch_jacobi_round(djt, (int)active.size(), pairs, round, st));
+      HIP_TRY(launch_jacobi_round(djt, (int)active.size(), pairs, 0, round, st));
     HIP_TRY(hipMemcpyAsync(hcount, d_counts, 2 * (size_t)C * sizeof(int), hipMemcpyDeviceToHost, st));
     HIP_TRY(hipStreamSynchronize(st));
     std::vector<int> next;
@@ -2605,12 +2597,13 @@ int hipmps_engine_create(const hipmps_engine_opts* opts, hipmps_engine* out) {
   for (int l = 1; l < hipmps_engine_s::MAX_LANES; ++l)
     ok = ok && hipStreamCreateWithFlags(&e->lane_stream[l], hipStreamNonBlocking) == hipSuccess;
   for (auto& ev : e->lane_ev) ok = ok && hipEventCreateWithFlags(&ev, hipEventDisableTiming) == hipSuccess;
-  if (hipEventCreateWithFlags(&e->stage_ev, hipEventDisableTiming) != hipSuccess) {
-    e->stage_ev = nullptr;
-    (void)hipGetLastError();
-    (void)hipmps_engine_destroy(e);
-    return fail(HIPMPS_E_DEVICE, "event creation failed");
-  }
+  for (auto& ev : e->sweep_ev)
+    if (hipEventCreateWithFlags(&ev, hipEventDisableTiming) != hipSuccess) {
+      ev = nullptr;
+      (void)hipGetLastError();
+      (void)hipmps_engine_destroy(e);
+      return fail(HIPMPS_E_DEVICE, "event creation failed");
+    }
   bool lq_ok = true;
   for (auto& ev : e->lq_ev) lq_ok = lq_ok && hipEventCreateWithFlags(&ev, hipEventDisableTiming) == hipSuccess;
   if (!lq_ok) {
@@ -2681,7 +2674,8 @@ int hipmps_engine_destroy(hipmps_engine e) {
     if (ev) (void)hipEventDestroy(ev);
   for (auto& ev : e->lq_ev)
     if (ev) (void)hipEventDestroy(ev);
-  if (e->stage_ev) (void)hipEventDestroy(e->stage_ev);
+  for (auto& ev : e->sweep_ev)
+    if (ev) (void)hipEventDestroy(ev);
   for (int l = 1; l < hipmps_engine_s::MAX_LANES; ++l)
     if (e->lane_stream[l]) {
       (void)hipStreamSynchronize(e->lane_stream[l]);

@@ -37,14 +37,14 @@ struct JacTask {
   int c_tot;
   int nb;            // r_pad / JB (even)
   int pair_begin;    // first block of this task in the grid
-  int* counter;      // rotated block pairs in the current sweep
-  int* visited;      // block pairs visited in the current sweep
+  int* counts;       // per sweep s: counts[s * cstride] block pairs rotated, [s * cstride + 1] visited
   double* fro2;      // ||X||_F^2 (k_fro2), or null: rows with squared norm below JAC_FLOOR2 * fro2 are
                      // numerically zero (rounding residue) and neither rotate nor count against
                      // convergence
   double tol;        // relative off-diagonal below which a block pair counts as orthogonal
-  int gram32;        // this sweep forms the Gram with FP32 MFMA (rotations and updates stay FP64)
-  int pad;
+  int gram32;        // the first gram32 sweeps form the Gram with FP32 MFMA (rotations and updates stay
+                     // FP64); such a sweep never counts as the converged one
+  int cstride;
   double2* Yt;       // the same rows in tiles (jac_tile_offset), or null: the sweeps of the main path
                      // run on Yt (launch_to_tiles before, launch_from_tiles after)
   int ntc;           // 16-column tiles per 16-row block of Yt: ceil(c_tot / 16)
@@ -195,10 +195,15 @@ hipError_t launch_jacobi_prep(const SplitTask* d_split, const JacTask* d_jac, in
 // (1e-15)^2: a row whose norm is below 1e-15 ||X||_F lies under FP64 resolution of any result
 // computed from X, so the relative convergence test has no meaning for it
 constexpr double JAC_FLOOR2 = 1e-30;
-// *jt[t].fro2 = ||theta'_t||_F^2 (= ||X||_F^2 = ||R2||_F^2), one workgroup per task, fixed order
-hipError_t launch_fro2(const SplitTask* d_split, const JacTask* d_jac, int ntasks, hipStream_t s);
-hipError_t launch_jacobi_round(const JacTask* d_tasks, int ntasks, int total_pairs, int round, hipStream_t s,
-                               bool tiled = false);
+// *jt[t].fro2 = ||theta'_t||_F^2 (= ||X||_F^2 = ||R2||_F^2): FRO_BLOCKS partial sums per task in `part`, added
+// in order by the last workgroup of the task to finish (`done`: a zeroed int per task)
+constexpr int FRO_BLOCKS = 32;
+hipError_t launch_fro2(const SplitTask* d_split, const JacTask* d_jac, double* part, int* done, int ntasks,
+                       hipStream_t s);
+// One round of sweep `sweep`.  A task whose previous sweep (not a gram32 one) rotated nothing has converged
+// and its workgroups return at once, so that a sweep can be queued before the host has seen the last one.
+hipError_t launch_jacobi_round(const JacTask* d_tasks, int ntasks, int total_pairs, int sweep, int round,
+                               hipStream_t s, bool tiled = false);
 // Y (row-major, ldy) <-> Yt (tiled, ntc) for every task: rows [0, r_pad), columns [0, c_tot);
 // to_tiles writes zeros into the tile columns past c_tot.  max_blocks = largest r_pad / 16.
 hipError_t launch_to_tiles(const JacTask* d_tasks, int ntasks, int max_blocks, int max_ntc, hipStream_t s);

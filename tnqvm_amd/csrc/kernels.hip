@@ -478,7 +478,7 @@ __device__ __forceinline__ void inner_sweep(InnerShared& S, double itol, double 
 // BLK is the block size JB (a template parameter: the kernel's register allocation on
 // gfx950 comes out at 168 VGPRs, three waves per SIMD, in the tiled form).
 template <int BLK, bool TILED>
-__global__ __launch_bounds__(256, 2) void k_jacobi_round(const JacTask* tasks, int ntasks, int round) {
+__global__ __launch_bounds__(256, 2) void k_jacobi_round(const JacTask* tasks, int ntasks, int sweep, int round) {
   static_assert(BLK == 16 && JB == BLK && JP == 2 * BLK, "256 threads map onto 16 x 16 rotation-pair blocks");
   __shared__ InnerShared S;
   double2 (*sG)[JP + 1] = S.G[0];
@@ -489,6 +489,8 @@ __global__ __launch_bounds__(256, 2) void k_jacobi_round(const JacTask* tasks, i
   const int pi = blockIdx.x - T.pair_begin;
   const int nb = T.nb;
   if (pi >= nb / 2 || round >= nb - 1) return;
+  int* counts = T.counts + (size_t)sweep * T.cstride;
+  if (sweep > T.gram32 && counts[-T.cstride] == 0) return;  // converged in the sweep before
   const int ba = circle_slot(pi, round, nb), bb = circle_slot(nb - 1 - pi, round, nb);
   const int C = T.c, CT = T.c_tot;
   const size_t ld = T.ldy;
@@ -530,7 +532,7 @@ __global__ __launch_bounds__(256, 2) void k_jacobi_round(const JacTask* tasks, i
   //    K3 = -Ai (Br + Bi)^T;  Re = K1 - K3, Im = K1 + K2.
   // Each partial sum of the four waves goes to LDS as (Re, X) for the diagonal tiles and
   // (Re, Im) for the off-diagonal one; Im of the diagonal tiles is formed after the sum.
-  if (!T.gram32) {
+  if (sweep >= T.gram32) {
     mfma_d4 a00r = {0, 0, 0, 0}, a00x = {0, 0, 0, 0}, a11r = {0, 0, 0, 0}, a11x = {0, 0, 0, 0};
     mfma_d4 k1 = {0, 0, 0, 0}, k2 = {0, 0, 0, 0}, k3 = {0, 0, 0, 0};
     double2 x0[PD], x1[PD];
@@ -650,7 +652,7 @@ __global__ __launch_bounds__(256, 2) void k_jacobi_round(const JacTask* tasks, i
     if (lane == 0) S.rot[wave] = above;
     __syncthreads();
   }
-  if (tid == 0) atomicAdd(T.visited, 1);
+  if (tid == 0) atomicAdd(counts + 1, 1);
   if (!(S.rot[0] | S.rot[1] | S.rot[2] | S.rot[3])) return;
 
   // ---- apply prefetch: this wave's first column tile, all 32 rows ----
@@ -699,37 +701,49 @@ __global__ __launch_bounds__(256, 2) void k_jacobi_round(const JacTask* tasks, i
       }
     }
   }
-  if (tid == 0) atomicAdd(T.counter, 1);
+  if (tid == 0) atomicAdd(counts, 1);
 }
 
-__global__ __launch_bounds__(256) void k_fro2(const SplitTask* sp, const JacTask* jt) {
-  __shared__ double red[256];
-  const SplitTask& S = sp[blockIdx.x];
+// Bound by the read of theta'; one workgroup a task took 2.5 ms at 1536 x 1536 and 220 us a wave of 512 x 512.
+__global__ __launch_bounds__(256) void k_fro2(const SplitTask* sp, const JacTask* jt, double* part, int* done) {
+  __shared__ double red[4];
+  __shared__ int last;
+  const SplitTask& S = sp[blockIdx.y];
   const size_t n = (size_t)S.m * S.n;
+  const double2* x = S.theta;
   double a = 0.0;
-  for (size_t e = threadIdx.x; e < n; e += 256) a += cabs2(S.theta[e]);
-  red[threadIdx.x] = a;
+  for (size_t e = (size_t)blockIdx.x * 256 + threadIdx.x; e < n; e += (size_t)FRO_BLOCKS * 256) a += cabs2(gld(x + e));
+  a = wave_sum(a);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = a;
   __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if (threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-    __syncthreads();
+  double* mine = part + (size_t)blockIdx.y * FRO_BLOCKS;
+  if (threadIdx.x == 0) {
+    __hip_atomic_store(mine + blockIdx.x, (red[0] + red[1]) + (red[2] + red[3]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    last = __hip_atomic_fetch_add(done + blockIdx.y, 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == FRO_BLOCKS - 1;
   }
-  if (threadIdx.x == 0 && jt[blockIdx.x].fro2) *jt[blockIdx.x].fro2 = red[0];
+  __syncthreads();
+  if (!last || threadIdx.x != 0) return;
+  double t = 0.0;
+  for (int b = 0; b < FRO_BLOCKS; ++b) t += __hip_atomic_load(mine + b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  *jt[blockIdx.y].fro2 = t;
 }
 
-hipError_t launch_fro2(const SplitTask* d_split, const JacTask* d_jac, int ntasks, hipStream_t s) {
+hipError_t launch_fro2(const SplitTask* d_split, const JacTask* d_jac, double* part, int* done, int ntasks,
+                       hipStream_t s) {
   if (ntasks <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_fro2, dim3(ntasks), dim3(256), 0, s, d_split, d_jac);
+  hipLaunchKernelGGL(k_fro2, dim3(FRO_BLOCKS, ntasks), dim3(256), 0, s, d_split, d_jac, part, done);
   return hipGetLastError();
 }
 
-hipError_t launch_jacobi_round(const JacTask* d_tasks, int ntasks, int total_pairs, int round, hipStream_t s,
-                               bool tiled) {
+hipError_t launch_jacobi_round(const JacTask* d_tasks, int ntasks, int total_pairs, int sweep, int round,
+                               hipStream_t s, bool tiled) {
   if (total_pairs <= 0) return hipSuccess;
   if (tiled)
-    hipLaunchKernelGGL((k_jacobi_round<JB, true>), dim3(total_pairs), dim3(256), 0, s, d_tasks, ntasks, round);
+    hipLaunchKernelGGL((k_jacobi_round<JB, true>), dim3(total_pairs), dim3(256), 0, s, d_tasks, ntasks, sweep,
+                       round);
   else
-    hipLaunchKernelGGL((k_jacobi_round<JB, false>), dim3(total_pairs), dim3(256), 0, s, d_tasks, ntasks, round);
+    hipLaunchKernelGGL((k_jacobi_round<JB, false>), dim3(total_pairs), dim3(256), 0, s, d_tasks, ntasks, sweep,
+                       round);
   return hipGetLastError();
 }
 
