@@ -163,6 +163,10 @@ int hipmps_amplitudes_noalloc(hipmps_state s, const int8_t* bits, int k, double*
 /* <psi| (x)_k diag(d[2k], d[2k+1]) |psi>: Z strings, projectors (sequential sampling,
  * getMeasureSample :2211-2364), occupation numbers */
 int hipmps_expval_diag(hipmps_state s, const double* diag_2n, double* out);
+/* P(outcome) of k <= 16 listed qubits: out[x], x = sum_i b_i 2^i with b_i the bit of qubits[i], is the
+ * value of hipmps_expval_diag for the projectors of that outcome (unnormalised), all 2^k at once.  The
+ * reference's noisy visitor reads them off the density matrix (ExaTnPmpsVisitor.cpp:657-761). */
+int hipmps_outcome_probabilities(hipmps_state s, const int* qubits, int k, double* out);
 /* getMeasureSample (ExaTnMpsVisitor.cpp:2211-2364, the reference's sampling for n >= 20) for `shots`
  * shots at once, every shot's marginals advanced together on the device.  qubits: the k measured
  * qubits in Measure order, which must be increasing (HIPMPS_E_UNSUPPORTED otherwise); draws: shots * k

@@ -64,6 +64,12 @@ def test_observables(eng, bonds, precision):
     assert abs(s.norm() - expval(sites, diag([]))) < 1e-11
     assert abs(s.expval_z_parity(range(0, n, 2)) - expval(sites, diag(list(range(0, n, 2))))) < 1e-11
     assert abs(s.expval_diag(d) / np.abs(d).max(1).prod() - expval(sites, d) / np.abs(d).max(1).prod()) < 1e-11
+    qs = [n - 1, 0]
+    want = np.zeros(4)
+    for x in range(4):
+        pr = {qs[0]: x & 1, qs[1]: x >> 1}
+        want[x] = expval(sites, [(1.0, 1.0) if k not in pr else (float(pr[k] == 0), float(pr[k] == 1)) for k in range(n)])
+    assert np.abs(s.outcome_probabilities(qs) - want).max() < 1e-11
     s.close()
 
 

@@ -35,7 +35,7 @@ EXPORTS = [
     "hipmps_amplitudes", "hipmps_wavefunction_slice", "hipmps_state_vector", "hipmps_get_site",
     "hipmps_set_site", "hipmps_run_batch", "hipmps_serve_submit", "hipmps_serve_step",
     "hipmps_serve_poll", "hipmps_serve_pending", "hipmps_engine_profile", "hipmps_engine_set_timing", "hipmps_engine_set_lq_precondition",
-    "hipmps_expval_diag", "hipmps_state_clone", "hipmps_apply_kraus", "hipmps_kraus_dims",
+    "hipmps_expval_diag", "hipmps_outcome_probabilities", "hipmps_state_clone", "hipmps_apply_kraus", "hipmps_kraus_dims",
     "hipmps_reduced_density_matrix", "hipmps_engine_get_tuning", "hipmps_engine_set_tuning",
     "hipmps_queue_gates", "hipmps_queue_kraus", "hipmps_run_waves", "hipmps_circuit_footprint",
     "hipmps_amplitudes_noalloc", "hipmps_sample_sequential",
@@ -152,6 +152,7 @@ def lib():
         "hipmps_engine_set_timing": ([vp, ip], ip),
         "hipmps_engine_set_lq_precondition": ([vp, ip], ip),
         "hipmps_expval_diag": ([vp, dp, dp], ip),
+        "hipmps_outcome_probabilities": ([vp, pint, ip, dp], ip),
         "hipmps_state_clone": ([vp, ctypes.POINTER(vp)], ip),
         "hipmps_apply_kraus": ([vp, ip, ip, dp], ip),
         "hipmps_kraus_dims": ([vp, pint], ip),

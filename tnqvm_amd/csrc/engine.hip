@@ -1854,9 +1854,59 @@ int trace_products(hipmps_engine E, const std::vector<const double2*>& A, const 
   return 0;
 }
 
+// Values of `m` diagonals at once on a state of small bonds (k_env_chain), when that is estimated to take
+// less than the sweeps of products launched one by one that they replace (`sweeps` of them): a step of a
+// site takes about 1000 clocks and 20 per contraction index and 256 elements, and 512 workgroups run at a
+// time; a sweep's two products a site take 10 us.
+bool chain_fits(const hipmps_state_s* s, size_t m, size_t sweeps) {
+  double clocks = 0.0;
+  for (int k = 0; k < s->n; ++k) {
+    const int cl = s->chi[k], cr = s->chi[k + 1];
+    if (cl > CHAIN_MAX_BOND || cr > CHAIN_MAX_BOND) return false;
+    const int steps = (2 * s->kap[k] + chain_slots(cl, cr) - 1) / chain_slots(cl, cr);
+    clocks += steps * (1000.0 + 20.0 * cl * ((cl * cr + 255) / 256 + (cr * cr + 255) / 256)) + 1500.0;
+  }
+  return clocks * (double)((m + 511) / 512) < 24000.0 * s->n * sweeps;
+}
+
+// out[t] = value of diagonal t; set(t, d): diagonal t's 2n values into d
+int chain_values(hipmps_state_s* s, size_t m, const std::function<void(size_t, double*)>& set, double* out) {
+  hipmps_engine E = s->e;
+  const int n = s->n;
+  constexpr size_t BLK = 4096;
+  const size_t sb = align_up(n * sizeof(ChainSite)), cb = std::min(m, BLK), db = align_up(cb * 2 * n * sizeof(double));
+  RC_TRY(E->desc.ensure(sb + db + cb * sizeof(double)));
+  RC_TRY(E->hdesc.ensure(sb + db + cb * sizeof(double)));
+  char* h = (char*)E->hdesc.p;
+  char* d = (char*)E->desc.p;
+  for (int k = 0; k < n; ++k)
+    ((ChainSite*)h)[k] = {s->sites[k].p, s->chi[k], s->chi[k + 1], s->kap[k], 0};
+  for (size_t t0 = 0; t0 < m; t0 += BLK) {
+    const size_t b = std::min(BLK, m - t0);
+    for (size_t t = 0; t < b; ++t) set(t0 + t, (double*)(h + sb) + t * 2 * n);
+    HIP_TRY(hipMemcpyAsync(d, h, sb + b * 2 * n * sizeof(double), hipMemcpyHostToDevice, E->stream));
+    HIP_TRY(launch_env_chain((const ChainSite*)d, n, (const double*)(d + sb), (double*)(d + sb + db), (int)b, s->fp32,
+                             E->stream));
+    HIP_TRY(hipMemcpyAsync(h + sb + db, d + sb + db, b * sizeof(double), hipMemcpyDeviceToHost, E->stream));
+    HIP_TRY(hipStreamSynchronize(E->stream));  // staging reuse
+    memcpy(out + t0, h + sb + db, b * sizeof(double));
+  }
+  return 0;
+}
+
 // <Z_i> for every site; with norm, also <psi|psi> (the closed left environment)
 int measure_z_all(hipmps_state_s* s, double* out, double* norm = nullptr) {
   hipmps_engine E = s->e;
+  if (chain_fits(s, (size_t)s->n + 1, 1)) {
+    std::vector<double> v(s->n + 1);
+    RC_TRY(chain_values(s, v.size(), [&](size_t t, double* d) {
+      std::fill(d, d + 2 * s->n, 1.0);
+      if (t < (size_t)s->n) d[2 * t + 1] = -1.0;
+    }, v.data()));
+    std::copy(v.begin(), v.end() - 1, out);
+    if (norm) *norm = v.back();
+    return 0;
+  }
   const EnvLayout L = env_layout(s, true, true);
   RC_TRY(E->env.ensure(L.total));
   char* base = (char*)E->env.p;
@@ -1880,6 +1930,12 @@ int measure_zz(hipmps_state_s* s, const int* pairs, int k, double* out) {
     if (a < 0 || a >= n || b < 0 || b >= n) return fail(HIPMPS_E_ARG, "zz pair out of range");
     if (a != b) ends[std::min(a, b)].push_back(std::max(a, b));
   }
+  if (chain_fits(s, (size_t)k, 2))
+    return chain_values(s, (size_t)k, [&](size_t t, double* d) {
+      std::fill(d, d + 2 * n, 1.0);
+      d[2 * pairs[2 * t] + 1] *= -1.0;
+      d[2 * pairs[2 * t + 1] + 1] *= -1.0;  // Z_i Z_i = I
+    }, out);
   EnvLayout L = env_layout(s, true, true);
   size_t xmax = 1;
   for (int q = 0; q < n; ++q) xmax = std::max(xmax, site_elems(s, q));
@@ -1950,11 +2006,32 @@ int measure_zz(hipmps_state_s* s, const int* pairs, int k, double* out) {
 // <psi| (x)_k diag(d[2k], d[2k+1]) |psi>, diag empty: <psi|psi>
 int measure_diag(hipmps_state_s* s, const std::vector<double>& diag, double* out) {
   hipmps_engine E = s->e;
+  if (chain_fits(s, 1, 1))
+    return chain_values(s, 1, [&](size_t, double* d) {
+      if (diag.empty()) std::fill(d, d + 2 * s->n, 1.0);
+      else std::copy(diag.begin(), diag.end(), d);
+    }, out);
   const EnvLayout L = env_layout(s, false, false);
   RC_TRY(E->env.ensure(L.total));
   EnvPlan P;
   env_sweeps(P, left_jobs(s, L, (char*)E->env.p, diag), {});
   return env_run(s, L, P, nullptr, out);
+}
+
+// P(outcome x) of the listed qubits for every x = sum_i b_i 2^i
+int measure_outcomes(hipmps_state_s* s, const int* qubits, int k, double* out) {
+  const size_t m = (size_t)1 << k;
+  auto set = [&](size_t x, double* d) {
+    std::fill(d, d + 2 * s->n, 1.0);
+    for (int i = 0; i < k; ++i) d[2 * qubits[i] + (1 - ((x >> i) & 1))] = 0.0;
+  };
+  if (chain_fits(s, m, m)) return chain_values(s, m, set, out);
+  std::vector<double> diag(2 * s->n);
+  for (size_t x = 0; x < m; ++x) {
+    set(x, diag.data());
+    RC_TRY(measure_diag(s, diag, out + x));
+  }
+  return 0;
 }
 
 int measure_parity(hipmps_state_s* s, const std::vector<int>& zmask, double* out) {
@@ -3008,6 +3085,15 @@ int hipmps_expval_diag(hipmps_state s, const double* diag, double* out) {
   RC_TRY(state_flush(s));
   std::vector<double> d(diag, diag + 2 * s->n);
   return measure_diag(s, d, out);
+}
+
+int hipmps_outcome_probabilities(hipmps_state s, const int* qubits, int k, double* out) {
+  if (!s || !out || k < 0 || (k > 0 && !qubits)) return fail(HIPMPS_E_ARG, "bad arguments");
+  if (k > 16) return fail(HIPMPS_E_UNSUPPORTED, "at most 16 measured qubits");
+  for (int i = 0; i < k; ++i)
+    if (qubits[i] < 0 || qubits[i] >= s->n) return fail(HIPMPS_E_ARG, "measured qubit out of range");
+  RC_TRY(state_flush(s));
+  return measure_outcomes(s, qubits, k, out);
 }
 
 int hipmps_sample_sequential(hipmps_state s, const int* qubits, int k, int shots, const double* draws, char* out) {

@@ -127,6 +127,21 @@ inline bool gate_small(int r, int c) {
 // lo: every task fits SMALL_CAP_LO
 hipError_t launch_gate_small(const GateTask* d_tasks, int ntasks, int fp32, bool lo, hipStream_t s);
 
+// <psi| (x)_k diag(d[2k], d[2k+1]) |psi> of one state of small bonds for many diagonals at once
+// (k_env_chain, small.hip): one workgroup per diagonal, its whole left environment chain.
+struct ChainSite {
+  const void* A;  // cl x 2 x kap x cr
+  int cl, cr, kap, pad;
+};
+constexpr int CHAIN_MAX_BOND = 32;
+// the s of a site that a step of the chain takes side by side
+__host__ __device__ inline int chain_slots(int cl, int cr) {
+  const int w = cl > cr ? cl * cr : cr * cr;
+  return w > 128 ? 1 : (256 / w < 16 ? 256 / w : 16);
+}
+hipError_t launch_env_chain(const ChainSite* d_sites, int n, const double* d_diags, double* d_out, int nchains,
+                            int fp32, hipStream_t s);
+
 // Generic batched complex GEMM: C (M x N) = rowscale . op(A) op(B) . colscale
 // op codes: 0 N, 1 C (conjugate), 2 H (conjugate transpose), 3 T (transpose).
 struct GemmTask {

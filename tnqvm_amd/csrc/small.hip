@@ -284,4 +284,100 @@ hipError_t launch_gate_small(const GateTask* d_tasks, int ntasks, int fp32, bool
   return hipGetLastError();
 }
 
+// ------------------------------------------------------------------ environment chain of small bonds
+// E <- sum_s d_s A_s^H (E A_s) over the sites, s = (p, kap), E and A_s in LDS.  A chain of products launched
+// one by one costs two launches a site, 8 to 20 us, for a few us of work on few workgroups; here a site is
+// a few steps of three barriers, and every diagonal of a measurement -- one per <Z_i>, per pair, per outcome
+// string -- is a workgroup of the same launch.  A step takes as many s side by side as fit the workgroup's
+// threads (chain_slots); the next A_s are read while these are used.
+template <typename S>
+__global__ __launch_bounds__(256) void k_env_chain(const ChainSite* sites, int n, const double* diags, double* out) {
+  constexpr int B = CHAIN_MAX_BOND, Q = B * B / 256;
+  __shared__ double2 sE[B * (B + 1)], sA[B * (B + 1)], sX[B * (B + 1)];
+  const int tid = threadIdx.x;
+  const double* diag = diags + (size_t)blockIdx.x * 2 * n;
+  if (tid == 0) sE[0] = make_double2(1.0, 0.0);
+  for (int k = 0; k < n; ++k) {
+    const ChainSite site = sites[k];
+    const int cl = site.cl, cr = site.cr, kap = site.kap, na = cl * cr, ne = cr * cr;
+    const S* A = (const S*)site.A;
+    const double dg[2] = {diag[2 * k], diag[2 * k + 1]};
+    const int slots = chain_slots(cl, cr), w = max(na, ne);
+    const int slot = slots > 1 ? tid / w : 0;
+    const int i0 = tid - slot * w;  // first element of this thread
+    const bool on = slot < slots;
+    const double2* eA = sA + slot * na;
+    double2* eX = sX + slot * na;
+    int al[Q], ar[Q];  // this thread's elements (l, r) of A_s and X, and (i, j) of the result
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+      al[q] = (i0 + 256 * q) / cr;
+      ar[q] = (i0 + 256 * q) - al[q] * cr;
+    }
+    auto has = [&](int q, int count) { return on && (q == 0 || slots == 1) && i0 + 256 * q < count; };
+    double2 acc[Q], next[Q];
+#pragma unroll
+    for (int q = 0; q < Q; ++q) acc[q] = make_double2(0, 0);
+    // the s with a nonzero diagonal: [s0, s1)
+    const int s0 = dg[0] != 0.0 ? 0 : kap, s1 = dg[1] != 0.0 ? 2 * kap : kap;
+    auto fetch = [&](int s) __attribute__((always_inline)) {
+#pragma unroll
+      for (int q = 0; q < Q; ++q) {
+        next[q] = make_double2(0, 0);
+        if (has(q, na) && s < s1) next[q] = ld(A, ((size_t)al[q] * 2 * kap + s) * cr + ar[q]);
+      }
+    };
+    if (s0 < s1) fetch(s0 + slot);
+    for (int sb = s0; sb < s1; sb += slots) {
+      const int s = sb + slot;
+#pragma unroll
+      for (int q = 0; q < Q; ++q)
+        if (has(q, na)) sA[slot * na + i0 + 256 * q] = next[q];
+      __syncthreads();
+      if (sb + slots < s1) fetch(s + slots);
+#pragma unroll
+      for (int q = 0; q < Q; ++q)
+        if (has(q, na)) {
+          double2 x = make_double2(0, 0);
+          for (int l = 0; l < cl; ++l) x = cfma(sE[al[q] * cl + l], eA[l * cr + ar[q]], x);
+          eX[i0 + 256 * q] = x;
+        }
+      __syncthreads();
+      const double d = s < kap ? dg[0] : dg[1];
+#pragma unroll
+      for (int q = 0; q < Q; ++q)
+        if (has(q, ne)) {
+          double2 x = make_double2(0, 0);
+          for (int l = 0; l < cl; ++l) x = cfmac(eA[l * cr + al[q]], eX[l * cr + ar[q]], x);
+          acc[q] = make_double2(fma(d, x.x, acc[q].x), fma(d, x.y, acc[q].y));
+        }
+      __syncthreads();
+    }
+    __syncthreads();
+    if (slots > 1) {  // the slots' sums, in order
+      if (has(0, ne)) sX[slot * ne + i0] = acc[0];
+      __syncthreads();
+      if (tid < ne) {
+        double2 t = make_double2(0, 0);
+        for (int q = 0; q < slots; ++q) t = cadd(t, sX[q * ne + tid]);
+        sE[tid] = t;
+      }
+    } else {
+#pragma unroll
+      for (int q = 0; q < Q; ++q)
+        if (has(q, ne)) sE[i0 + 256 * q] = acc[q];
+    }
+    __syncthreads();
+  }
+  if (tid == 0) out[blockIdx.x] = sE[0].x;
+}
+
+hipError_t launch_env_chain(const ChainSite* d_sites, int n, const double* d_diags, double* d_out, int nchains,
+                            int fp32, hipStream_t s) {
+  if (nchains <= 0) return hipSuccess;
+  if (fp32) hipLaunchKernelGGL(k_env_chain<float2>, dim3(nchains), dim3(256), 0, s, d_sites, n, d_diags, d_out);
+  else hipLaunchKernelGGL(k_env_chain<double2>, dim3(nchains), dim3(256), 0, s, d_sites, n, d_diags, d_out);
+  return hipGetLastError();
+}
+
 }  // namespace hipmps

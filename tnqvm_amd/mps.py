@@ -380,13 +380,10 @@ class MpsState:
         k = len(qubits)
         if k > 16:
             raise ValueError("at most 16 measured qubits")
+        q = np.asarray(qubits, dtype=np.int32).reshape(-1)
+        q = np.ascontiguousarray(np.where(q < 0, q + self.n, q), dtype=np.int32)
         out = np.zeros(1 << k)
-        for x in range(1 << k):
-            d = np.ones(2 * self.n)
-            for i, q in enumerate(qubits):
-                b = (x >> i) & 1
-                d[2 * q + (1 - b)] = 0.0
-            out[x] = self.expval_diag(d)
+        check(lib().hipmps_outcome_probabilities(self.h, q.ctypes.data_as(_ip), k, out.ctypes.data_as(_dp)))
         return out
 
     def reduced_density_matrix(self, qubits) -> np.ndarray:
