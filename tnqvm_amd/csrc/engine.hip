@@ -1344,31 +1344,54 @@ int state_flush(hipmps_state_s* s) {
 // and one readback of the new extents.  A 1-qubit gate pending on the site when its channel
 // is queued is folded into the operators (K_o P); a gate on a site with a queued channel opens
 // the next wave.
+// Channels whose rows fit k_kraus_small run there, one workgroup each, beside the others.
 constexpr double KRAUS_EPS = 1e-9;
+static_assert(MAX_KRAUS_OPS == HIPMPS_MAX_KRAUS_OPS, "operators of a channel");
+
+// adj: more rows (kap n_ops) than columns (2 cl cr); the Jacobi then runs on the rows of X^H (jr = c rows),
+// a sweep of few rounds instead of many, in the general path on [X^H | I] (ld = rows + c)
+struct KrausItem {
+  hipmps_state_s* s;
+  const hipmps_state_s::QK* k;
+  int q, cl, cr, kap, n_ops, rows, r_pad, jr, jc, ld, max_bond;
+  bool adj;
+  size_t c, off_x, off_v, off_k;
+  int K;          // kept
+  double w[WS_N];
+};
+
+int run_kraus_general(hipmps_engine E, std::vector<KrausItem*>& ch);
+
+// the new sites of the channels of run_kraus_general
+int write_kraus_general(hipmps_engine E, const std::vector<KrausItem*>& ch) {
+  char* ws = (char*)E->ws.p;
+  const int* d_K = (const int*)E->small.p + 2 * ch.size();
+  for (size_t i = 0; i < ch.size(); ++i) {
+    const KrausItem& h = *ch[i];
+    const int* perm = (const int*)(ws + h.off_v + 40 * (size_t)h.r_pad);
+    if (h.adj)
+      HIP_TRY(launch_kraus_gather_adj((double2*)(ws + h.off_x), h.ld, h.rows, (const double*)(ws + h.off_v), perm,
+                                      d_K + i, h.K, h.s->sites[h.q].p, h.s->fp32, h.cl, h.cr, E->stream));
+    else
+      HIP_TRY(launch_kraus_gather((double2*)(ws + h.off_x), h.ld, perm, d_K + i, h.K, h.s->sites[h.q].p, h.s->fp32,
+                                  h.cl, h.cr, E->stream));
+  }
+  return 0;
+}
 
 int run_kraus_waves(hipmps_engine E, const std::vector<hipmps_state_s*>& states) {
-  std::vector<std::pair<hipmps_state_s*, const hipmps_state_s::QK*>> list;
-  for (auto* st_ : states)
-    for (const auto& k : st_->cwave) list.push_back({st_, &k});
-  if (list.empty()) return 0;
   const hipStream_t st = E->stream;
-  const int C = (int)list.size();
-  // adj: more rows (kap n_ops) than columns (2 cl cr); the Jacobi then runs on the rows of
-  // [X^H | I] (jr = c rows, ld = rows + c), a sweep of few rounds instead of many
-  struct Ch {
-    hipmps_state_s* s;
-    const hipmps_state_s::QK* k;
-    int q, cl, cr, kap, n_ops, rows, r_pad, jr, jc, ld;
-    bool adj;
-    size_t c, off_x, off_v, off_k;
-  };
-  std::vector<Ch> ch(C);
-  size_t off = 0, kbytes = 0;
-  int max_rows = 1;
-  for (int i = 0; i < C; ++i) {
-    Ch& h = ch[i];
-    h.s = list[i].first;
-    h.k = list[i].second;
+  std::vector<KrausItem> ch;
+  for (auto* st_ : states)
+    for (const auto& k : st_->cwave) {
+      ch.push_back({});
+      ch.back().s = st_;
+      ch.back().k = &k;
+    }
+  if (ch.empty()) return 0;
+  std::vector<KrausItem*> small[4], general;  // small: by launch variant (precision, LDS size)
+  size_t off = 0, ns = 0;
+  for (auto& h : ch) {
     h.q = h.k->q;
     h.n_ops = h.k->n_ops;
     h.cl = h.s->chi[h.q];
@@ -1377,21 +1400,129 @@ int run_kraus_waves(hipmps_engine E, const std::vector<hipmps_state_s*>& states)
     h.rows = h.kap * h.n_ops;
     if (h.rows > 4096) return fail(HIPMPS_E_UNSUPPORTED, "Kraus leg above 4096 rows");
     h.c = (size_t)2 * h.cl * h.cr;
+    h.max_bond = (int)std::min<size_t>(h.c, (size_t)2 * h.kap);
     h.adj = (size_t)h.rows > h.c;
     h.jr = h.adj ? (int)h.c : h.rows;
     h.jc = h.adj ? h.rows : (int)h.c;
     h.ld = h.adj ? h.rows + (int)h.c : (int)h.c;
     h.r_pad = (h.jr + JP - 1) / JP * JP;
     h.off_x = off;
+    if (gate_small(h.jr, h.jc)) {
+      off = align_up(off + h.c * std::min(h.jr, h.max_bond) * h.s->es);
+      small[2 * h.s->fp32 + (small_rows(h.jr) * small_stride(h.jc) > SMALL_CAP_LO)].push_back(&h);
+      ++ns;
+      continue;
+    }
     off = align_up(off + (size_t)h.r_pad * h.ld * 16);
     h.off_v = off;
     off = align_up(off + (size_t)h.r_pad * (8 * 5 + 4));
     h.off_k = off;
     off = align_up(off + (size_t)h.n_ops * 4 * 16);
-    kbytes += (size_t)h.n_ops * 4 * sizeof(double2);
-    max_rows = std::max(max_rows, h.jr);
+    general.push_back(&h);
   }
   RC_TRY(E->ws.ensure(off));
+  char* ws = (char*)E->ws.p;
+  // descriptors and results, read and written by the device in place
+  RC_TRY(E->hgate.ensure(ns * (sizeof(KrausTask) + sizeof(CopyTask) + sizeof(GateResult))));
+  KrausTask* ht = (KrausTask*)E->hgate.p;
+  CopyTask* hc = (CopyTask*)(ht + ns);
+  const GateResult* hr = (const GateResult*)(hc + ns);
+  KrausTask* dt = nullptr;
+  if (ns) {
+    HIP_TRY(hipHostGetDevicePointer((void**)&dt, E->hgate.p, 0));
+    GateResult* dr = (GateResult*)((CopyTask*)(dt + ns) + ns);
+    size_t i = 0;
+    for (auto& v : small)
+      for (auto* h : v) {
+        KrausTask& T = ht[i];
+        T.site = h->s->sites[h->q].p;
+        T.out = ws + h->off_x;
+        T.res = dr + i;
+        T.cl = h->cl;
+        T.cr = h->cr;
+        T.kap = h->kap;
+        T.n_ops = h->n_ops;
+        T.adj = h->adj;
+        T.r = h->jr;
+        T.c = h->jc;
+        T.max_bond = h->max_bond;
+        T.pn_l2 = h->s->t.partial_norm == HIPMPS_PN_L2;
+        T.max_sweeps = E->max_sweeps;
+        T.cutoff = KRAUS_EPS;
+        T.tol = h->s->fp32 ? E->tol_mixed : E->tol;
+        for (int t = 0; t < 4 * h->n_ops; ++t) T.K[t] = make_double2(h->k->K[t].real(), h->k->K[t].imag());
+        ++i;
+      }
+    const KrausTask* d = dt;
+    for (int v = 0; v < 4; ++v) {
+      HIP_TRY(launch_kraus_small(d, (int)small[v].size(), v >> 1, (v & 1) == 0, st));
+      d += small[v].size();
+    }
+  }
+  const int rc = general.empty() ? 0 : run_kraus_general(E, general);
+  HIP_TRY(hipStreamSynchronize(st));
+  RC_TRY(rc);
+  {
+    size_t i = 0;
+    for (auto& v : small)
+      for (auto* h : v) {
+        const GateResult& R = hr[i++];
+        h->K = R.K;
+        memcpy(h->w, R.w, sizeof(h->w));
+        if (!R.converged) {
+          if (h->s->status == 0) h->s->status = HIPMPS_E_CONVERGENCE;
+          h->s->nonconverged++;
+        }
+      }
+  }
+  // new Kraus extents: every site that must grow is reserved before any is written (all or
+  // nothing, as in run_wave), so a failure leaves every state and its queued channels as they were
+  {
+    std::vector<SiteGrowth> grow;
+    for (auto& h : ch) {
+      if (h.K < 1 || h.K > h.jr) return fail(HIPMPS_E_NUMERIC, "Kraus compression returned no rows");
+      const size_t need = h.c * h.K;
+      const Site& S = h.s->sites[h.q];
+      if (need > S.cap) grow.push_back({h.s, h.q, std::max(need, S.cap * 2), nullptr});
+    }
+    if (!grow.empty()) RC_TRY(grow_sites(E, grow));
+  }
+  if (ns) {
+    size_t i = 0;
+    for (auto& v : small)
+      for (auto* h : v) {
+        hc[i].src = ws + h->off_x;
+        hc[i].dst = h->s->sites[h->q].p;
+        hc[i].units = h->c * h->K * (h->s->es / 8);
+        ++i;
+      }
+    HIP_TRY(launch_copy_sites((const CopyTask*)(dt + ns), (int)ns, st));
+  }
+  RC_TRY(write_kraus_general(E, general));
+  for (auto& h : ch) {
+    if (h.w[5] != 0.0 || !std::isfinite(h.w[0] + h.w[1])) h.s->status = HIPMPS_E_NUMERIC;
+    h.s->kap[h.q] = h.K;
+    h.s->kraus_ops++;
+  }
+  HIP_TRY(hipStreamSynchronize(st));
+  for (auto* st_ : states) {
+    st_->cwave.clear();
+    std::fill(st_->cbusy.begin(), st_->cbusy.end(), 0);
+    release_deferred(st_);
+  }
+  return 0;
+}
+
+// the channels that do not fit k_kraus_small: Jacobi sweeps and selection as batched launches
+int run_kraus_general(hipmps_engine E, std::vector<KrausItem*>& ch) {
+  const hipStream_t st = E->stream;
+  const int C = (int)ch.size();
+  size_t kbytes = 0;
+  int max_rows = 1;
+  for (const auto* h : ch) {
+    kbytes += (size_t)h->n_ops * 4 * sizeof(double2);
+    max_rows = std::max(max_rows, h->jr);
+  }
   char* ws = (char*)E->ws.p;
   const size_t cnt_bytes = align_up((size_t)3 * C * sizeof(int));
   RC_TRY(E->small.ensure(cnt_bytes + (size_t)C * WS_N * sizeof(double)));
@@ -1414,7 +1545,7 @@ int run_kraus_waves(hipmps_engine E, const std::vector<hipmps_state_s*>& states)
   memset(hs, 0, desc_bytes);
   size_t ko = 0;
   for (int i = 0; i < C; ++i) {
-    const Ch& h = ch[i];
+    const KrausItem& h = *ch[i];
     hipmps_state_s* s = h.s;
     for (int t = 0; t < 4 * h.n_ops; ++t) hk[ko + t] = make_double2(h.k->K[t].real(), h.k->K[t].imag());
     char* v = ws + h.off_v;
@@ -1435,7 +1566,7 @@ int run_kraus_waves(hipmps_engine E, const std::vector<hipmps_state_s*>& states)
     S.K = d_K + i;
     S.wstats = d_w + (size_t)i * WS_N;
     S.cutoff = KRAUS_EPS;
-    S.max_bond = (int)std::min<size_t>(h.c, (size_t)2 * h.kap);
+    S.max_bond = h.max_bond;
     S.pn_l2 = s->t.partial_norm == HIPMPS_PN_L2;
     S.site_fp32 = s->fp32;
     S.keep_rule = 1;
@@ -1463,7 +1594,7 @@ int run_kraus_waves(hipmps_engine E, const std::vector<hipmps_state_s*>& states)
   HIP_TRY(hipMemcpyAsync(dd, hd, sp_bytes, hipMemcpyHostToDevice, st));
   ko = 0;
   for (int i = 0; i < C; ++i) {
-    const Ch& h = ch[i];
+    const KrausItem& h = *ch[i];
     hipmps_state_s* s = h.s;
     HIP_TRY(hipMemcpyAsync(ws + h.off_k, hk + ko, (size_t)h.n_ops * 4 * sizeof(double2), hipMemcpyHostToDevice, st));
     if (h.adj)
@@ -1497,49 +1628,17 @@ int run_kraus_waves(hipmps_engine E, const std::vector<hipmps_state_s*>& states)
     active.swap(next);
   }
   for (int i : active) {
-    if (ch[i].s->status == 0) ch[i].s->status = HIPMPS_E_CONVERGENCE;
-    ch[i].s->nonconverged++;
+    if (ch[i]->s->status == 0) ch[i]->s->status = HIPMPS_E_CONVERGENCE;
+    ch[i]->s->nonconverged++;
   }
   HIP_TRY(launch_rownorm(dsp, C, max_rows, st));
   HIP_TRY(launch_select(dsp, C, st));
   HIP_TRY(hipMemcpyAsync(hcount + 2 * C, d_K, (size_t)C * sizeof(int), hipMemcpyDeviceToHost, st));
   HIP_TRY(hipMemcpyAsync(hw, d_w, (size_t)C * WS_N * sizeof(double), hipMemcpyDeviceToHost, st));
   HIP_TRY(hipStreamSynchronize(st));
-  // new Kraus extents: every site that must grow is reserved before any is written (all or
-  // nothing, as in run_wave), so a failure leaves every state and its queued channels as they were
-  {
-    std::vector<SiteGrowth> grow;
-    for (int i = 0; i < C; ++i) {
-      const Ch& h = ch[i];
-      const int Kn = hcount[2 * C + i];
-      if (Kn < 1 || Kn > h.jr) return fail(HIPMPS_E_NUMERIC, "Kraus compression returned no rows");
-      const size_t need = (size_t)h.cl * 2 * Kn * h.cr;
-      const Site& S = h.s->sites[h.q];
-      if (need > S.cap) grow.push_back({h.s, h.q, std::max(need, S.cap * 2), nullptr});
-    }
-    if (!grow.empty()) RC_TRY(grow_sites(E, grow));
-  }
   for (int i = 0; i < C; ++i) {
-    const Ch& h = ch[i];
-    hipmps_state_s* s = h.s;
-    const int Kn = hcount[2 * C + i];
-    const double* w = hw + (size_t)i * WS_N;
-    if (w[5] != 0.0 || !std::isfinite(w[0] + w[1])) s->status = HIPMPS_E_NUMERIC;
-    const int* perm = (const int*)(ws + h.off_v + 40 * (size_t)h.r_pad);
-    if (h.adj)
-      HIP_TRY(launch_kraus_gather_adj((double2*)(ws + h.off_x), h.ld, h.rows, (const double*)(ws + h.off_v), perm,
-                                      d_K + i, Kn, s->sites[h.q].p, s->fp32, h.cl, h.cr, st));
-    else
-      HIP_TRY(launch_kraus_gather((double2*)(ws + h.off_x), h.ld, perm, d_K + i, Kn, s->sites[h.q].p, s->fp32,
-                                  h.cl, h.cr, st));
-    s->kap[h.q] = Kn;
-    s->kraus_ops++;
-  }
-  HIP_TRY(hipStreamSynchronize(st));
-  for (auto* st_ : states) {
-    st_->cwave.clear();
-    std::fill(st_->cbusy.begin(), st_->cbusy.end(), 0);
-    release_deferred(st_);
+    ch[i]->K = hcount[2 * C + i];
+    memcpy(ch[i]->w, hw + (size_t)i * WS_N, sizeof(ch[i]->w));
   }
   return 0;
 }

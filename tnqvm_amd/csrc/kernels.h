@@ -125,6 +125,25 @@ inline bool gate_small(int r, int c) {
   return r <= SMALL_MAX_ROWS && c <= 128 && small_rows(r) * small_stride(c) <= SMALL_CAP;
 }
 // lo: every task fits SMALL_CAP_LO
+// A noise channel of a small site (k_kraus_small): the same limits on its rows and columns.
+constexpr int MAX_KRAUS_OPS = 16;
+struct KrausTask {
+  const void* site;  // cl x 2 x kap x cr
+  void* out;         // cl x 2 x K x cr
+  GateResult* res;
+  int cl, cr, kap, n_ops;
+  int adj, r, c;     // X^H instead of X (kap n_ops rows, 2 cl cr columns); its rows and columns
+  int max_bond, pn_l2, max_sweeps;
+  double cutoff, tol;
+  double2 K[4 * MAX_KRAUS_OPS];
+};
+hipError_t launch_kraus_small(const KrausTask* d_tasks, int ntasks, int fp32, bool lo, hipStream_t s);
+struct CopyTask {
+  const void* src;
+  void* dst;
+  size_t units;  // of 8 bytes
+};
+hipError_t launch_copy_sites(const CopyTask* d_tasks, int ntasks, hipStream_t s);
 hipError_t launch_gate_small(const GateTask* d_tasks, int ntasks, int fp32, bool lo, hipStream_t s);
 
 // <psi| (x)_k diag(d[2k], d[2k+1]) |psi> of one state of small bonds for many diagonals at once

@@ -14,6 +14,7 @@
 // products, four DPP sums, the rotation, LDS write, barrier), and at 64 rows by FP64 issue of the one CU.
 // Measured, a wave: 13 us at bonds up to 4, 60 to 80 us up to 16, 320 to 465 us up to 32.
 #include <cfloat>
+#include <cstddef>
 
 #include "kernels.h"
 #include "device_util.h"
@@ -95,6 +96,64 @@ __device__ __forceinline__ int jacobi_rows_n(double2* Y, int stride, int nr, dou
   }
 }
 
+// Norms of the rows of Y, sorted descending, ties by row: sig[rank], perm[rank].  NaN / Inf sorted as 0 and
+// flagged.  tmp, sig, perm: LDS, SMALL_MAX_ROWS entries.
+template <int NT>
+__device__ __forceinline__ void sort_rows(const double2* Y, int stride, int r, int c, double* tmp, double* sig,
+                                          int* perm, int* bad) {
+  const int tid = threadIdx.x, group = tid >> 4, l16 = tid & 15;
+  for (int i = group; i < r; i += NT / 16) {
+    double a = 0.0;
+    for (int j = l16; j < c; j += 16) a += cabs2(Y[i * stride + j]);
+    a = sqrt(row16_sum(a));
+    if (l16 == 0) {
+      if (!(a >= 0.0 && a <= DBL_MAX)) {
+        a = 0.0;
+        *bad = 1;
+      }
+      tmp[i] = a;
+    }
+  }
+  __syncthreads();
+  if (tid < r) {
+    const double a = tmp[tid];
+    int rank = 0;
+    for (int j = 0; j < r; ++j) {
+      const double b = tmp[j];
+      rank += b > a || (b == a && j < tid);
+    }
+    sig[rank] = a;
+    perm[rank] = tid;
+  }
+  __syncthreads();
+}
+
+// One vector of X's other side per 16 lanes: u[i] = <y, X row i> * scale for the rows i = l16 + 16 q < r;
+// returns the sum of |u|^2 over all rows.  The lanes start at different columns: rows are a multiple of 256
+// bytes apart, the same column of 16 rows is one LDS bank (measured 27 of 320 us at 64 rows).
+__device__ __forceinline__ double other_side(const double2* X, const double2* y, int stride, int r, int c,
+                                             double scale, double2 (&u)[SMALL_MAX_ROWS / 16]) {
+  const int l16 = threadIdx.x & 15;
+  double t = 0.0;
+#pragma unroll
+  for (int q = 0; q < SMALL_MAX_ROWS / 16; ++q) {
+    u[q] = make_double2(0, 0);
+    const int i = l16 + 16 * q;
+    if (i < r) {
+      const double2* x = X + i * stride;
+      double2 d = make_double2(0, 0);
+      int j = l16 % c;
+      for (int e = 0; e < c; ++e) {
+        d = cfmac(y[j], x[j], d);
+        j = j + 1 == c ? 0 : j + 1;
+      }
+      u[q] = cscale(d, scale);
+      t += cabs2(u[q]);
+    }
+  }
+  return row16_sum(t);
+}
+
 template <typename S, int NT, int CAP>
 __global__ __launch_bounds__(NT) void k_gate_small(const GateTask* tasks) {
   __shared__ GateTask T;
@@ -158,31 +217,7 @@ __global__ __launch_bounds__(NT) void k_gate_small(const GateTask* tasks) {
   __syncthreads();
   const int sweeps = jacobi_rows_n<NT>(sY, stride, nr, T.tol, JAC_FLOOR2 * f2, T.max_sweeps, &s_flag);
   __syncthreads();
-  // ---- singular values (row norms), sorted descending, ties by row; NaN / Inf sorted as 0 and flagged ----
-  for (int i = group; i < r; i += NT / 16) {
-    double a = 0.0;
-    for (int j = l16; j < T.c; j += 16) a += cabs2(sY[i * stride + j]);
-    a = sqrt(row16_sum(a));
-    if (l16 == 0) {
-      if (!(a >= 0.0 && a <= DBL_MAX)) {
-        a = 0.0;
-        s_bad = 1;
-      }
-      s_inv[i] = a;
-    }
-  }
-  __syncthreads();
-  if (tid < r) {
-    const double a = s_inv[tid];
-    int rank = 0;
-    for (int j = 0; j < r; ++j) {
-      const double b = s_inv[j];
-      rank += b > a || (b == a && j < tid);
-    }
-    s_sig[rank] = a;
-    s_perm[rank] = tid;
-  }
-  __syncthreads();
+  sort_rows<NT>(sY, stride, r, T.c, s_inv, s_sig, s_perm, &s_bad);
   // ---- truncation rule and factor scales, as k_select ----
   if (wave == 0) {
     const double sg = lane < r ? s_sig[lane] : 0.0;
@@ -244,23 +279,8 @@ __global__ __launch_bounds__(NT) void k_gate_small(const GateTask* tasks) {
   }
   // ---- the other factor: X's rows on the kept rows of Y, each vector scaled to its length ----
   for (int k = group; k < K; k += NT / 16) {
-    const double2* y = sY + s_perm[k] * stride;
-    const double is = s_inv[k];
     double2 u[SMALL_MAX_ROWS / 16];
-    double t = 0.0;
-#pragma unroll
-    for (int q = 0; q < SMALL_MAX_ROWS / 16; ++q) {
-      u[q] = make_double2(0, 0);
-      const int i = l16 + 16 * q;
-      if (i < r) {
-        const double2* x = sX + i * stride;
-        double2 d = make_double2(0, 0);
-        for (int c = 0; c < T.c; ++c) d = cfmac(y[c], x[c], d);
-        u[q] = cscale(d, is);
-        t += cabs2(u[q]);
-      }
-    }
-    t = row16_sum(t);
+    const double t = other_side(sX, sY + s_perm[k] * stride, stride, r, T.c, s_inv[k], u);
     const double f = t > 0.0 ? s_scw[k] / sqrt(t) : 0.0;
 #pragma unroll
     for (int q = 0; q < SMALL_MAX_ROWS / 16; ++q) {
@@ -281,6 +301,125 @@ hipError_t launch_gate_small(const GateTask* d_tasks, int ntasks, int fp32, bool
     if (lo) hipLaunchKernelGGL((k_gate_small<double2, 256, SMALL_CAP_LO>), dim3(ntasks), dim3(256), 0, s, d_tasks);
     else hipLaunchKernelGGL((k_gate_small<double2, 512, SMALL_CAP>), dim3(ntasks), dim3(512), 0, s, d_tasks);
   }
+  return hipGetLastError();
+}
+
+// ------------------------------------------------------------------ noise channels of small sites
+// A whole channel in one workgroup: the rows of X (one per old Kraus index and operator, columns (l, p, r))
+// or of X^H when X has more rows than columns, their Jacobi sweeps, the kept rows, and the new site in its
+// final layout, K of its Kraus index known here, in T.out.  The general path (kraus.hip) takes a copy, an
+// expansion, a launch per Jacobi round, a synchronisation per sweep and a gather per channel; at these sizes
+// each of them is a launch for a few us of work.  From X^H: W X^H = Y with orthogonal rows of length sigma_j
+// makes Sigma W a square root of X^H X like X itself, and its row j is (Y_j X) / sigma_j, scaled to length
+// sigma_j; no identity is carried through the rotations.
+template <typename S, int NT, int CAP>
+__global__ __launch_bounds__(NT) void k_kraus_small(const KrausTask* tasks) {
+  __shared__ KrausTask T;
+  __shared__ double2 sX[CAP], sY[CAP];
+  __shared__ double s_sig[SMALL_MAX_ROWS], s_tmp[SMALL_MAX_ROWS];
+  __shared__ int s_perm[SMALL_MAX_ROWS];
+  __shared__ int s_flag, s_K, s_bad;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, group = tid >> 4, l16 = tid & 15;
+  {
+    const KrausTask* t = tasks + blockIdx.x;
+    const int words = (int)(offsetof(KrausTask, K) / 4) + 16 * t->n_ops;
+    for (int e = tid; e < words; e += NT) ((int*)&T)[e] = ((const int*)t)[e];
+  }
+  if (tid == 0) {
+    s_flag = 0;
+    s_bad = 0;
+  }
+  __syncthreads();
+  const int cr = T.cr, kap = T.kap, n_ops = T.n_ops, adj = T.adj, r = T.r, c = T.c;
+  const int nr = small_rows(r), stride = small_stride(c);
+  for (int e = tid; e < nr * stride; e += NT) sX[e] = sY[e] = make_double2(0, 0);
+  __syncthreads();
+  {  // one thread per (l, k, r): its 2 n_ops elements of X
+    const S* A = (const S*)T.site;
+    for (int e = tid; e < T.cl * kap * cr; e += NT) {
+      const int rr = e % cr, lk = e / cr, l = lk / kap, k = lk - l * kap;
+      const double2 a0 = ld(A, ((size_t)(2 * l) * kap + k) * cr + rr);
+      const double2 a1 = ld(A, ((size_t)(2 * l + 1) * kap + k) * cr + rr);
+      for (int op = 0; op < 2 * n_ops; ++op) {  // (operator, new physical index)
+        const int row = k * n_ops + (op >> 1), col = (2 * l + (op & 1)) * cr + rr;
+        const double2 v = cadd(cmul(T.K[2 * op], a0), cmul(T.K[2 * op + 1], a1));
+        const int at = adj ? col * stride + row : row * stride + col;
+        sX[at] = sY[at] = adj ? cconj(v) : v;
+      }
+    }
+  }
+  __syncthreads();
+  const int sweeps = jacobi_rows_n<NT>(sY, stride, nr, T.tol, 0.0, T.max_sweeps, &s_flag);
+  __syncthreads();
+  sort_rows<NT>(sY, stride, r, c, s_tmp, s_sig, s_perm, &s_bad);
+  if (wave == 0) {  // kept rows, as k_select's keep_rule
+    const double sg = lane < r ? s_sig[lane] : 0.0;
+    const double pn = T.pn_l2 ? sg : sg * sg;
+    const unsigned long long below = __ballot(lane < r && pn < T.cutoff);
+    const int K = max(1, min(below ? (int)__ffsll(below) - 1 : r, T.max_bond));
+    const double kept = wave_sum(lane < K ? sg * sg : 0.0), disc = wave_sum(lane >= K ? sg * sg : 0.0);
+    if (lane == 0) {
+      s_K = K;
+      GateResult R;
+      R.K = K;
+      R.sweeps = sweeps;
+      R.converged = s_flag == 0;
+      R.pad = 0;
+      R.w[0] = disc;
+      R.w[1] = kept;
+      R.w[2] = kept + disc;
+      R.w[3] = 1.0;
+      R.w[4] = 0.0;
+      R.w[5] = s_bad ? 1.0 : 0.0;
+      *T.res = R;
+    }
+  }
+  __syncthreads();
+  const int K = s_K;
+  S* out = (S*)T.out;
+  if (!adj) {
+    for (int e = tid; e < K * c; e += NT) {  // e = (lp, j, r)
+      const int rr = e % cr, lpj = e / cr, lp = lpj / K, j = lpj - lp * K;
+      st(out, (size_t)e, sY[s_perm[j] * stride + lp * cr + rr]);
+    }
+    return;
+  }
+  for (int j = group; j < K; j += NT / 16) {
+    const double sg = s_sig[j];
+    double2 u[SMALL_MAX_ROWS / 16];
+    const double t = other_side(sX, sY + s_perm[j] * stride, stride, r, c, sg > 1e-150 ? 1.0 / sg : 0.0, u);
+    const double f = t > 0.0 ? sg / sqrt(t) : 0.0;
+#pragma unroll
+    for (int q = 0; q < SMALL_MAX_ROWS / 16; ++q) {
+      const int i = l16 + 16 * q;
+      if (i < r) st(out, ((size_t)(i / cr) * K + j) * cr + i % cr, cscale(cconj(u[q]), f));
+    }
+  }
+}
+
+hipError_t launch_kraus_small(const KrausTask* d_tasks, int ntasks, int fp32, bool lo, hipStream_t s) {
+  if (ntasks <= 0) return hipSuccess;
+  if (fp32) {
+    if (lo) hipLaunchKernelGGL((k_kraus_small<float2, 256, SMALL_CAP_LO>), dim3(ntasks), dim3(256), 0, s, d_tasks);
+    else hipLaunchKernelGGL((k_kraus_small<float2, 512, SMALL_CAP>), dim3(ntasks), dim3(512), 0, s, d_tasks);
+  } else {
+    if (lo) hipLaunchKernelGGL((k_kraus_small<double2, 256, SMALL_CAP_LO>), dim3(ntasks), dim3(256), 0, s, d_tasks);
+    else hipLaunchKernelGGL((k_kraus_small<double2, 512, SMALL_CAP>), dim3(ntasks), dim3(512), 0, s, d_tasks);
+  }
+  return hipGetLastError();
+}
+
+// The new sites of a wave of channels from scratch to their buffers, one workgroup each (units of 8 bytes).
+__global__ __launch_bounds__(256) void k_copy_sites(const CopyTask* tasks) {
+  const CopyTask T = tasks[blockIdx.x];
+  const HIPMPS_GLOBAL double* src = (const HIPMPS_GLOBAL double*)T.src;
+  HIPMPS_GLOBAL double* dst = (HIPMPS_GLOBAL double*)T.dst;
+#pragma unroll 8
+  for (size_t e = threadIdx.x; e < T.units; e += 256) dst[e] = src[e];
+}
+
+hipError_t launch_copy_sites(const CopyTask* d_tasks, int ntasks, hipStream_t s) {
+  if (ntasks > 0) hipLaunchKernelGGL(k_copy_sites, dim3(ntasks), dim3(256), 0, s, d_tasks);
   return hipGetLastError();
 }
 
