@@ -42,6 +42,7 @@
 
 #include "hipmps.h"
 #include "kernels.h"
+#include "site_pool.h"
 
 using cd = std::complex<double>;
 using namespace hipmps;
@@ -161,6 +162,16 @@ void kron2(const cd* A, const cd* B, cd* K) {  // A (x) B, A on the most signifi
 // ======================================================================================
 // engine / state
 // ======================================================================================
+struct SiteDevice {
+  static void* alloc(size_t bytes) {
+    void* p = nullptr;
+    if (hipMalloc(&p, bytes) == hipSuccess) return p;
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  static void free(void* p) { (void)hipFree(p); }
+};
+
 struct Site {
   void* p = nullptr;
   size_t cap = 0;  // elements
@@ -203,6 +214,7 @@ struct hipmps_engine_s {
   DevBuf desc;   // task descriptors
   DevBuf small;  // counters / K / stats
   DevBuf env;    // environments for measurements
+  SitePool<SiteDevice> pool;  // site buffers
   HostBuf hdesc;
   HostBuf hsmall;
   HostBuf hgate;  // descriptors and results of k_gate_small, read and written by the device in place
@@ -404,14 +416,11 @@ int ensure_site(hipmps_state_s* s, int k, size_t elems, bool keep_old_for_read, 
   hipmps_engine e = s->e;
   if (e->used + nbytes > e->budget)
     return fail(HIPMPS_E_NOMEM, "HBM budget exceeded growing site " + std::to_string(k));
-  void* p = nullptr;
-  if (hipMalloc(&p, nbytes) != hipSuccess) {
-    (void)hipGetLastError();
-    return fail(HIPMPS_E_NOMEM, "device allocation for site " + std::to_string(k) + " failed");
-  }
+  void* p = e->pool.get(nbytes);
+  if (!p) return fail(HIPMPS_E_NOMEM, "device allocation for site " + std::to_string(k) + " failed");
   if (S.p) {
     if (keep_old_for_read) s->deferred.push_back(S.p);
-    else (void)hipFree(S.p);
+    else e->pool.put(S.p);
     e->used -= S.cap * s->es;
     s->bytes -= S.cap * s->es;
   }
@@ -424,7 +433,7 @@ int ensure_site(hipmps_state_s* s, int k, size_t elems, bool keep_old_for_read, 
 }
 
 void release_deferred(hipmps_state_s* s) {
-  for (void* p : s->deferred) (void)hipFree(p);
+  for (void* p : s->deferred) s->e->pool.put(p);
   s->deferred.clear();
 }
 
@@ -446,9 +455,9 @@ int grow_sites(hipmps_engine E, std::vector<SiteGrowth>& g) {
     return fail(HIPMPS_E_NOMEM, "HBM budget exceeded growing " + std::to_string(g.size()) + " site(s) by " +
                                     std::to_string(add) + " bytes");
   for (size_t a = 0; a < g.size(); ++a) {
-    if (hipMalloc(&g[a].p, g[a].ncap * g[a].s->es) != hipSuccess) {
-      (void)hipGetLastError();
-      for (size_t b = 0; b < a; ++b) (void)hipFree(g[b].p);
+    g[a].p = E->pool.get(g[a].ncap * g[a].s->es);
+    if (!g[a].p) {
+      for (size_t b = 0; b < a; ++b) E->pool.put(g[b].p);
       for (auto& x : g) x.p = nullptr;
       return fail(HIPMPS_E_NOMEM, "device allocation for site " + std::to_string(g[a].k) + " failed");
     }
@@ -497,11 +506,14 @@ int state_init_product(hipmps_state_s* s) {
   // |0..0>: every site 1 x 2 x 1 with body {1, 0} (ExaTnMpsVisitor.cpp:46, :323)
   s->chi.assign(s->n + 1, 1);
   s->kap.assign(s->n, 1);
-  const cd body[2] = {1.0, 0.0};
-  for (int k = 0; k < s->n; ++k) {
-    RC_TRY(ensure_site(s, k, 2, false, nullptr));
-    RC_TRY(upload_site_host(s, k, body, 2));
-  }
+  hipmps_engine e = s->e;
+  for (int k = 0; k < s->n; ++k) RC_TRY(ensure_site(s, k, 2, false, nullptr));
+  RC_TRY(e->hgate.ensure((size_t)s->n * sizeof(void*)));
+  void* dev = nullptr;
+  HIP_TRY(hipHostGetDevicePointer(&dev, e->hgate.p, 0));
+  for (int k = 0; k < s->n; ++k) ((void**)e->hgate.p)[k] = s->sites[k].p;
+  HIP_TRY(launch_zero_state((void* const*)dev, s->n, s->fp32, e->stream));
+  HIP_TRY(hipStreamSynchronize(e->stream));
   s->pend.assign(s->n, {cd(1), cd(0), cd(0), cd(1)});
   s->has_pend.assign(s->n, 0);
   s->busy.assign(s->n, 0);
@@ -2844,6 +2856,7 @@ int hipmps_engine_destroy(hipmps_engine e) {
   e->hdesc.release();
   e->hsmall.release();
   e->hgate.release();
+  e->pool.release();
   for (auto& ev : e->ev)
     if (ev) (void)hipEventDestroy(ev);
   for (auto& ev : e->lane_ev)
@@ -2980,7 +2993,7 @@ int hipmps_state_destroy(hipmps_state s) {
   (void)hipStreamSynchronize(s->e->stream);
   release_deferred(s);
   for (auto& S : s->sites) {
-    if (S.p) (void)hipFree(S.p);
+    s->e->pool.put(S.p);
     s->e->used -= S.cap * s->es;
   }
   delete s;

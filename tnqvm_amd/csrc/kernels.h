@@ -143,6 +143,8 @@ struct CopyTask {
   void* dst;
   size_t units;  // of 8 bytes
 };
+// sites[k] <- 1 x 2 x 1 body {1, 0}, k < n
+hipError_t launch_zero_state(void* const* sites, int n, int fp32, hipStream_t s);
 hipError_t launch_copy_sites(const CopyTask* d_tasks, int ntasks, hipStream_t s);
 hipError_t launch_gate_small(const GateTask* d_tasks, int ntasks, int fp32, bool lo, hipStream_t s);
 

@@ -423,6 +423,23 @@ hipError_t launch_copy_sites(const CopyTask* d_tasks, int ntasks, hipStream_t s)
   return hipGetLastError();
 }
 
+// |0..0>: one launch for all sites instead of an upload and a synchronisation each.
+template <typename S>
+__global__ __launch_bounds__(256) void k_zero_state(void* const* sites, int n) {
+  const int k = blockIdx.x * 256 + threadIdx.x;
+  if (k >= n) return;
+  S* A = (S*)sites[k];
+  st(A, 0, make_double2(1, 0));
+  st(A, 1, make_double2(0, 0));
+}
+
+hipError_t launch_zero_state(void* const* sites, int n, int fp32, hipStream_t s) {
+  const dim3 grid((n + 255) / 256);
+  if (fp32) hipLaunchKernelGGL(k_zero_state<float2>, grid, dim3(256), 0, s, sites, n);
+  else hipLaunchKernelGGL(k_zero_state<double2>, grid, dim3(256), 0, s, sites, n);
+  return hipGetLastError();
+}
+
 // ------------------------------------------------------------------ environment chain of small bonds
 // E <- sum_s d_s A_s^H (E A_s) over the sites, s = (p, kap), E and A_s in LDS.  A chain of products launched
 // one by one costs two launches a site, 8 to 20 us, for a few us of work on few workgroups; here a site is
