@@ -16,6 +16,7 @@
 #include <algorithm>
 #include <cfloat>
 #include <cmath>
+#include <type_traits>
 
 namespace hipmps {
 
@@ -310,12 +311,13 @@ struct InnerShared {
   double2 tau[2][JB];  // rotations of the current / next step
   double c[2][JB];
   double d[2][JP];     // diagonal by slot, rotated
-  int rot[4];          // per wave: an entry of the Gram is above the tolerance
+  int rot[8];          // per wave: an entry of the Gram is above the tolerance
 };
 
 // One cyclic two-sided Jacobi sweep on the Hermitian S.G[0]; leaves W (its rotations) in S.G[0].
 // Waves 0 and 1 hold one 2x2 block each of rotation pairs k < l (the other half is its conjugate,
 // a rotated diagonal block is diag(d) with a zero off-diagonal entry), waves 2 and 3 hold W.
+// Further waves only keep the barriers.
 template <bool CROSS>
 __device__ __forceinline__ void inner_sweep(InnerShared& S, double itol, double floor2) {
   const int tid = threadIdx.x, wave = tid >> 6, l16 = tid & 15;
@@ -414,6 +416,9 @@ __device__ __forceinline__ void inner_sweep(InnerShared& S, double itol, double 
       gB = tmp;
     }
     __syncthreads();  // W is in place
+  } else if (wave >= 4) {
+#pragma unroll 1
+    for (int st = 0; st <= STEPS; ++st) __syncthreads();
   } else {
     // W rows wr .. wr + 3 at slots l16 (t) and JP-1-l16 (b)
     const int wr = 4 * ((tid - 128) >> 4);
@@ -473,13 +478,19 @@ __device__ __forceinline__ void inner_sweep(InnerShared& S, double itol, double 
 //  by LDS bandwidth: the whole G and W in LDS (20 16-byte accesses a thread and step, all four
 //  waves) took 1590 clocks a step, a half of G on two waves and W in registers 1200.
 //  Measured, 768 workgroups on 32 rows x 512 columns (three per CU): 156 us a launch before
-//  (inner sweep 93k clocks), 142 us with the full ordering, 126 us with the cross one, which is
-//  4.8 TB/s over its three passes; one workgroup alone on 32 x 32: 32 us before, 26 and 18 us.
+//  (inner sweep 93k clocks), 143 us with the full ordering, 126 us with the cross one, which is
+//  4.8 TB/s over its three passes, 115 us with the diagonal tiles' products left out of cross rounds.
+//  * A launch that leaves CUs idle is bound by one workgroup's chain.  At 32 x 256, four waves: Gram
+//    26.7k clocks (1700 a unit of 9 MFMA, 576 of them MFMA: two loads in flight do not cover the
+//    latency), inner 20.6k, apply 19.3k.  Eight waves with four loads in flight and cross rounds of
+//    three MFMA a unit: 12.5k, 20.6k, 16.6k; 35.2 -> 29.4 -> 26.8 us a launch (512 columns:
+//    54.4 -> 43.5 -> 37.3).
 // BLK is the block size JB (a template parameter: the kernel's register allocation on
 // gfx950 comes out at 168 VGPRs, three waves per SIMD, in the tiled form).
-template <int BLK, bool TILED>
-__global__ __launch_bounds__(256, 2) void k_jacobi_round(const JacTask* tasks, int ntasks, int sweep, int round) {
-  static_assert(BLK == 16 && JB == BLK && JP == 2 * BLK, "256 threads map onto 16 x 16 rotation-pair blocks");
+template <int BLK, bool TILED, int NW>
+__global__ __launch_bounds__(64 * NW, 2) void k_jacobi_round(const JacTask* tasks, int ntasks, int sweep, int round) {
+  static_assert(BLK == 16 && JB == BLK && JP == 2 * BLK && NW % 4 == 0, "rotation-pair blocks of the inner sweep");
+  constexpr int NT = 64 * NW;
   __shared__ InnerShared S;
   double2 (*sG)[JP + 1] = S.G[0];
   double2 (*sG2)[JP + 1] = S.G[1];
@@ -505,22 +516,23 @@ __global__ __launch_bounds__(256, 2) void k_jacobi_round(const JacTask* tasks, i
   auto at = [&](int row, int col) -> size_t { return (size_t)row * ld + col; };
   const int rowa = ba * JB + l16, rowb = bb * JB + l16;  // pair rows l16 and 16 + l16
 
-  // ---- Gram tiles (0,0), (0,1), (1,1) over this wave's 4-column units u = wave, wave + 4, ... ----
+  // ---- Gram tiles (0,0), (0,1), (1,1), or in a cross round (0,1) and the diagonal, over this wave's 4-column units u = wave, wave + NW, ... ----
   // FP64 MFMA, or in the early sweeps of large SVDs FP32 MFMA at twice the rate: the rotations
   // they give are still applied in FP64 and are unitary, so the rows only lose the accuracy of
   // the rotation angles, which the FP64 sweeps that end every SVD make up for.
-  // Tiled rows (c = c_tot, the last tile's missing columns zero): unit wave + 4 d is the wave's
-  // quarter of tile d, so both operands advance by one tile a step; row-major rows are bounded by
-  // their columns.
-  const int nd = TILED ? ntc : (((C + 3) >> 2) + 3) >> 2;
-  const double2* ga = TILED ? Y + (size_t)ba * ntc * 256 + (l16 >> 2) * 64 + wave * 16 + (l16 & 3) * 4 + k4 : Y;
-  const double2* gb = TILED ? Y + (size_t)bb * ntc * 256 + (l16 >> 2) * 64 + wave * 16 + (l16 & 3) * 4 + k4 : Y;
-  constexpr int PD = 2;
+  // Tiled rows (c = c_tot, the last tile's missing columns zero): unit wave + NW d is a quarter of
+  // tile (wave / 4) + (NW / 4) d, so both operands advance by NW / 4 tiles a step; row-major rows are
+  // bounded by their columns.
+  constexpr int TS = NW / 4;  // tiles a step
+  const int nd = ((TILED ? ntc : (((C + 3) >> 2) + 3) >> 2) + TS - 1) / TS;
+  const double2* ga = TILED ? Y + (size_t)ba * ntc * 256 + (l16 >> 2) * 64 + (wave & 3) * 16 + (l16 & 3) * 4 + k4 : Y;
+  const double2* gb = TILED ? Y + (size_t)bb * ntc * 256 + (l16 >> 2) * 64 + (wave & 3) * 16 + (l16 & 3) * 4 + k4 : Y;
+  constexpr int PD = NW == 4 ? 2 : 4;
   auto ld_unit = [&](int d, double2& v0, double2& v1) {
-    const int col = 4 * (wave + 4 * d) + k4;
-    if (TILED ? d < nd : col < C) {
-      v0 = gld(TILED ? ga + (size_t)d * 256 : Y + at(rowa, col));
-      v1 = gld(TILED ? gb + (size_t)d * 256 : Y + at(rowb, col));
+    const int col = 4 * (wave + NW * d) + k4, tile = (wave >> 2) + TS * d;
+    if (TILED ? tile < ntc : col < C) {
+      v0 = gld(TILED ? ga + (size_t)tile * 256 : Y + at(rowa, col));
+      v1 = gld(TILED ? gb + (size_t)tile * 256 : Y + at(rowb, col));
     } else {
       v0 = make_double2(0, 0);
       v1 = make_double2(0, 0);
@@ -530,120 +542,152 @@ __global__ __launch_bounds__(256, 2) void k_jacobi_round(const JacTask* tasks, i
   //  * diagonal tiles (Hermitian): Re = Ar Ar^T + Ai Ai^T, and Im = X - X^T with X = Ar Ai^T;
   //  * off-diagonal tile conj(A) B^T (Gauss): K1 = (Ar - Ai) Br^T, K2 = Ar (Bi - Br)^T,
   //    K3 = -Ai (Br + Bi)^T;  Re = K1 - K3, Im = K1 + K2.
-  // Each partial sum of the four waves goes to LDS as (Re, X) for the diagonal tiles and
+  // A cross round takes only the rows' norms of the diagonal tiles, three products a unit instead of
+  // nine: what its sweep leaves out there is second order (see jacobi_full_round).
+  // Each partial sum of the waves goes to LDS as (Re, X) for the diagonal tiles and
   // (Re, Im) for the off-diagonal one; Im of the diagonal tiles is formed after the sum.
-  if (sweep >= T.gram32) {
-    mfma_d4 a00r = {0, 0, 0, 0}, a00x = {0, 0, 0, 0}, a11r = {0, 0, 0, 0}, a11x = {0, 0, 0, 0};
-    mfma_d4 k1 = {0, 0, 0, 0}, k2 = {0, 0, 0, 0}, k3 = {0, 0, 0, 0};
-    double2 x0[PD], x1[PD];
-#pragma unroll
-    for (int d = 0; d < PD; ++d) ld_unit(d, x0[d], x1[d]);
-#pragma unroll 1
-    for (int e0 = 0; e0 < nd; e0 += PD) {
-#pragma unroll
-      for (int d = 0; d < PD; ++d) {
-        const double2 v0 = x0[d], v1 = x1[d];
-        ld_unit(e0 + d + PD, x0[d], x1[d]);
-        a00r = mfma64(v0.x, v0.x, a00r);
-        a11r = mfma64(v1.x, v1.x, a11r);
-        a00x = mfma64(v0.x, v0.y, a00x);
-        a11x = mfma64(v1.x, v1.y, a11x);
-        k1 = mfma64(v0.x - v0.y, v1.x, k1);
-        k2 = mfma64(v0.x, v1.y - v1.x, k2);
-        k3 = mfma64(-v0.y, v1.x + v1.y, k3);
-        a00r = mfma64(v0.y, v0.y, a00r);
-        a11r = mfma64(v1.y, v1.y, a11r);
-      }
+  // to_lds(value of the tile entry v of this lane, its row): waves 0, 1 store, then 2, 3 (and so on) add
+  const bool full = jacobi_full_round(round, nb);
+  double n0 = 0.0, n1 = 0.0;  // cross: squared norms of the rows l16 and 16 + l16 over this lane's columns
+  auto to_lds = [&](auto row, auto e00, auto e01, auto e11) __attribute__((always_inline)) {
+    if (!full) {
+      n0 += __shfl_xor(n0, 16);
+      n1 += __shfl_xor(n1, 16);
+      n0 += __shfl_xor(n0, 32);
+      n1 += __shfl_xor(n1, 32);
     }
-    // f64 D[i][j]: lane j + 16 (i % 4), register i / 4
-    for (int w = 0; w < 4; w += 2) {  // waves 0, 1 store, then 2, 3 add: two partial sums
-      if ((wave & 2) == w) {
+    for (int w = 0; w < NW; w += 2) {
+      if ((wave & ~1) == w) {
         double2 (*P)[JP + 1] = S.G[wave & 1];
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-          const int i = 4 * v + k4, j = l16;
-          double2 g00 = make_double2(a00r[v], a00x[v]);
-          double2 g01 = make_double2(k1[v] - k3[v], k1[v] + k2[v]);
-          double2 g11 = make_double2(a11r[v], a11x[v]);
-          if (w) {
-            g00 = cadd(g00, P[i][j]);
-            g01 = cadd(g01, P[i][JB + j]);
-            g11 = cadd(g11, P[JB + i][JB + j]);
+          const int i = row(v), j = l16;
+          const double2 g01 = e01(v);
+          P[i][JB + j] = w ? cadd(g01, P[i][JB + j]) : g01;
+          if (full) {
+            const double2 g00 = e00(v), g11 = e11(v);
+            P[i][j] = w ? cadd(g00, P[i][j]) : g00;
+            P[JB + i][JB + j] = w ? cadd(g11, P[JB + i][JB + j]) : g11;
           }
-          P[i][j] = g00;
-          P[i][JB + j] = g01;
-          P[JB + i][JB + j] = g11;
+        }
+        if (!full && k4 == 0) {
+          P[l16][l16].x = w ? P[l16][l16].x + n0 : n0;
+          P[JB + l16][JB + l16].x = w ? P[JB + l16][JB + l16].x + n1 : n1;
         }
       }
       __syncthreads();
     }
+  };
+  if (sweep >= T.gram32) {
+    mfma_d4 k1 = {0, 0, 0, 0}, k2 = {0, 0, 0, 0}, k3 = {0, 0, 0, 0};
+    mfma_d4 a00r = {0, 0, 0, 0}, a00x = {0, 0, 0, 0}, a11r = {0, 0, 0, 0}, a11x = {0, 0, 0, 0};
+    auto products = [&](auto diag) __attribute__((always_inline)) {
+      double2 x0[PD], x1[PD];
+#pragma unroll
+      for (int d = 0; d < PD; ++d) ld_unit(d, x0[d], x1[d]);
+#pragma unroll 1
+      for (int e0 = 0; e0 < nd; e0 += PD) {
+#pragma unroll
+        for (int d = 0; d < PD; ++d) {
+          const double2 v0 = x0[d], v1 = x1[d];
+          ld_unit(e0 + d + PD, x0[d], x1[d]);
+          if (diag) {
+            a00r = mfma64(v0.x, v0.x, a00r);
+            a11r = mfma64(v1.x, v1.x, a11r);
+            a00x = mfma64(v0.x, v0.y, a00x);
+            a11x = mfma64(v1.x, v1.y, a11x);
+          } else {
+            n0 = fma(v0.x, v0.x, fma(v0.y, v0.y, n0));
+            n1 = fma(v1.x, v1.x, fma(v1.y, v1.y, n1));
+          }
+          k1 = mfma64(v0.x - v0.y, v1.x, k1);
+          k2 = mfma64(v0.x, v1.y - v1.x, k2);
+          k3 = mfma64(-v0.y, v1.x + v1.y, k3);
+          if (diag) {
+            a00r = mfma64(v0.y, v0.y, a00r);
+            a11r = mfma64(v1.y, v1.y, a11r);
+          }
+        }
+      }
+    };
+    if (full) products(std::true_type());
+    else products(std::false_type());
+    // f64 D[i][j]: lane j + 16 (i % 4), register i / 4
+    to_lds([&](int v) { return 4 * v + k4; }, [&](int v) { return make_double2(a00r[v], a00x[v]); },
+           [&](int v) { return make_double2(k1[v] - k3[v], k1[v] + k2[v]); },
+           [&](int v) { return make_double2(a11r[v], a11x[v]); });
   } else {
     typedef float mfma_f4 __attribute__((ext_vector_type(4)));
-    mfma_f4 b00r = {0, 0, 0, 0}, b00x = {0, 0, 0, 0}, b11r = {0, 0, 0, 0}, b11x = {0, 0, 0, 0};
     mfma_f4 h1 = {0, 0, 0, 0}, h2 = {0, 0, 0, 0}, h3 = {0, 0, 0, 0};
-    double2 x0[PD], x1[PD];
+    mfma_f4 b00r = {0, 0, 0, 0}, b00x = {0, 0, 0, 0}, b11r = {0, 0, 0, 0}, b11x = {0, 0, 0, 0};
+    auto products = [&](auto diag) __attribute__((always_inline)) {
+      double2 x0[PD], x1[PD];
 #pragma unroll
-    for (int d = 0; d < PD; ++d) ld_unit(d, x0[d], x1[d]);
+      for (int d = 0; d < PD; ++d) ld_unit(d, x0[d], x1[d]);
 #pragma unroll 1
-    for (int e0 = 0; e0 < nd; e0 += PD) {
+      for (int e0 = 0; e0 < nd; e0 += PD) {
 #pragma unroll
-      for (int d = 0; d < PD; ++d) {
-        const float p0 = (float)x0[d].x, q0 = (float)x0[d].y, p1 = (float)x1[d].x, q1 = (float)x1[d].y;
-        ld_unit(e0 + d + PD, x0[d], x1[d]);
-        b00r = __builtin_amdgcn_mfma_f32_16x16x4f32(p0, p0, b00r, 0, 0, 0);
-        b11r = __builtin_amdgcn_mfma_f32_16x16x4f32(p1, p1, b11r, 0, 0, 0);
-        b00x = __builtin_amdgcn_mfma_f32_16x16x4f32(p0, q0, b00x, 0, 0, 0);
-        b11x = __builtin_amdgcn_mfma_f32_16x16x4f32(p1, q1, b11x, 0, 0, 0);
-        h1 = __builtin_amdgcn_mfma_f32_16x16x4f32(p0 - q0, p1, h1, 0, 0, 0);
-        h2 = __builtin_amdgcn_mfma_f32_16x16x4f32(p0, q1 - p1, h2, 0, 0, 0);
-        h3 = __builtin_amdgcn_mfma_f32_16x16x4f32(-q0, p1 + q1, h3, 0, 0, 0);
-        b00r = __builtin_amdgcn_mfma_f32_16x16x4f32(q0, q0, b00r, 0, 0, 0);
-        b11r = __builtin_amdgcn_mfma_f32_16x16x4f32(q1, q1, b11r, 0, 0, 0);
-      }
-    }
-    // f32 D[i][j]: lane j + 16 (i / 4), register i % 4; the four waves' partial tiles are
-    // summed in FP64
-    for (int w = 0; w < 4; w += 2) {  // waves 0, 1 store, then 2, 3 add: two partial sums
-      if ((wave & 2) == w) {
-        double2 (*P)[JP + 1] = S.G[wave & 1];
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const int i = 4 * k4 + v, j = l16;
-          double2 g00 = make_double2((double)b00r[v], (double)b00x[v]);
-          double2 g01 = make_double2((double)h1[v] - (double)h3[v], (double)h1[v] + (double)h2[v]);
-          double2 g11 = make_double2((double)b11r[v], (double)b11x[v]);
-          if (w) {
-            g00 = cadd(g00, P[i][j]);
-            g01 = cadd(g01, P[i][JB + j]);
-            g11 = cadd(g11, P[JB + i][JB + j]);
+        for (int d = 0; d < PD; ++d) {
+          const double2 v0 = x0[d], v1 = x1[d];
+          const float p0 = (float)v0.x, q0 = (float)v0.y, p1 = (float)v1.x, q1 = (float)v1.y;
+          ld_unit(e0 + d + PD, x0[d], x1[d]);
+          if (diag) {
+            b00r = __builtin_amdgcn_mfma_f32_16x16x4f32(p0, p0, b00r, 0, 0, 0);
+            b11r = __builtin_amdgcn_mfma_f32_16x16x4f32(p1, p1, b11r, 0, 0, 0);
+            b00x = __builtin_amdgcn_mfma_f32_16x16x4f32(p0, q0, b00x, 0, 0, 0);
+            b11x = __builtin_amdgcn_mfma_f32_16x16x4f32(p1, q1, b11x, 0, 0, 0);
+          } else {
+            n0 = fma(v0.x, v0.x, fma(v0.y, v0.y, n0));
+            n1 = fma(v1.x, v1.x, fma(v1.y, v1.y, n1));
           }
-          P[i][j] = g00;
-          P[i][JB + j] = g01;
-          P[JB + i][JB + j] = g11;
+          h1 = __builtin_amdgcn_mfma_f32_16x16x4f32(p0 - q0, p1, h1, 0, 0, 0);
+          h2 = __builtin_amdgcn_mfma_f32_16x16x4f32(p0, q1 - p1, h2, 0, 0, 0);
+          h3 = __builtin_amdgcn_mfma_f32_16x16x4f32(-q0, p1 + q1, h3, 0, 0, 0);
+          if (diag) {
+            b00r = __builtin_amdgcn_mfma_f32_16x16x4f32(q0, q0, b00r, 0, 0, 0);
+            b11r = __builtin_amdgcn_mfma_f32_16x16x4f32(q1, q1, b11r, 0, 0, 0);
+          }
         }
       }
-      __syncthreads();
-    }
+    };
+    if (full) products(std::true_type());
+    else products(std::false_type());
+    // f32 D[i][j]: lane j + 16 (i / 4), register i % 4; the waves' partial tiles are summed in FP64
+    to_lds([&](int v) { return 4 * k4 + v; }, [&](int v) { return make_double2((double)b00r[v], (double)b00x[v]); },
+           [&](int v) {
+             return make_double2((double)h1[v] - (double)h3[v], (double)h1[v] + (double)h2[v]);
+           },
+           [&](int v) { return make_double2((double)b11r[v], (double)b11x[v]); });
   }
   {
-    // the two partial sums; Im of the diagonal tiles from X (X[i][j] - X[j][i]), and the lower
-    // off-diagonal tile
-    const int i = tid >> 4, j = tid & 15;
-    const double2 g00 = cadd(sG[i][j], sG2[i][j]), g11 = cadd(sG[JB + i][JB + j], sG2[JB + i][JB + j]);
-    const double y00 = sG[j][i].y + sG2[j][i].y, y11 = sG[JB + j][JB + i].y + sG2[JB + j][JB + i].y;
+    // the two partial sums; Im of the diagonal tiles from X (X[i][j] - X[j][i]), or nothing but the
+    // diagonal in a cross round; and the lower off-diagonal tile
+    const int i = (tid >> 4) & 15, j = tid & 15;
+    double2 g00 = make_double2(0, 0), g11 = make_double2(0, 0);
+    if (full) {
+      g00 = cadd(sG[i][j], sG2[i][j]);
+      g11 = cadd(sG[JB + i][JB + j], sG2[JB + i][JB + j]);
+      g00.y -= sG[j][i].y + sG2[j][i].y;
+      g11.y -= sG[JB + j][JB + i].y + sG2[JB + j][JB + i].y;
+    } else if (i == j) {
+      g00.x = sG[i][i].x + sG2[i][i].x;
+      g11.x = sG[JB + i][JB + i].x + sG2[JB + i][JB + i].x;
+    }
     const double2 g01 = cadd(sG[i][JB + j], sG2[i][JB + j]), g10 = cadd(sG[j][JB + i], sG2[j][JB + i]);
     __syncthreads();
-    sG[i][j] = make_double2(g00.x, g00.y - y00);
-    sG[JB + i][JB + j] = make_double2(g11.x, g11.y - y11);
-    sG[i][JB + j] = g01;
-    sG[JB + i][j] = cconj(g10);
+    if (tid < 256) {
+      sG[i][j] = g00;
+      sG[JB + i][JB + j] = g11;
+      sG[i][JB + j] = g01;
+      sG[JB + i][j] = cconj(g10);
+    }
   }
   __syncthreads();
   // ---- convergence test of this block pair: |G_ij|^2 > tol^2 G_ii G_jj for some i < j ----
   {
     int above = 0;
     const double tol2 = tol * tol;
-    for (int e = tid; e < JP * JP; e += 256) {
+    for (int e = tid; e < JP * JP; e += NT) {
       const int i = e / JP, j = e % JP;
       const double aii = sG[i][i].x, ajj = sG[j][j].x;
       if (i < j && aii > floor2 && ajj > floor2 && cabs2(sG[i][j]) > tol2 * (aii * ajj)) above = 1;
@@ -653,7 +697,10 @@ __global__ __launch_bounds__(256, 2) void k_jacobi_round(const JacTask* tasks, i
     __syncthreads();
   }
   if (tid == 0) atomicAdd(counts + 1, 1);
-  if (!(S.rot[0] | S.rot[1] | S.rot[2] | S.rot[3])) return;
+  int any = 0;
+#pragma unroll
+  for (int w = 0; w < NW; ++w) any |= S.rot[w];
+  if (!any) return;
 
   // ---- apply prefetch: this wave's first column tile, all 32 rows ----
   // element (4 kk + k4, column l16 of the tile) of the pair's rows, kk = 0..7
@@ -667,24 +714,24 @@ __global__ __launch_bounds__(256, 2) void k_jacobi_round(const JacTask* tasks, i
 #pragma unroll
   for (int kk = 0; kk < 8; ++kk) bq[kk] = ok_tile(wave) ? gld(elem(kk, wave)) : make_double2(0, 0);
 
-  if (jacobi_full_round(round, nb)) inner_sweep<false>(S, tol * 0.25, floor2);
+  if (full) inner_sweep<false>(S, tol * 0.25, floor2);
   else inner_sweep<true>(S, tol * 0.25, floor2);
   double2 (*sW)[JP + 1] = S.G[0];
 
-  // ---- apply Y' = W^T Y; wave owns column tiles wave, wave + 4, ... (all 32 rows) ----
+  // ---- apply Y' = W^T Y; wave owns column tiles wave, wave + NW, ... (all 32 rows) ----
 #pragma unroll 1
-  for (int ctile = wave; ctile < nt; ctile += 4) {
+  for (int ctile = wave; ctile < nt; ctile += NW) {
     // (A + iB)(C + iD) with three real products (Gauss): K1 = (A + B) C, K2 = A (D - C),
     // K3 = B (C + D); Re = K1 - K3, Im = K1 + K2
     mfma_d4 e0 = {0, 0, 0, 0}, f0 = {0, 0, 0, 0}, g0 = {0, 0, 0, 0};
     mfma_d4 e1 = {0, 0, 0, 0}, f1 = {0, 0, 0, 0}, g1 = {0, 0, 0, 0};
-    const bool nok = ok_tile(ctile + 4);
+    const bool nok = ok_tile(ctile + NW);
 #pragma unroll
     for (int kk = 0; kk < 8; ++kk) {
       const double2 b = bq[kk];
       const double2 w0 = sW[kk * 4 + k4][l16];       // A[i][k] = W[k][i], rows 0..15
       const double2 w1 = sW[kk * 4 + k4][16 + l16];  // rows 16..31
-      bq[kk] = nok ? gld(elem(kk, ctile + 4)) : make_double2(0, 0);
+      bq[kk] = nok ? gld(elem(kk, ctile + NW)) : make_double2(0, 0);
       const double dmc = b.y - b.x, cpd = b.x + b.y;
       e0 = mfma64(w0.x + w0.y, b.x, e0);
       e1 = mfma64(w1.x + w1.y, b.x, e1);
@@ -735,15 +782,20 @@ hipError_t launch_fro2(const SplitTask* d_split, const JacTask* d_jac, double* p
   return hipGetLastError();
 }
 
+// Launches of at most one workgroup per CU take eight waves each: 256 workgroups on 32 x 512 took 71 us
+// with four waves and 56 with eight; from two per CU on, the second one's waves do the same.
+constexpr int JAC_WIDE_PAIRS = 256;
 hipError_t launch_jacobi_round(const JacTask* d_tasks, int ntasks, int total_pairs, int sweep, int round,
                                hipStream_t s, bool tiled) {
   if (total_pairs <= 0) return hipSuccess;
-  if (tiled)
-    hipLaunchKernelGGL((k_jacobi_round<JB, true>), dim3(total_pairs), dim3(256), 0, s, d_tasks, ntasks, sweep,
-                       round);
-  else
-    hipLaunchKernelGGL((k_jacobi_round<JB, false>), dim3(total_pairs), dim3(256), 0, s, d_tasks, ntasks, sweep,
-                       round);
+  const dim3 grid(total_pairs);
+  if (total_pairs <= JAC_WIDE_PAIRS) {
+    if (tiled) hipLaunchKernelGGL((k_jacobi_round<JB, true, 8>), grid, dim3(512), 0, s, d_tasks, ntasks, sweep, round);
+    else hipLaunchKernelGGL((k_jacobi_round<JB, false, 8>), grid, dim3(512), 0, s, d_tasks, ntasks, sweep, round);
+  } else {
+    if (tiled) hipLaunchKernelGGL((k_jacobi_round<JB, true, 4>), grid, dim3(256), 0, s, d_tasks, ntasks, sweep, round);
+    else hipLaunchKernelGGL((k_jacobi_round<JB, false, 4>), grid, dim3(256), 0, s, d_tasks, ntasks, sweep, round);
+  }
   return hipGetLastError();
 }
 
