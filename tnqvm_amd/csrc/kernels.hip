@@ -486,9 +486,9 @@ __device__ __forceinline__ void inner_sweep(InnerShared& S, double itol, double 
 //    three MFMA a unit: 12.5k, 20.6k, 16.6k; 35.2 -> 29.4 -> 26.8 us a launch (512 columns:
 //    54.4 -> 43.5 -> 37.3).
 // BLK is the block size JB (a template parameter: the kernel's register allocation on
-// gfx950 comes out at 168 VGPRs, three waves per SIMD, in the tiled form).
+// gfx950 comes out at 128 VGPRs with four waves, four waves per SIMD, in the tiled form).
 template <int BLK, bool TILED, int NW>
-__global__ __launch_bounds__(64 * NW, 2) void k_jacobi_round(const JacTask* tasks, int ntasks, int sweep, int round) {
+__global__ __launch_bounds__(64 * NW, NW == 4 && TILED ? 4 : 2) void k_jacobi_round(const JacTask* tasks, int ntasks, int sweep, int round) {
   static_assert(BLK == 16 && JB == BLK && JP == 2 * BLK && NW % 4 == 0, "rotation-pair blocks of the inner sweep");
   constexpr int NT = 64 * NW;
   __shared__ InnerShared S;
@@ -711,40 +711,53 @@ __global__ __launch_bounds__(64 * NW, 2) void k_jacobi_round(const JacTask* task
   auto ok_tile = [&](int ctile) { return TILED ? ctile < nt : ctile < nt && ctile * 16 + l16 < CT; };
   auto elem = [&](int kk, int ctile) { return (kk < 4 ? ya + kk * step_row : yb + (kk - 4) * step_row) + ctile * step_tile; };
   double2 bq[8];
+  auto first_tile = [&]() __attribute__((always_inline)) {
 #pragma unroll
-  for (int kk = 0; kk < 8; ++kk) bq[kk] = ok_tile(wave) ? gld(elem(kk, wave)) : make_double2(0, 0);
-
+    for (int kk = 0; kk < 8; ++kk) bq[kk] = ok_tile(wave) ? gld(elem(kk, wave)) : make_double2(0, 0);
+  };
+  if (NW != 4) first_tile();
   if (full) inner_sweep<false>(S, tol * 0.25, floor2);
   else inner_sweep<true>(S, tol * 0.25, floor2);
+  if (NW == 4) first_tile();
   double2 (*sW)[JP + 1] = S.G[0];
 
+  // Several workgroups share a CU where NW = 4 and cover each other's phases: there 128 registers for four
+  // of them beat the first tile's loads ahead of the inner sweep, W in registers and both row tiles at a
+  // time (three per CU): 1024 workgroups on 32 x 256 95 -> 81 us, on 32 x 512 154 -> 145 us.
+  constexpr int RT = NW == 4 ? 1 : 2;  // 16-row tiles at a time
   // ---- apply Y' = W^T Y; wave owns column tiles wave, wave + NW, ... (all 32 rows) ----
 #pragma unroll 1
   for (int ctile = wave; ctile < nt; ctile += NW) {
+    if (NW == 4) asm volatile("" ::: "memory");  // W from LDS for each tile, not held in registers over the tiles
     // (A + iB)(C + iD) with three real products (Gauss): K1 = (A + B) C, K2 = A (D - C),
     // K3 = B (C + D); Re = K1 - K3, Im = K1 + K2
-    mfma_d4 e0 = {0, 0, 0, 0}, f0 = {0, 0, 0, 0}, g0 = {0, 0, 0, 0};
-    mfma_d4 e1 = {0, 0, 0, 0}, f1 = {0, 0, 0, 0}, g1 = {0, 0, 0, 0};
-    const bool nok = ok_tile(ctile + NW);
+    const bool ok = ok_tile(ctile), nok = ok_tile(ctile + NW);
 #pragma unroll
-    for (int kk = 0; kk < 8; ++kk) {
-      const double2 b = bq[kk];
-      const double2 w0 = sW[kk * 4 + k4][l16];       // A[i][k] = W[k][i], rows 0..15
-      const double2 w1 = sW[kk * 4 + k4][16 + l16];  // rows 16..31
-      bq[kk] = nok ? gld(elem(kk, ctile + NW)) : make_double2(0, 0);
-      const double dmc = b.y - b.x, cpd = b.x + b.y;
-      e0 = mfma64(w0.x + w0.y, b.x, e0);
-      e1 = mfma64(w1.x + w1.y, b.x, e1);
-      f0 = mfma64(w0.x, dmc, f0);
-      f1 = mfma64(w1.x, dmc, f1);
-      g0 = mfma64(w0.y, cpd, g0);
-      g1 = mfma64(w1.y, cpd, g1);
-    }
-    if (ok_tile(ctile)) {
+    for (int h = 0; h < 2; h += RT) {
+      mfma_d4 e[RT], f[RT], g[RT];
 #pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        gst(elem(v, ctile), make_double2(e0[v] - g0[v], e0[v] + f0[v]));
-        gst(elem(4 + v, ctile), make_double2(e1[v] - g1[v], e1[v] + f1[v]));
+      for (int q = 0; q < RT; ++q) e[q] = f[q] = g[q] = mfma_d4{0, 0, 0, 0};
+#pragma unroll
+      for (int kk = 0; kk < 8; ++kk) {
+        const double2 b = bq[kk];
+        double2 w[RT];
+#pragma unroll
+        for (int q = 0; q < RT; ++q) w[q] = sW[kk * 4 + k4][16 * (h + q) + l16];  // A[i][k] = W[k][i]
+        if (h + RT == 2) bq[kk] = nok ? gld(elem(kk, ctile + NW)) : make_double2(0, 0);
+        const double dmc = b.y - b.x, cpd = b.x + b.y;
+#pragma unroll
+        for (int q = 0; q < RT; ++q) {
+          e[q] = mfma64(w[q].x + w[q].y, b.x, e[q]);
+          f[q] = mfma64(w[q].x, dmc, f[q]);
+          g[q] = mfma64(w[q].y, cpd, g[q]);
+        }
+      }
+      if (ok) {
+#pragma unroll
+        for (int q = 0; q < RT; ++q)
+#pragma unroll
+          for (int v = 0; v < 4; ++v)
+            gst(elem(4 * (h + q) + v, ctile), make_double2(e[q][v] - g[q][v], e[q][v] + f[q][v]));
       }
     }
   }
