@@ -2687,8 +2687,8 @@ int measure_rdm(hipmps_state_s* s, const std::vector<int>& qubits, double* out) 
   return 0;
 }
 
-// amplitude / slice chain
-int chain_contract(hipmps_state_s* s, int rows0, const int8_t* d_bits, const int* slice_bits, std::vector<double2>& out) {
+// amplitude chain (bits: rows0 x n on the host) or slice chain (slice_bits)
+int chain_contract(hipmps_state_s* s, int rows0, const int8_t* bits, const int* slice_bits, std::vector<double2>& out) {
   if (is_purified(s))
     return fail(HIPMPS_E_UNSUPPORTED, "amplitudes are not defined for a purified (mixed) state");
   hipmps_engine E = s->e;
@@ -2700,44 +2700,42 @@ int chain_contract(hipmps_state_s* s, int rows0, const int8_t* d_bits, const int
   size_t maxv = 1;
   for (int k = 0; k <= n; ++k) maxv = std::max(maxv, (size_t)rows[k] * s->chi[k]);
   if (maxv > ((size_t)1 << 31)) return fail(HIPMPS_E_UNSUPPORTED, "slice too large");
-  size_t vb = align_up(maxv * 16);
-  RC_TRY(E->env.ensure(2 * vb + 4096));
+  const size_t vb = align_up(maxv * 16), bb = bits ? (size_t)rows0 * n : 0;
+  RC_TRY(E->env.ensure(2 * vb + bb + 4096));
   char* base = (char*)E->env.p;
   double2* v0 = (double2*)base;
   double2* v1 = (double2*)(base + vb);
-  // v0 = ones (rows0 x 1)
-  {
-    std::vector<double2> ones(rows0, make_double2(1.0, 0.0));
-    HIP_TRY(hipMemcpyAsync(v0, ones.data(), rows0 * sizeof(double2), hipMemcpyHostToDevice, E->stream));
-    HIP_TRY(hipStreamSynchronize(E->stream));
-  }
-  RC_TRY(E->hdesc.ensure(sizeof(ChainTask)));
-  RC_TRY(E->desc.ensure(sizeof(ChainTask)));
+  int8_t* d_bits = (int8_t*)(base + 2 * vb);
+  const hipStream_t st = E->stream;
+  // every site's descriptor in one upload; the chain itself needs no synchronisation
+  const size_t db = (size_t)n * sizeof(ChainTask);
+  RC_TRY(E->hdesc.ensure(db));
+  RC_TRY(E->desc.ensure(db));
+  ChainTask* h = (ChainTask*)E->hdesc.p;
+  memset(h, 0, db);
   for (int k = 0; k < n; ++k) {
-    ChainTask* h = (ChainTask*)E->hdesc.p;
-    memset(h, 0, sizeof(*h));
-    h->vin = v0;
-    h->vout = v1;
-    h->A = s->sites[k].p;
-    h->cl = s->chi[k];
-    h->cr = s->chi[k + 1];
-    h->rows_in = (int)rows[k];
-    h->rows_out = (int)rows[k + 1];
-    h->bits = d_bits;
-    h->n = n;
-    h->site = k;
-    h->mode = slice_bits ? 1 : 0;
-    h->slice_bit = slice_bits ? slice_bits[k] : 0;
-    h->block_begin = 0;
-    h->blocks = (int)rows[k + 1] * ((h->cr + 255) / 256);
-    HIP_TRY(hipMemcpyAsync(E->desc.p, h, sizeof(ChainTask), hipMemcpyHostToDevice, E->stream));
-    HIP_TRY(launch_chain((const ChainTask*)E->desc.p, 1, h->blocks, s->fp32, E->stream));
-    HIP_TRY(hipStreamSynchronize(E->stream));
-    std::swap(v0, v1);
+    h[k].vin = (k & 1) ? v1 : v0;
+    h[k].vout = (k & 1) ? v0 : v1;
+    h[k].A = s->sites[k].p;
+    h[k].cl = s->chi[k];
+    h[k].cr = s->chi[k + 1];
+    h[k].rows_in = (int)rows[k];
+    h[k].rows_out = (int)rows[k + 1];
+    h[k].bits = d_bits;
+    h[k].n = n;
+    h[k].site = k;
+    h[k].mode = slice_bits ? 1 : 0;
+    h[k].slice_bit = slice_bits ? slice_bits[k] : 0;
+    h[k].blocks = chain_blocks(rows[k + 1], h[k].cr);
   }
+  HIP_TRY(hipMemcpyAsync(E->desc.p, h, db, hipMemcpyHostToDevice, st));
+  if (bits) HIP_TRY(hipMemcpyAsync(d_bits, bits, bb, hipMemcpyHostToDevice, st));
+  HIP_TRY(launch_fill_c(v0, (size_t)rows0, make_double2(1.0, 0.0), st));  // rows of ones (chi_0 = 1)
+  for (int k = 0; k < n; ++k)
+    HIP_TRY(launch_chain((const ChainTask*)E->desc.p + k, 1, h[k].blocks, s->fp32, st));
   out.resize(rows[n]);
-  HIP_TRY(hipMemcpyAsync(out.data(), v0, rows[n] * sizeof(double2), hipMemcpyDeviceToHost, E->stream));
-  HIP_TRY(hipStreamSynchronize(E->stream));
+  HIP_TRY(hipMemcpyAsync(out.data(), (n & 1) ? v1 : v0, rows[n] * sizeof(double2), hipMemcpyDeviceToHost, st));
+  HIP_TRY(hipStreamSynchronize(st));
   return 0;
 }
 
@@ -3261,16 +3259,8 @@ int hipmps_amplitudes(hipmps_state s, const int8_t* bits, int k, double* out) {
   RC_TRY(state_flush(s));
   for (size_t t = 0; t < (size_t)k * s->n; ++t)
     if (bits[t] != 0 && bits[t] != 1) return fail(HIPMPS_E_ARG, "bits must be 0 or 1");
-  hipmps_engine E = s->e;
-  // bits live after the chain buffers; upload into a dedicated small buffer
-  DevBuf db;
-  RC_TRY(db.ensure((size_t)k * s->n));
-  HIP_TRY(hipMemcpy(db.p, bits, (size_t)k * s->n, hipMemcpyHostToDevice));
   std::vector<double2> v;
-  int rc = chain_contract(s, k, (const int8_t*)db.p, nullptr, v);
-  db.release();
-  (void)E;
-  if (rc) return rc;
+  RC_TRY(chain_contract(s, k, bits, nullptr, v));
   for (int t = 0; t < k; ++t) {
     out[2 * t] = v[t].x;
     out[2 * t + 1] = v[t].y;
@@ -3331,15 +3321,14 @@ int hipmps_amplitudes_noalloc(hipmps_state s, const int8_t* bits, int k, double*
       c.site = site;
       c.mode = 0;
       c.block_begin = 0;
-      c.blocks = k * ((c.cr + 255) / 256);
+      c.blocks = chain_blocks(k, c.cr);
     }
     HIP_TRY(hipMemcpy(d_desc + k0, h, (size_t)m * sizeof(ChainTask), hipMemcpyHostToDevice));
   }
   HIP_TRY(hipMemcpy(d_bits, bits, (size_t)k * n, hipMemcpyHostToDevice));
   HIP_TRY(launch_fill_c(v0, (size_t)k, make_double2(1.0, 0.0), E->stream));  // rows of ones (chi_0 = 1)
   for (int site = 0; site < n; ++site) {
-    const int blocks = k * ((s->chi[site + 1] + 255) / 256);
-    HIP_TRY(launch_chain(d_desc + site, 1, blocks, s->fp32, E->stream));
+    HIP_TRY(launch_chain(d_desc + site, 1, chain_blocks(k, s->chi[site + 1]), s->fp32, E->stream));
   }
   const double2* res = (n & 1) ? v1 : v0;
   HIP_TRY(hipMemcpyAsync(out, res, (size_t)k * sizeof(double2), hipMemcpyDeviceToHost, E->stream));

@@ -210,9 +210,13 @@ struct TriTask {
 hipError_t launch_rank_cut(const TriTask* d_tasks, const double* d_sigma_cut, int ntasks, hipStream_t s);
 
 // Chain step for amplitudes / slices: rows of partial contractions v[row][l].
+constexpr int CHAIN_ROWS = 64;  // rows of a workgroup of k_chain
+inline int chain_blocks(long long rows_out, int cr) {
+  return (int)((rows_out + CHAIN_ROWS - 1) / CHAIN_ROWS * ((cr + 15) / 16));
+}
 struct ChainTask {
-  const double2* vin;   // rows_in x cl
-  double2* vout;        // rows_out x cr
+  const double2* vin;   // cl x rows_in
+  double2* vout;        // cr x rows_out
   const void* A;        // cl x 2 x cr
   int cl, cr, rows_in, rows_out;
   const int8_t* bits;   // amplitude mode: bits[row * n + site]; slice mode: unused

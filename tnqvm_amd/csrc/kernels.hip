@@ -1244,38 +1244,144 @@ hipError_t launch_gemm(const GemmTask* d_tasks, int ntasks, int total_tiles, int
 }
 
 // ------------------------------------------------------------------ chain step (amplitudes / slices)
-// amplitude: vout[row][r] = sum_l vin[row][l] A[l][bits[row][site]][r]
-// slice:     vout[o][r]   = sum_l vin[o % rows_in][l] A[l][p][r], p = open ? o / rows_in : bit
+// amplitude: vout[r][row] = sum_l vin[l][row] A[l][bits[row][site]][r]
+// slice:     vout[r][o]   = sum_l vin[l][o % rows_in] A[l][p][r], p = open ? o / rows_in : bit
+//
+// FP64 MFMA.  A workgroup owns CHAIN_ROWS rows x 16 columns: it lists its rows with p = 0 and then those
+// with p = 1, so that each 16-row tile takes one of the two matrices A[.][p][.] (at most one tile more than
+// the rows alone need), and its eight waves split l (unit u of 4 to wave u mod 8).  The vectors lie with the
+// rows together; a wave reads them in whole lines, CHAIN_PD units ahead, and picks its tiles' rows through
+// LDS of its own, without a barrier.  The partial tiles are summed in LDS in a fixed order.
+// Measured, 1000 strings at bond 256, a site: a thread a column with l in series 54 us; tiles read straight
+// from rows of vectors, a gather of 64-byte pieces with two units in flight, 24 us; this 21 us, of which
+// the MFMA of five tiles for 64 rows take 9.
 template <typename T>
-__global__ __launch_bounds__(256) void k_chain(const ChainTask* tasks, int ntasks) {
+__global__ __launch_bounds__(512) void k_chain(const ChainTask* tasks, int ntasks) {
+  constexpr int NTILE = CHAIN_ROWS / 16 + 1, PD = 4, NW = 8;
+  __shared__ int s_row[16 * NTILE];  // of the tiles' rows: the workgroup's row, or -1
+  __shared__ double2 sV[NW][2][4][CHAIN_ROWS];
+  __shared__ double2 sC[NW / 2][NTILE][16][17];
+  __shared__ int s_tiles[2];
   const int t = find_task(tasks, ntasks, (int)blockIdx.x, [](const ChainTask& x) { return x.block_begin; });
   const ChainTask& C = tasks[t];
   const int b = blockIdx.x - C.block_begin;
   if (b >= C.blocks) return;
-  const int rblocks = (C.cr + 255) / 256;
-  const int row = b / rblocks, r = (b % rblocks) * 256 + threadIdx.x;
-  if (row >= C.rows_out || r >= C.cr) return;
-  int src, p;
-  if (C.mode == 0) {
-    src = row;
-    p = C.bits[(size_t)row * C.n + C.site];
-  } else {
-    src = row % C.rows_in;
-    p = C.slice_bit < 0 ? row / C.rows_in : C.slice_bit;
+  const int cl = C.cl, cr = C.cr, rows_in = C.rows_in;
+  // blocks of the same rows 8 apart in launch order: on one XCD, which reads an eighth of the vectors, those
+  // it wrote at the site before, and all of A (the other way round: all vectors, an eighth of A)
+  const int rblocks = (C.rows_out + CHAIN_ROWS - 1) / CHAIN_ROWS;
+  const int r0 = b % rblocks * CHAIN_ROWS, j0 = b / rblocks * 16;
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, l16 = lane & 15,
+            k4 = lane >> 4;
+  const T* A = (const T*)C.A + min(j0 + l16, cr - 1);
+  static_assert(CHAIN_ROWS == 64, "a lane a row");
+  const int row = min(r0 + lane, C.rows_out - 1);
+  const double2* v = C.vin + (C.mode == 0 ? row : row % rows_in);
+  const int nu = (cl + 3) >> 2, nd = (nu - wave + NW - 1) / NW;
+  double2 x[PD][4], y[PD][2];  // a unit's vectors (a row a lane) and rows of A (p = 0, 1)
+  auto load = [&](int d, double2 (&xs)[4], double2 (&ys)[2]) __attribute__((always_inline)) {
+    const int l0 = 4 * (wave + NW * d);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) xs[i] = gld(v + (size_t)min(l0 + i, cl - 1) * rows_in);
+    const size_t at = (size_t)min(l0 + k4, cl - 1) * 2 * cr;
+    ys[0] = ld(A, at);
+    ys[1] = ld(A, at + cr);
+  };
+#pragma unroll
+  for (int d = 0; d < PD; ++d) load(d, x[d], y[d]);
+  if (wave == 0) {
+    const bool in = r0 + lane < C.rows_out;
+    int p = 0;
+    if (in) p = C.mode == 0 ? C.bits[(size_t)row * C.n + C.site] : (C.slice_bit < 0 ? row / rows_in : C.slice_bit);
+    const unsigned long long m0 = __ballot(in && p == 0), m1 = __ballot(in && p != 0);
+    const unsigned long long below = (1ull << lane) - 1;
+    const int t0 = (__popcll(m0) + 15) / 16 * 16;
+    for (int e = lane; e < 16 * NTILE; e += 64) s_row[e] = -1;
+    __builtin_amdgcn_wave_barrier();
+    if (in) s_row[p == 0 ? __popcll(m0 & below) : t0 + __popcll(m1 & below)] = lane;
+    if (lane == 0) {
+      s_tiles[0] = t0 / 16;
+      s_tiles[1] = t0 / 16 + (__popcll(m1) + 15) / 16;
+    }
   }
-  const T* A = (const T*)C.A;
-  const double2* v = C.vin + (size_t)src * C.cl;
-  double2 acc = make_double2(0, 0);
-  for (int l = 0; l < C.cl; ++l) acc = cfma(v[l], ld(A, ((size_t)l * 2 + p) * C.cr + r), acc);
-  C.vout[(size_t)row * C.cr + r] = acc;
+  __syncthreads();
+  const int n0 = __builtin_amdgcn_readfirstlane(s_tiles[0]);  // tiles with p = 0
+  const int nt = __builtin_amdgcn_readfirstlane(s_tiles[1]);  // all tiles
+  int pick[NTILE];  // past the end of a tile: any row, not stored
+#pragma unroll
+  for (int q = 0; q < NTILE; ++q) pick[q] = max(s_row[16 * q + l16], 0);
+  mfma_d4 re[NTILE], im[NTILE];
+#pragma unroll
+  for (int q = 0; q < NTILE; ++q) re[q] = im[q] = mfma_d4{0, 0, 0, 0};
+  // the loads are not conditional, past the end they repeat the last row: a wait for one unit's would
+  // otherwise be a wait for all that may have followed
+#pragma unroll 1
+  for (int d0 = 0; d0 < nd; d0 += PD) {
+#pragma unroll
+    for (int d = 0; d < PD; ++d) {
+      const int l0 = 4 * (wave + NW * (d0 + d));
+      double2 (*mine)[CHAIN_ROWS] = sV[wave][d & 1];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) mine[i][lane] = l0 + i < cl ? x[d][i] : make_double2(0, 0);
+      const double2 b0 = y[d][0], b1 = y[d][1];
+      load(d0 + d + PD, x[d], y[d]);
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      if (l0 < cl) {
+        double2 a[NTILE];
+#pragma unroll
+        for (int q = 0; q < NTILE; ++q) a[q] = mine[k4][pick[q]];
+#pragma unroll
+        for (int q = 0; q < NTILE; ++q)
+          if (q < nt) {
+            re[q] = mfma64(a[q].x, q < n0 ? b0.x : b1.x, re[q]);
+            im[q] = mfma64(a[q].x, q < n0 ? b0.y : b1.y, im[q]);
+          }
+#pragma unroll
+        for (int q = 0; q < NTILE; ++q)
+          if (q < nt) {
+            re[q] = mfma64(-a[q].y, q < n0 ? b0.y : b1.y, re[q]);
+            im[q] = mfma64(a[q].y, q < n0 ? b0.x : b1.x, im[q]);
+          }
+      }
+    }
+  }
+  // sums of the eight waves: the upper four to the lower, then those four; no barrier after a store
+  auto put = [&](int w) __attribute__((always_inline)) {
+#pragma unroll
+    for (int q = 0; q < NTILE; ++q)
+      if (q < nt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) sC[w][q][4 * i + k4][l16] = make_double2(re[q][i], im[q][i]);
+  };
+  if (wave >= 4) put(wave - 4);
+  __syncthreads();
+  if (wave < 4) {
+#pragma unroll
+    for (int q = 0; q < NTILE; ++q)
+      if (q < nt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const double2 x = sC[wave][q][4 * i + k4][l16];
+          re[q][i] += x.x;
+          im[q][i] += x.y;
+        }
+    put(wave);  // where this wave read
+  }
+  __syncthreads();
+  for (int e = tid; e < 256 * nt; e += 64 * NW) {
+    const int q = e >> 8, j = (e >> 4) & 15, i = e & 15, mine = s_row[16 * q + i];
+    if (mine < 0 || j0 + j >= cr) continue;
+    const double2 o = cadd(cadd(sC[0][q][i][j], sC[1][q][i][j]), cadd(sC[2][q][i][j], sC[3][q][i][j]));
+    gst(C.vout + (size_t)(j0 + j) * C.rows_out + r0 + mine, o);
+  }
 }
 
 hipError_t launch_chain(const ChainTask* d_tasks, int ntasks, int total_blocks, int fp32, hipStream_t s) {
   if (total_blocks <= 0) return hipSuccess;
   if (fp32)
-    hipLaunchKernelGGL(k_chain<float2>, dim3(total_blocks), dim3(256), 0, s, d_tasks, ntasks);
+    hipLaunchKernelGGL(k_chain<float2>, dim3(total_blocks), dim3(512), 0, s, d_tasks, ntasks);
   else
-    hipLaunchKernelGGL(k_chain<double2>, dim3(total_blocks), dim3(256), 0, s, d_tasks, ntasks);
+    hipLaunchKernelGGL(k_chain<double2>, dim3(total_blocks), dim3(512), 0, s, d_tasks, ntasks);
   return hipGetLastError();
 }
 
