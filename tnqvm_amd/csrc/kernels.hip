@@ -510,7 +510,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && TILED ? 4 : 2) void k_jacobi_ro
   double2* Y = TILED ? T.Yt : T.Y;
   const int ntc = T.ntc;
   const int tid = threadIdx.x;
-  const int wave = tid >> 6, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int l16 = lane & 15, k4 = lane >> 4;
   // element (row, col) of the row-major layout
   auto at = [&](int row, int col) -> size_t { return (size_t)row * ld + col; };
@@ -528,15 +528,16 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && TILED ? 4 : 2) void k_jacobi_ro
   const double2* ga = TILED ? Y + (size_t)ba * ntc * 256 + (l16 >> 2) * 64 + (wave & 3) * 16 + (l16 & 3) * 4 + k4 : Y;
   const double2* gb = TILED ? Y + (size_t)bb * ntc * 256 + (l16 >> 2) * 64 + (wave & 3) * 16 + (l16 & 3) * 4 + k4 : Y;
   constexpr int PD = NW == 4 ? 2 : 4;
-  auto ld_unit = [&](int d, double2& v0, double2& v1) {
-    const int col = 4 * (wave + NW * d) + k4, tile = (wave >> 2) + TS * d;
-    if (TILED ? tile < ntc : col < C) {
-      v0 = gld(TILED ? ga + (size_t)tile * 256 : Y + at(rowa, col));
-      v1 = gld(TILED ? gb + (size_t)tile * 256 : Y + at(rowb, col));
-    } else {
-      v0 = make_double2(0, 0);
-      v1 = make_double2(0, 0);
-    }
+  // The loads are not conditional, past the end they repeat the last tile or column: behind a load that may
+  // not have been issued, the wait for an older one is a wait for all.
+  auto ld_unit = [&](int d, double2& v0, double2& v1) __attribute__((always_inline)) {
+    const int col = min(4 * (wave + NW * d) + k4, C - 1), tile = min((wave >> 2) + TS * d, ntc - 1);
+    v0 = gld(TILED ? ga + (size_t)tile * 256 : Y + at(rowa, col));
+    v1 = gld(TILED ? gb + (size_t)tile * 256 : Y + at(rowb, col));
+  };
+  auto skip_unit = [&](int d) { return TILED && (wave >> 2) + TS * d >= ntc; };
+  auto unit = [&](int d, double2 v) __attribute__((always_inline)) {  // row-major: nothing past the columns
+    return TILED || 4 * (wave + NW * d) + k4 < C ? v : make_double2(0, 0);
   };
   // Complex products on real MFMA with three real products each instead of four:
   //  * diagonal tiles (Hermitian): Re = Ar Ar^T + Ai Ai^T, and Im = X - X^T with X = Ar Ai^T;
@@ -589,8 +590,9 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && TILED ? 4 : 2) void k_jacobi_ro
       for (int e0 = 0; e0 < nd; e0 += PD) {
 #pragma unroll
         for (int d = 0; d < PD; ++d) {
-          const double2 v0 = x0[d], v1 = x1[d];
+          const double2 v0 = unit(e0 + d, x0[d]), v1 = unit(e0 + d, x1[d]);
           ld_unit(e0 + d + PD, x0[d], x1[d]);
+          if (skip_unit(e0 + d)) continue;
           if (diag) {
             a00r = mfma64(v0.x, v0.x, a00r);
             a11r = mfma64(v1.x, v1.x, a11r);
@@ -628,9 +630,10 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && TILED ? 4 : 2) void k_jacobi_ro
       for (int e0 = 0; e0 < nd; e0 += PD) {
 #pragma unroll
         for (int d = 0; d < PD; ++d) {
-          const double2 v0 = x0[d], v1 = x1[d];
+          const double2 v0 = unit(e0 + d, x0[d]), v1 = unit(e0 + d, x1[d]);
           const float p0 = (float)v0.x, q0 = (float)v0.y, p1 = (float)v1.x, q1 = (float)v1.y;
           ld_unit(e0 + d + PD, x0[d], x1[d]);
+          if (skip_unit(e0 + d)) continue;
           if (diag) {
             b00r = __builtin_amdgcn_mfma_f32_16x16x4f32(p0, p0, b00r, 0, 0, 0);
             b11r = __builtin_amdgcn_mfma_f32_16x16x4f32(p1, p1, b11r, 0, 0, 0);
@@ -1143,7 +1146,7 @@ __global__ __launch_bounds__(256) void k_gemm(const GemmTask* tasks, int ntasks,
   const TB* B = (const TB*)T.B;
   const int sign_div = T.sign_div;
   const double kd0 = T.kd0, kd1 = T.kd1;
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int l16 = lane & 15, k4 = lane >> 4;
   // rows of A and columns of B of this lane; past the end: a repeat, not stored
   const int ia = min(i0 + l16, M - 1), ib = min(i0 + 16 + l16, M - 1), jb = min(j0 + l16, N - 1);
@@ -1153,30 +1156,34 @@ __global__ __launch_bounds__(256) void k_gemm(const GemmTask* tasks, int ntasks,
   const TB* pj = B + (OPB == 0 ? (size_t)jb : (size_t)(T.gatherB ? T.gatherB[jb] : jb) * ldb);
   const size_t sa = a_rows ? 1 : lda, sb = OPB == 0 ? ldb : 1;
   const int nu = (K + 3) >> 2, nd = (nu - wave + 3) >> 2;  // this wave's units wave, wave + 4, ...
+  // past the end of K a load repeats the last element: behind a load that may not have been issued, the wait
+  // for an older one is a wait for all
   auto load = [&](int d, double2& x0, double2& x1, double2& y) __attribute__((always_inline)) {
-    const int k = 4 * (wave + 4 * d) + k4, kc = min(k, K - 1);
+    const int kc = min(4 * (wave + 4 * d) + k4, K - 1);
     x0 = ld(pa, (size_t)kc * sa);
     x1 = ld(pb, (size_t)kc * sa);
     y = ld(pj, (size_t)kc * sb);
-    double f = k < K ? 1.0 : 0.0;
-    if (sign_div > 0) f *= ((kc / sign_div) & 1) ? kd1 : kd0;
-    if (k >= K || sign_div > 0) {
-      x0 = cscale(x0, f);
-      x1 = cscale(x1, f);
-    }
   };
   mfma_d4 re0 = {0, 0, 0, 0}, im0 = {0, 0, 0, 0}, re1 = {0, 0, 0, 0}, im1 = {0, 0, 0, 0};
   double2 x0[GEMM_PD], x1[GEMM_PD], y[GEMM_PD];
 #pragma unroll
-  for (int d = 0; d < GEMM_PD; ++d)
-    if (d < nd) load(d, x0[d], x1[d], y[d]);
+  for (int d = 0; d < GEMM_PD; ++d) load(d, x0[d], x1[d], y[d]);
 #pragma unroll 1
   for (int d0 = 0; d0 < nd; d0 += GEMM_PD) {
 #pragma unroll
     for (int d = 0; d < GEMM_PD; ++d) {
+      double2 a0 = x0[d], a1 = x1[d];
+      const double2 b = y[d];
+      load(d0 + d + GEMM_PD, x0[d], x1[d], y[d]);
       if (d0 + d < nd) {
-        const double2 a0 = x0[d], a1 = x1[d], b = y[d];
-        if (d0 + d + GEMM_PD < nd) load(d0 + d + GEMM_PD, x0[d], x1[d], y[d]);
+        const int k0 = 4 * (wave + 4 * (d0 + d));
+        if (k0 + 4 > K || sign_div > 0) {
+          const int k = k0 + k4;
+          double f = k < K ? 1.0 : 0.0;
+          if (sign_div > 0) f *= ((k / sign_div) & 1) ? kd1 : kd0;
+          a0 = cscale(a0, f);
+          a1 = cscale(a1, f);
+        }
         // conj(A) (OPA 1, 2): -a.y for a.y; conj(B) (OPB 2): -b.y for b.y
         const double a0y = OPA == 1 || OPA == 2 ? -a0.y : a0.y, a1y = OPA == 1 || OPA == 2 ? -a1.y : a1.y;
         const double by = OPB == 2 ? -b.y : b.y;
