@@ -110,10 +110,9 @@ __device__ __forceinline__ void lq_factor_panel(const LqTask& T, int k0, double2
 // T' = T (conjT = 0) or T^H (conjT = 1), W the reflector rows [k0, k1) of the panel at k0 (at most
 // LQB).  P = Y W^H (16 x LQB) by MFMA with the column range split over the 4 waves, Q = P T' with T'
 // staged in LDS, then Y -= Q W by MFMA, each wave owning whole 16-column tiles.  PD units of P and a
-// whole tile of the update are in flight; the loads of whole 16-column groups past the panel's own
-// columns, nearly all, are plain (no reflector starts there, no column is past the end).  With one
-// unit ahead and a branch around every load, a workgroup alone on its CU waited for one load latency
-// per 16 columns.  Run by teams of four waves (a workgroup of 256 threads is one team, one of 512
+// whole tile of the update are in flight.  No load is under a condition (behind a load that may not have
+// been issued, the wait for an older one is a wait for all): past the end they repeat the last group, and
+// the panel's own columns, where its reflectors start, and columns past the end are put right at use.  Run by teams of four waves (a workgroup of 256 threads is one team, one of 512
 // threads two, each with rows and LDS of its own).
 template <int PD>
 __device__ __forceinline__ void lq_apply_panel(const LqTask& T, int k0, int k1, double2* Y, size_t ly, int r0, int r1,
@@ -123,68 +122,63 @@ __device__ __forceinline__ void lq_apply_panel(const LqTask& T, int k0, int k1, 
   const double2* W0 = T.W0;
   const size_t ld = T.ld;
   const int C = T.cols;
-  const int tid = threadIdx.x & 255, wave = tid >> 6, lane = tid & 63;
+  const int tid = threadIdx.x & 255, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int l16 = lane & 15, k4 = lane >> 4;
-  // element w_j[col] of reflector j (support col >= j; head in W0, tail in M's row j).  A reflector
-  // past k1 repeats the last one: its rows and columns of T are zero.
-  auto wload = [&](int j, int g, int off) __attribute__((always_inline)) {  // 16-column group at k0 + 16 g
-    const int c0 = k0 + 16 * g, col = c0 + off;
-    const unsigned row = (unsigned)min(j, k1 - 1) * (unsigned)ld;
-    if (g > 0 && c0 + 16 <= C) return gld_at(M, row + col);
-    const int jc = min(j, k1 - 1), cc = min(col, C - 1);
-    const double2 v = gld_at(M, row + cc), h = gld_at(W0, jc);
-    const bool head = col == jc, zero = col < jc || col >= C;
-    return make_double2(zero ? 0.0 : (head ? h.x : v.x), zero ? 0.0 : (head ? h.y : v.y));
+  // a reflector past k1 repeats the last one: its rows and columns of T are zero
+  const int jl = min(k0 + l16, k1 - 1);
+  const unsigned wrow = (unsigned)jl * (unsigned)ld;
+  const double2 head = gld_at(W0, jl);  // of reflector k0 + l16
+  // element w_j[col] of reflector j (support col >= j; head in W0, tail in M's row j), M's element being v
+  auto own = [&](double2 v, double2 h, int j, int col) __attribute__((always_inline)) {
+    const bool is_head = col == j, zero = col < j || col >= C;
+    return make_double2(zero ? 0.0 : (is_head ? h.x : v.x), zero ? 0.0 : (is_head ? h.y : v.y));
   };
+  auto special = [&](int g) { return g == 0 || k0 + 16 * g + 16 > C; };
   // ---- P[i][j] = sum_c Y[r0+i][c] conj(w_j[c]); B operand: reflector k0 + l16 ----
   const unsigned yrow = (unsigned)min(r0 + l16, r1 - 1) * (unsigned)ly;  // a row past the end: a repeat, not stored
-  auto yload = [&](int g, int off) __attribute__((always_inline)) {
-    const int c0 = k0 + 16 * g, col = c0 + off;
-    if (c0 + 16 <= C) return gld_at(Y, yrow + col);
-    const double2 v = gld_at(Y, yrow + min(col, C - 1));
-    return make_double2(col < C ? v.x : 0.0, col < C ? v.y : 0.0);
-  };
   mfma_d4 pr = {0, 0, 0, 0}, pim = {0, 0, 0, 0};
   const int nt = (C - k0 + 15) >> 4;  // 16-column groups; this wave's unit of a group: 4 columns
-  const int uo = 4 * wave + k4;
+  const int uo = k0 + 4 * wave + k4;
   double2 a[PD], w[PD];
+  auto load = [&](int g, double2& y, double2& m) __attribute__((always_inline)) {
+    const unsigned col = min(uo + 16 * g, C - 1);
+    y = gld_at(Y, yrow + col);
+    m = gld_at(M, wrow + col);
+  };
 #pragma unroll
-  for (int d = 0; d < PD; ++d)
-    if (d < nt) {
-      a[d] = yload(d, uo);
-      w[d] = wload(k0 + l16, d, uo);
-    }
+  for (int d = 0; d < PD; ++d) load(d, a[d], w[d]);
 #pragma unroll 1
   for (int d0 = 0; d0 < nt; d0 += PD) {
 #pragma unroll
     for (int d = 0; d < PD; ++d) {
-      if (d0 + d < nt) {
-        const double2 x = a[d], y = w[d];
-        if (d0 + d + PD < nt) {
-          a[d] = yload(d0 + d + PD, uo);
-          w[d] = wload(k0 + l16, d0 + d + PD, uo);
-        }
-        // x conj(y): re = x.x y.x + x.y y.y, im = x.y y.x - x.x y.y
-        pr = mfma64(x.x, y.x, pr);
-        pim = mfma64(x.y, y.x, pim);
-        pr = mfma64(x.y, y.y, pr);
-        pim = mfma64(-x.x, y.y, pim);
-      }
+      const int g = d0 + d;
+      const double2 x = a[d];
+      double2 y = w[d];
+      load(g + PD, a[d], w[d]);
+      if (g >= nt) continue;
+      if (special(g)) y = own(y, head, jl, uo + 16 * g);
+      // x conj(y): re = x.x y.x + x.y y.y, im = x.y y.x - x.x y.y
+      pr = mfma64(x.x, y.x, pr);
+      pim = mfma64(x.y, y.x, pim);
+      pr = mfma64(x.y, y.y, pr);
+      pim = mfma64(-x.x, y.y, pim);
     }
   }
   // first tile of the update, while P is summed
   double2 tw[LQB / 4], ty[4];
-  unsigned ry[4];
+  unsigned ry[4], rw[LQB / 4];
 #pragma unroll
   for (int v = 0; v < 4; ++v) ry[v] = (unsigned)min(r0 + 4 * v + k4, r1 - 1) * (unsigned)ly;
-  auto tile = [&](int t) __attribute__((always_inline)) {
-    const int c = min(k0 + 16 * t + l16, C - 1);
 #pragma unroll
-    for (int kk = 0; kk < LQB / 4; ++kk) tw[kk] = wload(k0 + kk * 4 + k4, t, l16);  // B[k][c] = w_j[c]
+  for (int kk = 0; kk < LQB / 4; ++kk) rw[kk] = (unsigned)min(k0 + kk * 4 + k4, k1 - 1) * (unsigned)ld;
+  auto tile = [&](int t) __attribute__((always_inline)) {
+    const unsigned c = min(k0 + 16 * t + l16, C - 1);
+#pragma unroll
+    for (int kk = 0; kk < LQB / 4; ++kk) tw[kk] = gld_at(M, rw[kk] + c);  // B[k][c] = w_j[c]
 #pragma unroll
     for (int v = 0; v < 4; ++v) ty[v] = gld_at(Y, ry[v] + c);
   };
-  if (wave < nt) tile(wave);
+  tile(wave);
   for (int q = 0; q < 4; ++q) {
     if (wave == q) {
 #pragma unroll
@@ -224,7 +218,14 @@ __device__ __forceinline__ void lq_apply_panel(const LqTask& T, int k0, int k1, 
     for (int kk = 0; kk < LQB / 4; ++kk) cwv[kk] = tw[kk];
 #pragma unroll
     for (int v = 0; v < 4; ++v) cy[v] = ty[v];
-    if (t + 4 < nt) tile(t + 4);
+    tile(t + 4);
+    if (special(t)) {
+#pragma unroll
+      for (int kk = 0; kk < LQB / 4; ++kk) {
+        const double2 h = make_double2(__shfl(head.x, kk * 4 + k4), __shfl(head.y, kk * 4 + k4));
+        cwv[kk] = own(cwv[kk], h, min(k0 + kk * 4 + k4, k1 - 1), c);
+      }
+    }
     mfma_d4 dr = {0, 0, 0, 0}, di = {0, 0, 0, 0};
 #pragma unroll
     for (int kk = 0; kk < LQB / 4; ++kk) {
@@ -278,7 +279,7 @@ __global__ __launch_bounds__(256) void k_lq_update(const LqTask* tasks, int p) {
 // Tgt <- Tgt (I - W_p^H T_p^H W_p) for every panel p from the last to the first, on rows [16x, 16x +
 // 16) of Tgt: the rows are independent of each other, so one launch applies all panels, each
 // workgroup to its rows (one launch a panel left gaps of several us between launches of 7 to 20 us).
-__global__ __launch_bounds__(256) void k_lq_apply_q(const LqTask* tasks) {
+__global__ __launch_bounds__(256, 4) void k_lq_apply_q(const LqTask* tasks) {
   __shared__ double2 sP[LQB][LQB + 1];
   __shared__ double2 sQ[LQB][LQB + 1];
   __shared__ double2 sT[LQR][LQB + 1];
@@ -553,7 +554,7 @@ __global__ __launch_bounds__(512) void k_lq_step(const LqTask* tasks, int p) {
 }
 
 // Rows beyond panel p + 1 with the block reflector of panel p, 16 rows per workgroup
-__global__ __launch_bounds__(256) void k_lq_rest(const LqTask* tasks, int p) {
+__global__ __launch_bounds__(256, 4) void k_lq_rest(const LqTask* tasks, int p) {
   __shared__ double2 sP[LQB][LQB + 1];
   __shared__ double2 sQ[LQB][LQB + 1];
   __shared__ double2 sT[LQR][LQB + 1];
