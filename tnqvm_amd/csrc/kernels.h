@@ -118,11 +118,11 @@ struct GateTask {
 __host__ __device__ inline int small_rows(int r) { return r + (r & 1); }
 __host__ __device__ inline int small_stride(int c) { return (c <= 16 ? 16 : c <= 32 ? 32 : c <= 64 ? 64 : 128) + 1; }
 // complex128 elements of X (and of Y) that fit a workgroup's LDS, and the largest row count
-constexpr int SMALL_MAX_ROWS = 64;
+constexpr int SMALL_MAX_ROWS = 64, SMALL_MAX_COLS = 128;
 constexpr int SMALL_CAP = 64 * 65;
 constexpr int SMALL_CAP_LO = 32 * 33;  // variant of 256 threads, several workgroups per CU
 inline bool gate_small(int r, int c) {
-  return r <= SMALL_MAX_ROWS && c <= 128 && small_rows(r) * small_stride(c) <= SMALL_CAP;
+  return r <= SMALL_MAX_ROWS && c <= SMALL_MAX_COLS && small_rows(r) * small_stride(c) <= SMALL_CAP;
 }
 // lo: every task fits SMALL_CAP_LO
 // A noise channel of a small site (k_kraus_small): the same limits on its rows and columns.

@@ -7,12 +7,14 @@
 // took 0.3 to 0.9 ms.  Here theta', its rows and every intermediate stay in LDS, convergence is tested
 // on the device, and a wave is one launch.
 //
-// The SVD is the one-sided Jacobi of the general path on single rows: the rows of X = theta' (or
-// theta'^H) in circle order, r / 2 disjoint pairs a step.  A pair belongs to 16 lanes (one DPP row): they
-// form both squared norms and the inner product from the rows, rotate and write them back, so every angle
-// comes from the rows themselves and no Gram matrix is carried.  A step is bound by its chain (LDS read,
-// products, four DPP sums, the rotation, LDS write, barrier), and at 64 rows by FP64 issue of the one CU.
-// Measured, a wave: 13 us at bonds up to 4, 60 to 80 us up to 16, 320 to 465 us up to 32.
+// The SVD is an LQ and the one-sided Jacobi of the general path on single rows: the rows of L^H in circle
+// order, r / 2 disjoint pairs a step.  A pair belongs to 16 lanes (one DPP row): they form the inner product
+// from the rows, rotate and write them back, so every angle comes from the rows themselves and no Gram matrix
+// is carried.  A step is bound by its chain (LDS read, products, two DPP sums, the rotation, LDS write,
+// barrier: 1050 clocks up to 16 rows, 1200 at 32), and at 64 rows by LDS bandwidth and FP64 issue of the one
+// CU one after the other (2290).  Measured, random theta' (8 to 9 sweeps): 18 us at 4 x 4, 31 at 8 x 8, 68 at
+// 16 x 16, 160 at 32 x 32, 620 at 64 x 64; a line of 12 qubits whose waves are at most 64 x 64 took 9.6 ms
+// with the sweeps on the rows of theta' and norms formed at every step, 7.7 ms with these.
 #include <cfloat>
 #include <cstddef>
 
@@ -31,24 +33,100 @@ __device__ __forceinline__ double row16_sum(double v) {
   return dpp_add<0x140>(v);      // row_mirror
 }
 
+// X = L Q by Householder reflections from the right, X (r x c, r <= c, in Y) replaced by L^H: its first r
+// columns upper triangular, columns r .. 16 NJ - 1 (of the sweeps that follow) zero.  At a step every 16 lanes
+// form the reflector of row k from the row themselves and apply it to their rows below: one barrier a step,
+// the diagonal kept aside in d (LDS, r entries) because the others still read row k.
+template <int NT, int NC>
+__device__ __forceinline__ void lq_rows(double2* Y, int stride, int r, int c, int zero_to, double2* d) {
+  const int tid = threadIdx.x, group = tid >> 4, l16 = tid & 15;
+  for (int k = 0; k < r; ++k) {
+    const double2* yk = Y + k * stride;
+    const double2 head = yk[k];
+    double2 w[NC];
+    double tail = 0.0;
+#pragma unroll
+    for (int q = 0; q < NC; ++q) {
+      w[q] = yk[l16 + 16 * q];
+      if (l16 + 16 * q <= k) w[q] = make_double2(0, 0);
+      tail = fma(w[q].x, w[q].x, fma(w[q].y, w[q].y, tail));
+    }
+    tail = row16_sum(tail);
+    if (tail > 1e-290) {  // below: nothing to reflect that a double would show
+      // w = x + e norm e_k with e = head / |head|; x becomes -e norm, other rows y - (y w^H) w / (norm (norm + |head|))
+      const double a2 = cabs2(head), n2 = a2 + tail, norm = n2 * nr_rsq(n2);
+      const double ra = a2 > 1e-290 ? nr_rsq(a2) : 0.0, a = a2 * ra;
+      const double2 e = ra > 0.0 ? cscale(head, ra) : make_double2(1, 0);
+      const double scale = nr_rcp(norm * (norm + a));
+      const double2 wk = cscale(e, a + norm);
+#pragma unroll
+      for (int q = 0; q < NC; ++q)
+        if (l16 + 16 * q == k) w[q] = wk;
+      for (int i = k + 1 + group; i < r; i += NT / 16) {
+        double2* y = Y + i * stride + l16;
+        double2 v[NC], t = make_double2(0, 0);
+#pragma unroll
+        for (int q = 0; q < NC; ++q) {
+          v[q] = y[16 * q];
+          t = cfmac(w[q], v[q], t);
+        }
+        t = cscale(make_double2(row16_sum(t.x), row16_sum(t.y)), -scale);
+#pragma unroll
+        for (int q = 0; q < NC; ++q) y[16 * q] = cfma(t, w[q], v[q]);
+      }
+      if (tid == 0) d[k] = cscale(e, -norm);
+    } else if (tid == 0) {
+      d[k] = head;
+    }
+    __syncthreads();
+  }
+  for (int e = tid; e < r * zero_to; e += NT) {
+    const int i = e / zero_to, j = e - i * zero_to;
+    double2* at = Y + i * stride + j;
+    if (j < i) {
+      Y[j * stride + i] = cconj(*at);
+      *at = make_double2(0, 0);
+    } else if (j == i) {
+      *at = cconj(d[i]);
+    } else if (j >= r) {
+      *at = make_double2(0, 0);
+    }
+  }
+  __syncthreads();
+}
+
 // One-sided Jacobi on the rows of Y (nr even, stride elements apart, 16 NJ columns): sweeps until no pair's
-// relative inner product exceeds tol.  Returns the sweeps used; *flag (LDS) is 0 when converged.
+// relative inner product exceeds tol.  A pair a group: nr / 2 <= NT / 16.  The squared norms travel with the
+// rotations in n2 (LDS) and are formed from the rows again at every sweep, so the sweep that finds nothing to
+// rotate has tested the rows' own.  Blocks of two rows a group, four rotations a step with half the LDS
+// traffic, are on four waves instead of eight and no faster (64 rows: 2310 clocks a rotation's step for 2290).
+// Returns the sweeps used; *flag (LDS) is 0 when converged.
 template <int NT, int NJ>
 __device__ __forceinline__ int jacobi_rows(double2* Y, int stride, int nr, double tol, double floor2, int max_sweeps,
-                                           int* flag) {
+                                           int* flag, double* n2) {
   const int tid = threadIdx.x, group = tid >> 4, l16 = tid & 15;
   const double itol = 0.25 * tol, tol2 = tol * tol;
   int sweep = 0;
   for (; sweep < max_sweeps; ++sweep) {
     if (tid == 0) *flag = 0;
+    for (int i = group; i < nr; i += NT / 16) {
+      double a = 0.0;
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) a += cabs2(Y[i * stride + l16 + 16 * j]);
+      a = row16_sum(a);
+      if (l16 == 0) n2[i] = a;
+    }
     __syncthreads();
+    bool above = false;
+    // the rows of this group's pair: slots group and nr - 1 - group of the circle ordering
+    int ip = group, iq = nr - 1 - group;
     for (int step = 0; step < nr - 1; ++step) {
-      for (int p = group; p < nr / 2; p += NT / 16) {
-        double2* yp = Y + circle_slot(p, step, nr) * stride + l16;
-        double2* yq = Y + circle_slot(nr - 1 - p, step, nr) * stride + l16;
+      if (group < nr / 2) {
+        double2* yp = Y + ip * stride + l16;
+        double2* yq = Y + iq * stride + l16;
+        double alpha = n2[ip], beta = n2[iq];
         double2 a[NJ], b[NJ];
-        double alpha = 0.0, beta = 0.0;
-        double2 g = make_double2(0, 0);
+        double2 g = make_double2(0, 0), g1 = make_double2(0, 0);
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
           a[j] = yp[16 * j];
@@ -56,14 +134,12 @@ __device__ __forceinline__ int jacobi_rows(double2* Y, int stride, int nr, doubl
         }
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
-          alpha = fma(a[j].x, a[j].x, fma(a[j].y, a[j].y, alpha));
-          beta = fma(b[j].x, b[j].x, fma(b[j].y, b[j].y, beta));
-          g = cfmac(a[j], b[j], g);
+          if (j & 1) g1 = cfmac(a[j], b[j], g1);
+          else g = cfmac(a[j], b[j], g);
         }
-        alpha = row16_sum(alpha);
-        beta = row16_sum(beta);
+        if (NJ > 1) g = cadd(g, g1);
         g = make_double2(row16_sum(g.x), row16_sum(g.y));
-        if (alpha > floor2 && beta > floor2 && cabs2(g) > tol2 * (alpha * beta) && l16 == 0) *flag = 1;
+        above |= (alpha > floor2) & (beta > floor2) & (cabs2(g) > tol2 * (alpha * beta));
         double c;
         double2 tau;
         jacobi_rotation(alpha, beta, g, itol, floor2, c, tau);
@@ -74,10 +150,18 @@ __device__ __forceinline__ int jacobi_rows(double2* Y, int stride, int nr, doubl
             yp[16 * j] = cscale(cfma(nt, b[j], a[j]), c);
             yq[16 * j] = cscale(cfma(tau, a[j], b[j]), c);
           }
+          if (l16 == 0) {
+            n2[ip] = alpha;
+            n2[iq] = beta;
+          }
         }
       }
+      ip = ip == 0 ? 0 : (ip + 1 == nr ? 1 : ip + 1);
+      iq = iq + 1 == nr ? 1 : iq + 1;
       __syncthreads();
     }
+    if (above) *flag = 1;
+    __syncthreads();
     const int again = *flag;
     __syncthreads();
     if (!again) return sweep + 1;
@@ -86,14 +170,31 @@ __device__ __forceinline__ int jacobi_rows(double2* Y, int stride, int nr, doubl
 }
 
 template <int NT>
-__device__ __forceinline__ int jacobi_rows_n(double2* Y, int stride, int nr, double tol, double floor2, int max_sweeps,
-                                             int* flag) {
-  switch (stride >> 4) {
-    case 1: return jacobi_rows<NT, 1>(Y, stride, nr, tol, floor2, max_sweeps, flag);
-    case 2: return jacobi_rows<NT, 2>(Y, stride, nr, tol, floor2, max_sweeps, flag);
-    case 4: return jacobi_rows<NT, 4>(Y, stride, nr, tol, floor2, max_sweeps, flag);
-    default: return jacobi_rows<NT, 8>(Y, stride, nr, tol, floor2, max_sweeps, flag);
+__device__ __forceinline__ int jacobi_rows_n(double2* Y, int stride, int nr, int cols, double tol, double floor2,
+                                             int max_sweeps, int* flag, double* n2) {
+  switch (cols >> 4) {
+    case 1: return jacobi_rows<NT, 1>(Y, stride, nr, tol, floor2, max_sweeps, flag, n2);
+    case 2: return jacobi_rows<NT, 2>(Y, stride, nr, tol, floor2, max_sweeps, flag, n2);
+    case 4: return jacobi_rows<NT, 4>(Y, stride, nr, tol, floor2, max_sweeps, flag, n2);
+    default: return jacobi_rows<NT, 8>(Y, stride, nr, tol, floor2, max_sweeps, flag, n2);
   }
+}
+
+// L of X = L Q (r x c in Y) and Jacobi sweeps on the rows of L^H: rows sigma_j u_j^H, r columns, u_j the left
+// singular vectors of X.  On theta' of decaying spectra the sweeps on the rows of X itself were 11 to 13 at 32
+// and 64 rows (24 over ten decades), on L^H 8 to 9, on rows of r columns instead of c; the LQ costs the
+// barriers of half a sweep.
+template <int NT>
+__device__ __forceinline__ int svd_rows(double2* Y, int stride, int r, int c, double tol, double floor2,
+                                        int max_sweeps, int* flag, double* n2, double2* d) {
+  const int zero_to = small_stride(r) - 1;
+  switch (stride >> 4) {
+    case 1: lq_rows<NT, 1>(Y, stride, r, c, zero_to, d); break;
+    case 2: lq_rows<NT, 2>(Y, stride, r, c, zero_to, d); break;
+    case 4: lq_rows<NT, 4>(Y, stride, r, c, zero_to, d); break;
+    default: lq_rows<NT, 8>(Y, stride, r, c, zero_to, d); break;
+  }
+  return jacobi_rows_n<NT>(Y, stride, small_rows(r), zero_to, tol, floor2, max_sweeps, flag, n2);
 }
 
 // Norms of the rows of Y, sorted descending, ties by row: sig[rank], perm[rank].  NaN / Inf sorted as 0 and
@@ -128,30 +229,36 @@ __device__ __forceinline__ void sort_rows(const double2* Y, int stride, int r, i
   __syncthreads();
 }
 
-// One vector of X's other side per 16 lanes: u[i] = <y, X row i> * scale for the rows i = l16 + 16 q < r;
-// returns the sum of |u|^2 over all rows.  The lanes start at different columns: rows are a multiple of 256
-// bytes apart, the same column of 16 rows is one LDS bank (measured 27 of 320 us at 64 rows).
-__device__ __forceinline__ double other_side(const double2* X, const double2* y, int stride, int r, int c,
-                                             double scale, double2 (&u)[SMALL_MAX_ROWS / 16]) {
+// X's other side: u[j] = sum_i y_i X_ij for the columns j = l16 + 16 q < c, two vectors y per 16 lanes.
+__device__ __forceinline__ void other_side(const double2* X, const double2* y0, const double2* y1, int stride, int r,
+                                           int c, double2 (&u0)[SMALL_MAX_COLS / 16],
+                                           double2 (&u1)[SMALL_MAX_COLS / 16]) {
   const int l16 = threadIdx.x & 15;
+#pragma unroll
+  for (int q = 0; q < SMALL_MAX_COLS / 16; ++q) u0[q] = u1[q] = make_double2(0, 0);
+  for (int i = 0; i < r; ++i) {
+    const double2 v0 = y0[i], v1 = y1[i];
+#pragma unroll
+    for (int q = 0; q < SMALL_MAX_COLS / 16; ++q)
+      if (16 * q < c) {
+        const double2 x = X[i * stride + l16 + 16 * q];  // X is zero from c to the stride
+        u0[q] = cfma(v0, x, u0[q]);
+        u1[q] = cfma(v1, x, u1[q]);
+      }
+  }
+}
+// u <- u times `scale`, then to the length `len`
+__device__ __forceinline__ void to_length(double2 (&u)[SMALL_MAX_COLS / 16], double scale, double len) {
   double t = 0.0;
 #pragma unroll
-  for (int q = 0; q < SMALL_MAX_ROWS / 16; ++q) {
-    u[q] = make_double2(0, 0);
-    const int i = l16 + 16 * q;
-    if (i < r) {
-      const double2* x = X + i * stride;
-      double2 d = make_double2(0, 0);
-      int j = l16 % c;
-      for (int e = 0; e < c; ++e) {
-        d = cfmac(y[j], x[j], d);
-        j = j + 1 == c ? 0 : j + 1;
-      }
-      u[q] = cscale(d, scale);
-      t += cabs2(u[q]);
-    }
+  for (int q = 0; q < SMALL_MAX_COLS / 16; ++q) {
+    u[q] = cscale(u[q], scale);
+    t += cabs2(u[q]);
   }
-  return row16_sum(t);
+  t = row16_sum(t);
+  const double f = t > 0.0 ? len / sqrt(t) : 0.0;
+#pragma unroll
+  for (int q = 0; q < SMALL_MAX_COLS / 16; ++q) u[q] = cscale(u[q], f);
 }
 
 template <typename S, int NT, int CAP>
@@ -159,6 +266,7 @@ __global__ __launch_bounds__(NT) void k_gate_small(const GateTask* tasks) {
   __shared__ GateTask T;
   __shared__ double2 sX[CAP], sY[CAP];
   __shared__ double s_sig[SMALL_MAX_ROWS], s_scy[SMALL_MAX_ROWS], s_scw[SMALL_MAX_ROWS], s_inv[SMALL_MAX_ROWS];
+  __shared__ double2 s_d[SMALL_MAX_ROWS];
   __shared__ int s_perm[SMALL_MAX_ROWS];
   __shared__ double s_red[NT / 64];
   __shared__ int s_flag, s_K, s_bad;
@@ -215,9 +323,9 @@ __global__ __launch_bounds__(NT) void k_gate_small(const GateTask* tasks) {
   f2 = 0.0;
   for (int w = 0; w < NT / 64; ++w) f2 += s_red[w];
   __syncthreads();
-  const int sweeps = jacobi_rows_n<NT>(sY, stride, nr, T.tol, JAC_FLOOR2 * f2, T.max_sweeps, &s_flag);
+  const int sweeps = svd_rows<NT>(sY, stride, r, T.c, T.tol, JAC_FLOOR2 * f2, T.max_sweeps, &s_flag, s_inv, s_d);
   __syncthreads();
-  sort_rows<NT>(sY, stride, r, T.c, s_inv, s_sig, s_perm, &s_bad);
+  sort_rows<NT>(sY, stride, r, r, s_inv, s_sig, s_perm, &s_bad);
   // ---- truncation rule and factor scales, as k_select ----
   if (wave == 0) {
     const double sg = lane < r ? s_sig[lane] : 0.0;
@@ -231,11 +339,11 @@ __global__ __launch_bounds__(NT) void k_gate_small(const GateTask* tasks) {
     if (lane < r) {
       double gy = 0.0, gw = 0.0, is = 0.0;
       if (lane < K && sg > 1e-150) {
-        // exponents of f sigma: left aL, right 1 - aL; Y's side is the right one unless transposed
+        // exponents of f sigma: left aL, right 1 - aL; Y's side is the left one unless transposed
         const double sf = sg * f, h = sqrt(sf);
         const double left = T.absorb == 0 ? h : 1.0, right = T.absorb == 0 ? h : sf;
-        gy = (tr ? left : right) / sg;
-        gw = tr ? right : left;
+        gy = (tr ? right : left) / sg;
+        gw = tr ? left : right;
         is = 1.0 / sg;
       }
       s_scy[lane] = gy;
@@ -268,26 +376,31 @@ __global__ __launch_bounds__(NT) void k_gate_small(const GateTask* tasks) {
     return ((size_t)(2 * l + (i & 1)) * ki + (lk - l * ki)) * K + k;
   };
   // ---- factor on Y's side ----
-  for (int e = tid; e < K * T.c; e += NT) {
+  for (int e = tid; e < K * r; e += NT) {
     if (!tr) {
-      const int k = e / n, j = e - k * n;
-      st(Oj, (size_t)e, cscale(sY[s_perm[k] * stride + j], s_scy[k]));
-    } else {
       const int i = e / K, k = e - i * K;
       st(Oi, left(i, k), cscale(cconj(sY[s_perm[k] * stride + i]), s_scy[k]));
+    } else {
+      const int k = e / r, i = e - k * r;
+      st(Oj, (size_t)e, cscale(sY[s_perm[k] * stride + i], s_scy[k]));
     }
   }
-  // ---- the other factor: X's rows on the kept rows of Y, each vector scaled to its length ----
-  for (int k = group; k < K; k += NT / 16) {
-    double2 u[SMALL_MAX_ROWS / 16];
-    const double t = other_side(sX, sY + s_perm[k] * stride, stride, r, T.c, s_inv[k], u);
-    const double f = t > 0.0 ? s_scw[k] / sqrt(t) : 0.0;
+  // ---- the other factor: the kept rows of Y on X, each vector scaled to its length ----
+  for (int k0 = 2 * group; k0 < K; k0 += NT / 8) {
+    const int k1 = min(k0 + 1, K - 1);
+    double2 u[2][SMALL_MAX_COLS / 16];
+    other_side(sX, sY + s_perm[k0] * stride, sY + s_perm[k1] * stride, stride, r, T.c, u[0], u[1]);
 #pragma unroll
-    for (int q = 0; q < SMALL_MAX_ROWS / 16; ++q) {
-      const int i = l16 + 16 * q;
-      if (i >= r) continue;
-      if (!tr) st(Oi, left(i, k), cscale(u[q], f));
-      else st(Oj, (size_t)k * n + i, cscale(cconj(u[q]), f));
+    for (int h = 0; h < 2; ++h) {
+      const int k = h ? k1 : k0;
+      to_length(u[h], s_inv[k], s_scw[k]);
+#pragma unroll
+      for (int q = 0; q < SMALL_MAX_COLS / 16; ++q) {
+        const int j = l16 + 16 * q;
+        if (j >= T.c) continue;
+        if (!tr) st(Oj, (size_t)k * n + j, u[h][q]);
+        else st(Oi, left(j, k), cconj(u[h][q]));
+      }
     }
   }
 }
@@ -302,6 +415,31 @@ hipError_t launch_gate_small(const GateTask* d_tasks, int ntasks, int fp32, bool
     else hipLaunchKernelGGL((k_gate_small<double2, 512, SMALL_CAP>), dim3(ntasks), dim3(512), 0, s, d_tasks);
   }
   return hipGetLastError();
+}
+
+// One vector per 16 lanes: u[i] = <y, X row i> * scale for the rows i = l16 + 16 q < r; returns the sum of |u|^2
+// over all rows.  The lanes start at different columns, for rows that start in the same LDS bank.
+__device__ __forceinline__ double other_rows(const double2* X, const double2* y, int stride, int r, int c,
+                                             double scale, double2 (&u)[SMALL_MAX_ROWS / 16]) {
+  const int l16 = threadIdx.x & 15;
+  double t = 0.0;
+#pragma unroll
+  for (int q = 0; q < SMALL_MAX_ROWS / 16; ++q) {
+    u[q] = make_double2(0, 0);
+    const int i = l16 + 16 * q;
+    if (i < r) {
+      const double2* x = X + i * stride;
+      double2 d = make_double2(0, 0);
+      int j = l16 % c;
+      for (int e = 0; e < c; ++e) {
+        d = cfmac(y[j], x[j], d);
+        j = j + 1 == c ? 0 : j + 1;
+      }
+      u[q] = cscale(d, scale);
+      t += cabs2(u[q]);
+    }
+  }
+  return row16_sum(t);
 }
 
 // ------------------------------------------------------------------ noise channels of small sites
@@ -349,7 +487,7 @@ __global__ __launch_bounds__(NT) void k_kraus_small(const KrausTask* tasks) {
     }
   }
   __syncthreads();
-  const int sweeps = jacobi_rows_n<NT>(sY, stride, nr, T.tol, 0.0, T.max_sweeps, &s_flag);
+  const int sweeps = jacobi_rows_n<NT>(sY, stride, nr, stride - 1, T.tol, 0.0, T.max_sweeps, &s_flag, s_tmp);
   __syncthreads();
   sort_rows<NT>(sY, stride, r, c, s_tmp, s_sig, s_perm, &s_bad);
   if (wave == 0) {  // kept rows, as k_select's keep_rule
@@ -387,7 +525,7 @@ __global__ __launch_bounds__(NT) void k_kraus_small(const KrausTask* tasks) {
   for (int j = group; j < K; j += NT / 16) {
     const double sg = s_sig[j];
     double2 u[SMALL_MAX_ROWS / 16];
-    const double t = other_side(sX, sY + s_perm[j] * stride, stride, r, c, sg > 1e-150 ? 1.0 / sg : 0.0, u);
+    const double t = other_rows(sX, sY + s_perm[j] * stride, stride, r, c, sg > 1e-150 ? 1.0 / sg : 0.0, u);
     const double f = t > 0.0 ? sg / sqrt(t) : 0.0;
 #pragma unroll
     for (int q = 0; q < SMALL_MAX_ROWS / 16; ++q) {
