@@ -764,7 +764,7 @@ int run_wave_general(hipmps_engine E, std::vector<WaveItem>& items, const std::f
   // sums; per sweep the counts (2N ints), and N ints, all zeroed at the start
   const size_t res_bytes = align_up(N * sizeof(int)) + align_up(WS_N * N * sizeof(double));
   const size_t fro_bytes = align_up((size_t)(1 + FRO_BLOCKS) * N * sizeof(double));
-  const size_t cnt_bytes = align_up(((size_t)2 * E->max_sweeps + 1) * N * sizeof(int));
+  const size_t cnt_bytes = align_up((size_t)2 * E->max_sweeps * N * sizeof(int));
   RC_TRY(E->small.ensure(res_bytes + fro_bytes + cnt_bytes));
   int* d_K = (int*)E->small.p;
   double* d_w = (double*)((char*)E->small.p + align_up(N * sizeof(int)));
@@ -987,7 +987,7 @@ int run_wave_general(hipmps_engine E, std::vector<WaveItem>& items, const std::f
   if (n64 > 0) HIP_TRY(launch_theta(dth, n64, tile_acc[0], 0, st));
   if (N - n64 > 0) HIP_TRY(launch_theta(dth + n64, N - n64, tile_acc[1], 1, st));
   HIP_TRY(launch_jacobi_prep(dsp, djt, N, max_rpad, max_c, st));
-  HIP_TRY(launch_fro2(dsp, djt, d_fro2 + N, d_counts + (size_t)2 * E->max_sweeps * N, N, st));
+  HIP_TRY(launch_fro2(dsp, djt, d_fro2 + N, N, st));
   if (E->timing) HIP_TRY(hipEventRecord(E->ev[6], st));
   // LQ lanes: with many items, contiguous slices of the LQ task arrays run their panel
   // sequences on separate streams, so that one slice's launch tails overlap another's work

@@ -235,11 +235,10 @@ hipError_t launch_jacobi_prep(const SplitTask* d_split, const JacTask* d_jac, in
 // (1e-15)^2: a row whose norm is below 1e-15 ||X||_F lies under FP64 resolution of any result
 // computed from X, so the relative convergence test has no meaning for it
 constexpr double JAC_FLOOR2 = 1e-30;
-// *jt[t].fro2 = ||theta'_t||_F^2 (= ||X||_F^2 = ||R2||_F^2): FRO_BLOCKS partial sums per task in `part`, added
-// in order by the last workgroup of the task to finish (`done`: a zeroed int per task)
+// *jt[t].fro2 = ||theta'_t||_F^2 (= ||X||_F^2 = ||R2||_F^2): FRO_BLOCKS partial sums per task in `part`, then added
+// in order
 constexpr int FRO_BLOCKS = 32;
-hipError_t launch_fro2(const SplitTask* d_split, const JacTask* d_jac, double* part, int* done, int ntasks,
-                       hipStream_t s);
+hipError_t launch_fro2(const SplitTask* d_split, const JacTask* d_jac, double* part, int ntasks, hipStream_t s);
 // One round of sweep `sweep`.  A task whose previous sweep (not a gram32 one) rotated nothing has converged
 // and its workgroups return at once, so that a sweep can be queued before the host has seen the last one.
 hipError_t launch_jacobi_round(const JacTask* d_tasks, int ntasks, int total_pairs, int sweep, int round,

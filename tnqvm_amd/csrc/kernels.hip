@@ -768,9 +768,10 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && TILED ? 4 : 2) void k_jacobi_ro
 }
 
 // Bound by the read of theta'; one workgroup a task took 2.5 ms at 1536 x 1536 and 220 us a wave of 512 x 512.
-__global__ __launch_bounds__(256) void k_fro2(const SplitTask* sp, const JacTask* jt, double* part, int* done) {
+// The partial sums are added by a launch of their own: the last workgroup to finish doing so, found by a
+// device-scope atomic, made every workgroup write back its XCD's L2 (126 us a wave of an uneven batch).
+__global__ __launch_bounds__(256) void k_fro2(const SplitTask* sp, double* part) {
   __shared__ double red[4];
-  __shared__ int last;
   const SplitTask& S = sp[blockIdx.y];
   const size_t n = (size_t)S.m * S.n;
   const double2* x = S.theta;
@@ -779,22 +780,21 @@ __global__ __launch_bounds__(256) void k_fro2(const SplitTask* sp, const JacTask
   a = wave_sum(a);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = a;
   __syncthreads();
-  double* mine = part + (size_t)blockIdx.y * FRO_BLOCKS;
-  if (threadIdx.x == 0) {
-    __hip_atomic_store(mine + blockIdx.x, (red[0] + red[1]) + (red[2] + red[3]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    last = __hip_atomic_fetch_add(done + blockIdx.y, 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == FRO_BLOCKS - 1;
-  }
-  __syncthreads();
-  if (!last || threadIdx.x != 0) return;
-  double t = 0.0;
-  for (int b = 0; b < FRO_BLOCKS; ++b) t += __hip_atomic_load(mine + b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  *jt[blockIdx.y].fro2 = t;
+  if (threadIdx.x == 0) part[(size_t)blockIdx.y * FRO_BLOCKS + blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);
 }
 
-hipError_t launch_fro2(const SplitTask* d_split, const JacTask* d_jac, double* part, int* done, int ntasks,
-                       hipStream_t s) {
+__global__ __launch_bounds__(256) void k_fro2_sum(const JacTask* jt, const double* part, int ntasks) {
+  const int t = blockIdx.x * 256 + threadIdx.x;
+  if (t >= ntasks) return;
+  double a = 0.0;
+  for (int b = 0; b < FRO_BLOCKS; ++b) a += part[(size_t)t * FRO_BLOCKS + b];
+  *jt[t].fro2 = a;
+}
+
+hipError_t launch_fro2(const SplitTask* d_split, const JacTask* d_jac, double* part, int ntasks, hipStream_t s) {
   if (ntasks <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_fro2, dim3(FRO_BLOCKS, ntasks), dim3(256), 0, s, d_split, d_jac, part, done);
+  hipLaunchKernelGGL(k_fro2, dim3(FRO_BLOCKS, ntasks), dim3(256), 0, s, d_split, part);
+  hipLaunchKernelGGL(k_fro2_sum, dim3((ntasks + 255) / 256), dim3(256), 0, s, d_jac, part, ntasks);
   return hipGetLastError();
 }
 
