@@ -1967,15 +1967,15 @@ int trace_products(hipmps_engine E, const std::vector<const double2*>& A, const 
 
 // Values of `m` diagonals at once on a state of small bonds (k_env_chain), when that is estimated to take
 // less than the sweeps of products launched one by one that they replace (`sweeps` of them): a step of a
-// site takes about 1000 clocks and 20 per contraction index and 256 elements, and 512 workgroups run at a
-// time; a sweep's two products a site take 10 us.
+// site takes about 1000 clocks and 40 per contraction index, and 512 workgroups run at a time; a sweep's two
+// products a site take 10 us.
 bool chain_fits(const hipmps_state_s* s, size_t m, size_t sweeps) {
   double clocks = 0.0;
   for (int k = 0; k < s->n; ++k) {
     const int cl = s->chi[k], cr = s->chi[k + 1];
     if (cl > CHAIN_MAX_BOND || cr > CHAIN_MAX_BOND) return false;
     const int steps = (2 * s->kap[k] + chain_slots(cl, cr) - 1) / chain_slots(cl, cr);
-    clocks += steps * (1000.0 + 20.0 * cl * ((cl * cr + 255) / 256 + (cr * cr + 255) / 256)) + 1500.0;
+    clocks += steps * (1000.0 + 20.0 * cl * 2) + 1500.0;
   }
   return clocks * (double)((m + 511) / 512) < 24000.0 * s->n * sweeps;
 }

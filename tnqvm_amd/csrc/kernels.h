@@ -154,11 +154,11 @@ struct ChainSite {
   const void* A;  // cl x 2 x kap x cr
   int cl, cr, kap, pad;
 };
-constexpr int CHAIN_MAX_BOND = 32;
+constexpr int CHAIN_MAX_BOND = 32, CHAIN_THREADS = 1024;
 // the s of a site that a step of the chain takes side by side
 __host__ __device__ inline int chain_slots(int cl, int cr) {
   const int w = cl > cr ? cl * cr : cr * cr;
-  return w > 128 ? 1 : (256 / w < 16 ? 256 / w : 16);
+  return w > CHAIN_THREADS / 2 ? 1 : (CHAIN_THREADS / w < 16 ? CHAIN_THREADS / w : 16);
 }
 hipError_t launch_env_chain(const ChainSite* d_sites, int n, const double* d_diags, double* d_out, int nchains,
                             int fp32, hipStream_t s);

@@ -585,8 +585,8 @@ hipError_t launch_zero_state(void* const* sites, int n, int fp32, hipStream_t s)
 // string -- is a workgroup of the same launch.  A step takes as many s side by side as fit the workgroup's
 // threads (chain_slots); the next A_s are read while these are used.
 template <typename S>
-__global__ __launch_bounds__(256) void k_env_chain(const ChainSite* sites, int n, const double* diags, double* out) {
-  constexpr int B = CHAIN_MAX_BOND, Q = B * B / 256;
+__global__ __launch_bounds__(CHAIN_THREADS) void k_env_chain(const ChainSite* sites, int n, const double* diags, double* out) {
+  constexpr int B = CHAIN_MAX_BOND, NT = CHAIN_THREADS, Q = B * B / NT;
   __shared__ double2 sE[B * (B + 1)], sA[B * (B + 1)], sX[B * (B + 1)];
   const int tid = threadIdx.x;
   const double* diag = diags + (size_t)blockIdx.x * 2 * n;
@@ -605,10 +605,10 @@ __global__ __launch_bounds__(256) void k_env_chain(const ChainSite* sites, int n
     int al[Q], ar[Q];  // this thread's elements (l, r) of A_s and X, and (i, j) of the result
 #pragma unroll
     for (int q = 0; q < Q; ++q) {
-      al[q] = (i0 + 256 * q) / cr;
-      ar[q] = (i0 + 256 * q) - al[q] * cr;
+      al[q] = (i0 + NT * q) / cr;
+      ar[q] = (i0 + NT * q) - al[q] * cr;
     }
-    auto has = [&](int q, int count) { return on && (q == 0 || slots == 1) && i0 + 256 * q < count; };
+    auto has = [&](int q, int count) { return on && (q == 0 || slots == 1) && i0 + NT * q < count; };
     double2 acc[Q], next[Q];
 #pragma unroll
     for (int q = 0; q < Q; ++q) acc[q] = make_double2(0, 0);
@@ -626,7 +626,7 @@ __global__ __launch_bounds__(256) void k_env_chain(const ChainSite* sites, int n
       const int s = sb + slot;
 #pragma unroll
       for (int q = 0; q < Q; ++q)
-        if (has(q, na)) sA[slot * na + i0 + 256 * q] = next[q];
+        if (has(q, na)) sA[slot * na + i0 + NT * q] = next[q];
       __syncthreads();
       if (sb + slots < s1) fetch(s + slots);
 #pragma unroll
@@ -634,7 +634,7 @@ __global__ __launch_bounds__(256) void k_env_chain(const ChainSite* sites, int n
         if (has(q, na)) {
           double2 x = make_double2(0, 0);
           for (int l = 0; l < cl; ++l) x = cfma(sE[al[q] * cl + l], eA[l * cr + ar[q]], x);
-          eX[i0 + 256 * q] = x;
+          eX[i0 + NT * q] = x;
         }
       __syncthreads();
       const double d = s < kap ? dg[0] : dg[1];
@@ -659,7 +659,7 @@ __global__ __launch_bounds__(256) void k_env_chain(const ChainSite* sites, int n
     } else {
 #pragma unroll
       for (int q = 0; q < Q; ++q)
-        if (has(q, ne)) sE[i0 + 256 * q] = acc[q];
+        if (has(q, ne)) sE[i0 + NT * q] = acc[q];
     }
     __syncthreads();
   }
@@ -669,8 +669,8 @@ __global__ __launch_bounds__(256) void k_env_chain(const ChainSite* sites, int n
 hipError_t launch_env_chain(const ChainSite* d_sites, int n, const double* d_diags, double* d_out, int nchains,
                             int fp32, hipStream_t s) {
   if (nchains <= 0) return hipSuccess;
-  if (fp32) hipLaunchKernelGGL(k_env_chain<float2>, dim3(nchains), dim3(256), 0, s, d_sites, n, d_diags, d_out);
-  else hipLaunchKernelGGL(k_env_chain<double2>, dim3(nchains), dim3(256), 0, s, d_sites, n, d_diags, d_out);
+  if (fp32) hipLaunchKernelGGL(k_env_chain<float2>, dim3(nchains), dim3(CHAIN_THREADS), 0, s, d_sites, n, d_diags, d_out);
+  else hipLaunchKernelGGL(k_env_chain<double2>, dim3(nchains), dim3(CHAIN_THREADS), 0, s, d_sites, n, d_diags, d_out);
   return hipGetLastError();
 }
 
