@@ -761,7 +761,7 @@ int run_wave_general(hipmps_engine E, std::vector<WaveItem>& items, const std::f
   RC_TRY(E->ws.ensure(off));
   char* ws = (char*)E->ws.p;
   // small: K (N ints) and wstats (WS_N doubles per item), read back together; ||X||_F^2 and its partial
-  // sums; per sweep the counts (2N ints), and N ints, all zeroed at the start
+  // sums; per sweep the counts (2N ints), zeroed at the start
   const size_t res_bytes = align_up(N * sizeof(int)) + align_up(WS_N * N * sizeof(double));
   const size_t fro_bytes = align_up((size_t)(1 + FRO_BLOCKS) * N * sizeof(double));
   const size_t cnt_bytes = align_up((size_t)2 * E->max_sweeps * N * sizeof(int));
@@ -774,7 +774,8 @@ int run_wave_general(hipmps_engine E, std::vector<WaveItem>& items, const std::f
   size_t desc_bytes = align_up(N * sizeof(ThetaTask)) + align_up(N * sizeof(SplitTask)) +
                       align_up(N * sizeof(JacTask)) + align_up(N * sizeof(GemmTask)) +
                       align_up(2 * N * sizeof(LqTask)) + align_up(3 * N * sizeof(TriTask)) +
-                      align_up(N * sizeof(double)) + 2 * align_up(N * sizeof(JacTask));
+                      align_up(N * sizeof(double)) + 2 * align_up(N * sizeof(JacTask)) +
+                      align_up(2 * N * sizeof(SwapTask));
   RC_TRY(E->desc.ensure(desc_bytes));
   // host staging: descriptors | active Jacobi lists of the last two sweeps queued | counts | results
   const size_t stage_bytes = desc_bytes + 2 * align_up(N * sizeof(JacTask)) + cnt_bytes + res_bytes;
@@ -791,6 +792,7 @@ int run_wave_general(hipmps_engine E, std::vector<WaveItem>& items, const std::f
   // Jacobi tasks of X (hjt: k_jacobi_prep), of the sweeps (hjs: R2 of LQ items, tiled), and a region for
   // the sweeps' active lists
   JacTask* hjs = (JacTask*)((char*)hcut + align_up(N * sizeof(double)));
+  SwapTask* hsw = (SwapTask*)((char*)hjs + 2 * align_up(N * sizeof(JacTask)));  // to and from the purified left sites
   char* dd = (char*)E->desc.p;
   ThetaTask* dth = (ThetaTask*)dd;
   SplitTask* dsp = (SplitTask*)(dd + align_up(N * sizeof(ThetaTask)));
@@ -801,6 +803,7 @@ int run_wave_general(hipmps_engine E, std::vector<WaveItem>& items, const std::f
   const double* dcut = (const double*)((char*)dtr + align_up(3 * N * sizeof(TriTask)));
   JacTask* djs = (JacTask*)((char*)dcut + align_up(N * sizeof(double)));
   JacTask* dja = (JacTask*)((char*)djs + align_up(N * sizeof(JacTask)));
+  const SwapTask* dsw = (const SwapTask*)((char*)dja + align_up(N * sizeof(JacTask)));
 
   // group boundaries
   int n64 = 0;
@@ -975,14 +978,22 @@ int run_wave_general(hipmps_engine E, std::vector<WaveItem>& items, const std::f
     hipLaunchKernelGGL(k_stage_delay, dim3(1), dim3(64), 0, st, E->stage_delay_ticks);
     HIP_TRY(hipGetLastError());
   }
+  // purified left sites, [l][p][k][m] -> [l][k][p][m] ahead of theta and [l][k][p][K] -> [l][p][k][K] after
+  int nsw = 0;
+  size_t sw_elems = 0;
+  for (int q = 0; q < N; ++q) {
+    const auto& it = items[q];
+    if (it.ki <= 1) continue;
+    const int L = it.s->chi[it.i];
+    hsw[nsw] = {it.old_i, ws + it.off_pin, nullptr, L, 2, it.ki, it.cm, it.fp32};
+    hsw[N + nsw++] = {ws + it.off_pout, it.s->sites[it.i].p, d_K + q, L, it.ki, 2, it.kub, it.fp32};
+    sw_elems = std::max(sw_elems, (size_t)L * 2 * it.ki * std::max(it.cm, it.kub));
+  }
   HIP_TRY(hipMemcpyAsync(dd, hd, desc_bytes, hipMemcpyHostToDevice, st));
   HIP_TRY(hipMemsetAsync(d_counts, 0, cnt_bytes, st));
 
   if (E->timing) HIP_TRY(hipEventRecord(E->ev[0], st));
-  // purified left sites: Kraus leg next to the left bond, [l][p][k][m] -> [l][k][p][m]
-  for (auto& it : items)
-    if (it.ki > 1)
-      HIP_TRY(launch_swap_mid(it.old_i, ws + it.off_pin, it.s->chi[it.i], 2, it.ki, it.cm, nullptr, it.fp32, st));
+  HIP_TRY(launch_swap_many(dsw, nsw, sw_elems, st));
   // ---- theta ----
   if (n64 > 0) HIP_TRY(launch_theta(dth, n64, tile_acc[0], 0, st));
   if (N - n64 > 0) HIP_TRY(launch_theta(dth + n64, N - n64, tile_acc[1], 1, st));
@@ -1204,13 +1215,7 @@ int run_wave_general(hipmps_engine E, std::vector<WaveItem>& items, const std::f
     if (n64 > 0) HIP_TRY(launch_normalize(dsp, n64, mk64, 0, st));
     if (N - n64 > 0) HIP_TRY(launch_normalize(dsp + n64, N - n64, mk32, 1, st));
   }
-  // purified left sites back to [l][p][k][K]
-  for (int q = 0; q < N; ++q) {
-    auto& it = items[q];
-    if (it.ki > 1)
-      HIP_TRY(launch_swap_mid(ws + it.off_pout, it.s->sites[it.i].p, it.s->chi[it.i], it.ki, 2, it.kub, d_K + q,
-                              it.fp32, st));
-  }
+  HIP_TRY(launch_swap_many(dsw + N, nsw, sw_elems, st));
   // results
   const int* hK = (const int*)((char*)hcounts + cnt_bytes);
   const double* hw = (const double*)((const char*)hK + align_up(N * sizeof(int)));

@@ -319,6 +319,13 @@ hipError_t launch_rdm_scatter(const double2* E, double2* out, const RdmPerm& P, 
 // ---- purified sites (Kraus leg), kraus.hip ------------------------------------------------
 // dst[l][b][a][m] = src[l][a][b][m] for m < M (M = *m_dyn when m_dyn is not null, at most
 // m_max); element type complex128 (fp32 = 0) or complex64.
+struct SwapTask {
+  const void* src;   // [L][A][B][m]
+  void* dst;         // [L][B][A][m]
+  const int* m_dyn;  // m, or null: m_max
+  int L, A, B, m_max, fp32;
+};
+hipError_t launch_swap_many(const SwapTask* d_tasks, int ntasks, size_t max_elems, hipStream_t s);
 hipError_t launch_swap_mid(const void* src, void* dst, int L, int A, int B, int m_max, const int* m_dyn,
                            int fp32, hipStream_t s);
 // X[k * M + o][(l * 2 + p) * cr + r] = sum_p' K_o[p][p'] A[l][p'][k][r] for the site A
