@@ -116,7 +116,7 @@ __device__ __forceinline__ void lq_factor_panel(const LqTask& T, int k0, double2
 // threads two, each with rows and LDS of its own).
 template <int PD>
 __device__ __forceinline__ void lq_apply_panel(const LqTask& T, int k0, int k1, double2* Y, size_t ly, int r0, int r1,
-                                               int conjT, double2 (*sP)[LQB + 1], double2 (*sQ)[LQB + 1],
+                                               int conjT, double2 (*sP)[LQR][LQB + 1], double2 (*sQ)[LQB + 1],
                                                double2 (*sT)[LQB + 1]) {
   const double2* M = T.M;
   const double2* W0 = T.W0;
@@ -124,6 +124,11 @@ __device__ __forceinline__ void lq_apply_panel(const LqTask& T, int k0, int k1, 
   const int C = T.cols;
   const int tid = threadIdx.x & 255, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int l16 = lane & 15, k4 = lane >> 4;
+  {  // T', wanted after P
+    const double2* Tp = T.T + (size_t)(k0 / LQB) * LQB * LQB;
+    const int i = tid >> 4, j = tid & 15;
+    sT[i][j] = conjT ? cconj(gld(Tp + j * LQB + i)) : gld(Tp + i * LQB + j);
+  }
   // a reflector past k1 repeats the last one: its rows and columns of T are zero
   const int jl = min(k0 + l16, k1 - 1);
   const unsigned wrow = (unsigned)jl * (unsigned)ld;
@@ -179,26 +184,22 @@ __device__ __forceinline__ void lq_apply_panel(const LqTask& T, int k0, int k1, 
     for (int v = 0; v < 4; ++v) ty[v] = gld_at(Y, ry[v] + c);
   };
   tile(wave);
-  for (int q = 0; q < 4; ++q) {
-    if (wave == q) {
 #pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        double2 e = make_double2(pr[v], pim[v]);
-        if (q) e = cadd(e, sP[4 * v + k4][l16]);
-        sP[4 * v + k4][l16] = e;
-      }
-    }
-    __syncthreads();
-  }
+  for (int v = 0; v < 4; ++v) sP[wave][4 * v + k4][l16] = make_double2(pr[v], pim[v]);
+  __syncthreads();
   // ---- Q = P T' (16 x LQB) ----
   {
-    const double2* Tp = T.T + (size_t)(k0 / LQB) * LQB * LQB;
     const int i = tid >> 4, j = tid & 15;
-    sT[i][j] = conjT ? cconj(gld(Tp + j * LQB + i)) : gld(Tp + i * LQB + j);
+    double2 p[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) p[q] = sP[q][i][j];
+    const double2 sum = cadd(cadd(p[0], p[1]), cadd(p[2], p[3]));
+    __syncthreads();
+    sP[0][i][j] = sum;
     __syncthreads();
     double2 acc = make_double2(0, 0);
 #pragma unroll 4
-    for (int m = 0; m < LQB; ++m) acc = cfma(sP[i][m], sT[m][j], acc);
+    for (int m = 0; m < LQB; ++m) acc = cfma(sP[0][i][m], sT[m][j], acc);
     sQ[i][j] = acc;
   }
   __syncthreads();
@@ -257,7 +258,7 @@ __global__ __launch_bounds__(256) void k_lq_panel0(const LqTask* tasks) {
 // panel p + 1, [k1, k1 + LQB), updates them and then factors them; workgroup (x > 0, task)
 // owns rows [k1 + LQB + 16 (x - 1), + 16).
 __global__ __launch_bounds__(256) void k_lq_update(const LqTask* tasks, int p) {
-  __shared__ double2 sP[LQB][LQB + 1];
+  __shared__ double2 sP[4][LQR][LQB + 1];
   __shared__ double2 sQ[LQB][LQB + 1];
   __shared__ double2 sT[LQR][LQB + 1];
   const LqTask& T = tasks[blockIdx.y];
@@ -268,7 +269,7 @@ __global__ __launch_bounds__(256) void k_lq_update(const LqTask* tasks, int p) {
     if (k1 >= T.rows) return;
     const int e1 = min(k1 + LQB, T.rows);
     lq_apply_panel<4>(T, k0, k1, T.M, T.ld, k1, e1, 0, sP, sQ, sT);
-    lq_factor_panel(T, k1, sP, sQ);
+    lq_factor_panel(T, k1, sP[0], sQ);
     return;
   }
   const int r0 = k1 + LQB + LQR * ((int)blockIdx.x - 1);
@@ -280,7 +281,7 @@ __global__ __launch_bounds__(256) void k_lq_update(const LqTask* tasks, int p) {
 // 16) of Tgt: the rows are independent of each other, so one launch applies all panels, each
 // workgroup to its rows (one launch a panel left gaps of several us between launches of 7 to 20 us).
 __global__ __launch_bounds__(256, 4) void k_lq_apply_q(const LqTask* tasks) {
-  __shared__ double2 sP[LQB][LQB + 1];
+  __shared__ double2 sP[4][LQR][LQB + 1];
   __shared__ double2 sQ[LQB][LQB + 1];
   __shared__ double2 sT[LQR][LQB + 1];
   const LqTask& T = tasks[blockIdx.x];
@@ -321,7 +322,7 @@ __global__ __launch_bounds__(256) void k_widen(const TriTask* tasks) {
 
 // ---- factorisation with the panel in registers ------------------------------------------------
 struct LqStepShared {
-  double2 P[2][LQB][LQB + 1], Q[2][LQB][LQB + 1], T[2][LQR][LQB + 1];  // lq_apply_panel, per team
+  double2 P[2][4][LQR][LQB + 1], Q[2][LQB][LQB + 1], T[2][LQR][LQB + 1];  // lq_apply_panel, per team
   double2 G[LQB][LQB + 1], Tf[LQB][LQB + 1];                           // lq_factor_regs
   double2 w0[LQB];
 };
@@ -556,7 +557,7 @@ __global__ __launch_bounds__(512) void k_lq_step(const LqTask* tasks, int p) {
 
 // Rows beyond panel p + 1 with the block reflector of panel p, 16 rows per workgroup
 __global__ __launch_bounds__(256, 4) void k_lq_rest(const LqTask* tasks, int p) {
-  __shared__ double2 sP[LQB][LQB + 1];
+  __shared__ double2 sP[4][LQR][LQB + 1];
   __shared__ double2 sQ[LQB][LQB + 1];
   __shared__ double2 sT[LQR][LQB + 1];
   const LqTask& T = tasks[blockIdx.x];
