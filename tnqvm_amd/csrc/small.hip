@@ -328,7 +328,10 @@ __global__ __launch_bounds__(NT) void k_gate_small(const GateTask* tasks) {
   sort_rows<NT>(sY, stride, r, r, s_inv, s_sig, s_perm, &s_bad);
   // ---- truncation rule and factor scales, as k_select ----
   if (wave == 0) {
-    const double sg = lane < r ? s_sig[lane] : 0.0;
+    // a row under the floor of the sweeps is rounding residue: its vectors, of length sqrt(sigma) in the sites,
+    // would come back in the next theta' as a singular value far above it
+    double sg = lane < r ? s_sig[lane] : 0.0;
+    if (!(sg * sg > JAC_FLOOR2 * f2)) sg = 0.0;
     const double pn = T.pn_l2 ? sqrt(sg) : sg;
     const unsigned long long below = __ballot(lane < r && pn < T.cutoff);
     int K = below ? (int)__ffsll(below) : r;  // first sub-threshold index i: keep i + 1
