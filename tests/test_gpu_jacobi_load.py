@@ -42,3 +42,27 @@ def test_many_svds(eng, count, m, n):
         assert np.abs((np.abs(left) ** 2).sum(0) - sref).max() < 1e-12
         assert np.abs(left @ right - a).max() < 1e-12
         s.close()
+
+
+def test_result_independent_of_load(eng):
+    """A gate's sites are the same to the bit alone and in a wave that fills the chip."""
+    print("load", flush=True)
+    rng = np.random.default_rng(9)
+    m, n = 130, 200
+    a = rng.standard_normal((m, n)) + 1j * rng.standard_normal((m, n))
+    out = []
+    for count in (1, 60):
+        states = []
+        for i in range(count):
+            s = mps.MpsState(eng, 4)
+            s.set_site(0, np.ones((1, 2, m // 2)) / m)
+            s.set_site(1, np.roll(a, i, axis=1).reshape(m // 2, 2, n))
+            s.set_site(2, np.eye(n).reshape(n, 2, n // 2))
+            s.set_site(3, np.ones((n // 2, 2, 1)) / n)
+            s.apply({"name": "unitary", "qubits": (1, 2), "matrix": np.eye(4)})
+            states.append(s)
+        mps.run_waves(states)
+        out.append((states[0].get_site(1), states[0].get_site(2)))
+        for s in states:
+            s.close()
+    assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])

@@ -488,7 +488,8 @@ __device__ __forceinline__ void inner_sweep(InnerShared& S, double itol, double 
 // BLK is the block size JB (a template parameter: the kernel's register allocation on
 // gfx950 comes out at 128 VGPRs with four waves, four waves per SIMD, in the tiled form).
 template <int BLK, bool TILED, int NW>
-__global__ __launch_bounds__(64 * NW, NW == 4 && TILED ? 4 : 2) void k_jacobi_round(const JacTask* tasks, int ntasks, int sweep, int round) {
+__global__ __launch_bounds__(64 * NW, NW == 4 && TILED ? 4 : 2) void k_jacobi_round(const JacTask* tasks, int ntasks,
+                                                                                    int sweep, int round) {
   static_assert(BLK == 16 && JB == BLK && JP == 2 * BLK && NW % 4 == 0, "rotation-pair blocks of the inner sweep");
   constexpr int NT = 64 * NW;
   __shared__ InnerShared S;
@@ -516,28 +517,31 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && TILED ? 4 : 2) void k_jacobi_ro
   auto at = [&](int row, int col) -> size_t { return (size_t)row * ld + col; };
   const int rowa = ba * JB + l16, rowb = bb * JB + l16;  // pair rows l16 and 16 + l16
 
-  // ---- Gram tiles (0,0), (0,1), (1,1), or in a cross round (0,1) and the diagonal, over this wave's 4-column units u = wave, wave + NW, ... ----
+  // ---- Gram tiles (0,0), (0,1), (1,1), or in a cross round (0,1) and the diagonal ----
   // FP64 MFMA, or in the early sweeps of large SVDs FP32 MFMA at twice the rate: the rotations
   // they give are still applied in FP64 and are unitary, so the rows only lose the accuracy of
   // the rotation angles, which the FP64 sweeps that end every SVD make up for.
-  // Tiled rows (c = c_tot, the last tile's missing columns zero): unit wave + NW d is a quarter of
-  // tile (wave / 4) + (NW / 4) d, so both operands advance by NW / 4 tiles a step; row-major rows are
+  // Eight partial sums whatever NW is, over the 4-column units u = vw, vw + 8, ..., added in the same order:
+  // an SVD's result does not depend on what else is in its launch.  Four waves take two of them each, one
+  // after the other.
+  // Tiled rows (c = c_tot, the last tile's missing columns zero): unit vw + 8 d is a quarter of
+  // tile (vw / 4) + 2 d, so both operands advance by two tiles a step; row-major rows are
   // bounded by their columns.
-  constexpr int TS = NW / 4;  // tiles a step
-  const int nd = ((TILED ? ntc : (((C + 3) >> 2) + 3) >> 2) + TS - 1) / TS;
+  const int nd = ((TILED ? ntc : (((C + 3) >> 2) + 3) >> 2) + 1) / 2;
   const double2* ga = TILED ? Y + (size_t)ba * ntc * 256 + (l16 >> 2) * 64 + (wave & 3) * 16 + (l16 & 3) * 4 + k4 : Y;
   const double2* gb = TILED ? Y + (size_t)bb * ntc * 256 + (l16 >> 2) * 64 + (wave & 3) * 16 + (l16 & 3) * 4 + k4 : Y;
   constexpr int PD = NW == 4 ? 2 : 4;
+  int vw = wave;
   // The loads are not conditional, past the end they repeat the last tile or column: behind a load that may
   // not have been issued, the wait for an older one is a wait for all.
   auto ld_unit = [&](int d, double2& v0, double2& v1) __attribute__((always_inline)) {
-    const int col = min(4 * (wave + NW * d) + k4, C - 1), tile = min((wave >> 2) + TS * d, ntc - 1);
+    const int col = min(4 * (vw + 8 * d) + k4, C - 1), tile = min((vw >> 2) + 2 * d, ntc - 1);
     v0 = gld(TILED ? ga + (size_t)tile * 256 : Y + at(rowa, col));
     v1 = gld(TILED ? gb + (size_t)tile * 256 : Y + at(rowb, col));
   };
-  auto skip_unit = [&](int d) { return TILED && (wave >> 2) + TS * d >= ntc; };
+  auto skip_unit = [&](int d) { return TILED && (vw >> 2) + 2 * d >= ntc; };
   auto unit = [&](int d, double2 v) __attribute__((always_inline)) {  // row-major: nothing past the columns
-    return TILED || 4 * (wave + NW * d) + k4 < C ? v : make_double2(0, 0);
+    return TILED || 4 * (vw + 8 * d) + k4 < C ? v : make_double2(0, 0);
   };
   // Complex products on real MFMA with three real products each instead of four:
   //  * diagonal tiles (Hermitian): Re = Ar Ar^T + Ai Ai^T, and Im = X - X^T with X = Ar Ai^T;
@@ -547,7 +551,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && TILED ? 4 : 2) void k_jacobi_ro
   // nine: what its sweep leaves out there is second order (see jacobi_full_round).
   // Each partial sum of the waves goes to LDS as (Re, X) for the diagonal tiles and
   // (Re, Im) for the off-diagonal one; Im of the diagonal tiles is formed after the sum.
-  // to_lds(value of the tile entry v of this lane, its row): waves 0, 1 store, then 2, 3 (and so on) add
+  // to_lds(value of the tile entry v of this lane, its row): sums 0, 1 store, then 2, 3 (and so on) add
   const bool full = jacobi_full_round(round, nb);
   double n0 = 0.0, n1 = 0.0;  // cross: squared norms of the rows l16 and 16 + l16 over this lane's columns
   auto to_lds = [&](auto row, auto e00, auto e01, auto e11) __attribute__((always_inline)) {
@@ -557,9 +561,9 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && TILED ? 4 : 2) void k_jacobi_ro
       n0 += __shfl_xor(n0, 32);
       n1 += __shfl_xor(n1, 32);
     }
-    for (int w = 0; w < NW; w += 2) {
-      if ((wave & ~1) == w) {
-        double2 (*P)[JP + 1] = S.G[wave & 1];
+    for (int w = vw - wave; w < vw - wave + NW; w += 2) {
+      if ((vw & ~1) == w) {
+        double2 (*P)[JP + 1] = S.G[vw & 1];
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
           const int i = row(v), j = l16;
@@ -579,88 +583,92 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && TILED ? 4 : 2) void k_jacobi_ro
       __syncthreads();
     }
   };
-  if (sweep >= T.gram32) {
-    mfma_d4 k1 = {0, 0, 0, 0}, k2 = {0, 0, 0, 0}, k3 = {0, 0, 0, 0};
-    mfma_d4 a00r = {0, 0, 0, 0}, a00x = {0, 0, 0, 0}, a11r = {0, 0, 0, 0}, a11x = {0, 0, 0, 0};
-    auto products = [&](auto diag) __attribute__((always_inline)) {
-      double2 x0[PD], x1[PD];
-#pragma unroll
-      for (int d = 0; d < PD; ++d) ld_unit(d, x0[d], x1[d]);
 #pragma unroll 1
-      for (int e0 = 0; e0 < nd; e0 += PD) {
+  for (; vw < 8; vw += NW) {
+    n0 = n1 = 0.0;
+    if (sweep >= T.gram32) {
+      mfma_d4 k1 = {0, 0, 0, 0}, k2 = {0, 0, 0, 0}, k3 = {0, 0, 0, 0};
+      mfma_d4 a00r = {0, 0, 0, 0}, a00x = {0, 0, 0, 0}, a11r = {0, 0, 0, 0}, a11x = {0, 0, 0, 0};
+      auto products = [&](auto diag) __attribute__((always_inline)) {
+        double2 x0[PD], x1[PD];
 #pragma unroll
-        for (int d = 0; d < PD; ++d) {
-          const double2 v0 = unit(e0 + d, x0[d]), v1 = unit(e0 + d, x1[d]);
-          ld_unit(e0 + d + PD, x0[d], x1[d]);
-          if (skip_unit(e0 + d)) continue;
-          if (diag) {
-            a00r = mfma64(v0.x, v0.x, a00r);
-            a11r = mfma64(v1.x, v1.x, a11r);
-            a00x = mfma64(v0.x, v0.y, a00x);
-            a11x = mfma64(v1.x, v1.y, a11x);
-          } else {
-            n0 = fma(v0.x, v0.x, fma(v0.y, v0.y, n0));
-            n1 = fma(v1.x, v1.x, fma(v1.y, v1.y, n1));
-          }
-          k1 = mfma64(v0.x - v0.y, v1.x, k1);
-          k2 = mfma64(v0.x, v1.y - v1.x, k2);
-          k3 = mfma64(-v0.y, v1.x + v1.y, k3);
-          if (diag) {
-            a00r = mfma64(v0.y, v0.y, a00r);
-            a11r = mfma64(v1.y, v1.y, a11r);
+        for (int d = 0; d < PD; ++d) ld_unit(d, x0[d], x1[d]);
+#pragma unroll 1
+        for (int e0 = 0; e0 < nd; e0 += PD) {
+#pragma unroll
+          for (int d = 0; d < PD; ++d) {
+            const double2 v0 = unit(e0 + d, x0[d]), v1 = unit(e0 + d, x1[d]);
+            ld_unit(e0 + d + PD, x0[d], x1[d]);
+            if (skip_unit(e0 + d)) continue;
+            if (diag) {
+              a00r = mfma64(v0.x, v0.x, a00r);
+              a11r = mfma64(v1.x, v1.x, a11r);
+              a00x = mfma64(v0.x, v0.y, a00x);
+              a11x = mfma64(v1.x, v1.y, a11x);
+            } else {
+              n0 = fma(v0.x, v0.x, fma(v0.y, v0.y, n0));
+              n1 = fma(v1.x, v1.x, fma(v1.y, v1.y, n1));
+            }
+            k1 = mfma64(v0.x - v0.y, v1.x, k1);
+            k2 = mfma64(v0.x, v1.y - v1.x, k2);
+            k3 = mfma64(-v0.y, v1.x + v1.y, k3);
+            if (diag) {
+              a00r = mfma64(v0.y, v0.y, a00r);
+              a11r = mfma64(v1.y, v1.y, a11r);
+            }
           }
         }
-      }
-    };
-    if (full) products(std::true_type());
-    else products(std::false_type());
-    // f64 D[i][j]: lane j + 16 (i % 4), register i / 4
-    to_lds([&](int v) { return 4 * v + k4; }, [&](int v) { return make_double2(a00r[v], a00x[v]); },
-           [&](int v) { return make_double2(k1[v] - k3[v], k1[v] + k2[v]); },
-           [&](int v) { return make_double2(a11r[v], a11x[v]); });
-  } else {
-    typedef float mfma_f4 __attribute__((ext_vector_type(4)));
-    mfma_f4 h1 = {0, 0, 0, 0}, h2 = {0, 0, 0, 0}, h3 = {0, 0, 0, 0};
-    mfma_f4 b00r = {0, 0, 0, 0}, b00x = {0, 0, 0, 0}, b11r = {0, 0, 0, 0}, b11x = {0, 0, 0, 0};
-    auto products = [&](auto diag) __attribute__((always_inline)) {
-      double2 x0[PD], x1[PD];
+      };
+      if (full) products(std::true_type());
+      else products(std::false_type());
+      // f64 D[i][j]: lane j + 16 (i % 4), register i / 4
+      to_lds([&](int v) { return 4 * v + k4; }, [&](int v) { return make_double2(a00r[v], a00x[v]); },
+             [&](int v) { return make_double2(k1[v] - k3[v], k1[v] + k2[v]); },
+             [&](int v) { return make_double2(a11r[v], a11x[v]); });
+    } else {
+      typedef float mfma_f4 __attribute__((ext_vector_type(4)));
+      mfma_f4 h1 = {0, 0, 0, 0}, h2 = {0, 0, 0, 0}, h3 = {0, 0, 0, 0};
+      mfma_f4 b00r = {0, 0, 0, 0}, b00x = {0, 0, 0, 0}, b11r = {0, 0, 0, 0}, b11x = {0, 0, 0, 0};
+      auto products = [&](auto diag) __attribute__((always_inline)) {
+        double2 x0[PD], x1[PD];
 #pragma unroll
-      for (int d = 0; d < PD; ++d) ld_unit(d, x0[d], x1[d]);
+        for (int d = 0; d < PD; ++d) ld_unit(d, x0[d], x1[d]);
 #pragma unroll 1
-      for (int e0 = 0; e0 < nd; e0 += PD) {
+        for (int e0 = 0; e0 < nd; e0 += PD) {
 #pragma unroll
-        for (int d = 0; d < PD; ++d) {
-          const double2 v0 = unit(e0 + d, x0[d]), v1 = unit(e0 + d, x1[d]);
-          const float p0 = (float)v0.x, q0 = (float)v0.y, p1 = (float)v1.x, q1 = (float)v1.y;
-          ld_unit(e0 + d + PD, x0[d], x1[d]);
-          if (skip_unit(e0 + d)) continue;
-          if (diag) {
-            b00r = __builtin_amdgcn_mfma_f32_16x16x4f32(p0, p0, b00r, 0, 0, 0);
-            b11r = __builtin_amdgcn_mfma_f32_16x16x4f32(p1, p1, b11r, 0, 0, 0);
-            b00x = __builtin_amdgcn_mfma_f32_16x16x4f32(p0, q0, b00x, 0, 0, 0);
-            b11x = __builtin_amdgcn_mfma_f32_16x16x4f32(p1, q1, b11x, 0, 0, 0);
-          } else {
-            n0 = fma(v0.x, v0.x, fma(v0.y, v0.y, n0));
-            n1 = fma(v1.x, v1.x, fma(v1.y, v1.y, n1));
-          }
-          h1 = __builtin_amdgcn_mfma_f32_16x16x4f32(p0 - q0, p1, h1, 0, 0, 0);
-          h2 = __builtin_amdgcn_mfma_f32_16x16x4f32(p0, q1 - p1, h2, 0, 0, 0);
-          h3 = __builtin_amdgcn_mfma_f32_16x16x4f32(-q0, p1 + q1, h3, 0, 0, 0);
-          if (diag) {
-            b00r = __builtin_amdgcn_mfma_f32_16x16x4f32(q0, q0, b00r, 0, 0, 0);
-            b11r = __builtin_amdgcn_mfma_f32_16x16x4f32(q1, q1, b11r, 0, 0, 0);
+          for (int d = 0; d < PD; ++d) {
+            const double2 v0 = unit(e0 + d, x0[d]), v1 = unit(e0 + d, x1[d]);
+            const float p0 = (float)v0.x, q0 = (float)v0.y, p1 = (float)v1.x, q1 = (float)v1.y;
+            ld_unit(e0 + d + PD, x0[d], x1[d]);
+            if (skip_unit(e0 + d)) continue;
+            if (diag) {
+              b00r = __builtin_amdgcn_mfma_f32_16x16x4f32(p0, p0, b00r, 0, 0, 0);
+              b11r = __builtin_amdgcn_mfma_f32_16x16x4f32(p1, p1, b11r, 0, 0, 0);
+              b00x = __builtin_amdgcn_mfma_f32_16x16x4f32(p0, q0, b00x, 0, 0, 0);
+              b11x = __builtin_amdgcn_mfma_f32_16x16x4f32(p1, q1, b11x, 0, 0, 0);
+            } else {
+              n0 = fma(v0.x, v0.x, fma(v0.y, v0.y, n0));
+              n1 = fma(v1.x, v1.x, fma(v1.y, v1.y, n1));
+            }
+            h1 = __builtin_amdgcn_mfma_f32_16x16x4f32(p0 - q0, p1, h1, 0, 0, 0);
+            h2 = __builtin_amdgcn_mfma_f32_16x16x4f32(p0, q1 - p1, h2, 0, 0, 0);
+            h3 = __builtin_amdgcn_mfma_f32_16x16x4f32(-q0, p1 + q1, h3, 0, 0, 0);
+            if (diag) {
+              b00r = __builtin_amdgcn_mfma_f32_16x16x4f32(q0, q0, b00r, 0, 0, 0);
+              b11r = __builtin_amdgcn_mfma_f32_16x16x4f32(q1, q1, b11r, 0, 0, 0);
+            }
           }
         }
-      }
-    };
-    if (full) products(std::true_type());
-    else products(std::false_type());
-    // f32 D[i][j]: lane j + 16 (i / 4), register i % 4; the waves' partial tiles are summed in FP64
-    to_lds([&](int v) { return 4 * k4 + v; }, [&](int v) { return make_double2((double)b00r[v], (double)b00x[v]); },
-           [&](int v) {
-             return make_double2((double)h1[v] - (double)h3[v], (double)h1[v] + (double)h2[v]);
-           },
-           [&](int v) { return make_double2((double)b11r[v], (double)b11x[v]); });
+      };
+      if (full) products(std::true_type());
+      else products(std::false_type());
+      // f32 D[i][j]: lane j + 16 (i / 4), register i % 4; the waves' partial tiles are summed in FP64
+      to_lds([&](int v) { return 4 * k4 + v; }, [&](int v) { return make_double2((double)b00r[v], (double)b00x[v]); },
+             [&](int v) {
+               return make_double2((double)h1[v] - (double)h3[v], (double)h1[v] + (double)h2[v]);
+             },
+             [&](int v) { return make_double2((double)b11r[v], (double)b11x[v]); });
+    }
   }
   {
     // the two partial sums; Im of the diagonal tiles from X (X[i][j] - X[j][i]), or nothing but the
