@@ -272,7 +272,7 @@ int hipmps_serve_pending(hipmps_engine e, int* queued, int* running);
 /* ---- measurement hooks for the bench ------------------------------------------------ */
 typedef struct {
   double ms_theta, ms_jacobi, ms_split, ms_other;
-  double ms_jacobi_rounds;  /* HIP-event time of the back-to-back k_jacobi_round launches */
+  double ms_jacobi_rounds;  /* HIP-event span of all sweeps' k_jacobi_round launches of a wave */
   long long jacobi_launches;
   long long jacobi_pairs_rotated;
   long long jacobi_pairs_visited;

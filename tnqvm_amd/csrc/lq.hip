@@ -335,8 +335,8 @@ struct LqStepShared {
 // -- <y_i, w_r> updates a row i > r, and is G_ir of the T factor for a row i < r -- and the wave with
 // row r + 1 goes on to the next reflector as soon as that row is updated; T's column r - 1 is formed by
 // another wave meanwhile.  One barrier per reflector.  Bound by that serial chain.  Measured, with the
-// update of the panel's rows by the panel before: 26, 34 and 48 us at up to 128, 256 and 512 columns
-// (rows in LDS, shuffle reductions: 55, 73 and 100 us), 80 us at 1024 and 218 us at 1536 (rows in L2:
+// update of the panel's rows by the panel before: 24, 31 and 44 us at up to 128, 256 and 512 columns
+// (rows in LDS, shuffle reductions: 55, 73 and 100 us), 77 us at 1024 and 193 us at 1536 (rows in L2:
 // 350 to 700 us).
 template <int NC, int RW>
 __device__ __forceinline__ void lq_factor_regs(const LqTask& T, int p, LqStepShared& S, double2* srow) {

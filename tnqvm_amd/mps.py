@@ -382,6 +382,8 @@ class MpsState:
             raise ValueError("at most 16 measured qubits")
         q = np.asarray(qubits, dtype=np.int32).reshape(-1)
         q = np.ascontiguousarray(np.where(q < 0, q + self.n, q), dtype=np.int32)
+        if (q < 0).any() or (q >= self.n).any():
+            raise IndexError("measured qubit out of range")
         out = np.zeros(1 << k)
         check(lib().hipmps_outcome_probabilities(self.h, q.ctypes.data_as(_ip), k, out.ctypes.data_as(_dp)))
         return out
