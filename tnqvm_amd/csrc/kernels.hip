@@ -720,7 +720,9 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && TILED ? 4 : 2) void k_jacobi_ro
   double2* yb = TILED ? Y + (size_t)bb * ntc * 256 + (l16 >> 2) * 16 + k4 * 4 + (l16 & 3) : Y + at(bb * JB + k4, l16);
   const size_t step_row = TILED ? 64 : 4 * ld, step_tile = TILED ? 256 : 16;
   auto ok_tile = [&](int ctile) { return TILED ? ctile < nt : ctile < nt && ctile * 16 + l16 < CT; };
-  auto elem = [&](int kk, int ctile) { return (kk < 4 ? ya + kk * step_row : yb + (kk - 4) * step_row) + ctile * step_tile; };
+  auto elem = [&](int kk, int ctile) {
+    return (kk < 4 ? ya + kk * step_row : yb + (kk - 4) * step_row) + ctile * step_tile;
+  };
   double2 bq[8];
   auto first_tile = [&]() __attribute__((always_inline)) {
 #pragma unroll

@@ -112,8 +112,9 @@ __device__ __forceinline__ void lq_factor_panel(const LqTask& T, int k0, double2
 // staged in LDS, then Y -= Q W by MFMA, each wave owning whole 16-column tiles.  PD units of P and a
 // whole tile of the update are in flight.  No load is under a condition (behind a load that may not have
 // been issued, the wait for an older one is a wait for all): past the end they repeat the last group, and
-// the panel's own columns, where its reflectors start, and columns past the end are put right at use.  Run by teams of four waves (a workgroup of 256 threads is one team, one of 512
-// threads two, each with rows and LDS of its own).
+// the panel's own columns, where its reflectors start, and columns past the end are put right at use.  Run
+// by teams of four waves (a workgroup of 256 threads is one team, one of 512 threads two, each with rows and
+// LDS of its own).
 template <int PD>
 __device__ __forceinline__ void lq_apply_panel(const LqTask& T, int k0, int k1, double2* Y, size_t ly, int r0, int r1,
                                                int conjT, double2 (*sP)[LQR][LQB + 1], double2 (*sQ)[LQB + 1],

@@ -588,7 +588,8 @@ hipError_t launch_zero_state(void* const* sites, int n, int fp32, hipStream_t s)
 // string -- is a workgroup of the same launch.  A step takes as many s side by side as fit the workgroup's
 // threads (chain_slots); the next A_s are read while these are used.
 template <typename S>
-__global__ __launch_bounds__(CHAIN_THREADS) void k_env_chain(const ChainSite* sites, int n, const double* diags, double* out) {
+__global__ __launch_bounds__(CHAIN_THREADS) void k_env_chain(const ChainSite* sites, int n, const double* diags,
+                                                             double* out) {
   constexpr int B = CHAIN_MAX_BOND, NT = CHAIN_THREADS, Q = B * B / NT;
   __shared__ double2 sE[B * (B + 1)], sA[B * (B + 1)], sX[B * (B + 1)];
   const int tid = threadIdx.x;
