@@ -322,6 +322,9 @@ __global__ __launch_bounds__(NT) void k_gate_small(const GateTask* tasks) {
   __syncthreads();
   f2 = 0.0;
   for (int w = 0; w < NT / 64; ++w) f2 += s_red[w];
+  // NaN / Inf anywhere in theta': the LQ drops what is right of a row's diagonal when its tail is a NaN, so the
+  // norms of the rows it leaves need not show it
+  if (tid == 0 && !(f2 <= DBL_MAX)) s_bad = 1;
   __syncthreads();
   const int sweeps = svd_rows<NT>(sY, stride, r, T.c, T.tol, JAC_FLOOR2 * f2, T.max_sweeps, &s_flag, s_inv, s_d);
   __syncthreads();
