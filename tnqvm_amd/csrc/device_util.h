@@ -57,8 +57,8 @@ __device__ __forceinline__ void gst(float2* p, float2 v) {
   *(HIPMPS_GLOBAL gvec_f2*)p = x;
 }
 
-// base uniform over the wave, idx < 2^28: one scalar base and a 32-bit offset instead of a 64-bit
-// address per load
+// base uniform over the wave, idx < 2^28 (the byte offset wraps at 2^32): one scalar base and a 32-bit offset
+// instead of a 64-bit address per load
 __device__ __forceinline__ double2 gld_at(const double2* base, unsigned idx) {
   const gvec_d2 v = *(const HIPMPS_GLOBAL gvec_d2*)((const HIPMPS_GLOBAL char*)base + (size_t)(idx * 16u));
   return make_double2(v.x, v.y);

@@ -609,7 +609,7 @@ int run_wave(hipmps_engine E, std::vector<WaveItem>& all) {
     int maxb = s->t.max_bond_dim > 0 ? s->t.max_bond_dim : INT_MAX - 1;
     it.kub = std::min(it.r, maxb);
     it.fp32 = s->fp32;
-    it.lq = E->lq_min_rank > 0 && it.r >= E->lq_min_rank;
+    it.lq = E->lq_min_rank > 0 && it.r >= E->lq_min_rank && it.c < LQ_MAX_COLS;
     it.small = gate_small(it.r, it.c);
   }
   std::stable_sort(all.begin(), all.end(), [](const WaveItem& a, const WaveItem& b) {

@@ -254,6 +254,9 @@ hipError_t launch_lq(const LqTask* d_tasks, int ntasks, int max_rows, hipStream_
 // block reflector meanwhile (events ea, eb order the two).  Rows of at most LQ_REG_MAX_COLS columns
 // (hipErrorNotSupported otherwise); on return every later launch on sa follows all of it.
 constexpr int LQ_REG_MAX_COLS = 2048;
+// Columns of a matrix whose LQ is taken: below this, 16 rows' elements are counted in 28 bits (gld_at).  Wider
+// ones (4 GiB a panel) are swept without it.
+constexpr int LQ_MAX_COLS = 1 << 24;
 hipError_t launch_lq_lookahead(const LqTask* d_tasks, int ntasks, int max_rows, int max_cols, hipStream_t sa,
                                hipStream_t sb, hipEvent_t ea, hipEvent_t eb);
 // Tgt <- Tgt Q~ (Q~ = H_{rows-1} ... H_0 restricted to the first rows of M's row space, applied

@@ -130,9 +130,14 @@ __device__ __forceinline__ void lq_apply_panel(const LqTask& T, int k0, int k1, 
     const int i = tid >> 4, j = tid & 15;
     sT[i][j] = conjT ? cconj(gld(Tp + j * LQB + i)) : gld(Tp + i * LQB + j);
   }
+  // 32-bit offsets (gld_at) from the panel's first row and from the first of Y's rows: 16 rows of fewer than
+  // LQ_MAX_COLS columns each
+  const int y0 = __builtin_amdgcn_readfirstlane(min(r0, r1 - 1));
+  const double2* Mk = M + (size_t)k0 * ld;
+  Y += (size_t)y0 * ly;
   // a reflector past k1 repeats the last one: its rows and columns of T are zero
   const int jl = min(k0 + l16, k1 - 1);
-  const unsigned wrow = (unsigned)jl * (unsigned)ld;
+  const unsigned wrow = (unsigned)(jl - k0) * (unsigned)ld;
   const double2 head = gld_at(W0, jl);  // of reflector k0 + l16
   // element w_j[col] of reflector j (support col >= j; head in W0, tail in M's row j), M's element being v
   auto own = [&](double2 v, double2 h, int j, int col) __attribute__((always_inline)) {
@@ -141,7 +146,7 @@ __device__ __forceinline__ void lq_apply_panel(const LqTask& T, int k0, int k1, 
   };
   auto special = [&](int g) { return g == 0 || k0 + 16 * g + 16 > C; };
   // ---- P[i][j] = sum_c Y[r0+i][c] conj(w_j[c]); B operand: reflector k0 + l16 ----
-  const unsigned yrow = (unsigned)min(r0 + l16, r1 - 1) * (unsigned)ly;  // a row past the end: a repeat, not stored
+  const unsigned yrow = (unsigned)min(l16, r1 - 1 - y0) * (unsigned)ly;  // a row past the end: a repeat, not stored
   mfma_d4 pr = {0, 0, 0, 0}, pim = {0, 0, 0, 0};
   const int nt = (C - k0 + 15) >> 4;  // 16-column groups; this wave's unit of a group: 4 columns
   const int uo = k0 + 4 * wave + k4;
@@ -149,7 +154,7 @@ __device__ __forceinline__ void lq_apply_panel(const LqTask& T, int k0, int k1, 
   auto load = [&](int g, double2& y, double2& m) __attribute__((always_inline)) {
     const unsigned col = min(uo + 16 * g, C - 1);
     y = gld_at(Y, yrow + col);
-    m = gld_at(M, wrow + col);
+    m = gld_at(Mk, wrow + col);
   };
 #pragma unroll
   for (int d = 0; d < PD; ++d) load(d, a[d], w[d]);
@@ -174,13 +179,13 @@ __device__ __forceinline__ void lq_apply_panel(const LqTask& T, int k0, int k1, 
   double2 tw[LQB / 4], ty[4];
   unsigned ry[4], rw[LQB / 4];
 #pragma unroll
-  for (int v = 0; v < 4; ++v) ry[v] = (unsigned)min(r0 + 4 * v + k4, r1 - 1) * (unsigned)ly;
+  for (int v = 0; v < 4; ++v) ry[v] = (unsigned)min(4 * v + k4, r1 - 1 - y0) * (unsigned)ly;
 #pragma unroll
-  for (int kk = 0; kk < LQB / 4; ++kk) rw[kk] = (unsigned)min(k0 + kk * 4 + k4, k1 - 1) * (unsigned)ld;
+  for (int kk = 0; kk < LQB / 4; ++kk) rw[kk] = (unsigned)min(kk * 4 + k4, k1 - 1 - k0) * (unsigned)ld;
   auto tile = [&](int t) __attribute__((always_inline)) {
     const unsigned c = min(k0 + 16 * t + l16, C - 1);
 #pragma unroll
-    for (int kk = 0; kk < LQB / 4; ++kk) tw[kk] = gld_at(M, rw[kk] + c);  // B[k][c] = w_j[c]
+    for (int kk = 0; kk < LQB / 4; ++kk) tw[kk] = gld_at(Mk, rw[kk] + c);  // B[k][c] = w_j[c]
 #pragma unroll
     for (int v = 0; v < 4; ++v) ty[v] = gld_at(Y, ry[v] + c);
   };
