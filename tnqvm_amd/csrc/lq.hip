@@ -21,6 +21,7 @@ namespace hipmps {
 
 constexpr int LQB = 16;  // rows per panel (reflectors per block reflector)
 constexpr int LQR = 16;  // rows per MFMA tile in the block-reflector application
+constexpr int LQ_TWO_ROWS_COLS = 64 * 16;  // widest panel of which a lane's registers hold two rows
 constexpr long long LQ_ONE_STREAM_ROWS = 4096;  // launch_lq_lookahead: rows of all tasks on one stream up to this
 
 // Element w_k[col] of reflector k of M (support col >= k; head in W0, tail in M's row k).
@@ -552,7 +553,10 @@ __global__ __launch_bounds__(512) void k_lq_step(const LqTask* tasks, int p) {
   if (blockIdx.y == 0) {
     const int e1 = min(k1 + LQB, T.rows);
     if (p >= 0) lq_apply_panel<4>(T, k0, k1, T.M, T.ld, k1, team ? k1 : e1, 0, S.P[team], S.Q[team], S.T[team]);
-    lq_factor_regs<NC, (NC <= 16 ? 2 : 1)>(T, p + 1, S, srow);
+    // one row of a lane or two is the task's own: the two round differently, and a matrix beside wider ones gives
+    // what it gives alone
+    if (NC <= 16 || T.cols - k1 <= LQ_TWO_ROWS_COLS) lq_factor_regs<(NC <= 16 ? NC : 16), 2>(T, p + 1, S, srow);
+    else lq_factor_regs<NC, 1>(T, p + 1, S, srow);
     return;
   }
   const int r0 = k1 + LQB + 2 * LQR * ((int)blockIdx.y - 1);
@@ -578,14 +582,15 @@ hipError_t launch_lq_lookahead(const LqTask* d_tasks, int ntasks, int max_rows, 
   if (ntasks <= 0 || max_rows <= 0) return hipSuccess;
   if (max_cols > LQ_REG_MAX_COLS) return hipErrorNotSupported;
   const int panels = (max_rows + LQB - 1) / LQB;
-  // columns per lane of the panel's registers; the results are the same for every NC that holds them
+  // columns per lane of the panel's registers, by the widest task; a task's results are the same for every NC
+  // that holds it
   auto step = [&](int p, int blocks) {
     const int w = max_cols - (p + 1) * LQB;
     const dim3 g(ntasks, blocks), b(512);
     if (w <= 128) hipLaunchKernelGGL(k_lq_step<2>, g, b, 0, sa, d_tasks, p);
     else if (w <= 256) hipLaunchKernelGGL(k_lq_step<4>, g, b, 0, sa, d_tasks, p);
     else if (w <= 512) hipLaunchKernelGGL(k_lq_step<8>, g, b, 0, sa, d_tasks, p);
-    else if (w <= 1024) hipLaunchKernelGGL(k_lq_step<16>, g, b, 0, sa, d_tasks, p);
+    else if (w <= LQ_TWO_ROWS_COLS) hipLaunchKernelGGL(k_lq_step<16>, g, b, 0, sa, d_tasks, p);
     else if (w <= 1536) hipLaunchKernelGGL(k_lq_step<24>, g, b, 0, sa, d_tasks, p);
     else hipLaunchKernelGGL(k_lq_step<32>, g, b, 0, sa, d_tasks, p);
   };
