@@ -55,3 +55,16 @@ def test_same_bits_beside_wider_ones(eng):
         got = run(eng, beside)
         assert [x for x, sites in zip(beside, got) if not same(sites, alone[SIZES.index(x)])] == []
 
+
+@pytest.mark.parametrize("lanes", [1, 2, 3, 4])
+def test_same_bits_on_any_lanes(eng, lanes):
+    """64 LQs or more are dealt to lanes."""
+    print("lq lanes", lanes, flush=True)
+    alone = run(eng, [(66, 130)])[0]
+    base = eng.tuning()
+    try:
+        eng.set_tuning(jacobi_lanes=lanes)
+        got = run(eng, [(66, 130)] * 66)
+    finally:
+        eng.set_tuning(**base)
+    assert all([same(sites, alone) for sites in got])

@@ -1020,15 +1020,15 @@ int run_wave_general(hipmps_engine E, std::vector<WaveItem>& items, const std::f
     }
     return 0;
   };
-  // one LQ of a lane's slice: with look-ahead on the lane's stream and a partner stream when the
-  // rows fit (lanes 0, 1 pair with streams 2, 3), else panel by panel on the lane's stream
-  const bool lookahead = E->lq_lookahead && 2 * lq_lanes <= hipmps_engine_s::MAX_LANES && E->lq_ev[0] != nullptr;
+  // one LQ of a lane's slice: with look-ahead when the rows fit, on the lane's stream and a partner stream
+  // where one is left (lanes 0, 1 pair with streams 2, 3), else panel by panel on the lane's stream
+  const bool la = E->lq_lookahead && E->lq_ev[0] != nullptr;
   // the LQ of tasks [b, b + n) of one array (second = 0: X, 1: L^H): look-ahead for the tasks of
   // items in the first group (columns <= LQ_REG_MAX_COLS), panel by panel for the others
   auto run_lq = [&](const LqTask* tasks, int b, int n, int second, int l) -> int {
     const hipStream_t ls = E->lane_stream[l];
     const int a_end = std::min(b + n, nlq_a), b_beg = std::max(b, nlq_a);
-    const bool la = lookahead && E->lane_stream[l + lq_lanes] != nullptr;
+    const hipStream_t partner = l + lq_lanes < hipmps_engine_s::MAX_LANES ? E->lane_stream[l + lq_lanes] : nullptr;
     auto extent = [&](int from, int to, int& rows, int& cols) {
       rows = cols = 0;
       for (int k = from; k < to; ++k) {
@@ -1040,8 +1040,8 @@ int run_wave_general(hipmps_engine E, std::vector<WaveItem>& items, const std::f
     int rows, cols;
     if (a_end > b) {
       extent(b, a_end, rows, cols);
-      if (la) HIP_TRY(launch_lq_lookahead(tasks + b, a_end - b, rows, cols, ls, E->lane_stream[l + lq_lanes],
-                                         E->lq_ev[2 * l], E->lq_ev[2 * l + 1]));
+      if (la) HIP_TRY(launch_lq_lookahead(tasks + b, a_end - b, rows, cols, ls, partner, E->lq_ev[2 * l],
+                                         E->lq_ev[2 * l + 1]));
       else HIP_TRY(launch_lq(tasks + b, a_end - b, rows, ls));
     }
     if (b + n > b_beg) {
