@@ -331,10 +331,7 @@ __global__ __launch_bounds__(NT) void k_gate_small(const GateTask* tasks) {
   sort_rows<NT>(sY, stride, r, r, s_inv, s_sig, s_perm, &s_bad);
   // ---- truncation rule and factor scales, as k_select ----
   if (wave == 0) {
-    // a row under the floor of the sweeps is rounding residue: its vectors, of length sqrt(sigma) in the sites,
-    // would come back in the next theta' as a singular value far above it
-    double sg = lane < r ? s_sig[lane] : 0.0;
-    if (!(sg * sg > JAC_FLOOR2 * f2)) sg = 0.0;
+    const double sg = lane < r ? s_sig[lane] : 0.0;
     const double pn = T.pn_l2 ? sqrt(sg) : sg;
     const unsigned long long below = __ballot(lane < r && pn < T.cutoff);
     int K = below ? (int)__ffsll(below) : r;  // first sub-threshold index i: keep i + 1
@@ -344,7 +341,10 @@ __global__ __launch_bounds__(NT) void k_gate_small(const GateTask* tasks) {
     const double f = T.renorm && kept > 0.0 ? sqrt((kept + disc) / kept) : 1.0;
     if (lane < r) {
       double gy = 0.0, gw = 0.0, is = 0.0;
-      if (lane < K && sg > 1e-150) {
+      // Of the index kept below the cutoff, a row under the floor of the sweeps is rounding residue: its vectors, of
+      // length sqrt(sigma) in the sites, would come back in the next theta' as a singular value far above both.
+      const bool residue = pn < T.cutoff && !(sg * sg > JAC_FLOOR2 * f2);
+      if (lane < K && sg > 1e-150 && !residue) {
         // exponents of f sigma: left aL, right 1 - aL; Y's side is the left one unless transposed
         const double sf = sg * f, h = sqrt(sf);
         const double left = T.absorb == 0 ? h : 1.0, right = T.absorb == 0 ? h : sf;
