@@ -379,16 +379,16 @@ __device__ __forceinline__ void lq_factor_regs(const LqTask& T, int p, LqStepSha
       if (j > 0 || lane > r) s += cabs2(v[j]);
     s = wave_sum(s);
     const double2 a = make_double2(lane_value(v[0].x, r), lane_value(v[0].y, r));
-    // reciprocal roots by one Newton step (nr_rsq): the library's square roots and divisions one after the
-    // other are most of a reflector's scalar chain
+    // reciprocal roots (full_rsq): the library's square roots and divisions one after the other are most of a
+    // reflector's scalar chain
     const double a2 = cabs2(a), n2 = a2 + s;
     double2 beta = make_double2(0, 0), w0 = make_double2(0, 0);
     double scale = 0.0;
     if (n2 > 0.0) {
-      const double2 ph = a2 > 0.0 ? cscale(a, nr_rsq(a2)) : make_double2(1.0, 0.0);
-      beta = cscale(ph, -(n2 * nr_rsq(n2)));  // -e^{i arg a} |x|: no cancellation in a - beta
+      const double2 ph = a2 > 0.0 ? cscale(a, full_rsq(a2)) : make_double2(1.0, 0.0);
+      beta = cscale(ph, -(n2 * full_rsq(n2)));  // -e^{i arg a} |x|: no cancellation in a - beta
       const double2 v0 = make_double2(a.x - beta.x, a.y - beta.y);
-      scale = nr_rsq(cabs2(v0) + s);
+      scale = full_rsq(cabs2(v0) + s);
       w0 = cscale(v0, scale);
     }
     double2* row = srow + (r & 1) * NC * 64;

@@ -54,10 +54,10 @@ __device__ __forceinline__ void lq_rows(double2* Y, int stride, int r, int c, in
     tail = row16_sum(tail);
     if (tail > 1e-290) {  // below: nothing to reflect that a double would show
       // w = x + e norm e_k with e = head / |head|; x becomes -e norm, other rows y - (y w^H) w / (norm (norm + |head|))
-      const double a2 = cabs2(head), n2 = a2 + tail, norm = n2 * nr_rsq(n2);
-      const double ra = a2 > 1e-290 ? nr_rsq(a2) : 0.0, a = a2 * ra;
+      const double a2 = cabs2(head), n2 = a2 + tail, norm = n2 * full_rsq(n2);
+      const double ra = a2 > 1e-290 ? full_rsq(a2) : 0.0, a = a2 * ra;
       const double2 e = ra > 0.0 ? cscale(head, ra) : make_double2(1, 0);
-      const double scale = nr_rcp(norm * (norm + a));
+      const double scale = full_rcp(norm * (norm + a));
       const double2 wk = cscale(e, a + norm);
 #pragma unroll
       for (int q = 0; q < NC; ++q)
