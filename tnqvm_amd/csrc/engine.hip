@@ -761,10 +761,10 @@ int run_wave_general(hipmps_engine E, std::vector<WaveItem>& items, const std::f
   RC_TRY(E->ws.ensure(off));
   char* ws = (char*)E->ws.p;
   // small: K (N ints) and wstats (WS_N doubles per item), read back together; ||X||_F^2 and its partial
-  // sums; per sweep the counts (2N ints), zeroed at the start
+  // sums; the counts (2N ints) of the last sweeps, zeroed at the start and when a slot comes round again
   const size_t res_bytes = align_up(N * sizeof(int)) + align_up(WS_N * N * sizeof(double));
   const size_t fro_bytes = align_up((size_t)(1 + FRO_BLOCKS) * N * sizeof(double));
-  const size_t cnt_bytes = align_up((size_t)2 * E->max_sweeps * N * sizeof(int));
+  const size_t cnt_bytes = align_up((size_t)2 * std::min(E->max_sweeps, JAC_COUNT_SLOTS) * N * sizeof(int));
   RC_TRY(E->small.ensure(res_bytes + fro_bytes + cnt_bytes));
   int* d_K = (int*)E->small.p;
   double* d_w = (double*)((char*)E->small.p + align_up(N * sizeof(int)));
@@ -1123,6 +1123,8 @@ int run_wave_general(hipmps_engine E, std::vector<WaveItem>& items, const std::f
       HIP_TRY(hipMemcpyAsync(dja, ha, nact * sizeof(JacTask), hipMemcpyHostToDevice, st));
       listed = active;
     }
+    const size_t at = (size_t)2 * N * (sweep % JAC_COUNT_SLOTS);
+    if (sweep >= JAC_COUNT_SLOTS) HIP_TRY(hipMemsetAsync(d_counts + at, 0, 2 * N * sizeof(int), st));
     if (E->timing && sweep == 0) HIP_TRY(hipEventRecord(E->ev[4], st));
     int max_rounds = 0;
     for (int l = 0; l < lanes; ++l) max_rounds = std::max(max_rounds, lane_rounds[l]);
@@ -1134,7 +1136,6 @@ int run_wave_general(hipmps_engine E, std::vector<WaveItem>& items, const std::f
                                       true));
     RC_TRY(join_lanes(lanes));
     for (int l = 0; l < lanes; ++l) E->prof.jacobi_launches += lane_rounds[l];
-    const size_t at = (size_t)2 * N * sweep;
     HIP_TRY(hipMemcpyAsync(hcounts + at, d_counts + at, 2 * N * sizeof(int), hipMemcpyDeviceToHost, st));
     HIP_TRY(hipEventRecord(E->sweep_ev[sweep & 1], st));
     return 0;
@@ -1143,7 +1144,7 @@ int run_wave_general(hipmps_engine E, std::vector<WaveItem>& items, const std::f
   bool nearly = false;
   auto finish = [&](int sweep) -> int {
     HIP_TRY(hipEventSynchronize(E->sweep_ev[sweep & 1]));
-    const int* cnt = hcounts + (size_t)2 * N * sweep;
+    const int* cnt = hcounts + (size_t)2 * N * (sweep % JAC_COUNT_SLOTS);
     long long R = 0, V = 0;
     std::vector<int> next;
     for (int q : active) {

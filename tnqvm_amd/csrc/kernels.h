@@ -28,6 +28,10 @@ struct ThetaTask {
   double2 G[16];     // G[(a,b)*4 + (a',b')], a = bit of the left site
 };
 
+// Sweeps whose counts are kept, at least three: the one that runs, the one before it (its counts say whether a task
+// has converged), and the one the host reads.  More of them only save clearing a slot per sweep.
+constexpr int JAC_COUNT_SLOTS = 64;
+
 // One Jacobi problem: orthogonalise the rows of Y (r_pad x c_tot, row-major, ld = ldy)
 // with respect to their first c columns (the data X); every rotation is applied to all
 // c_tot columns (c_tot = c: the rotation product is not carried).
@@ -37,7 +41,7 @@ struct JacTask {
   int c_tot;
   int nb;            // r_pad / JB (even)
   int pair_begin;    // first block of this task in the grid
-  int* counts;       // per sweep s: counts[s * cstride] block pairs rotated, [s * cstride + 1] visited
+  int* counts;       // of sweep s, at (s % JAC_COUNT_SLOTS) * cstride: block pairs rotated, then visited
   double* fro2;      // ||X||_F^2 (k_fro2), or null: rows with squared norm below JAC_FLOOR2 * fro2 are
                      // numerically zero (rounding residue) and neither rotate nor count against
                      // convergence

@@ -501,8 +501,8 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && TILED ? 4 : 2) void k_jacobi_ro
   const int pi = blockIdx.x - T.pair_begin;
   const int nb = T.nb;
   if (pi >= nb / 2 || round >= nb - 1) return;
-  int* counts = T.counts + (size_t)sweep * T.cstride;
-  if (sweep > T.gram32 && counts[-T.cstride] == 0) return;  // converged in the sweep before
+  int* counts = T.counts + sweep % JAC_COUNT_SLOTS * T.cstride;
+  if (sweep > T.gram32 && T.counts[(sweep - 1) % JAC_COUNT_SLOTS * T.cstride] == 0) return;  // converged in the sweep before
   const int ba = circle_slot(pi, round, nb), bb = circle_slot(nb - 1 - pi, round, nb);
   const int C = T.c, CT = T.c_tot;
   const size_t ld = T.ldy;
