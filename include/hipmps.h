@@ -74,7 +74,8 @@ typedef struct hipmps_state_s* hipmps_state;
 typedef struct {
   int device;               /* HIP device ordinal */
   size_t hbm_budget_bytes;  /* admission budget; 0 = 90% of the device's memory */
-  int jacobi_max_sweeps;    /* 0 = default (40) */
+  int jacobi_max_sweeps;    /* 0 = default (40); gates and channels that run in one workgroup, of at
+                               most 64 rows, stop at 1000 if it is larger */
   double jacobi_tol;        /* 0 = default: relative off-diagonal 1e-13 (fp64 states) */
   double jacobi_tol_mixed;  /* 0 = default: 1e-8 (mixed states, factors kept in complex64) */
 } hipmps_engine_opts;

@@ -61,3 +61,19 @@ def test_ends_at_the_cap(cap):
         s.close()
     finally:
         e.close()
+
+
+@pytest.mark.parametrize("m,cap,ends", [(4, 40, 40), (4, 1000, 1000), (4, 20000, 1000)])
+def test_one_launch_is_bounded(m, cap, ends):
+    """A gate in one workgroup sweeps within one launch, which has to end soon whatever the cap."""
+    print("one launch is bounded", m, cap, flush=True)
+    e = mps.Engine(jacobi_max_sweeps=cap, jacobi_tol=1e-30)
+    try:
+        s, a = planted(e, m)
+        with pytest.raises(capi.HipMpsError) as ei:
+            s.flush()
+        assert ei.value.code == capi.HIPMPS_E_CONVERGENCE
+        assert s.stats()["jacobi_sweeps_max"] == ends
+        s.close()
+    finally:
+        e.close()

@@ -677,7 +677,7 @@ int run_wave(hipmps_engine E, std::vector<WaveItem>& all) {
         T.pn_l2 = to.partial_norm == HIPMPS_PN_L2;
         T.absorb = to.absorb == HIPMPS_ABSORB_RIGHT ? 1 : 0;
         T.renorm = to.renormalize ? 1 : 0;
-        T.max_sweeps = E->max_sweeps;
+        T.max_sweeps = std::min(E->max_sweeps, SMALL_MAX_SWEEPS);
         T.cutoff = to.svd_cutoff;
         T.tol = it.fp32 ? E->tol_mixed : E->tol;
         for (int k = 0; k < 16; ++k) T.G[k] = make_double2(it.G[k].real(), it.G[k].imag());
@@ -1465,7 +1465,7 @@ int run_kraus_waves(hipmps_engine E, const std::vector<hipmps_state_s*>& states)
         T.c = h->jc;
         T.max_bond = h->max_bond;
         T.pn_l2 = h->s->t.partial_norm == HIPMPS_PN_L2;
-        T.max_sweeps = E->max_sweeps;
+        T.max_sweeps = std::min(E->max_sweeps, SMALL_MAX_SWEEPS);
         T.cutoff = KRAUS_EPS;
         T.tol = h->s->fp32 ? E->tol_mixed : E->tol;
         for (int t = 0; t < 4 * h->n_ops; ++t) T.K[t] = make_double2(h->k->K[t].real(), h->k->K[t].imag());

@@ -124,6 +124,8 @@ __host__ __device__ inline int small_stride(int c) { return (c <= 16 ? 16 : c <=
 // complex128 elements of X (and of Y) that fit a workgroup's LDS, and the largest row count
 constexpr int SMALL_MAX_ROWS = 64, SMALL_MAX_COLS = 128;
 constexpr int SMALL_CAP = 64 * 65;
+// sweeps of one launch at most, whatever the cap of the engine: 75 ms at 64 rows
+constexpr int SMALL_MAX_SWEEPS = 1000;
 constexpr int SMALL_CAP_LO = 32 * 33;  // variant of 256 threads, several workgroups per CU
 inline bool gate_small(int r, int c) {
   return r <= SMALL_MAX_ROWS && c <= SMALL_MAX_COLS && small_rows(r) * small_stride(c) <= SMALL_CAP;
