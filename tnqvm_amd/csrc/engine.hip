@@ -30,6 +30,7 @@
 #include <cmath>
 #include <complex>
 #include <cstdio>
+#include <cstdlib>
 #include <cstring>
 #include <deque>
 #include <functional>
@@ -214,6 +215,7 @@ struct hipmps_engine_s {
   DevBuf desc;   // task descriptors
   DevBuf small;  // counters / K / stats
   DevBuf env;    // environments for measurements
+  size_t env_keep = (size_t)4 << 30;  // largest workspace of a measurement that keeps every X and P
   SitePool<SiteDevice> pool;  // site buffers
   HostBuf hdesc;
   HostBuf hsmall;
@@ -1779,11 +1781,18 @@ int env_steps(hipmps_engine E, std::vector<EnvJob>& jobs, int fp32) {
 // are one dot product each, sum_e z_e X_e conj(P_e) (R is Hermitian), instead of two more products
 // and a trace.  Environments themselves only live from one step to the next (two buffers a chain),
 // so a sweep without `keep` holds one X.
+// X and P are twice the sites in complex128, of a large state or one with long Kraus legs more than can be
+// spared.  Above env_keep bytes, or when they cannot be had, every R is kept instead (one_site_layout) and X
+// and P of one site at a time, P formed again where it is wanted: five products a site instead of four and no
+// second stream (60 sites of bond 1024: <Z> 75 ms for 52, <ZZ> of the neighbours 101 ms both; 40 of bond 256: 2.3
+// for 1.2 and 2.7 for 1.5 ms), and less memory than an environment of either side per site and an X per pair.
 struct EnvLayout {
   size_t mat = 0;                 // bytes of one environment
   size_t L = 0, R = 0;            // two environments each
   std::vector<size_t> X, P;       // per site
+  std::vector<size_t> Rk;         // every R_k, or empty
   size_t total = 0;
+  size_t right(int k) const { return Rk.empty() ? R + (k & 1) * mat : Rk[k]; }
 };
 
 EnvLayout env_layout(const hipmps_state_s* s, bool keep, bool right) {
@@ -1811,6 +1820,26 @@ EnvLayout env_layout(const hipmps_state_s* s, bool keep, bool right) {
   return E;
 }
 
+// two: an X and a P at the same time
+EnvLayout one_site_layout(const hipmps_state_s* s, bool two) {
+  EnvLayout E;
+  int cmax = 1;
+  size_t xmax = 1;
+  for (int k = 0; k <= s->n; ++k) cmax = std::max(cmax, s->chi[k]);
+  for (int k = 0; k < s->n; ++k) xmax = std::max(xmax, site_elems(s, k));
+  E.mat = align_up((size_t)cmax * cmax * 16);
+  size_t off = 2 * E.mat;
+  for (int k = 0; k <= s->n; ++k) {
+    E.Rk.push_back(off);
+    off += align_up((size_t)s->chi[k] * s->chi[k] * 16);
+  }
+  const size_t x = align_up(xmax * 16);
+  E.X.assign(s->n, off);
+  E.P.assign(s->n, two ? off + x : off);
+  E.total = off + (two ? 2 : 1) * x;
+  return E;
+}
+
 // jobs of the left sweep (ends in environment buffer n % 2) and of the right one, in their order
 std::vector<EnvJob> left_jobs(hipmps_state_s* s, const EnvLayout& L, char* base, const std::vector<double>& diag) {
   std::vector<EnvJob> jobs(s->n);
@@ -1831,8 +1860,8 @@ std::vector<EnvJob> left_jobs(hipmps_state_s* s, const EnvLayout& L, char* base,
 std::vector<EnvJob> right_jobs(hipmps_state_s* s, const EnvLayout& L, char* base) {
   std::vector<EnvJob> jobs;
   for (int k = s->n - 1; k >= 0; --k) {
-    EnvJob j{s->sites[k].p, s->chi[k], s->chi[k + 1], (const double2*)(base + L.R + ((k + 1) & 1) * L.mat),
-             (double2*)(base + L.P[k]), (double2*)(base + L.R + (k & 1) * L.mat), 0};
+    EnvJob j{s->sites[k].p, s->chi[k], s->chi[k + 1], (const double2*)(base + L.right(k + 1)),
+             (double2*)(base + L.P[k]), (double2*)(base + L.right(k)), 0};
     j.kap = s->kap[k];
     jobs.push_back(j);
   }
@@ -1847,10 +1876,11 @@ struct EnvPlan {
   std::vector<DotTask> dots;
   struct Launch {
     size_t off;
-    int n, tiles, kind;  // kind 0: E A, 1: A^H X, 2: A R^T, 3: conj(A) X^T
+    int n, tiles, kind;  // kind 0: E A, 1: A^H X, 2: A R^T, 3: conj(A) X^T, 4: dot products
     bool second;         // on the right sweep's stream
   };
   std::vector<Launch> sweeps, steps;  // steps: after both sweeps
+  bool dots_last = true;              // all dot products after the steps, or those of kind 4 among them
   void add(std::vector<Launch>& to, const std::vector<GemmTask>& tasks, int kind, bool second) {
     Launch l{g.size(), (int)tasks.size(), 0, kind, second};
     for (GemmTask t : tasks) {
@@ -1858,6 +1888,11 @@ struct EnvPlan {
       g.push_back(t);
     }
     if (l.n > 0) to.push_back(l);
+  }
+  // the dot products from `first` on, among the steps
+  void add_dots(size_t first) {
+    dots_last = false;
+    if (first < dots.size()) steps.push_back({first, (int)(dots.size() - first), 0, 4, false});
   }
 };
 
@@ -1875,14 +1910,21 @@ int env_run(hipmps_state_s* s, const EnvLayout& L, EnvPlan& P, std::vector<doubl
   if (!P.g.empty()) memcpy(h, P.g.data(), P.g.size() * sizeof(GemmTask));
   if (!P.dots.empty()) memcpy(h + gb, P.dots.data(), P.dots.size() * sizeof(DotTask));
   HIP_TRY(hipMemcpyAsync(d, h, gb + db, hipMemcpyHostToDevice, st));
-  bool two = false;
-  for (const auto& l : P.sweeps) two = two || l.second;
+  bool two = false, right = false;
+  for (const auto& l : P.sweeps) {
+    two = two || l.second;
+    right = right || l.kind == 2;
+  }
   HIP_TRY(launch_fill_identity1((double2*)(base + L.L), st));
-  if (two) HIP_TRY(launch_fill_identity1((double2*)(base + L.R + (s->n & 1) * L.mat), st));
+  if (right) HIP_TRY(launch_fill_identity1((double2*)(base + L.right(s->n)), st));
   const hipStream_t s2 = two && E->lane_stream[1] && E->lane_ev[0] && E->lane_ev[1] ? E->lane_stream[1] : st;
   auto run = [&](const std::vector<EnvPlan::Launch>& v) -> int {
     static const int opa[4] = {0, 2, 0, 1}, opb[4] = {0, 0, 3, 3};
     for (const auto& l : v) {
+      if (l.kind == 4) {
+        HIP_TRY(launch_dot((const DotTask*)(d + gb) + l.off, (double*)(d + gb + db) + l.off * DOT_BLOCKS, l.n, st));
+        continue;
+      }
       const int ta = l.kind == 0 ? 0 : s->fp32, tb = l.kind == 0 ? s->fp32 : 0;
       HIP_TRY(launch_gemm((const GemmTask*)d + l.off, l.n, l.tiles, opa[l.kind], opb[l.kind], ta, tb, 0,
                           l.second ? s2 : st));
@@ -1902,7 +1944,7 @@ int env_run(hipmps_state_s* s, const EnvLayout& L, EnvPlan& P, std::vector<doubl
   double* hr = (double*)(h + gb + db);
   double2* hl = (double2*)(h + gb + db + rb);
   if (!P.dots.empty()) {
-    HIP_TRY(launch_dot((const DotTask*)(d + gb), (double*)(d + gb + db), (int)P.dots.size(), st));
+    if (P.dots_last) HIP_TRY(launch_dot((const DotTask*)(d + gb), (double*)(d + gb + db), (int)P.dots.size(), st));
     HIP_TRY(hipMemcpyAsync(hr, d + gb + db, rb, hipMemcpyDeviceToHost, st));
   }
   if (last)
@@ -1933,6 +1975,19 @@ void env_sweeps(EnvPlan& P, const std::vector<EnvJob>& left, const std::vector<E
     }
   }
 }
+
+// the right sweep alone, on the engine's stream (R_0 is of no use)
+void env_right_sweep(EnvPlan& P, const std::vector<EnvJob>& right) {
+  GemmTask a, b;
+  for (size_t k = 0; k + 1 < right.size(); ++k) {
+    env_tasks_right(right[k], a, b);
+    P.add(P.sweeps, {a}, 2, false);
+    P.add(P.sweeps, {b}, 3, false);
+  }
+}
+
+// whether the measurement's workspace with every X and P kept is had
+bool env_kept(hipmps_engine E, size_t bytes) { return bytes <= E->env_keep && E->env.ensure(bytes) == 0; }
 
 DotTask site_dot(const hipmps_state_s* s, int k, const void* x, const void* p, double z1) {
   return {(const double2*)x, (const double2*)p, s->chi[k], 2 * s->kap[k], s->chi[k + 1], 1.0, z1};
@@ -2024,12 +2079,29 @@ int measure_z_all(hipmps_state_s* s, double* out, double* norm = nullptr) {
     if (norm) *norm = v.back();
     return 0;
   }
-  const EnvLayout L = env_layout(s, true, true);
-  RC_TRY(E->env.ensure(L.total));
-  char* base = (char*)E->env.p;
+  EnvLayout L = env_layout(s, true, true);
   EnvPlan P;
-  env_sweeps(P, left_jobs(s, L, base, {}), right_jobs(s, L, base));
-  for (int i = 0; i < s->n; ++i) P.dots.push_back(site_dot(s, i, base + L.X[i], base + L.P[i], -1.0));
+  if (env_kept(E, L.total)) {
+    char* base = (char*)E->env.p;
+    env_sweeps(P, left_jobs(s, L, base, {}), right_jobs(s, L, base));
+    for (int i = 0; i < s->n; ++i) P.dots.push_back(site_dot(s, i, base + L.X[i], base + L.P[i], -1.0));
+  } else {
+    L = one_site_layout(s, true);
+    RC_TRY(E->env.ensure(L.total));
+    char* base = (char*)E->env.p;
+    const std::vector<EnvJob> left = left_jobs(s, L, base, {}), right = right_jobs(s, L, base);
+    env_right_sweep(P, right);
+    for (int i = 0; i < s->n; ++i) {
+      GemmTask x, e, p, r;
+      env_tasks_left(left[i], x, e);
+      env_tasks_right(right[s->n - 1 - i], p, r);
+      P.add(P.steps, {x}, 0, false);
+      P.add(P.steps, {p}, 2, false);
+      P.dots.push_back(site_dot(s, i, base + L.X[i], base + L.P[i], -1.0));
+      P.add_dots(i);
+      P.add(P.steps, {e}, 1, false);
+    }
+  }
   std::vector<double> v;
   RC_TRY(env_run(s, L, P, &v, norm));
   std::copy(v.begin(), v.end(), out);
@@ -2057,58 +2129,102 @@ int measure_zz(hipmps_state_s* s, const int* pairs, int k, double* out) {
   size_t xmax = 1;
   for (int q = 0; q < n; ++q) xmax = std::max(xmax, site_elems(s, q));
   // a chain holds two environments, the X of every site at which a pair ends (the dot products run
-  // after all steps) and one X for the sites between
+  // after all steps) and one X for the sites between; with R kept instead, whose dot products run at
+  // their site, the one X
   struct Chain {
     int i, last;
     size_t E, X;                 // offsets; X: scratch of the sites where no pair ends
-    std::vector<size_t> Xend;    // per site i + 1 .. last: offset, or 0
+    std::vector<char> end;       // per site i .. last: a pair ends there
+    std::vector<size_t> Xend;    // and the offset of its X
   };
   std::vector<Chain> chains;
-  size_t off = L.total;
   for (int i = 0; i < n; ++i) {
     if (ends[i].empty()) continue;
     Chain c;
     c.i = i;
     c.last = *std::max_element(ends[i].begin(), ends[i].end());
-    c.E = off;
-    off += 2 * L.mat;
-    c.X = off;
-    off += align_up(xmax * 16);
-    c.Xend.assign(c.last - i + 1, 0);
-    for (int j : ends[i])
-      if (!c.Xend[j - i]) {
-        c.Xend[j - i] = off;
-        off += align_up(site_elems(s, j) * 16);
-      }
+    c.end.assign(c.last - i + 1, 0);
+    for (int j : ends[i]) c.end[j - i] = 1;
     chains.push_back(std::move(c));
   }
-  RC_TRY(E->env.ensure(off));
+  auto place = [&](size_t off, bool keep) {
+    for (Chain& c : chains) {
+      c.E = off;
+      off += 2 * L.mat;
+      c.X = off;
+      off += align_up(xmax * 16);
+      c.Xend.assign(c.end.size(), c.X);
+      for (size_t q = 0; keep && q < c.end.size(); ++q)
+        if (c.end[q]) {
+          c.Xend[q] = off;
+          off += align_up(site_elems(s, c.i + (int)q) * 16);
+        }
+    }
+    return off;
+  };
+  const bool keep = env_kept(E, place(L.total, true));
+  if (!keep) {
+    L = one_site_layout(s, false);
+    RC_TRY(E->env.ensure(place(L.total, false)));
+  }
   char* base = (char*)E->env.p;
   EnvPlan P;
-  env_sweeps(P, left_jobs(s, L, base, {}), right_jobs(s, L, base));
   std::map<std::pair<int, int>, size_t> where;
-  for (int step = 0;; ++step) {
-    std::vector<GemmTask> ket, bra;
-    for (const Chain& c : chains) {
-      const int site = c.i + step;
-      if (site > c.last) continue;
-      const size_t xo = step == 0 ? L.X[site] : (c.Xend[step] ? c.Xend[step] : c.X);
-      EnvJob j{s->sites[site].p, s->chi[site], s->chi[site + 1],
-               (const double2*)(base + c.E + (step & 1) * L.mat), (double2*)(base + xo),
-               (double2*)(base + c.E + ((step + 1) & 1) * L.mat), step == 0 ? 1 : 0};
-      j.kap = s->kap[site];
-      GemmTask a, b;
-      env_tasks_left(j, a, b);
-      if (step > 0) ket.push_back(a);
-      if (site < c.last) bra.push_back(b);
-      if (step > 0 && c.Xend[step]) {
-        where[{c.i, site}] = P.dots.size();
-        P.dots.push_back(site_dot(s, site, base + xo, base + L.P[site], -1.0));
+  const std::vector<EnvJob> left = left_jobs(s, L, base, {}), right = right_jobs(s, L, base);
+  // the products of chain c at its site i + step: X = M A (but at the first site, where X is the left sweep's) and
+  // the next M = A^H X, with Z at the first site
+  auto chain_tasks = [&](const Chain& c, int step, GemmTask& a, GemmTask& b) {
+    const int site = c.i + step;
+    EnvJob j{s->sites[site].p, s->chi[site], s->chi[site + 1], (const double2*)(base + c.E + (step & 1) * L.mat),
+             (double2*)(base + (step == 0 ? L.X[site] : c.Xend[step])),
+             (double2*)(base + c.E + ((step + 1) & 1) * L.mat), step == 0 ? 1 : 0};
+    j.kap = s->kap[site];
+    env_tasks_left(j, a, b);
+  };
+  auto chain_dot = [&](const Chain& c, int step) {
+    if (step == 0 || !c.end[step]) return;
+    const int site = c.i + step;
+    where[{c.i, site}] = P.dots.size();
+    P.dots.push_back(site_dot(s, site, base + c.Xend[step], base + L.P[site], -1.0));
+  };
+  GemmTask a, b;
+  if (keep) {
+    env_sweeps(P, left, right);
+    for (int step = 0;; ++step) {
+      std::vector<GemmTask> ket, bra;
+      for (const Chain& c : chains) {
+        if (c.i + step > c.last) continue;
+        chain_tasks(c, step, a, b);
+        if (step > 0) ket.push_back(a);
+        if (c.i + step < c.last) bra.push_back(b);
+        chain_dot(c, step);
       }
+      if (ket.empty() && bra.empty()) break;
+      P.add(P.steps, ket, 0, false);
+      P.add(P.steps, bra, 1, false);
     }
-    if (ket.empty() && bra.empty()) break;
-    P.add(P.steps, ket, 0, false);
-    P.add(P.steps, bra, 1, false);
+  } else {
+    env_right_sweep(P, right);
+    for (int site = 0; site < n; ++site) {  // the left sweep, the chains beside it
+      env_tasks_left(left[site], a, b);
+      P.add(P.steps, {a}, 0, false);
+      std::vector<GemmTask> ket, bra{b};
+      const size_t first = P.dots.size();
+      for (const Chain& c : chains) {
+        if (site < c.i || site > c.last) continue;
+        chain_tasks(c, site - c.i, a, b);
+        if (site > c.i) ket.push_back(a);
+        if (site < c.last) bra.push_back(b);
+        chain_dot(c, site - c.i);
+      }
+      P.add(P.steps, ket, 0, false);
+      P.add(P.steps, bra, 1, false);
+      if (P.dots.size() > first) {  // P takes the place of the left sweep's X
+        env_tasks_right(right[n - 1 - site], a, b);
+        P.add(P.steps, {a}, 2, false);
+      }
+      P.add_dots(first);
+    }
   }
   std::vector<double> v;
   double norm = 0.0;
@@ -2811,6 +2927,7 @@ int hipmps_engine_create(const hipmps_engine_opts* opts, hipmps_engine* out) {
     }
     e->stage_delay_ticks = (long long)std::max(0, std::min(100000, atoi(v))) * khz / 1000;
   }
+  if (const char* v = getenv("HIPMPS_TEST_ENV_KEEP_BYTES")) e->env_keep = strtoull(v, nullptr, 10);
   if (const char* v = getenv("HIPMPS_WAVE_GROUPS")) e->wave_groups = std::max(1, std::min(2, atoi(v)));
   if (!ok) {
     (void)hipGetLastError();
