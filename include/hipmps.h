@@ -73,7 +73,9 @@ typedef struct hipmps_state_s* hipmps_state;
 
 typedef struct {
   int device;               /* HIP device ordinal */
-  size_t hbm_budget_bytes;  /* admission budget; 0 = 90% of the device's memory */
+  size_t hbm_budget_bytes;  /* admission budget; 0 = 90% of the device's memory.  Counts the bytes of
+                               site tensors; those up to 2 MiB lie in slabs of 16 MiB, whose ends lose
+                               an eighth at most and of which two are kept when unused */
   int jacobi_max_sweeps;    /* 0 = default (40); gates and channels that run in one workgroup, of at
                                most 64 rows, stop at 1000 if it is larger */
   double jacobi_tol;        /* 0 = default: relative off-diagonal 1e-13 (fp64 states) */
