@@ -702,12 +702,20 @@ int run_wave(hipmps_engine E, std::vector<WaveItem>& all) {
     if (ss != st) HIP_TRY(hipStreamSynchronize(ss));
     return 0;
   };
+  int rc;
   if (items.empty()) {
-    RC_TRY(start());
-    HIP_TRY(hipStreamSynchronize(st));
-    E->prof.waves += 1;
+    rc = start();
+    if (rc == 0) {
+      HIP_TRY(hipStreamSynchronize(st));
+      E->prof.waves += 1;
+    }
   } else {
-    RC_TRY(run_wave_general(E, items, start, join));
+    rc = run_wave_general(E, items, start, join);
+  }
+  if (rc != 0) {  // what the wave has queued still reads its descriptors and writes sites
+    for (hipStream_t l : E->lane_stream)
+      if (l) (void)hipStreamSynchronize(l);
+    return rc;
   }
   int q = 0;
   for (auto& v : small)
@@ -1448,6 +1456,7 @@ int run_kraus_waves(hipmps_engine E, const std::vector<hipmps_state_s*>& states)
   CopyTask* hc = (CopyTask*)(ht + ns);
   const GateResult* hr = (const GateResult*)(hc + ns);
   KrausTask* dt = nullptr;
+  hipError_t launched = hipSuccess;
   if (ns) {
     HIP_TRY(hipHostGetDevicePointer((void**)&dt, E->hgate.p, 0));
     GateResult* dr = (GateResult*)((CopyTask*)(dt + ns) + ns);
@@ -1474,13 +1483,14 @@ int run_kraus_waves(hipmps_engine E, const std::vector<hipmps_state_s*>& states)
         ++i;
       }
     const KrausTask* d = dt;
-    for (int v = 0; v < 4; ++v) {
-      HIP_TRY(launch_kraus_small(d, (int)small[v].size(), v >> 1, (v & 1) == 0, st));
+    for (int v = 0; v < 4 && launched == hipSuccess; ++v) {
+      launched = launch_kraus_small(d, (int)small[v].size(), v >> 1, (v & 1) == 0, st);
       d += small[v].size();
     }
   }
-  const int rc = general.empty() ? 0 : run_kraus_general(E, general);
-  HIP_TRY(hipStreamSynchronize(st));
+  const int rc = general.empty() || launched != hipSuccess ? 0 : run_kraus_general(E, general);
+  HIP_TRY(hipStreamSynchronize(st));  // also on a failure: what is queued reads the descriptors
+  HIP_TRY(launched);
   RC_TRY(rc);
   {
     size_t i = 0;
