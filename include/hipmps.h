@@ -274,6 +274,9 @@ int hipmps_serve_pending(hipmps_engine e, int* queued, int* running);
 
 /* ---- measurement hooks for the bench ------------------------------------------------ */
 typedef struct {
+  /* HIP-event times.  A gate of at most 64 rows runs whole in one workgroup: waves of such gates alone
+   * are ms_other, and those beside larger ones run within the other fields' spans.  The jacobi_*
+   * counts but jacobi_sweeps leave these gates out. */
   double ms_theta, ms_jacobi, ms_split, ms_other;
   double ms_jacobi_rounds;  /* HIP-event span of all sweeps' k_jacobi_round launches of a wave */
   long long jacobi_launches;
@@ -298,7 +301,9 @@ int hipmps_engine_profile(hipmps_engine e, hipmps_profile_t* out, int reset);
 int hipmps_engine_set_timing(hipmps_engine e, int enabled);
 /* Preconditioning of the SVD: for min(m, n) >= min_rank the one-sided Jacobi runs on R2 of the
  * double Householder LQ (X = L Q, L^H = L_Z Q_Z, R2 = L_Z^H) instead of on X, which it
- * converges on in fewer sweeps; 0 turns it off.  Default 64.  No counterpart in the reference,
+ * converges on in fewer sweeps; 0 turns it off.  Default 64.  Gates that run in one workgroup
+ * (at most 64 rows, the other side at most 64 too, or 128 up to 32 rows) take a single LQ of their
+ * own whatever this says.  No counterpart in the reference,
  * whose SVD is ExaTN's (ExaTnMpsVisitor.cpp:1623); the singular values and the truncation are
  * the same either way. */
 int hipmps_engine_set_lq_precondition(hipmps_engine e, int min_rank);

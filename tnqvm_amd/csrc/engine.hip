@@ -704,9 +704,16 @@ int run_wave(hipmps_engine E, std::vector<WaveItem>& all) {
   };
   int rc;
   if (items.empty()) {
+    if (E->timing) HIP_TRY(hipEventRecord(E->ev[0], st));
     rc = start();
     if (rc == 0) {
+      if (E->timing) HIP_TRY(hipEventRecord(E->ev[1], st));
       HIP_TRY(hipStreamSynchronize(st));
+      if (E->timing) {
+        float ms = 0;
+        (void)hipEventElapsedTime(&ms, E->ev[0], E->ev[1]);
+        E->prof.ms_other += ms;
+      }
       E->prof.waves += 1;
     }
   } else {
