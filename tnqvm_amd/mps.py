@@ -6,6 +6,7 @@ operation runs in the HIP library.  Gate dicts follow tnqvm_amd.circuits.
 from __future__ import annotations
 
 import ctypes
+import operator
 import sys
 import weakref
 
@@ -380,12 +381,24 @@ class MpsState:
         k = len(qubits)
         if k > 16:
             raise ValueError("at most 16 measured qubits")
-        q = np.asarray(qubits, dtype=np.int32).reshape(-1)
-        q = np.ascontiguousarray(np.where(q < 0, q + self.n, q), dtype=np.int32)
-        if (q < 0).any() or (q >= self.n).any():
+        try:
+            q = [operator.index(x) for x in qubits]
+        except TypeError:  # arrays as elements: what they mean, and what is refused, is a diagonal's matter
+            return self._outcomes_one_by_one(qubits)
+        if any(x < -self.n or x >= self.n for x in q):
             raise IndexError("measured qubit out of range")
+        q = np.array([x % self.n for x in q], dtype=np.int32)
         out = np.zeros(1 << k)
         check(lib().hipmps_outcome_probabilities(self.h, q.ctypes.data_as(_ip), k, out.ctypes.data_as(_dp)))
+        return out
+
+    def _outcomes_one_by_one(self, qubits) -> np.ndarray:
+        out = np.zeros(1 << len(qubits))
+        for x in range(len(out)):
+            d = np.ones(2 * self.n)
+            for i, q in enumerate(qubits):
+                d[2 * q + (1 - ((x >> i) & 1))] = 0.0
+            out[x] = self.expval_diag(d)
         return out
 
     def reduced_density_matrix(self, qubits) -> np.ndarray:
