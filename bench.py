@@ -664,7 +664,7 @@ def main():
         traffic_ratio = round(per_pair * prof["jacobi_pairs_visited"] / max(1.0, applies * 2 * 512 * 512 * 16), 2)
     roofline = {"bound": "mfma", "achieved": round(svd_tflops, 3), "peak": PEAK_FP64_TFLOPS, "unit": "TFLOP/s",
                 "frac": round(svd_tflops / PEAK_FP64_TFLOPS, 4), "traffic": traffic,
-                "kernel": "SVD of theta' 512x512: double LQ (k_lq_factor_lds/k_lq_next/k_lq_rest with look-ahead, "
+                "kernel": "SVD of theta' 512x512: double LQ (k_lq_step/k_lq_rest with look-ahead, "
                           "k_lq_panel0/k_lq_update), k_jacobi_round, k_lq_apply_q",
                 "flops_per_unit": NOMINAL_SVD * CHI ** 3, "unit_of_work": "one chi=256 apply's SVD (nominal 704 chi^3)",
                 "wave_groups": groups, "svd_event_ms": round(svd_ms, 2),

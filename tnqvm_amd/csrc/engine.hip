@@ -205,7 +205,7 @@ struct hipmps_engine_s {
   double tol_mixed = 1e-8;  // mixed path: factors are stored in complex64
   int debug_sweeps = 0;  // HIPMPS_DEBUG_SWEEPS: per-sweep rotated / visited block pairs on stderr
   int lq_min_rank = 64;  // Jacobi on the double-LQ factor when min(m, n) >= this (0: never)
-  // LQ with look-ahead (next panel factored in LDS on one stream while the trailing rows update
+  // LQ with look-ahead (next panel factored in registers on one stream while the trailing rows update
   // on another) for rows of at most LQ_REG_MAX_COLS columns; HIPMPS_LQ_LOOKAHEAD=0 turns it off
   int lq_lookahead = 1;
   hipEvent_t lq_ev[2 * MAX_LANES] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
@@ -2008,12 +2008,6 @@ bool env_kept(hipmps_engine E, size_t bytes) { return bytes <= E->env_keep && E-
 
 DotTask site_dot(const hipmps_state_s* s, int k, const void* x, const void* p, double z1) {
   return {(const double2*)x, (const double2*)p, s->chi[k], 2 * s->kap[k], s->chi[k + 1], 1.0, z1};
-}
-
-int read_scalar(hipmps_engine E, const void* dptr, double2* out) {
-  HIP_TRY(hipMemcpyAsync(out, dptr, sizeof(double2), hipMemcpyDeviceToHost, E->stream));
-  HIP_TRY(hipStreamSynchronize(E->stream));
-  return 0;
 }
 
 // sum over pairs M_t o R_t (elementwise), results to host

@@ -130,7 +130,6 @@ constexpr int SMALL_CAP_LO = 32 * 33;  // variant of 256 threads, several workgr
 inline bool gate_small(int r, int c) {
   return r <= SMALL_MAX_ROWS && c <= SMALL_MAX_COLS && small_rows(r) * small_stride(c) <= SMALL_CAP;
 }
-// lo: every task fits SMALL_CAP_LO
 // A noise channel of a small site (k_kraus_small): the same limits on its rows and columns.
 constexpr int MAX_KRAUS_OPS = 16;
 struct KrausTask {
@@ -143,6 +142,7 @@ struct KrausTask {
   double cutoff, tol;
   double2 K[4 * MAX_KRAUS_OPS];
 };
+// lo: every task fits SMALL_CAP_LO
 hipError_t launch_kraus_small(const KrausTask* d_tasks, int ntasks, int fp32, bool lo, hipStream_t s);
 struct CopyTask {
   const void* src;
