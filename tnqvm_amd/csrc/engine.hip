@@ -192,7 +192,12 @@ struct hipmps_engine_s {
   hipStream_t lane_stream[MAX_LANES] = {nullptr, nullptr, nullptr, nullptr};
   hipEvent_t lane_ev[MAX_LANES + 1] = {nullptr, nullptr, nullptr, nullptr, nullptr};
   int jacobi_lanes = 2;
-  int lane_min_pairs = 1536;  // two generations of the 768 resident Jacobi workgroups
+  // Block pairs of a sweep from which its SVDs are dealt to several lanes: 1536 was two generations of the Jacobi
+  // workgroups that fit the chip three a CU.  They fit four a CU now, and two lanes against one, in one wave group
+  // (applies/s of 40-qubit circuits), are 0.98 at 220 pairs, 0.99 at 430, 1.01 at 650, 1.06 at 860 and 1.08 to
+  // 1.10 above, rows of 256; 1.07 at 420, 1.09 at 830, 1.13 at 1250, 1.12 at 1660 and 1.06 at 3300, rows of 512.
+  // With two wave groups the other group fills the tails: 1.00 either way.
+  int lane_min_pairs = 1536;
   // mixed path: the first sweeps of SVDs with min(m, n) >= 256 form the Gram with FP32 MFMA;
   // such a sweep never counts as the converged one, so every SVD ends with FP64 sweeps.  The
   // FP64 path never does: rotation angles good to ~1e-7 mix large rows into small ones, which
@@ -1105,8 +1110,8 @@ int run_wave_general(hipmps_engine E, std::vector<WaveItem>& items, const std::f
     if (active != listed) {
       const int nact = (int)active.size();
       JacTask* ha = hja[sweep & 1];  // its last reader, an upload two sweeps back, has run
-      // lanes only pay when one launch would already fill the chip twice over (768 resident
-      // workgroups: 256 CUs x 3 at the kernel's register count); below that they add launches
+      // lanes pay when a launch has more workgroups than are resident at a time (see lane_min_pairs); well
+      // below that they only add launches
       int total_pairs = 0;
       for (int q : active) total_pairs += hjs[q].nb / 2;
       lanes = total_pairs >= E->lane_min_pairs ? std::max(1, std::min(E->jacobi_lanes, nact)) : 1;

@@ -22,7 +22,12 @@ namespace hipmps {
 constexpr int LQB = 16;  // rows per panel (reflectors per block reflector)
 constexpr int LQR = 16;  // rows per MFMA tile in the block-reflector application
 constexpr int LQ_TWO_ROWS_COLS = 64 * 16;  // widest panel of which a lane's registers hold two rows
-constexpr long long LQ_ONE_STREAM_ROWS = 4096;  // launch_lq_lookahead: rows of all tasks on one stream up to this
+// launch_lq_lookahead: rows of all tasks on one stream up to this.  The line is that of an earlier form of the panel
+// kernels, whose workgroups beside the factoring one held its registers.  With these, one stream against two, both
+// LQs of a wave alone: 8 of 512 x 512 2.44 for 3.37 ms, 64 of them (32768 rows) 4.29 for 5.51, 32 of 1024 x 1024
+// 17.3 for 20.7; the 8-circuit chi 256 load 2375 for 2355 applies/s (two wave groups).  One is the faster at every
+// size measured, so the line costs a few percent above it.
+constexpr long long LQ_ONE_STREAM_ROWS = 4096;
 
 // Element w_k[col] of reflector k of M (support col >= k; head in W0, tail in M's row k).
 __device__ __forceinline__ double2 refl(const double2* M, size_t ld, const double2* W0, int k, int col) {
