@@ -42,6 +42,7 @@
 #include <vector>
 
 #include "hipmps.h"
+#include "chain_rule.h"
 #include "kernels.h"
 #include "site_pool.h"
 
@@ -2043,19 +2044,21 @@ int trace_products(hipmps_engine E, const std::vector<const double2*>& A, const 
 }
 
 // Values of `m` diagonals at once on a state of small bonds (k_env_chain), when that is estimated to take
-// less than the sweeps of products launched one by one that they replace (`sweeps` of them): a step of a
-// site takes about 1000 clocks and 40 per contraction index, and 512 workgroups run at a time; a sweep's two
-// products a site take 10 us.
-bool chain_fits(const hipmps_state_s* s, size_t m, size_t sweeps) {
-  double clocks = 0.0;
+// less than the `products` us of the sweeps of products launched one by one that they replace.
+bool chain_fits(const hipmps_state_s* s, size_t m, double products) {
+  double sites = 0.0;
+  int cmax = 1;
   for (int k = 0; k < s->n; ++k) {
     const int cl = s->chi[k], cr = s->chi[k + 1];
     if (cl > CHAIN_MAX_BOND || cr > CHAIN_MAX_BOND) return false;
-    const int steps = (2 * s->kap[k] + chain_slots(cl, cr) - 1) / chain_slots(cl, cr);
-    clocks += steps * (1000.0 + 20.0 * cl * 2) + 1500.0;
+    sites += chain_site_us(cl, (2 * s->kap[k] + chain_slots(cl, cr) - 1) / chain_slots(cl, cr));
+    cmax = std::max(cmax, cl);
   }
-  return clocks * (double)((m + 511) / 512) < 24000.0 * s->n * sweeps;
+  return chain_us(sites, cmax, m, s->n) < products;
 }
+
+// one sweep of products on this state
+double state_sweep_us(const hipmps_state_s* s) { return sweep_us(s->n, *std::max_element(s->chi.begin(), s->chi.end())); }
 
 // out[t] = value of diagonal t; set(t, d): diagonal t's 2n values into d
 int chain_values(hipmps_state_s* s, size_t m, const std::function<void(size_t, double*)>& set, double* out) {
@@ -2085,7 +2088,7 @@ int chain_values(hipmps_state_s* s, size_t m, const std::function<void(size_t, d
 // <Z_i> for every site; with norm, also <psi|psi> (the closed left environment)
 int measure_z_all(hipmps_state_s* s, double* out, double* norm = nullptr) {
   hipmps_engine E = s->e;
-  if (chain_fits(s, (size_t)s->n + 1, 1)) {
+  if (chain_fits(s, (size_t)s->n + 1, both_sweeps_us(s->n))) {
     std::vector<double> v(s->n + 1);
     RC_TRY(chain_values(s, v.size(), [&](size_t t, double* d) {
       std::fill(d, d + 2 * s->n, 1.0);
@@ -2135,7 +2138,14 @@ int measure_zz(hipmps_state_s* s, const int* pairs, int k, double* out) {
     if (a < 0 || a >= n || b < 0 || b >= n) return fail(HIPMPS_E_ARG, "zz pair out of range");
     if (a != b) ends[std::min(a, b)].push_back(std::max(a, b));
   }
-  if (chain_fits(s, (size_t)k, 2))
+  size_t longest = 0, steps = 0;  // of the chains below
+  for (int i = 0; i < n; ++i)
+    if (!ends[i].empty()) {
+      const size_t len = *std::max_element(ends[i].begin(), ends[i].end()) - i;
+      longest = std::max(longest, len);
+      steps += len;
+    }
+  if (chain_fits(s, (size_t)k, zz_us(n, longest, steps)))
     return chain_values(s, (size_t)k, [&](size_t t, double* d) {
       std::fill(d, d + 2 * n, 1.0);
       d[2 * pairs[2 * t] + 1] *= -1.0;
@@ -2255,7 +2265,7 @@ int measure_zz(hipmps_state_s* s, const int* pairs, int k, double* out) {
 // <psi| (x)_k diag(d[2k], d[2k+1]) |psi>, diag empty: <psi|psi>
 int measure_diag(hipmps_state_s* s, const std::vector<double>& diag, double* out) {
   hipmps_engine E = s->e;
-  if (chain_fits(s, 1, 1))
+  if (chain_fits(s, 1, state_sweep_us(s)))
     return chain_values(s, 1, [&](size_t, double* d) {
       if (diag.empty()) std::fill(d, d + 2 * s->n, 1.0);
       else std::copy(diag.begin(), diag.end(), d);
@@ -2274,7 +2284,7 @@ int measure_outcomes(hipmps_state_s* s, const int* qubits, int k, double* out) {
     std::fill(d, d + 2 * s->n, 1.0);
     for (int i = 0; i < k; ++i) d[2 * qubits[i] + (1 - ((x >> i) & 1))] = 0.0;
   };
-  if (chain_fits(s, m, m)) return chain_values(s, m, set, out);
+  if (chain_fits(s, m, (double)m * state_sweep_us(s))) return chain_values(s, m, set, out);
   std::vector<double> diag(2 * s->n);
   for (size_t x = 0; x < m; ++x) {
     set(x, diag.data());
